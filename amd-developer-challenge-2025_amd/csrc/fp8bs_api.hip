@@ -20,14 +20,20 @@ namespace {
 
 constexpr int KBLK = 128;
 
+// A kernel is named by its variant (FP8BS_VARIANT_*) and, for the variants that have two, its form: tile = variant + 256 * form.
 struct VariantInfo { int bm, bn, threads; };
+constexpr int FORM1 = 256;
+constexpr int variant_of(int tile) { return tile & 255; }
+constexpr int form_of(int tile) { return tile >> 8; }
 
-bool variant_info(int variant, VariantInfo* out) {
-    switch (variant) {
+bool variant_info(int tile, VariantInfo* out) {
+    switch (tile) {
         case FP8BS_VARIANT_GENERIC:  *out = {16, 16, 256}; return true;
         case FP8BS_VARIANT_T256x256: *out = {256, 256, 512}; return true;
         case FP8BS_VARIANT_T128x128: *out = {128, 128, 256}; return true;
-        case FP8BS_VARIANT_T64x128:  *out = {64, 128, 256}; return true;
+        case FP8BS_VARIANT_T64x256S3 | FORM1: *out = {128, 128, 512}; return true;
+        case FP8BS_VARIANT_T64x128:  *out = {64, 128, 512}; return true;
+        case FP8BS_VARIANT_T64x128 | FORM1: *out = {64, 64, 256}; return true;
         case FP8BS_VARIANT_T256x128: *out = {256, 128, 512}; return true;
         case FP8BS_VARIANT_SKINNY64x144: *out = {64, 144, 256}; return true;
         case FP8BS_VARIANT_SKINNY64x256: *out = {64, 256, 256}; return true;
@@ -44,10 +50,10 @@ inline long cdiv(long a, long b) { return (a + b - 1) / b; }
 
 // Workgroups of a call that deals K blocks instead of tiles: one per place on the chip (what the tile's LDS
 // and thread count let a CU hold), never more than there are (tile, K block) pairs.
-int streamk_grid(int variant, int m, int n, int k, int num_cus) {
+int streamk_grid(int tile, int m, int n, int k, int num_cus) {
     VariantInfo vi{};
-    if (!variant_info(variant, &vi) || variant == FP8BS_VARIANT_GENERIC || k < KBLK) return 0;
-    const int lds = fp8bs::variant_lds_bytes(variant);
+    if (!variant_info(tile, &vi) || tile == FP8BS_VARIANT_GENERIC || form_of(tile) != 0 || k < KBLK) return 0;
+    const int lds = fp8bs::variant_lds_bytes(tile);
     if (lds <= 0 || lds > 163840) return 0;
     if (num_cus <= 0) num_cus = 256;
     const long by_lds = 163840 / lds, by_threads = 2048 / vi.threads;
@@ -58,6 +64,9 @@ int streamk_grid(int variant, int m, int n, int k, int num_cus) {
     return (int)(g < fp8bs::StreamK::MAX_GRID ? g : fp8bs::StreamK::MAX_GRID);
 }
 
+// The tile of a forced variant argument: FP8BS_VARIANT_FORM(variant, form) names a form, a plain variant its first.
+int forced_tile(int variant) { return variant < 256 ? variant : variant_of(variant) | ((variant >> 8) - 1) * FORM1; }
+
 bool is_streaming_variant(int v) { return v == FP8BS_VARIANT_SKINNY64x144 || v == FP8BS_VARIANT_SKINNY64x256 || v == FP8BS_VARIANT_SKINNY64x288; }
 
 // The fp32 partial planes of a K split followed by the reduce kernel.
@@ -65,32 +74,32 @@ uint64_t planes_bytes(int m, int n, int split_k) { return split_k > 1 ? (uint64_
 
 // Can the partial tiles of a K split of this tile shape be summed in the kernel that writes them (one counter per
 // tile in the head of the workspace, the partition count in the counter's low 16 bits)?
-bool can_sum_in_kernel(int m, int n, int variant, int split_k) {
+bool can_sum_in_kernel(int m, int n, int tile, int split_k) {
     VariantInfo vi{};
-    if (variant == FP8BS_VARIANT_GENERIC || is_streaming_variant(variant) || !variant_info(variant, &vi)) return false;
+    if (tile == FP8BS_VARIANT_GENERIC || is_streaming_variant(tile) || !variant_info(tile, &vi)) return false;
     return split_k >= 2 && split_k <= 255 && cdiv(m, vi.bm) * cdiv(n, vi.bn) <= fp8bs::StreamK::MAX_GRID;
 }
 
-// Fill a plan for a given variant and split count.  in_kernel: the split's partial tiles are summed by the last
+// Fill a plan for a given tile and split count.  in_kernel: the split's partial tiles are summed by the last
 // workgroup to finish each tile (where the shape allows it, see above; else the reduce kernel follows).
-void fill_plan(int m, int n, int k, int variant, int split_k, fp8bs_plan_t* out, int stream_k = 0, bool in_kernel = false) {
+void fill_plan(int m, int n, int k, int tile, int split_k, fp8bs_plan_t* out, int stream_k = 0, bool in_kernel = false) {
     VariantInfo vi{};
-    variant_info(variant, &vi);
+    variant_info(tile, &vi);
     int kbt = k / KBLK;
-    if (variant == FP8BS_VARIANT_GENERIC) { split_k = 1; stream_k = 0; }
+    if (tile == FP8BS_VARIANT_GENERIC) { split_k = 1; stream_k = 0; }
     if (stream_k > 0) split_k = 1;
     if (split_k < 1) split_k = 1;
     if (split_k > kbt) split_k = kbt > 0 ? kbt : 1;
-    out->variant = variant;
+    out->variant = variant_of(tile);
+    out->form = form_of(tile);
     out->tile_m = vi.bm;
     out->tile_n = vi.bn;
     out->split_k = split_k;
     out->block_threads = vi.threads;
-    out->lds_bytes = fp8bs::variant_lds_bytes(variant);
+    out->lds_bytes = fp8bs::variant_lds_bytes(tile);
     out->stream_k = stream_k > 0 ? stream_k : 0;
-    out->sum_in_kernel = in_kernel && stream_k <= 0 && can_sum_in_kernel(m, n, variant, split_k) ? 1 : 0;
-    out->reserved = 0;
-    if (variant == FP8BS_VARIANT_GENERIC) {
+    out->sum_in_kernel = in_kernel && stream_k <= 0 && can_sum_in_kernel(m, n, tile, split_k) ? 1 : 0;
+    if (tile == FP8BS_VARIANT_GENERIC) {
         out->grid_x = (int)cdiv(n, 16); out->grid_y = (int)cdiv(m, 16); out->grid_z = 1;
     } else {
         out->grid_x = stream_k > 0 ? stream_k : (int)(cdiv(m, vi.bm) * cdiv(n, vi.bn) * split_k); out->grid_y = 1; out->grid_z = 1;
@@ -114,45 +123,53 @@ bool skinny_shape(int m, int n, int k) { return m <= 64 && (double)n * (double)k
 void choose_tiled(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_split = true) {
     if (num_cus <= 0) num_cus = 256;
     int kbt = k / KBLK;
-    // The tile shape and K split that finish soonest under a cost model in microseconds.  A workgroup advances one
-    // K block in max(t_alone x f(r), t_power x w / CUs): t_alone is the tile's time per block at the full clock
-    // (f(r) = 1, 1.30, 1.71 with r = 1, 2, 3 workgroups sharing a CU), t_power what the board's power limit allows
-    // when every CU runs one such workgroup - with w workgroups running together the limit is shared by w, so fewer
-    // busy CUs clock higher until the full clock is reached.  A round of workgroups (CUs x the most that fit a CU; a
-    // last partial round with fewer) costs a fixed time for the first copies' latency, the output and the drain.  A
-    // K split adds the fp32 partial planes (written and read back, mostly through the 256 MB cache) and the reduce
-    // launch.  The constants are a least-squares fit (of logarithms) of this model to the measured time of every
-    // (tile, split) pair on 38 shapes on MI355X - the 18 of the upstream benchmark and 20 others, M 96 .. 16384,
-    // N 1024 .. 28672, K 1024 .. 14336 - (rms error 10 %; picking by the model costs 1.2 % against picking the
-    // measured best, geometric mean over the shapes, worst shape +13 %).
-    struct Cand { int variant; int rmax; double t_alone, t_power, t_fixed; };
-    const Cand cands[7] = {
-        {FP8BS_VARIANT_T256x256, 1, 1.181, 1.462, 6.75},
-        {FP8BS_VARIANT_T256x192, 1, 1.011, 1.163, 5.51},
-        {FP8BS_VARIANT_T192x192S3, 1, 0.881, 1.059, 4.11},
-        {FP8BS_VARIANT_T256x128S3, 1, 0.783, 0.906, 3.70},
-        {FP8BS_VARIANT_T128x128, 2, 0.797, 0.570, 2.86},
-        {FP8BS_VARIANT_T64x128, 3, 0.645, 0.400, 1.91},
-        // the 64x256 three-stage tile: many small tiles and a deep copy ring; what shapes of a few hundred rows, or
-        // with few K blocks per tile, finish soonest on (1536 x 1536 x 4096: 21.4 us against 25.0 with the best of the others)
-        {FP8BS_VARIANT_T64x256S3, 1, 0.576, 0.618, 2.03},
+    // The tile and K split that finish soonest under a cost model in microseconds.  A workgroup advances one K block in
+    // max(t_alone x shared, t_power x w / CUs): t_alone is the tile's time per block with one workgroup on a CU, shared
+    // the factor with two, t_power what the board's power limit allows when every CU runs one such workgroup - with w
+    // workgroups running together the limit is shared by w, so fewer busy CUs clock higher until the full clock is
+    // reached.  A round of workgroups (CUs x the most that fit a CU; a last partial round with fewer) costs a fixed time
+    // for the launch, the first copies' latency, the output and the drain.  A K split adds the fp32 partial planes
+    // (written and read back, mostly through the 256 MB cache) and the reduce launch.  The constants are fits (of
+    // logarithms) to measured times on MI355X: those of the four largest tiles to 38 shapes, M 96 .. 16384, N 1024 ..
+    // 28672, K 1024 .. 14336; those of the other tiles and of the splits, with the former held fixed, to every (tile,
+    // split, form) of 93 shapes - the 18 of the upstream benchmark, 60 log-uniform draws of M 1 .. 8192, N 512 .. 18432,
+    // K 256 .. 7168, and 15 others.  Picking by the model costs 0.7 % against the measured best of each of the 93 shapes
+    // in the geometric mean, worst 14 %.
+    struct Cand { int tile; int rmax; double t_alone, t_power, t_fixed, shared; int kb_min; };
+    // kb_min: the fewest K blocks a workgroup of a split keeps.  4; 8 with the 64x256 tile, whose short blocks leave a
+    // workgroup's first copies and its partial plane as most of its time (1024 x 512 x 7168: split 8 20.9 us, split 4
+    // 18.6); 2 with the small tiles, where the splits are what fills the chip (1 x 2048 x 2048: split 8 6.5 us, 4 6.9).
+    const Cand cands[9] = {
+        {FP8BS_VARIANT_T256x256, 1, 1.181, 1.462, 6.75, 1.0, 4},
+        {FP8BS_VARIANT_T256x192, 1, 1.011, 1.163, 5.51, 1.0, 4},
+        {FP8BS_VARIANT_T192x192S3, 1, 0.881, 1.059, 4.11, 1.0, 4},
+        {FP8BS_VARIANT_T256x128S3, 1, 0.783, 0.906, 3.70, 1.0, 4},
+        {FP8BS_VARIANT_T128x128, 2, 0.765, 0.511, 4.86, 1.38, 4},
+        // few output tiles or few K blocks: the call is a chain of K blocks and barriers, so the tile with the shortest
+        // block wins (512 x 2048 x 1024: 64x64 5.8 us, 64x128 6.3, 128x128 in eight waves 7.5, 64x256 7.7)
+        {FP8BS_VARIANT_T64x128, 2, 0.398, 0.093, 4.76, 1.90, 2},
+        {FP8BS_VARIANT_T64x128 | FORM1, 2, 0.323, 0.108, 4.00, 1.76, 2},
+        {FP8BS_VARIANT_T64x256S3, 1, 0.552, 0.540, 5.00, 1.0, 8},
+        // 128x128 in eight waves: see fp8bs_tile_64x256s3.hip (2048^3 12.6 us against 14.2 with 64x256, the best of the others)
+        {FP8BS_VARIANT_T64x256S3 | FORM1, 1, 0.467, 0.531, 4.57, 1.0, 4},
     };
-    const double shared[3] = {1.0, 1.30, 1.71};
     const int splits[6] = {1, 2, 3, 4, 6, 8};
-    int best_variant = 0, best_split = 1; double best_cost = 0; bool best_fused = false;
+    int best_tile = 0, best_split = 1; double best_cost = 0; bool best_fused = false;
     for (const Cand& c : cands) {
         VariantInfo vi{};
-        variant_info(c.variant, &vi);
+        variant_info(c.tile, &vi);
         const long tiles = cdiv(m, vi.bm) * cdiv(n, vi.bn);
         auto t_block = [&](long w) {          // w workgroups running together
             const long r = cdiv(w, num_cus) < c.rmax ? cdiv(w, num_cus) : c.rmax;
-            const double alone = c.t_alone * shared[r - 1], power = c.t_power * (double)w / (double)num_cus;
+            const double alone = r > 1 ? c.t_alone * c.shared : c.t_alone, power = c.t_power * (double)w / (double)num_cus;
             return alone > power ? alone : power;
         };
         for (int s : splits) {
-            // keep at least 4 K blocks per workgroup - 8 with the 64x256 tile, whose short blocks leave a workgroup's
-            // first copies and its partial plane as most of its time (1024 x 512 x 7168: split 8 20.9 us, split 4 18.6)
-            if (s > 1 && (kbt / s < (c.variant == FP8BS_VARIANT_T64x256S3 ? 8 : 4) || !may_split)) continue;
+            if (s > 1 && (kbt / s < c.kb_min || !may_split)) continue;
+            // Chains of more than 48 K blocks are left to the other tiles, which split K or walk them in fewer, larger
+            // steps: 6144 x 576 x 7168 (56 blocks, 240 tiles) takes 35-38 us with this tile unsplit and 39-40 with the
+            // best split of the others, but the split form is what the tests of the sum in the kernel run at full size.
+            if (c.tile == (FP8BS_VARIANT_T64x256S3 | FORM1) && cdiv(kbt, s) > 48) continue;
             const long wgs = tiles * s, per_round = (long)num_cus * c.rmax;
             const long full = wgs / per_round, rem = wgs % per_round;
             const double kb = (double)cdiv(kbt, s);
@@ -162,15 +179,19 @@ void choose_tiled(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_
             // launch and no pass over whole planes, but the last workgroup of a tile reads s - 1 partial tiles alone
             // (measured on the same 38 shapes: two partitions 1-50 us faster than with the reduce launch, median 4.7;
             // three: median 2.3 faster; four and more: the serial sums cost more than the launch)
-            const double planes = 4.85 + 1.10e-6 * s * (double)m * (double)n;
-            const double in_kernel = 3.77 + 0.752e-6 * s * (double)m * (double)n
-                                     + 5.90 * (s - 1) * (vi.bm * vi.bn * 4e-6) * (double)cdiv(wgs, num_cus);
-            const bool fuse = (s == 2 || s == 3) && can_sum_in_kernel(m, n, c.variant, s) && in_kernel < planes;
+            const double planes = 2.66 + 1.656e-6 * s * (double)m * (double)n;
+            const double in_kernel = 2.34 + 0.891e-6 * s * (double)m * (double)n
+                                     + 13.2 * (s - 1) * (vi.bm * vi.bn * 4e-6) * (double)cdiv(wgs, num_cus);
+            const bool fuse = (s == 2 || s == 3) && can_sum_in_kernel(m, n, c.tile, s) && in_kernel < planes;
             if (s > 1) cost += fuse ? in_kernel : planes;
-            if (best_variant == 0 || cost < best_cost) { best_variant = c.variant; best_split = s; best_cost = cost; best_fused = fuse; }
+            // calls issued one after another are never faster than the host launches them: the reduce launch of a split
+            // pays only beyond that (2 x 700 x 3200 in eight partitions: done on the GPU after 7.2 us, 9.5 us a call)
+            const double host = s > 1 && !fuse ? 7.8 : 4.5;
+            if (cost < host) cost = host;
+            if (best_tile == 0 || cost < best_cost) { best_tile = c.tile; best_split = s; best_cost = cost; best_fused = fuse; }
         }
     }
-    fill_plan(m, n, k, best_variant, best_split, out, 0, best_fused);
+    fill_plan(m, n, k, best_tile, best_split, out, 0, best_fused);
 }
 
 // Skinny shapes: the 64 x 256 tile with three LDS stages (two K blocks of b, 64 KB, in flight per workgroup) and
@@ -346,18 +367,21 @@ int fp8bs_gemm_ex(const void* a, const void* b, const float* a_scale, const floa
     const int cus = fp8bs::device_cus();
     if (variant == FP8BS_VARIANT_AUTO) {
         choose(m, n, k, cus, &plan);
-        if (split_k > 0) fill_plan(m, n, k, plan.variant, split_k & ~FP8BS_SPLIT_SUM_IN_KERNEL, &plan, 0, (split_k & FP8BS_SPLIT_SUM_IN_KERNEL) != 0);
-        else if (split_k < 0) fill_plan(m, n, k, plan.variant, 1, &plan, streamk_grid(plan.variant, m, n, k, cus));
+        const int tile = plan.variant | plan.form * FORM1;
+        if (split_k > 0) fill_plan(m, n, k, tile, split_k & ~FP8BS_SPLIT_SUM_IN_KERNEL, &plan, 0, (split_k & FP8BS_SPLIT_SUM_IN_KERNEL) != 0);
+        else if (split_k < 0) fill_plan(m, n, k, plan.variant, 1, &plan, streamk_grid(plan.variant, m, n, k, cus));   // (the first form only)
         // the plan needs a workspace the caller did not bring: the best plan that needs none
         else if (plan.workspace_bytes > 0 && (!ws || ws_bytes < plan.workspace_bytes)) {
             // too small for the partial tiles of a sum in the kernel but not for the planes (tiles that overhang
             // the matrix): the same split with the reduce kernel
-            if (plan.sum_in_kernel && ws && ws_bytes >= planes_bytes(m, n, plan.split_k)) fill_plan(m, n, k, plan.variant, plan.split_k, &plan);
+            if (plan.sum_in_kernel && ws && ws_bytes >= planes_bytes(m, n, plan.split_k)) fill_plan(m, n, k, tile, plan.split_k, &plan);
             else choose(m, n, k, cus, &plan, false);
         }
     } else {
         VariantInfo vi{};
-        if (!variant_info(variant, &vi)) return FP8BS_ERR_BAD_VARIANT;
+        const int tile = forced_tile(variant);
+        variant = variant_of(variant);
+        if (!variant_info(tile, &vi)) return FP8BS_ERR_BAD_VARIANT;
         if (is_streaming_variant(variant) && !simple) return FP8BS_ERR_BAD_VARIANT;
         if (is_streaming_variant(variant) && variant != FP8BS_VARIANT_SKINNY64x144 && (m % 4) != 0) return FP8BS_ERR_BAD_VARIANT;   // only the planner's width repairs a
         if (split_k < 0) {
@@ -366,7 +390,7 @@ int fp8bs_gemm_ex(const void* a, const void* b, const float* a_scale, const floa
         } else {
             const bool in_kernel = split_k > 0 && (split_k & FP8BS_SPLIT_SUM_IN_KERNEL) != 0;
             if (in_kernel && (is_streaming_variant(variant) || variant == FP8BS_VARIANT_GENERIC)) return FP8BS_ERR_BAD_VARIANT;   // the tiled kernel only
-            fill_plan(m, n, k, variant, split_k > 0 ? (split_k & ~FP8BS_SPLIT_SUM_IN_KERNEL) : 1, &plan, 0, in_kernel);
+            fill_plan(m, n, k, tile, split_k > 0 ? (split_k & ~FP8BS_SPLIT_SUM_IN_KERNEL) : 1, &plan, 0, in_kernel);
         }
     }
     if (plan.workspace_bytes > 0 && (!ws || ws_bytes < plan.workspace_bytes)) return FP8BS_ERR_WORKSPACE;
@@ -389,7 +413,7 @@ int fp8bs_gemm_ex(const void* a, const void* b, const float* a_scale, const floa
         g.sk_nonce = next_nonce();
         g.sk_spin = streamk_spin_limit();
     }
-    if (fp8bs::launch_gemm(plan.variant, mode, g, s) != hipSuccess) return FP8BS_ERR_LAUNCH;
+    if (fp8bs::launch_gemm(plan.variant | plan.form * FORM1, mode, g, s) != hipSuccess) return FP8BS_ERR_LAUNCH;
     if (mode == 1) {
         if (fp8bs::launch_splitk_reduce(g.ws, g.c, (size_t)m * n, plan.split_k, s) != hipSuccess) return FP8BS_ERR_LAUNCH;
     }
@@ -449,6 +473,7 @@ int fp8bs_gemm_grouped_ex(const void* a, const void* b, const float* a_scale, co
         variant = k == 0 ? FP8BS_VARIANT_GENERIC : ((long)total_rows <= 32L * num_experts ? FP8BS_VARIANT_T64x256S3 : FP8BS_VARIANT_T256x256);
     } else {
         VariantInfo vi{};
+        variant = forced_tile(variant);
         if (!variant_info(variant, &vi) || is_streaming_variant(variant)) return FP8BS_ERR_BAD_VARIANT;   // no grouped mode in the streaming kernels
         if (variant != FP8BS_VARIANT_GENERIC && k == 0) return FP8BS_ERR_BAD_VARIANT;
     }

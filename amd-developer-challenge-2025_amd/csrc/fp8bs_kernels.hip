@@ -257,8 +257,10 @@ void gemm_skinny_kernel(const GemmArgs p) {
 // Split-K reduction: sums `split_k` fp32 planes in a fixed order and rounds to bf16, 8 outputs per
 // thread with one 16-byte store (role of fp8_mm_128x128_ft2_split4_merge,
 // 1-amd-fp8-mm/amd-fp8-mm-submission.py:485-511, for any split count).  The planes and c are walked as flat
-// arrays of m*n elements, so the row length plays no part.  VEC: m*n is a multiple of 8 and c starts on a
-// 16-byte boundary; otherwise the same sums, element by element, with the last group cut at m*n.
+// arrays of m*n elements, so the row length plays no part: with c on a 16-byte boundary (VEC) every group of 8 outputs
+// is one aligned store, and where m*n is not a multiple of 4 the later planes' 16-byte loads start on 4-byte boundaries,
+// which the memory system takes (11 x 911 x 6400 in eight partitions, the whole call: 11.4 us against 17.8 element by
+// element).  The last m*n % 8 outputs, and a c off the 16-byte grid, go element by element.
 // ---------------------------------------------------------------------------------------------------
 // SPLIT > 0: the number of planes is a compile-time fact, so all of a thread's loads are issued before the first add
 // (with a run-time count the compiler keeps the loop and every plane's load waits for the previous plane's add: the
@@ -269,23 +271,24 @@ __global__ __launch_bounds__(256)
 void splitk_reduce_kernel(const float* __restrict__ ws, uint16_t* __restrict__ c, size_t mn, int split_k) {
     size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8;
     if (i >= mn) return;
-    if constexpr (VEC) {
+    if (VEC && i + 8 <= mn) {
+        typedef v4f v4f_any __attribute__((aligned(4)));
         v4f s0, s1;
         if constexpr (SPLIT > 0) {
             v4f p0[SPLIT], p1[SPLIT];
 #pragma unroll
             for (int z = 0; z < SPLIT; z++) {
-                p0[z] = __builtin_nontemporal_load((const v4f*)(ws + (size_t)z * mn + i));
-                p1[z] = __builtin_nontemporal_load((const v4f*)(ws + (size_t)z * mn + i + 4));
+                p0[z] = __builtin_nontemporal_load((const v4f_any*)(ws + (size_t)z * mn + i));
+                p1[z] = __builtin_nontemporal_load((const v4f_any*)(ws + (size_t)z * mn + i + 4));
             }
             s0 = p0[0]; s1 = p1[0];
 #pragma unroll
             for (int z = 1; z < SPLIT; z++) { s0 += p0[z]; s1 += p1[z]; }
         } else {
-            s0 = *(const v4f*)(ws + i); s1 = *(const v4f*)(ws + i + 4);
+            s0 = *(const v4f_any*)(ws + i); s1 = *(const v4f_any*)(ws + i + 4);
             for (int z = 1; z < split_k; z++) {
-                s0 += *(const v4f*)(ws + (size_t)z * mn + i);
-                s1 += *(const v4f*)(ws + (size_t)z * mn + i + 4);
+                s0 += *(const v4f_any*)(ws + (size_t)z * mn + i);
+                s1 += *(const v4f_any*)(ws + (size_t)z * mn + i + 4);
             }
         }
         v4i o;
@@ -383,8 +386,8 @@ static hipError_t launch_skinny(const GemmArgs& a, int mode, hipStream_t stream)
     return hipGetLastError();
 }
 
-hipError_t launch_gemm(int variant, int mode, const GemmArgs& a, hipStream_t stream) {
-    switch (variant) {
+hipError_t launch_gemm(int tile, int mode, const GemmArgs& a, hipStream_t stream) {
+    switch (tile) {
         case 1: {
             dim3 grid(((a.epi == 1 ? a.n / 2 : a.n) + 15) / 16, (a.m + 15) / 16);
             hipLaunchKernelGGL(gemm_generic_kernel, grid, dim3(256), 0, stream, a);
@@ -393,6 +396,7 @@ hipError_t launch_gemm(int variant, int mode, const GemmArgs& a, hipStream_t str
         case 2: return launch_tile_256x256(a, mode, stream);
         case 3: return launch_tile_128x128(a, mode, stream);
         case 4: return launch_tile_64x128(a, mode, stream);
+        case 4 | 256: return launch_tile_64x64(a, mode, stream);
         case 5: return launch_tile_256x128(a, mode, stream);
         case 6: return launch_skinny<144, 4>(a, mode, stream);
         case 7: return launch_skinny<256, 3>(a, mode, stream);
@@ -401,6 +405,7 @@ hipError_t launch_gemm(int variant, int mode, const GemmArgs& a, hipStream_t str
         case 10: return launch_tile_256x128s3(a, mode, stream);
         case 11: return launch_tile_192x192s3(a, mode, stream);
         case 12: return launch_tile_64x256s3(a, mode, stream);
+        case 12 | 256: return launch_tile_128x128s4(a, mode, stream);
         default: return hipErrorInvalidValue;
     }
 }
@@ -408,7 +413,7 @@ hipError_t launch_gemm(int variant, int mode, const GemmArgs& a, hipStream_t str
 hipError_t launch_splitk_reduce(const float* ws, uint16_t* c, size_t mn, int split_k, hipStream_t stream) {
     size_t threads = (mn + 7) / 8;
     unsigned blocks = (unsigned)((threads + 255) / 256);
-    if ((mn & 7) == 0 && ((uintptr_t)c & 15) == 0 && ((uintptr_t)ws & 15) == 0) {
+    if (((uintptr_t)c & 15) == 0 && ((uintptr_t)ws & 3) == 0) {
         void (*kern)(const float*, uint16_t*, size_t, int) = splitk_reduce_kernel<true, 0>;
         switch (split_k) {
             case 2: kern = splitk_reduce_kernel<true, 2>; break;
@@ -427,11 +432,12 @@ hipError_t launch_splitk_reduce(const float* ws, uint16_t* c, size_t mn, int spl
     return hipGetLastError();
 }
 
-int variant_lds_bytes(int variant) {
-    switch (variant) {
+int variant_lds_bytes(int tile) {
+    switch (tile) {
         case 2: return TileCfg<256, 256, 64, 128, 0>::LDS_BYTES;
         case 3: return TileCfg<128, 128, 64, 64, 0>::LDS_BYTES;
-        case 4: return TileCfg<64, 128, 32, 64, 0>::LDS_BYTES;
+        case 4: return TileCfg<64, 128, 32, 32, 0, 3>::LDS_BYTES;
+        case 4 | 256: return TileCfg<64, 64, 32, 32, 0, 4>::LDS_BYTES;
         case 5: return TileCfg<256, 128, 64, 64, 0>::LDS_BYTES;
         case 6: return SkinnyCfg<144, 4>::LDS_BYTES;
         case 7: return SkinnyCfg<256, 3>::LDS_BYTES;
@@ -440,6 +446,7 @@ int variant_lds_bytes(int variant) {
         case 10: return TileCfg<256, 128, 64, 64, 0, 3>::LDS_BYTES;
         case 11: return TileCfg<192, 192, 48, 96, 0, 3>::LDS_BYTES;
         case 12: return TileCfg<64, 256, 32, 64, 0, 3>::LDS_BYTES;
+        case 12 | 256: return TileCfg<128, 128, 32, 64, 0, 4>::LDS_BYTES;
         default: return 0;
     }
 }

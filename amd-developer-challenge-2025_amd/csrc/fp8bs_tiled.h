@@ -105,7 +105,7 @@ __device__ __forceinline__ void band_tile(int v, int tiles_m, int tiles_n, int g
 //   MODE 2  : grouped (row_offsets), bf16 output
 //   MODE 3  : dense, K blocks instead of tiles dealt to the workgroups, partial tiles through the workspace, bf16 output
 //   MODE 4  : dense split-K, partial tiles to the workspace, summed by the last workgroup to finish a tile, bf16 output
-// LDS: 2 stages, each [128 k][BM] bytes of A then [128 k][BN] bytes of B, 16-byte chunks XOR-swizzled
+// LDS: NSTAGE stages, each [128 k][BM] bytes of A then [128 k][BN] bytes of B, 16-byte chunks XOR-swizzled
 // so that the 16 k rows touched by half a wave in one transposing read fall on 16 different 16-byte
 // bank groups, then the k block's a_scale row and b_scale values.
 // ---------------------------------------------------------------------------------------------------
@@ -123,15 +123,15 @@ struct TileCfg {
     static constexpr int BS_AREA = 256;                              // the k block's b_scale values of the tile's n blocks
     static constexpr int STAGE_BYTES = A_BYTES + B_BYTES + AS_AREA + BS_AREA;
     static constexpr int LDS_BYTES = NSTAGE * STAGE_BYTES;
-    static_assert(NSTAGE == 2 || NSTAGE == 3, "two or three stages");
+    static_assert(NSTAGE >= 2, "at least two stages");
     static_assert(LDS_BYTES <= 160 * 1024, "LDS");
     static constexpr int A_LOADS = A_BYTES / 16 / NTHREADS;         // 16-byte loads per thread per block
     static constexpr int B_LOADS = B_BYTES / 16 / NTHREADS;
     static_assert(A_BYTES % (16 * NTHREADS) == 0 && B_BYTES % (16 * NTHREADS) == 0, "tile/threads");
-    // A wave's n range lies inside one b_scale block when the tile starts on a block boundary and the
-    // wave width divides 128.  Otherwise (BN = 192, WN = 96) it may cross one boundary, at an n tile that
+    // A wave's n range lies inside one b_scale block when the wave width divides 128 and tiles start on a block
+    // boundary or, narrower than a block, divide it.  Otherwise (BN = 192, WN = 96) it may cross one boundary, at an n tile that
     // depends on the tile and the wave: the K loop is instantiated per boundary position.
-    static constexpr bool SPLIT_SCALES = !(BN % 128 == 0 && 128 % WN == 0);
+    static constexpr bool SPLIT_SCALES = !(128 % WN == 0 && (BN % 128 == 0 || 128 % BN == 0));
     static_assert(WN <= 128, "a wave's n range crosses at most one b_scale block boundary");
     static_assert(!SPLIT_SCALES || (BN == 192 && WN == 96), "boundary positions are enumerated for the 192-wide tile only");
     static_assert(CPR_A <= 16 && CPR_B <= 16, "swizzle assumes a k row spans at most 256 bytes");
@@ -536,8 +536,9 @@ void gemm_tr_kernel(const GemmArgs p) {
     // enforced by hand: s_waitcnt vmcnt(0) + workgroup barrier before the first read of a stage.
     const uint32_t lds_base = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)lds;
     constexpr int NLOADS = C::A_LOADS + C::B_LOADS + 1;     // + the scales
-    // the counted waits below name up to two blocks of copies and a tile's output stores; the counter has six bits
-    static_assert(2 * NLOADS + EPI_STORES <= 63, "vmcnt wait thresholds must fit the counter");
+    // the counted waits below name the copies of the blocks that may stay in flight and a tile's output stores; the
+    // counter has six bits
+    static_assert((NSTAGE - 2) * NLOADS + EPI_STORES <= 63, "vmcnt wait thresholds must fit the counter");
     // copy q (compile-time) of k block `blk` (relative to the tile's first) into `stage`
     auto issue_one = [&](const CopyPlan& cp, int stage, int blk, auto q_tag) {
         constexpr int q = decltype(q_tag)::value;
@@ -562,6 +563,13 @@ void gemm_tr_kernel(const GemmArgs p) {
         [&]<int... Q>(std::integer_sequence<int, Q...>) {
             (issue_one(cp, stage, blk, std::integral_constant<int, Q>{}), ...);
         }(std::make_integer_sequence<int, NLOADS>{});
+    };
+
+    // blocks 0 .. NSTAGE-2 of a tile, as many as it has
+    auto issue_first = [&](const CopyPlan& cp, int blocks) {
+        issue_all(cp, 0, 0);
+#pragma unroll
+        for (int s = 1; s < NSTAGE - 1; s++) if (blocks > s) issue_all(cp, s, s);
     };
 
     // ---- per-lane LDS read addresses -----------------------------------------------------------
@@ -653,7 +661,7 @@ void gemm_tr_kernel(const GemmArgs p) {
     const bool wave_active = __builtin_amdgcn_readfirstlane((m0 + wave_m * WM < row_hi && m0 + wave_m * WM + WM > row_lo &&
                                                              n0 + wave_n * WN < p.n) ? 1 : 0) != 0;
     // b_scale of the wave's n tiles: slot bs_off for n tiles [0, ub), the next slot for [ub, NT)
-    const int wave_col = (C::SPLIT_SCALES ? (n0 & 127) : 0) + wave_n * WN;               // from the start of the tile's first n block
+    const int wave_col = (BN % 128 != 0 ? (n0 & 127) : 0) + wave_n * WN;               // from the start of the tile's first n block
     const int bs_off = bs_base + (wave_col >> 7) * 4;
     const int ub = C::SPLIT_SCALES ? (128 - (wave_col & 127)) >> 4 : C::NT;
 
@@ -676,7 +684,8 @@ void gemm_tr_kernel(const GemmArgs p) {
         // (the 192-wide tile is the exception, measured: one copy per step gives it 0.92 us per K block on
         // one CU against 1.02, while the 256-wide tile loses 4 % that way)
         constexpr int DMA_EVERY = BN == 192 ? 1 : ((STEPS - C::MT) / NL_EARLY >= 2 ? 2 : 1), DMA_FIRST = DMA_EVERY - 1;
-        static_assert(NL_EARLY * DMA_EVERY <= STEPS - C::MT, "not enough steps to issue the copies before the barrier");
+        // (a small wave tile has fewer steps before the barrier than copies: several go into one step)
+        constexpr int DMA_PER_STEP = NL_EARLY * DMA_EVERY <= STEPS - C::MT ? 1 : (NL_EARLY + STEPS - C::MT - 1) / (STEPS - C::MT);
 
         // ---- prologue: blocks 0 .. NSTAGE-2 -> stages 0 .. NSTAGE-2 (unless the previous tile already
         //      sent them), wait for block 0; first copies of block NSTAGE-1 -> the last stage.  The
@@ -684,19 +693,15 @@ void gemm_tr_kernel(const GemmArgs p) {
         //      output ----
         // The vector memory counter retires loads and stores in the order they were issued.  If block 0
         // was sent ahead of the previous tile's NSTORES output stores, "at most NSTORES outstanding" means
-        // the block has landed, and the stores are left to finish under the first K block.  With three
-        // stages block 1 (NLOADS copies) sits between block 0 and the stores.
-        if (!prefetched) {
-            issue_all(cp, 0, 0);
-            if constexpr (NSTAGE == 3) { if (nkb > 1) issue_all(cp, 1, 1); }
-        }
-        if constexpr (NSTAGE == 2) {
-            if (prefetched && stores_behind) wait_vmcnt<EPI_STORES>();
-            else wait_vmcnt<0>();
-        } else {
+        // the block has landed, and the stores are left to finish under the first K block.  With more than
+        // two stages the next blocks (NLOADS copies each) sit between block 0 and the stores.
+        if (!prefetched) issue_first(cp, nkb);
+        {
             const bool sb = prefetched && stores_behind;
-            if (nkb > 1) { if (sb) wait_vmcnt<NLOADS + EPI_STORES>(); else wait_vmcnt<NLOADS>(); }
-            else { if (sb) wait_vmcnt<EPI_STORES>(); else wait_vmcnt<0>(); }
+            const int behind = (nkb < NSTAGE - 1 ? nkb : NSTAGE - 1) - 1;       // blocks sent after block 0
+            [&]<int... I>(std::integer_sequence<int, I...>) {
+                ((behind == I ? (sb ? wait_vmcnt<I * NLOADS + EPI_STORES>() : wait_vmcnt<I * NLOADS>()) : (void)0), ...);
+            }(std::make_integer_sequence<int, NSTAGE - 1>{});
         }
         __syncthreads();
         if (TAILS && nkb == 1) FP8BS_PATCH_TAILS(0, 1);
@@ -722,20 +727,21 @@ void gemm_tr_kernel(const GemmArgs p) {
         // Block j lives in stage j % NSTAGE.  While it is multiplied, the rest of block j+NSTAGE-1 is
         // copied into the stage that the barrier of block j-1 freed; behind the barrier of block j the
         // first copies of block j+NSTAGE go into the stage just read.  With two stages a copy has one
-        // block's time to land, with three stages two.
-        auto k_block = [&](int j, auto h1_tag, auto h2_tag, auto h3_tag) {
-            constexpr bool HAS_NEXT = decltype(h1_tag)::value;                                              // block j+1 exists
-            constexpr bool HAS_EARLY = NSTAGE == 2 ? decltype(h1_tag)::value : decltype(h2_tag)::value;    // block j+NSTAGE-1 exists
-            constexpr bool HAS_LATE = NSTAGE == 2 ? decltype(h2_tag)::value : decltype(h3_tag)::value;     // block j+NSTAGE exists
-            constexpr bool LANDS_LAST = decltype(h1_tag)::value && !decltype(h2_tag)::value;               // block j+1 is the tile's last
+        // block's time to land, with three stages two, with four three.
+        auto k_block = [&](int j, auto rem_tag) {
+            constexpr int REM = decltype(rem_tag)::value;                      // blocks behind block j; NSTAGE stands for that many or more
+            constexpr bool HAS_NEXT = REM >= 1;                                // block j+1 exists
+            constexpr bool HAS_EARLY = REM >= NSTAGE - 1;                      // block j+NSTAGE-1 exists
+            constexpr bool HAS_LATE = REM >= NSTAGE;                           // block j+NSTAGE exists
+            constexpr bool LANDS_LAST = REM == 1;                              // block j+1 is the tile's last
             const int cur_stage = NSTAGE == 2 ? (j & 1) : j % NSTAGE;
             const int next_stage = cur_stage + 1 == NSTAGE ? 0 : cur_stage + 1;
-            const int early_stage = NSTAGE == 2 ? next_stage : (next_stage + 1 == NSTAGE ? 0 : next_stage + 1);
-            // what must have landed at the barrier is block j+1; with three stages the NLOADS copies of
-            // block j+2 were all issued after it and may stay in flight
+            const int early_stage = NSTAGE == 2 ? next_stage : (cur_stage == 0 ? NSTAGE - 1 : cur_stage - 1);
+            // what must have landed at the barrier is block j+1; the copies of the blocks behind it (j+2 up to
+            // j+NSTAGE-1, as far as they exist) were all issued after it and may stay in flight
             auto wait_next_block = [&]() {
-                if constexpr (NSTAGE == 3 && HAS_EARLY) wait_vmcnt_lgkm0<NLOADS>();
-                else __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0)
+                constexpr int BEHIND = (REM < NSTAGE - 1 ? REM : NSTAGE - 1) - 1;
+                wait_vmcnt_lgkm0<(BEHIND > 0 ? BEHIND : 0) * NLOADS>();
             };
             if (!wave_active) {
                 // none of this wave's rows is stored: it only does its share of the copies, in the
@@ -771,8 +777,15 @@ void gemm_tr_kernel(const GemmArgs p) {
                 constexpr int s = decltype(s_tag)::value;
                 if constexpr (s < STEPS) {
                     constexpr int u = s / C::MT, t = s % C::MT;
-                    if constexpr (HAS_EARLY && s % DMA_EVERY == DMA_FIRST && s / DMA_EVERY < NL_EARLY)
-                        issue_one(cp, early_stage, j + NSTAGE - 1, std::integral_constant<int, NL_LATE + s / DMA_EVERY>{});
+                    if constexpr (HAS_EARLY && DMA_PER_STEP == 1) {
+                        if constexpr (s % DMA_EVERY == DMA_FIRST && s / DMA_EVERY < NL_EARLY)
+                            issue_one(cp, early_stage, j + NSTAGE - 1, std::integral_constant<int, NL_LATE + s / DMA_EVERY>{});
+                    } else if constexpr (HAS_EARLY && s * DMA_PER_STEP < NL_EARLY) {
+                        constexpr int FIRST = s * DMA_PER_STEP, COUNT = NL_EARLY - FIRST < DMA_PER_STEP ? NL_EARLY - FIRST : DMA_PER_STEP;
+                        [&]<int... Q>(std::integer_sequence<int, Q...>) {
+                            (issue_one(cp, early_stage, j + NSTAGE - 1, std::integral_constant<int, NL_LATE + FIRST + Q>{}), ...);
+                        }(std::make_integer_sequence<int, COUNT>{});
+                    }
                     if constexpr (t == 0 && u + 1 < C::NT) read_b(breg[(u + 1) & 1], u + 1, sbase);
                     if constexpr (t == 0 && u == C::NT - 1) {
                         // All reads of this stage are issued.  Wait for them and for this wave's part
@@ -804,18 +817,12 @@ void gemm_tr_kernel(const GemmArgs p) {
             }(std::make_integer_sequence<int, STEPS + LAG>{});
         };
 
-        constexpr std::true_type T{};
-        constexpr std::false_type F{};
         int j = 0;
-        if constexpr (NSTAGE == 2) {
-            for (; j + 2 < nkb; j++) k_block(j, T, T, F);
-            if (j + 1 < nkb) { k_block(j, T, F, F); j++; }
-        } else {
-            for (; j + 3 < nkb; j++) k_block(j, T, T, T);
-            if (j + 2 < nkb) { k_block(j, T, T, F); j++; }
-            if (j + 1 < nkb) { k_block(j, T, F, F); j++; }
-        }
-        k_block(j, F, F, F);
+        for (; j + NSTAGE < nkb; j++) k_block(j, std::integral_constant<int, NSTAGE>{});
+        [&]<int... R>(std::integer_sequence<int, R...>) {
+            ((j + (NSTAGE - 1 - R) < nkb ? (k_block(j, std::integral_constant<int, NSTAGE - 1 - R>{}), (void)j++) : (void)0), ...);
+        }(std::make_integer_sequence<int, NSTAGE - 1>{});
+        k_block(j, std::integral_constant<int, 0>{});
         };   // run_blocks
         if constexpr (C::SPLIT_SCALES) {
             // 96-column wave tiles of a 192-column tile start 0, 96, 64 or 160 columns into a block
@@ -839,8 +846,7 @@ void gemm_tr_kernel(const GemmArgs p) {
     if (nxt.valid) {
         ncp = copy_plan(nxt);
         if (nxt.kb_end > nxt.kb_begin) {
-            issue_all(ncp, 0, 0);
-            if constexpr (NSTAGE == 3) { if (nxt.kb_end - nxt.kb_begin > 1) issue_all(ncp, 1, 1); }
+            issue_first(ncp, nxt.kb_end - nxt.kb_begin);
             prefetched = true;
         }
     }
@@ -1082,10 +1088,16 @@ void gemm_tr_kernel(const GemmArgs p) {
                 if constexpr (!TAILS) {
                     *(v4f*)dst = acc[t][u];
                 } else {
-                    // rows of the plane start on any 4-byte boundary and may end inside the lane's four columns
+                    // rows of the plane start on any 4-byte boundary, which a 16-byte store takes, and may end inside the
+                    // lane's four columns
+                    typedef v4f v4f_any __attribute__((aligned(4)));
+                    if (col + 3 < p.n) {
+                        *(v4f_any*)dst = acc[t][u];
+                    } else {
 #pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        if (col + r < p.n) dst[r] = acc[t][u][r];
+                        for (int r = 0; r < 3; r++)
+                            if (col + r < p.n) dst[r] = acc[t][u][r];
+                    }
                 }
             }
         }
@@ -1279,8 +1291,8 @@ static inline hipError_t launch_shape(const GemmArgs& a, int mode, hipStream_t s
         // the fused silu-mul epilogue exists for the 256x256 tile, dense or grouped, without K split
         if constexpr (WITH_EPI) {
             if (a.epi != 1 || mode == 1) return hipErrorInvalidValue;
-            if (mode == 2) return launch_tr<BM, BN, WM, WN, 2, 1>(a, grid, stream);
-            return launch_tr<BM, BN, WM, WN, 0, 1>(a, grid, stream);
+            if (mode == 2) return launch_tr<BM, BN, WM, WN, 2, 1, NSTAGE>(a, grid, stream);
+            return launch_tr<BM, BN, WM, WN, 0, 1, NSTAGE>(a, grid, stream);
         } else {
             return hipErrorInvalidValue;
         }

@@ -53,7 +53,8 @@ enum {
     FP8BS_VARIANT_GENERIC = 1,    /* scalar kernel, any m/n: the planner uses it for k = 0 only */
     FP8BS_VARIANT_T256x256 = 2,   /* compute-bound: 256x256 tile, 8 waves                    */
     FP8BS_VARIANT_T128x128 = 3,   /* mid-size: 128x128 tile, 4 waves                         */
-    FP8BS_VARIANT_T64x128 = 4,    /* skinny-M: 64(m) x 128(n) tile, 4 waves, split-K         */
+    FP8BS_VARIANT_T64x128 = 4,    /* small: form 0: 64(m) x 128(n) tile, 8 waves, three LDS stages; form 1: 64 x 64 tile,
+                                     4 waves, four stages                                     */
     FP8BS_VARIANT_T256x128 = 5,   /* 256(m) x 128(n) tile, 8 waves                           */
     FP8BS_VARIANT_SKINNY64x144 = 6, /* streaming kernel: 64(m) x 144(n) tile, 4-stage copy ring (forced only: needs m <= 64
                                        per tile row to pay, n % 8 == 0 and operands on 16-byte boundaries) */
@@ -62,9 +63,13 @@ enum {
     FP8BS_VARIANT_T256x192 = 9,   /* 256(m) x 192(n) tile, 8 waves: fills more CUs when n/256 rounds up badly */
     FP8BS_VARIANT_T256x128S3 = 10, /* 256 x 128 tile, three LDS stages (a copy has two K blocks' time to land) */
     FP8BS_VARIANT_T192x192S3 = 11, /* 192 x 192 tile, 8 waves of 48 x 96, three LDS stages     */
-    FP8BS_VARIANT_T64x256S3 = 12,  /* 64(m) x 256(n) tile, 8 waves of 32 x 64, three LDS stages: few rows against much of b */
+    FP8BS_VARIANT_T64x256S3 = 12,  /* 8 waves of 32 x 64.  Form 0: 64(m) x 256(n) tile, three LDS stages: few rows against much of
+                                     b; form 1: 128 x 128 tile, four stages: mid-size, one tile per CU */
     FP8BS_VARIANT_COUNT = 13
 };
+
+/* A forced variant argument that names one of the two forms of a variant (without it: the first form). */
+#define FP8BS_VARIANT_FORM(variant, form) ((variant) | (((form) + 1) << 8))
 
 /* What fp8bs_plan() decides for a shape. Replaces the exact-(m,n,k) if-ladder of the reference
  * (1-amd-fp8-mm/amd-fp8-mm-submission.py:528-578) with a shape-family rule. */
@@ -80,7 +85,7 @@ typedef struct fp8bs_plan_t {
     int32_t sum_in_kernel;  /* 1 (with split_k > 1): one launch - the workgroups of a tile's K partitions leave fp32
                                partial tiles in the workspace and the last one to finish adds them in ascending K and
                                writes c; 0: partial planes and a reduce kernel (two launches)      */
-    int32_t reserved;
+    int32_t form;           /* form of the variant (0 unless the variant has two)  */
     uint64_t workspace_bytes;
 } fp8bs_plan_t;
 
