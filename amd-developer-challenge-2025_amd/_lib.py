@@ -13,9 +13,10 @@ LIB_PATH = os.path.join(HERE, "libfp8bs.so")
 EXPORTS = (
     "fp8bs_version", "fp8bs_strerror", "fp8bs_plan", "fp8bs_workspace_bytes",
     "fp8bs_gemm", "fp8bs_gemm_ex", "fp8bs_gemm_noalloc", "fp8bs_gemm_grouped", "fp8bs_gemm_grouped_ex",
+    "fp8bs_gemm_grouped_ws", "fp8bs_grouped_workspace_bytes",
     "fp8bs_quantize_a", "fp8bs_quantize_b", "fp8bs_gather_a",
     "fp8bs_moe_topk", "fp8bs_moe_route_workspace_bytes", "fp8bs_moe_route",
-    "fp8bs_gemm_silu_mul", "fp8bs_moe_combine", "fp8bs_convert_fnuz_to_fn", "fp8bs_diag_mfma_mix",
+    "fp8bs_gemm_silu_mul", "fp8bs_gemm_silu_mul_ws", "fp8bs_silu_mul_workspace_bytes", "fp8bs_moe_combine", "fp8bs_convert_fnuz_to_fn", "fp8bs_diag_mfma_mix",
 )
 
 VARIANT_NAMES = {0: "auto", 1: "generic", 2: "t256x256", 3: "t128x128", 4: "t64x128", 5: "t256x128", 6: "skinny64x144", 7: "skinny64x256", 8: "skinny64x288", 9: "t256x192", 10: "t256x128s3", 11: "t192x192s3", 12: "t64x256s3"}
@@ -72,6 +73,14 @@ def load() -> ctypes.CDLL:
     lib.fp8bs_gemm_grouped.argtypes = [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, vp]
     lib.fp8bs_gemm_grouped_ex.restype = i32
     lib.fp8bs_gemm_grouped_ex.argtypes = [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, vp]
+    lib.fp8bs_gemm_grouped_ws.restype = i32
+    lib.fp8bs_gemm_grouped_ws.argtypes = [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp, sz, vp]
+    lib.fp8bs_grouped_workspace_bytes.restype = sz
+    lib.fp8bs_grouped_workspace_bytes.argtypes = [i32, i32, i32, i32]
+    lib.fp8bs_gemm_silu_mul_ws.restype = i32
+    lib.fp8bs_gemm_silu_mul_ws.argtypes = [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp, sz, vp]
+    lib.fp8bs_silu_mul_workspace_bytes.restype = sz
+    lib.fp8bs_silu_mul_workspace_bytes.argtypes = [i32, i32, i32]
     i64 = ctypes.c_int64
     lib.fp8bs_quantize_a.restype = i32
     lib.fp8bs_quantize_a.argtypes = [vp, i32, i64, vp, i32, vp, vp, i32, i32, vp]

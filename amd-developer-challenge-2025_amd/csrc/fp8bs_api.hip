@@ -80,6 +80,20 @@ bool can_sum_in_kernel(int m, int n, int tile, int split_k) {
     return split_k >= 2 && split_k <= 255 && cdiv(m, vi.bm) * cdiv(n, vi.bn) <= fp8bs::StreamK::MAX_GRID;
 }
 
+// Tiles with the fused silu-mul epilogue.
+bool has_epilogue(int tile) {
+    switch (tile) {
+        case FP8BS_VARIANT_T256x256: case FP8BS_VARIANT_T256x128S3: case FP8BS_VARIANT_T64x128: case FP8BS_VARIANT_T64x128 | FORM1:
+        case FP8BS_VARIANT_T64x256S3: case FP8BS_VARIANT_T64x256S3 | FORM1: return true;
+        default: return false;
+    }
+}
+
+// Tiles with the grouped walk in K partitions.
+bool has_grouped_split(int tile) {
+    return tile == (FP8BS_VARIANT_T64x128 | FORM1) || tile == FP8BS_VARIANT_T64x256S3 || tile == (FP8BS_VARIANT_T64x256S3 | FORM1);
+}
+
 // Fill a plan for a given tile and split count.  in_kernel: the split's partial tiles are summed by the last
 // workgroup to finish each tile (where the shape allows it, see above; else the reduce kernel follows).
 void fill_plan(int m, int n, int k, int tile, int split_k, fp8bs_plan_t* out, int stream_k = 0, bool in_kernel = false) {
@@ -120,7 +134,7 @@ bool vector_shape(int n) { return (n % 8) == 0; }
 bool skinny_shape(int m, int n, int k) { return m <= 64 && (double)n * (double)k >= 24.0e6; }
 
 // The tile shape and K split of the tiled MFMA kernel that finish soonest (any m, any n).
-void choose_tiled(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_split = true) {
+void choose_tiled(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_split, bool epi) {
     if (num_cus <= 0) num_cus = 256;
     int kbt = k / KBLK;
     // The tile and K split that finish soonest under a cost model in microseconds.  A workgroup advances one K block in
@@ -156,6 +170,7 @@ void choose_tiled(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_
     const int splits[6] = {1, 2, 3, 4, 6, 8};
     int best_tile = 0, best_split = 1; double best_cost = 0; bool best_fused = false;
     for (const Cand& c : cands) {
+        if (epi && !has_epilogue(c.tile)) continue;
         VariantInfo vi{};
         variant_info(c.tile, &vi);
         const long tiles = cdiv(m, vi.bm) * cdiv(n, vi.bn);
@@ -203,7 +218,7 @@ void choose_tiled(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_
 // streaming kernel and the 64 x 128 tile: 64 x 18432 x 7168 34.3 us (split 3) against 37.7 and 38.4;
 // 64 x 7168 x 7168 20.4 against 32.4 and 21.0; 1 x 18432 x 7168 29.2 against 31.8 and 34.1;
 // 1 x 28672 x 4096 26.7 against 34.6 and 30.6.
-void choose_skinny(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_split = true) {
+void choose_skinny(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_split) {
     if (num_cus <= 0) num_cus = 256;
     const int kbt = k / KBLK;
     const long tiles = cdiv(m, 64) * cdiv(n, 256);
@@ -231,9 +246,9 @@ void choose_skinny(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may
 
 // Shape-family rule.  A few rows against a large b -> the 64 x 256 three-stage tile.  Everything else -> the
 // tile and K split that the cost model of the tiled kernel picks.
-void choose(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_split = true) {
+void choose(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_split = true, bool epi = false) {
     if (skinny_shape(m, n, k)) choose_skinny(m, n, k, num_cus, out, may_split);
-    else choose_tiled(m, n, k, num_cus, out, may_split);
+    else choose_tiled(m, n, k, num_cus, out, may_split, epi);
 }
 
 // Order of the tiles of a grouped call (the row counts themselves are on the device).  With a tile or more of
@@ -242,6 +257,77 @@ void choose(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_split 
 // configuration 5: 2-3 % faster).  With fewer rows every expert is one tile row and the call streams the weights;
 // the order across the experts is then 0.7-1.2 % ahead (8 or 100 rows per expert), so it is kept there.
 int group_order(int total_rows, int num_experts) { return (long)total_rows >= 256L * num_experts ? 1 : 0; }
+
+struct GroupedPlan { int tile, split; };
+
+// The counters and partial tiles of a grouped K split, for as many tiles as the routing can give.
+uint64_t grouped_bytes(const GroupedPlan& p, int experts, int rows, int n) {
+    if (p.split <= 1) return 0;
+    VariantInfo vi{};
+    variant_info(p.tile, &vi);
+    return (uint64_t)fp8bs::StreamK::SLOTS_OFF + (uint64_t)(fp8bs::grouped_slots_bound(rows, experts, vi.bm) * cdiv(n, vi.bn)) * (uint64_t)p.split * (uint64_t)vi.bm * (uint64_t)vi.bn * 4u;
+}
+
+bool can_split_grouped(const GroupedPlan& p, int experts, int rows, int n, int k) {
+    VariantInfo vi{};
+    if (!has_grouped_split(p.tile) || !variant_info(p.tile, &vi)) return false;
+    return p.split >= 2 && p.split <= 255 && p.split <= k / KBLK && fp8bs::grouped_slots_bound(rows, experts, vi.bm) * cdiv(n, vi.bn) <= fp8bs::StreamK::MAX_GRID;
+}
+
+// The tile and K split of a grouped call.  The row counts themselves are on the device, so the model below works with
+// averages: experts that get rows, tiles per such expert (its rows plus, on average, half of the 16 it may start late, and
+// the last, partial tile), and the share of a tile's rows that exist - waves without rows only copy, so a tile with few
+// rows takes its shorter time per K block, t_few.  Terms as in choose_tiled; bw is the rate in TB/s at which tiles of this
+// width stream the experts' weights from HBM together (row segments of 256 bytes are taken best), shared by the tiles that
+// read the same panel.  The constants are fits to the measured times of every (tile, split) on 210 shapes on MI355X (8, 16
+// or 32 experts, 1 .. 4096 tokens to 2, 4 or 8 of them, N 512 .. 7168, K 512 .. 7168, log-uniform): picking by the model
+// costs 2.2 % against the best of each shape in the geometric mean and takes 17 % off the rule it replaced (the 256x256
+// tile above 32 rows per expert on average, 64x256 below): 194 tokens to 4 of 16 experts, 1299 x 5760: 90.8 -> 49.2 us;
+// 801 to 4 of 8, 840 x 1664: 23.2 -> 15.0; 35 to 4 of 8, 1375 x 5504: 43.6 -> 22.8.
+GroupedPlan choose_grouped(int experts, int rows, int n, int k, int num_cus, bool may_split) {
+    if (num_cus <= 0) num_cus = 256;
+    struct Cand { int tile; int rmax; double t_full, t_few, t_power, t_fixed, shared, bw; };
+    const Cand cands[5] = {
+        {FP8BS_VARIANT_T256x256, 1, 2.010, 1.259, 1.681, 6.01, 1.0, 5.18},
+        {FP8BS_VARIANT_T256x128S3, 1, 1.122, 0.618, 0.605, 5.58, 1.0, 5.06},
+        {FP8BS_VARIANT_T64x256S3, 1, 0.794, 0.578, 0.500, 5.09, 1.0, 5.32},
+        {FP8BS_VARIANT_T64x256S3 | FORM1, 1, 0.728, 0.497, 0.661, 4.34, 1.0, 5.27},
+        {FP8BS_VARIANT_T64x128 | FORM1, 2, 0.570, 0.313, 0.100, 3.59, 1.65, 4.02},
+    };
+    double unused = 1.0;                                           // (1 - 1/E)^rows: an expert's chance to get none
+    for (int r = 0; r < rows && unused > 1e-3; r++) unused *= 1.0 - 1.0 / experts;
+    const double active = experts * (1.0 - unused), average = rows / active;
+    const int kbt = k / KBLK;
+    GroupedPlan best{FP8BS_VARIANT_T256x256, 1};
+    double best_cost = 0;
+    for (const Cand& c : cands) {
+        VariantInfo vi{};
+        variant_info(c.tile, &vi);
+        double slots = (average + 8.0) / vi.bm + 0.4;
+        if (slots < 1.0) slots = 1.0;
+        double fill = (average / slots + 24.0) / vi.bm;
+        if (fill > 1.0) fill = 1.0;
+        const double t_alone = c.t_few + (c.t_full - c.t_few) * fill;
+        for (int s = 1; s <= 4; s++) {
+            const GroupedPlan p{c.tile, s};
+            // (partial tiles of 64 MB at most: beyond that a call has tiles enough without a split)
+            if (s > 1 && (!may_split || kbt / s < 2 || !can_split_grouped(p, experts, rows, n, k) || grouped_bytes(p, experts, rows, n) > (64u << 20))) break;
+            const double wgs = active * slots * (double)cdiv(n, vi.bn) * s, per_round = (double)num_cus * c.rmax, kb = (double)cdiv(kbt, s);
+            auto t_block = [&](double w) {
+                double t = t_alone * (w > num_cus && c.rmax > 1 ? c.shared : 1.0);
+                const double power = c.t_power * fill * w / num_cus, stream = w * 128.0 * vi.bn / slots / (c.bw * 1e6);
+                t = power > t ? power : t;
+                return stream > t ? stream : t;
+            };
+            const double full = (double)(long)(wgs / per_round), rem = wgs - full * per_round;
+            double cost = full * (c.t_fixed + kb * t_block(per_round));
+            if (rem > 0.5) cost += c.t_fixed + kb * t_block(rem);
+            if (s > 1) cost += 3.56 + 0.757e-6 * s * (double)rows * (double)n;
+            if (best_cost == 0 || cost < best_cost) { best = p; best_cost = cost; }
+        }
+    }
+    return best;
+}
 
 // The value a flag takes in one call that deals K blocks: never zero, different from call to call (and, through
 // the clock and the process id, from run to run), so that whatever an earlier call or an uninitialised workspace
@@ -345,9 +431,9 @@ size_t fp8bs_workspace_bytes(int m, int n, int k) {
     return (size_t)p.workspace_bytes;
 }
 
-int fp8bs_gemm_ex(const void* a, const void* b, const float* a_scale, const float* b_scale,
-                  void* c, void* ws, size_t ws_bytes, int m, int n, int k,
-                  int variant, int split_k, void* stream) {
+// A dense call, plain or with the silu-mul epilogue (epi 1: c has n/2 columns).
+static int dense_call(const void* a, const void* b, const float* a_scale, const float* b_scale, void* c, void* ws, size_t ws_bytes,
+                      int m, int n, int k, int variant, int split_k, int epi, void* stream) {
     int st = check_common(a, b, a_scale, b_scale, c, m, n, k);
     if (st != FP8BS_OK) return st;
     if (m == 0 || n == 0) return FP8BS_OK;
@@ -366,7 +452,7 @@ int fp8bs_gemm_ex(const void* a, const void* b, const float* a_scale, const floa
     const bool simple = aligned && vector_shape(n);      // streaming kernels possible
     const int cus = fp8bs::device_cus();
     if (variant == FP8BS_VARIANT_AUTO) {
-        choose(m, n, k, cus, &plan);
+        choose(m, n, k, cus, &plan, true, epi != 0);
         const int tile = plan.variant | plan.form * FORM1;
         if (split_k > 0) fill_plan(m, n, k, tile, split_k & ~FP8BS_SPLIT_SUM_IN_KERNEL, &plan, 0, (split_k & FP8BS_SPLIT_SUM_IN_KERNEL) != 0);
         else if (split_k < 0) fill_plan(m, n, k, plan.variant, 1, &plan, streamk_grid(plan.variant, m, n, k, cus));   // (the first form only)
@@ -375,7 +461,7 @@ int fp8bs_gemm_ex(const void* a, const void* b, const float* a_scale, const floa
             // too small for the partial tiles of a sum in the kernel but not for the planes (tiles that overhang
             // the matrix): the same split with the reduce kernel
             if (plan.sum_in_kernel && ws && ws_bytes >= planes_bytes(m, n, plan.split_k)) fill_plan(m, n, k, tile, plan.split_k, &plan);
-            else choose(m, n, k, cus, &plan, false);
+            else choose(m, n, k, cus, &plan, false, epi != 0);
         }
     } else {
         VariantInfo vi{};
@@ -394,6 +480,7 @@ int fp8bs_gemm_ex(const void* a, const void* b, const float* a_scale, const floa
         }
     }
     if (plan.workspace_bytes > 0 && (!ws || ws_bytes < plan.workspace_bytes)) return FP8BS_ERR_WORKSPACE;
+    if (epi && plan.variant != FP8BS_VARIANT_GENERIC && (!has_epilogue(plan.variant | plan.form * FORM1) || plan.stream_k > 0)) return FP8BS_ERR_BAD_VARIANT;
 
     fp8bs::GemmArgs g{};
     g.a = (const uint8_t*)a; g.b = (const uint8_t*)b; g.as = a_scale; g.bs = b_scale;
@@ -403,6 +490,7 @@ int fp8bs_gemm_ex(const void* a, const void* b, const float* a_scale, const floa
     g.kb_per_split = (int)cdiv(k / KBLK, plan.split_k);
     g.band_h = 4;
     g.num_experts = 0;
+    g.epi = epi;
     int mode = plan.split_k > 1 ? 1 : 0;
     if (plan.sum_in_kernel && plan.split_k > 1) {
         mode = 4;
@@ -415,9 +503,15 @@ int fp8bs_gemm_ex(const void* a, const void* b, const float* a_scale, const floa
     }
     if (fp8bs::launch_gemm(plan.variant | plan.form * FORM1, mode, g, s) != hipSuccess) return FP8BS_ERR_LAUNCH;
     if (mode == 1) {
-        if (fp8bs::launch_splitk_reduce(g.ws, g.c, (size_t)m * n, plan.split_k, s) != hipSuccess) return FP8BS_ERR_LAUNCH;
+        if (fp8bs::launch_splitk_reduce(g.ws, g.c, (size_t)m * n, plan.split_k, epi, s) != hipSuccess) return FP8BS_ERR_LAUNCH;
     }
     return FP8BS_OK;
+}
+
+int fp8bs_gemm_ex(const void* a, const void* b, const float* a_scale, const float* b_scale,
+                  void* c, void* ws, size_t ws_bytes, int m, int n, int k,
+                  int variant, int split_k, void* stream) {
+    return dense_call(a, b, a_scale, b_scale, c, ws, ws_bytes, m, n, k, variant, split_k, 0, stream);
 }
 
 int fp8bs_gemm(const void* a, const void* b, const float* a_scale, const float* b_scale,
@@ -446,39 +540,68 @@ int fp8bs_gemm_noalloc(const void* a, const void* b, const float* a_scale, const
     return fp8bs_gemm_ex(a, b, a_scale, b_scale, c, ws, (size_t)FP8BS_NOALLOC_SCRATCH_BYTES, m, n, k, FP8BS_VARIANT_AUTO, 0, stream);
 }
 
+// A grouped call, plain or with the silu-mul epilogue.
+static int grouped_call(const void* a, const void* b, const float* a_scale, const float* b_scale, void* c, const int32_t* row_offsets,
+                        int num_experts, int rows, int n, int k, int variant, int split_k, int epi, void* ws, size_t ws_bytes, void* stream) {
+    if (num_experts <= 0) return FP8BS_ERR_BAD_OFFSETS;
+    if (!row_offsets) return FP8BS_ERR_NULL_POINTER;
+    int st = check_common(a, b, a_scale, b_scale, c, rows, n, k);
+    if (st != FP8BS_OK) return st;
+    if (rows == 0 || n == 0) return FP8BS_OK;
+    if (ws && ((uintptr_t)ws & 15) != 0) {
+        const size_t skip = 16 - ((uintptr_t)ws & 15);
+        if (ws_bytes > skip) { ws = (char*)ws + skip; ws_bytes -= skip; }
+        else { ws = nullptr; ws_bytes = 0; }
+    }
+    fp8bs::GemmArgs g{};
+    g.a = (const uint8_t*)a; g.b = (const uint8_t*)b; g.as = a_scale; g.bs = b_scale;
+    g.c = (uint16_t*)c; g.ws = (float*)ws; g.row_offsets = row_offsets;
+    g.m = rows; g.n = n; g.k = k; g.lda = rows; g.nb = (n + 127) / 128;
+    g.band_h = 4; g.num_experts = num_experts;
+    g.by_expert = group_order(rows, num_experts);
+    g.epi = epi;
+    GroupedPlan plan{forced_tile(variant), split_k > 1 ? split_k : 1};
+    if (k == 0 && variant == FP8BS_VARIANT_AUTO) plan = {FP8BS_VARIANT_GENERIC, 1};
+    else if (variant == FP8BS_VARIANT_AUTO) {
+        plan = choose_grouped(num_experts, rows, n, k, fp8bs::device_cus(), true);
+        if (plan.split > 1 && (!ws || ws_bytes < grouped_bytes(plan, num_experts, rows, n))) plan = choose_grouped(num_experts, rows, n, k, fp8bs::device_cus(), false);
+    } else {
+        VariantInfo vi{};
+        if (!variant_info(plan.tile, &vi) || is_streaming_variant(plan.tile)) return FP8BS_ERR_BAD_VARIANT;   // no grouped mode in the streaming kernels
+        if (plan.tile != FP8BS_VARIANT_GENERIC && k == 0) return FP8BS_ERR_BAD_VARIANT;
+        if (epi && plan.tile != FP8BS_VARIANT_GENERIC && !has_epilogue(plan.tile)) return FP8BS_ERR_BAD_VARIANT;
+        if (plan.split > 1 && !can_split_grouped(plan, num_experts, rows, n, k)) return FP8BS_ERR_BAD_VARIANT;
+        if (plan.split > 1 && (!ws || ws_bytes < grouped_bytes(plan, num_experts, rows, n))) return FP8BS_ERR_WORKSPACE;
+    }
+    g.split_k = plan.split;
+    g.kb_per_split = (int)cdiv(k / KBLK, plan.split);
+    if (plan.split > 1) g.sk_nonce = next_nonce();
+    if (fp8bs::launch_gemm(plan.tile, plan.split > 1 ? 5 : 2, g, (hipStream_t)stream) != hipSuccess) return FP8BS_ERR_LAUNCH;
+    return FP8BS_OK;
+}
+
+size_t fp8bs_grouped_workspace_bytes(int num_experts, int total_rows, int n, int k) {
+    if (num_experts <= 0 || total_rows <= 0 || n <= 0 || k <= 0 || (k % KBLK) != 0) return 0;
+    return (size_t)grouped_bytes(choose_grouped(num_experts, total_rows, n, k, fp8bs::device_cus(), true), num_experts, total_rows, n);
+}
+
+size_t fp8bs_silu_mul_workspace_bytes(int rows, int n, int k) {
+    if (rows <= 0 || n <= 0 || k <= 0 || (k % KBLK) != 0) return 0;
+    fp8bs_plan_t p{};
+    choose(rows, n, k, fp8bs::device_cus(), &p, true, true);
+    return (size_t)p.workspace_bytes;
+}
+
 int fp8bs_gemm_grouped_ex(const void* a, const void* b, const float* a_scale, const float* b_scale,
                           void* c, const int32_t* row_offsets, int num_experts, int total_rows,
                           int n, int k, int variant, void* stream) {
-    if (num_experts <= 0) return FP8BS_ERR_BAD_OFFSETS;
-    if (!row_offsets) return FP8BS_ERR_NULL_POINTER;
-    int st = check_common(a, b, a_scale, b_scale, c, total_rows, n, k);
-    if (st != FP8BS_OK) return st;
-    if (total_rows == 0 || n == 0) return FP8BS_OK;
-    hipStream_t s = (hipStream_t)stream;
-    fp8bs::GemmArgs g{};
-    g.a = (const uint8_t*)a; g.b = (const uint8_t*)b; g.as = a_scale; g.bs = b_scale;
-    g.c = (uint16_t*)c; g.ws = nullptr; g.row_offsets = row_offsets;
-    g.m = total_rows; g.n = n; g.k = k; g.lda = total_rows; g.nb = (n + 127) / 128;
-    g.split_k = 1; g.kb_per_split = k / KBLK; g.band_h = 4; g.num_experts = num_experts;
-    g.by_expert = group_order(total_rows, num_experts);
-    if (variant == FP8BS_VARIANT_AUTO) {
-        // The 256x256 tile for every routing with more than 32 rows per expert on average: measured with 32
-        // experts of 8 .. 1024 rows each (even and random counts, n x k = 4096 x 7168 and 7168 x 2048) it is the
-        // fastest of the two-stage tiles throughout - the waves without rows only copy, and the widest tile moves
-        // the fewest bytes of a per byte of b.  With 32 rows or fewer per expert the call streams every expert's
-        // weights once and little else: the 64 x 256 tile with three stages keeps two K blocks of b in flight per
-        // workgroup (32 experts x 4096 x 7168: 1 / 8 / 32 rows each 165 / 167 / 173 us against 181 / 185 / 186;
-        // from 100 rows on an expert needs a second row of its tiles and the 256x256 tile wins).  Any n and any
-        // operand alignment (the instantiation that repairs every expert's last bytes of b).
-        variant = k == 0 ? FP8BS_VARIANT_GENERIC : ((long)total_rows <= 32L * num_experts ? FP8BS_VARIANT_T64x256S3 : FP8BS_VARIANT_T256x256);
-    } else {
-        VariantInfo vi{};
-        variant = forced_tile(variant);
-        if (!variant_info(variant, &vi) || is_streaming_variant(variant)) return FP8BS_ERR_BAD_VARIANT;   // no grouped mode in the streaming kernels
-        if (variant != FP8BS_VARIANT_GENERIC && k == 0) return FP8BS_ERR_BAD_VARIANT;
-    }
-    if (fp8bs::launch_gemm(variant, 2, g, s) != hipSuccess) return FP8BS_ERR_LAUNCH;
-    return FP8BS_OK;
+    return grouped_call(a, b, a_scale, b_scale, c, row_offsets, num_experts, total_rows, n, k, variant, 1, 0, nullptr, 0, stream);
+}
+
+int fp8bs_gemm_grouped_ws(const void* a, const void* b, const float* a_scale, const float* b_scale,
+                          void* c, const int32_t* row_offsets, int num_experts, int total_rows,
+                          int n, int k, int variant, int split_k, void* ws, size_t ws_bytes, void* stream) {
+    return grouped_call(a, b, a_scale, b_scale, c, row_offsets, num_experts, total_rows, n, k, variant, split_k, 0, ws, ws_bytes, stream);
 }
 
 int fp8bs_gemm_grouped(const void* a, const void* b, const float* a_scale, const float* b_scale,
@@ -487,24 +610,20 @@ int fp8bs_gemm_grouped(const void* a, const void* b, const float* a_scale, const
     return fp8bs_gemm_grouped_ex(a, b, a_scale, b_scale, c, row_offsets, num_experts, total_rows, n, k, FP8BS_VARIANT_AUTO, stream);
 }
 
+int fp8bs_gemm_silu_mul_ws(const void* a, const void* b, const float* a_scale, const float* b_scale, void* h,
+                           const int32_t* row_offsets, int num_experts, int rows, int n, int k,
+                           int variant, int split_k, void* ws, size_t ws_bytes, void* stream) {
+    if ((n & 1) != 0) return FP8BS_ERR_BAD_SHAPE;
+    if (split_k < 0) return FP8BS_ERR_BAD_VARIANT;               // K blocks are dealt without an epilogue only
+    // any even n and any operand alignment: rows of h that do not keep 16-byte stores aligned are stored in pieces
+    if (row_offsets)
+        return grouped_call(a, b, a_scale, b_scale, h, row_offsets, num_experts, rows, n, k, variant, split_k & ~FP8BS_SPLIT_SUM_IN_KERNEL, 1, ws, ws_bytes, stream);
+    return dense_call(a, b, a_scale, b_scale, h, ws, ws_bytes, rows, n, k, variant, split_k, 1, stream);
+}
+
 int fp8bs_gemm_silu_mul(const void* a, const void* b, const float* a_scale, const float* b_scale, void* h,
                         const int32_t* row_offsets, int num_experts, int rows, int n, int k, void* stream) {
-    if (row_offsets && num_experts <= 0) return FP8BS_ERR_BAD_OFFSETS;
-    if ((n & 1) != 0) return FP8BS_ERR_BAD_SHAPE;
-    int st = check_common(a, b, a_scale, b_scale, h, rows, n, k);
-    if (st != FP8BS_OK) return st;
-    if (rows == 0 || n == 0) return FP8BS_OK;
-    fp8bs::GemmArgs g{};
-    g.a = (const uint8_t*)a; g.b = (const uint8_t*)b; g.as = a_scale; g.bs = b_scale;
-    g.c = (uint16_t*)h; g.ws = nullptr; g.row_offsets = row_offsets;
-    g.m = rows; g.n = n; g.k = k; g.lda = rows; g.nb = (n + 127) / 128;
-    g.split_k = 1; g.kb_per_split = k / KBLK; g.band_h = 4; g.num_experts = row_offsets ? num_experts : 0;
-    g.epi = 1;
-    g.by_expert = row_offsets ? group_order(rows, num_experts) : 0;
-    // any even n and any operand alignment: rows of h that do not keep 16-byte stores aligned are stored in pieces
-    int variant = k == 0 ? FP8BS_VARIANT_GENERIC : FP8BS_VARIANT_T256x256;
-    if (fp8bs::launch_gemm(variant, row_offsets ? 2 : 0, g, (hipStream_t)stream) != hipSuccess) return FP8BS_ERR_LAUNCH;
-    return FP8BS_OK;
+    return fp8bs_gemm_silu_mul_ws(a, b, a_scale, b_scale, h, row_offsets, num_experts, rows, n, k, FP8BS_VARIANT_AUTO, 0, nullptr, 0, stream);
 }
 
 }  // extern "C"

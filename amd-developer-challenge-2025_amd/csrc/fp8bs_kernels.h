@@ -71,7 +71,11 @@ inline int device_cus() {
     return n;
 }
 
-// mode: 0 dense bf16, 1 dense split-K partials, 2 grouped.  tile: FP8BS_VARIANT_* (not AUTO) + 256 * form.
+// Upper bound on the m-tile slots of a grouped call of `rows` rows: an expert of r rows starts up to 15 rows into its first
+// tile and has ceil((r + 15) / bm) <= 1 + r / (bm - 14) of them, and no more experts have rows than there are rows.
+inline long grouped_slots_bound(long rows, long experts, int bm) { return (rows < experts ? rows : experts) + rows / (bm - 14); }
+
+// mode: 0 dense bf16, 1 dense split-K partials, 2 grouped, 3 K blocks dealt, 4 dense split-K summed in the kernel, 5 grouped likewise.  tile: FP8BS_VARIANT_* (not AUTO) + 256 * form.
 hipError_t launch_gemm(int tile, int mode, const GemmArgs& args, hipStream_t stream);
 // one per tile shape of the tiled kernel, each in a translation unit of its own
 hipError_t launch_tile_256x256(const GemmArgs& args, int mode, hipStream_t stream);
@@ -84,7 +88,7 @@ hipError_t launch_tile_64x128(const GemmArgs& args, int mode, hipStream_t stream
 hipError_t launch_tile_64x64(const GemmArgs& args, int mode, hipStream_t stream);
 hipError_t launch_tile_192x192s3(const GemmArgs& args, int mode, hipStream_t stream);
 hipError_t launch_tile_64x256s3(const GemmArgs& args, int mode, hipStream_t stream);
-hipError_t launch_splitk_reduce(const float* ws, uint16_t* c, size_t mn, int split_k, hipStream_t stream);
+hipError_t launch_splitk_reduce(const float* ws, uint16_t* c, size_t mn, int split_k, int epi, hipStream_t stream);
 int variant_lds_bytes(int tile);
 
 }  // namespace fp8bs

@@ -266,7 +266,8 @@ void gemm_skinny_kernel(const GemmArgs p) {
 // (with a run-time count the compiler keeps the loop and every plane's load waits for the previous plane's add: the
 // kernel then takes one memory latency per plane); SPLIT == 0: any count.  The sum is taken in ascending order of
 // the planes either way.
-template <bool VEC, int SPLIT>
+// EPI 1: the sums are (gate, up) pairs, every thread's 8 sums become 4 outputs (m*n is even).
+template <bool VEC, int SPLIT, int EPI>
 __global__ __launch_bounds__(256)
 void splitk_reduce_kernel(const float* __restrict__ ws, uint16_t* __restrict__ c, size_t mn, int split_k) {
     size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8;
@@ -291,16 +292,27 @@ void splitk_reduce_kernel(const float* __restrict__ ws, uint16_t* __restrict__ c
                 s1 += *(const v4f_any*)(ws + (size_t)z * mn + i + 4);
             }
         }
-        v4i o;
-        o[0] = (int)pack_bf16x2(s0[0], s0[1]); o[1] = (int)pack_bf16x2(s0[2], s0[3]);
-        o[2] = (int)pack_bf16x2(s1[0], s1[1]); o[3] = (int)pack_bf16x2(s1[2], s1[3]);
-        *(v4i*)(c + i) = o;
+        if constexpr (EPI == 1) {
+            const v2i o = {(int)pack_bf16x2(silu_mul(s0[0], s0[1]), silu_mul(s0[2], s0[3])), (int)pack_bf16x2(silu_mul(s1[0], s1[1]), silu_mul(s1[2], s1[3]))};
+            *(v2i*)(c + i / 2) = o;
+        } else {
+            v4i o;
+            o[0] = (int)pack_bf16x2(s0[0], s0[1]); o[1] = (int)pack_bf16x2(s0[2], s0[3]);
+            o[2] = (int)pack_bf16x2(s1[0], s1[1]); o[3] = (int)pack_bf16x2(s1[2], s1[3]);
+            *(v4i*)(c + i) = o;
+        }
     } else {
         const int cnt = mn - i < 8 ? (int)(mn - i) : 8;
+        float even = 0.f;
         for (int j = 0; j < cnt; j++) {
             float s = ws[i + j];
             for (int z = 1; z < split_k; z++) s += ws[(size_t)z * mn + i + j];
-            c[i + j] = (uint16_t)(pack_bf16x2(s, 0.f) & 0xFFFFu);
+            if constexpr (EPI == 1) {
+                if (j & 1) c[(i + j) / 2] = (uint16_t)(pack_bf16x2(silu_mul(even, s), 0.f) & 0xFFFFu);
+                else even = s;
+            } else {
+                c[i + j] = (uint16_t)(pack_bf16x2(s, 0.f) & 0xFFFFu);
+            }
         }
     }
 }
@@ -410,25 +422,26 @@ hipError_t launch_gemm(int tile, int mode, const GemmArgs& a, hipStream_t stream
     }
 }
 
-hipError_t launch_splitk_reduce(const float* ws, uint16_t* c, size_t mn, int split_k, hipStream_t stream) {
-    size_t threads = (mn + 7) / 8;
-    unsigned blocks = (unsigned)((threads + 255) / 256);
-    if (((uintptr_t)c & 15) == 0 && ((uintptr_t)ws & 3) == 0) {
-        void (*kern)(const float*, uint16_t*, size_t, int) = splitk_reduce_kernel<true, 0>;
-        switch (split_k) {
-            case 2: kern = splitk_reduce_kernel<true, 2>; break;
-            case 3: kern = splitk_reduce_kernel<true, 3>; break;
-            case 4: kern = splitk_reduce_kernel<true, 4>; break;
-            case 5: kern = splitk_reduce_kernel<true, 5>; break;
-            case 6: kern = splitk_reduce_kernel<true, 6>; break;
-            case 7: kern = splitk_reduce_kernel<true, 7>; break;
-            case 8: kern = splitk_reduce_kernel<true, 8>; break;
-            default: break;
-        }
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, stream, ws, c, mn, split_k);
-    } else {
-        hipLaunchKernelGGL((splitk_reduce_kernel<false, 0>), dim3(blocks), dim3(256), 0, stream, ws, c, mn, split_k);
+template <int EPI>
+static void (*splitk_reduce_for(bool vec, int split_k))(const float*, uint16_t*, size_t, int) {
+    if (!vec) return splitk_reduce_kernel<false, 0, EPI>;
+    switch (split_k) {
+        case 2: return splitk_reduce_kernel<true, 2, EPI>;
+        case 3: return splitk_reduce_kernel<true, 3, EPI>;
+        case 4: return splitk_reduce_kernel<true, 4, EPI>;
+        case 5: return splitk_reduce_kernel<true, 5, EPI>;
+        case 6: return splitk_reduce_kernel<true, 6, EPI>;
+        case 7: return splitk_reduce_kernel<true, 7, EPI>;
+        case 8: return splitk_reduce_kernel<true, 8, EPI>;
+        default: return splitk_reduce_kernel<true, 0, EPI>;
     }
+}
+
+hipError_t launch_splitk_reduce(const float* ws, uint16_t* c, size_t mn, int split_k, int epi, hipStream_t stream) {
+    const unsigned blocks = (unsigned)(((mn + 7) / 8 + 255) / 256);
+    const bool vec = ((uintptr_t)c & 15) == 0 && ((uintptr_t)ws & 3) == 0;
+    void (*kern)(const float*, uint16_t*, size_t, int) = epi == 1 ? splitk_reduce_for<1>(vec, split_k) : splitk_reduce_for<0>(vec, split_k);
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, stream, ws, c, mn, split_k);
     return hipGetLastError();
 }
 

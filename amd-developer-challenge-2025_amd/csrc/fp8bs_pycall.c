@@ -1,4 +1,4 @@
-/* CPython binding of the two GEMM entry points of libfp8bs.so (include/fp8bs.h), for callers that issue many
+/* CPython binding of the GEMM entry points of libfp8bs.so (include/fp8bs.h), for callers that issue many
  * small calls from Python: ctypes spends ~1.2 us marshalling the 13 arguments of fp8bs_gemm_ex, this module
  * ~0.15 us.  Pointers and the stream arrive as Python ints (tensor.data_ptr(), the raw hipStream_t) or None;
  * the status code is returned as an int.  Nothing else lives here: checks, planning and launches are the
@@ -55,9 +55,27 @@ static PyObject* py_gemm_grouped_ex(PyObject* self, PyObject* const* args, Py_ss
     return PyLong_FromLong(st);
 }
 
+/* gemm_grouped_ws / gemm_silu_mul_ws(a, b, a_scale, b_scale, c, row_offsets, num_experts, rows, n, k, variant, split_k, ws, ws_bytes, stream) -> status */
+typedef int (*grouped_fn)(const void*, const void*, const float*, const float*, void*, const int32_t*, int, int, int, int, int, int, void*, size_t, void*);
+static PyObject* call_grouped(grouped_fn fn, PyObject* const* args, Py_ssize_t nargs) {
+    if (nargs != 15) { PyErr_SetString(PyExc_TypeError, "15 arguments expected"); return NULL; }
+    void* p[6]; void* stream; void* ws; int v[6];
+    for (int i = 0; i < 6; i++) if (as_pointer(args[i], &p[i]) < 0) return NULL;
+    for (int i = 0; i < 6; i++) if (as_int(args[6 + i], &v[i]) < 0) return NULL;
+    if (as_pointer(args[12], &ws) < 0) return NULL;
+    size_t ws_bytes = PyLong_AsSize_t(args[13]);
+    if (ws_bytes == (size_t)-1 && PyErr_Occurred()) return NULL;
+    if (as_pointer(args[14], &stream) < 0) return NULL;
+    return PyLong_FromLong(fn(p[0], p[1], (const float*)p[2], (const float*)p[3], p[4], (const int32_t*)p[5], v[0], v[1], v[2], v[3], v[4], v[5], ws, ws_bytes, stream));
+}
+static PyObject* py_gemm_grouped_ws(PyObject* self, PyObject* const* args, Py_ssize_t nargs) { (void)self; return call_grouped(fp8bs_gemm_grouped_ws, args, nargs); }
+static PyObject* py_gemm_silu_mul_ws(PyObject* self, PyObject* const* args, Py_ssize_t nargs) { (void)self; return call_grouped(fp8bs_gemm_silu_mul_ws, args, nargs); }
+
 static PyMethodDef methods[] = {
     {"gemm_ex", (PyCFunction)(void (*)(void))py_gemm_ex, METH_FASTCALL, "fp8bs_gemm_ex with addresses as ints; returns the status code"},
     {"gemm_grouped_ex", (PyCFunction)(void (*)(void))py_gemm_grouped_ex, METH_FASTCALL, "fp8bs_gemm_grouped_ex with addresses as ints; returns the status code"},
+    {"gemm_grouped_ws", (PyCFunction)(void (*)(void))py_gemm_grouped_ws, METH_FASTCALL, "fp8bs_gemm_grouped_ws with addresses as ints; returns the status code"},
+    {"gemm_silu_mul_ws", (PyCFunction)(void (*)(void))py_gemm_silu_mul_ws, METH_FASTCALL, "fp8bs_gemm_silu_mul_ws with addresses as ints; returns the status code"},
     {NULL, NULL, 0, NULL},
 };
 

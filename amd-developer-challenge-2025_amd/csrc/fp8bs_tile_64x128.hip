@@ -6,6 +6,6 @@
 #include "fp8bs_tiled.h"
 
 namespace fp8bs {
-hipError_t launch_tile_64x128(const GemmArgs& a, int mode, hipStream_t stream) { return launch_shape<64, 128, 32, 32, false, 3>(a, mode, stream); }
-hipError_t launch_tile_64x64(const GemmArgs& a, int mode, hipStream_t stream) { return launch_shape<64, 64, 32, 32, false, 4>(a, mode, stream); }
+hipError_t launch_tile_64x128(const GemmArgs& a, int mode, hipStream_t stream) { return launch_shape<64, 128, 32, 32, true, 3>(a, mode, stream); }
+hipError_t launch_tile_64x64(const GemmArgs& a, int mode, hipStream_t stream) { return launch_shape<64, 64, 32, 32, true, 4, true>(a, mode, stream); }
 }  // namespace fp8bs

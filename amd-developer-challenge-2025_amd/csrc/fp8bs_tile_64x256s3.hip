@@ -7,6 +7,6 @@
 #include "fp8bs_tiled.h"
 
 namespace fp8bs {
-hipError_t launch_tile_64x256s3(const GemmArgs& a, int mode, hipStream_t stream) { return launch_shape<64, 256, 32, 64, false, 3>(a, mode, stream); }
-hipError_t launch_tile_128x128s4(const GemmArgs& a, int mode, hipStream_t stream) { return launch_shape<128, 128, 32, 64, false, 4>(a, mode, stream); }
+hipError_t launch_tile_64x256s3(const GemmArgs& a, int mode, hipStream_t stream) { return launch_shape<64, 256, 32, 64, true, 3, true>(a, mode, stream); }
+hipError_t launch_tile_128x128s4(const GemmArgs& a, int mode, hipStream_t stream) { return launch_shape<128, 128, 32, 64, true, 4, true>(a, mode, stream); }
 }  // namespace fp8bs

@@ -105,6 +105,7 @@ __device__ __forceinline__ void band_tile(int v, int tiles_m, int tiles_n, int g
 //   MODE 2  : grouped (row_offsets), bf16 output
 //   MODE 3  : dense, K blocks instead of tiles dealt to the workgroups, partial tiles through the workspace, bf16 output
 //   MODE 4  : dense split-K, partial tiles to the workspace, summed by the last workgroup to finish a tile, bf16 output
+//   MODE 5  : grouped like MODE 2 with a K split summed like MODE 4's
 // LDS: NSTAGE stages, each [128 k][BM] bytes of A then [128 k][BN] bytes of B, 16-byte chunks XOR-swizzled
 // so that the 16 k rows touched by half a wave in one transposing read fall on 16 different 16-byte
 // bank groups, then the k block's a_scale row and b_scale values.
@@ -233,6 +234,7 @@ template <int BM, int BN, int WM, int WN, int MODE, int EPI = 0, int NSTAGE = 2,
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) __attribute__((amdgpu_waves_per_eu(waves_per_simd<BM, BN, WM, WN, MODE, NSTAGE>())))
 void gemm_tr_kernel(const GemmArgs p) {
     using C = TileCfg<BM, BN, WM, WN, MODE, NSTAGE>;
+    constexpr bool GROUPED = MODE == 2 || MODE == 5, SUMMED = MODE == 4 || MODE == 5;
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
 
     // global store instructions per wave and tile in the bf16 epilogue (always this many: lanes without
@@ -240,7 +242,8 @@ void gemm_tr_kernel(const GemmArgs p) {
     constexpr int EPI_WNO = EPI == 1 ? WN / 2 : WN;
     constexpr int EPI_ROW_CHUNKS = EPI_WNO * 2 / 16;
     constexpr int EPI_ROWS_PER_PASS = (EPI_ROW_CHUNKS & (EPI_ROW_CHUNKS - 1)) == 0 ? 64 / EPI_ROW_CHUNKS : 4;
-    constexpr int EPI_PARTS = (WM / 16) % 2 == 0 ? 2 : WM / 16;       // the wave tile is staged in parts of whole m tiles
+    // the wave tile is staged in parts of whole m tiles, in one part where a pass of stores covers more rows than half of it
+    constexpr int EPI_PARTS = WM / 2 < EPI_ROWS_PER_PASS ? 1 : (WM / 16) % 2 == 0 ? 2 : WM / 16;
     constexpr int EPI_STORES = MODE == 1 ? 0 : EPI_PARTS * ((WM / EPI_PARTS) / EPI_ROWS_PER_PASS);
 
     const int tid = threadIdx.x;
@@ -272,7 +275,7 @@ void gemm_tr_kernel(const GemmArgs p) {
     // between the last K block of one tile and the first copies of the next.  More experts: that loop.
     [[maybe_unused]] v4i* gtable = nullptr;
     bool use_table = false;
-    if constexpr (MODE == 2) {
+    if constexpr (GROUPED) {
         __shared__ v4i gtable_store[GROUP_TABLE_MAX];        // entry [num_experts]: the slots before the end = all of them
         gtable = gtable_store;
         use_table = p.num_experts < GROUP_TABLE_MAX;
@@ -352,7 +355,7 @@ void gemm_tr_kernel(const GemmArgs p) {
             t.kb_end = __builtin_amdgcn_readfirstlane(kb1);
             t.sk_contrib = t.kb_end < (int)kbt;
             t.sk_first = __builtin_amdgcn_readfirstlane(first);
-        } else if (MODE == 2) {
+        } else if (GROUPED) {
             // grouped: m-tile slots are laid over the experts in order; expert e's tiles start at
             // row_offsets[e] rounded down to 16 so that global 16-byte loads stay aligned; rows outside
             // [row_offsets[e], row_offsets[e+1]) are computed but never stored.  The gridDim.x tiles in
@@ -364,8 +367,13 @@ void gemm_tr_kernel(const GemmArgs p) {
             // tiles that read the same panel of the expert's weights.
             const int tiles_n = (p.n + BN - 1) / BN;
             const int total = total_slots * tiles_n;
-            const int v = it * G + xcd_virtual_id(blockIdx.x, G);
-            if (v >= total) return t;
+            int v = it * G + xcd_virtual_id(blockIdx.x, G);
+            if (v >= total * (MODE == 5 ? p.split_k : 1)) return t;
+            if (MODE == 5) {                           // partition by partition; the tile's number: its counter and its slots
+                t.split_z = __builtin_amdgcn_readfirstlane(v / total);
+                v -= t.split_z * total;
+                t.sk_first = v;
+            }
             const bool by_expert = p.by_expert != 0;
             int slot_all = 0, tn = 0;
             if (!by_expert) band_tile(v, total_slots, tiles_n, p.band_h, slot_all, tn);
@@ -413,7 +421,9 @@ void gemm_tr_kernel(const GemmArgs p) {
             t.row_lo = cnt_lo; t.row_hi = cnt_hi;
             t.bptr = p.b + (size_t)e * (size_t)p.k * (size_t)p.n;
             t.bsptr = p.bs + (size_t)e * (size_t)(p.k / KBLK) * (size_t)p.nb;
-            t.kb_begin = 0; t.kb_end = p.k / KBLK;
+            const int kbt = p.k / KBLK;
+            t.kb_begin = MODE == 5 ? t.split_z * p.kb_per_split : 0;
+            t.kb_end = MODE == 5 && t.kb_begin + p.kb_per_split < kbt ? t.kb_begin + p.kb_per_split : kbt;
         } else {
             const int tiles_m = (p.m + BM - 1) / BM, tiles_n = (p.n + BN - 1) / BN;
             const int per_split = tiles_m * tiles_n, total = per_split * p.split_k;
@@ -625,7 +635,7 @@ void gemm_tr_kernel(const GemmArgs p) {
         bcand0 = tail_candidate(end - 3, (uint32_t)p.n, end, (uint32_t)p.k);
         bcand1 = tail_candidate(end - 2, (uint32_t)p.n, end, (uint32_t)p.k);
         bcand2 = tail_candidate(end - 1, (uint32_t)p.n, end, (uint32_t)p.k);
-        if (MODE != 2) b_last = load_last_dword(p.b + (end - 4));     // grouped: every expert's matrix has last bytes of its own, read per tile
+        if (!GROUPED) b_last = load_last_dword(p.b + (end - 4));     // grouped: every expert's matrix has last bytes of its own, read per tile
     }
     // (the loads are consumed here, not inside the K loop)
     acand0 = __builtin_amdgcn_readfirstlane(acand0); acand1 = __builtin_amdgcn_readfirstlane(acand1);
@@ -652,7 +662,7 @@ void gemm_tr_kernel(const GemmArgs p) {
     const int m0 = cur.m0, n0 = cur.n0, kb_begin = cur.kb_begin, kb_end = cur.kb_end, split_z = cur.split_z;
     const int row_lo = cur.row_lo, row_hi = cur.row_hi;
     [[maybe_unused]] const int sk_contrib = cur.sk_contrib, sk_first = cur.sk_first;
-    if constexpr (TAILS && MODE == 2) {
+    if constexpr (TAILS && GROUPED) {
         if (b_tail) b_last = __builtin_amdgcn_readfirstlane(load_last_dword(cur.bptr + ((uint32_t)p.k * (uint32_t)p.n - 4u)));
     }
     // a_scale: lane's output row of m-tile t is tile row wave_m*WM + 16t + i16, read from the stage's
@@ -928,7 +938,7 @@ void gemm_tr_kernel(const GemmArgs p) {
                 }
             }
         }
-    } else if constexpr (MODE == 4) {
+    } else if constexpr (SUMMED) {
         // K split in one launch, nobody waits: every workgroup leaves its partial tile in the slot
         // (tile, K partition) and then counts itself in at the tile's counter; the one that finds all others
         // counted in before it adds the partial tiles in ascending order of K - ((P0 + P1) + P2) + ..., its own
@@ -1245,6 +1255,7 @@ static inline hipError_t launch_tr(const GemmArgs& a, dim3 grid, hipStream_t str
     // without assuming any alignment of its rows
     // (with the fused epilogue the rows of the output have n/2 columns: 16-byte stores need n/2 on the 8-column grid)
     const int out_cols = EPI == 1 ? a.n / 2 : a.n;
+    // (MODE 1 writes planes of n columns, not c)
     const bool tails = (a.lda & 3) != 0 || (a.n & 7) != 0 || (out_cols & 7) != 0 || (((uintptr_t)a.a | (uintptr_t)a.b | (uintptr_t)a.c) & 15) != 0;
     GemmArgs args = a;
     args.c_whole_lines = ((size_t)out_cols * 2u) % 128u == 0 && ((uintptr_t)a.c & 127) == 0;
@@ -1256,19 +1267,19 @@ static inline hipError_t launch_tr(const GemmArgs& a, dim3 grid, hipStream_t str
     return hipGetLastError();
 }
 
-template <int BM, int BN, int WM, int WN, bool WITH_EPI = false, int NSTAGE = 2>
+// WITH_EPI: the fused silu-mul epilogue is instantiated for this tile; GROUPED_SPLIT: the grouped walk with a K split is
+template <int BM, int BN, int WM, int WN, bool WITH_EPI = false, int NSTAGE = 2, bool GROUPED_SPLIT = false>
 static inline hipError_t launch_shape(const GemmArgs& a, int mode, hipStream_t stream) {
     using C = TileCfg<BM, BN, WM, WN, 0, NSTAGE>;
     // persistent workgroups: as many as fit the chip at once (LDS and thread limits), each walks
     // tiles  blockIdx.x, blockIdx.x + grid, ...
-    const int by_lds = 163840 / (C::LDS_BYTES + (mode == 2 ? GROUP_TABLE_MAX * 16 : 0)), by_threads = 2048 / C::NTHREADS;   // (grouped: + the table of the experts)
+    const int by_lds = 163840 / (C::LDS_BYTES + (mode == 2 || mode == 5 ? GROUP_TABLE_MAX * 16 : 0)), by_threads = 2048 / C::NTHREADS;   // (grouped: + the table of the experts)
     const long resident = (long)device_cus() * (by_lds < by_threads ? by_lds : by_threads);
     const int tiles_n = (a.n + BN - 1) / BN;
     long total;
-    if (mode == 2) {
-        // upper bound on m-tile slots: every expert can waste up to 15 rows (aligned-down start)
-        // plus one partial tile; workgroups beyond the real count find no tile and leave
-        total = (((long)a.m + BM - 1) / BM + 2L * a.num_experts) * tiles_n;
+    if (mode == 2 || mode == 5) {
+        // upper bound on m-tile slots; workgroups beyond the real count find no tile and leave
+        total = grouped_slots_bound(a.m, a.num_experts, BM) * tiles_n * (mode == 5 ? a.split_k : 1);
     } else {
         total = (long)((a.m + BM - 1) / BM) * tiles_n * a.split_k;
     }
@@ -1281,16 +1292,28 @@ static inline hipError_t launch_shape(const GemmArgs& a, int mode, hipStream_t s
         return launch_tr<BM, BN, WM, WN, 3, 0, NSTAGE>(a, dim3((unsigned)a.sk_grid), stream);
     }
     const dim3 grid((unsigned)(total < resident ? total : resident));
+    if (mode == 5) {
+        if constexpr (GROUPED_SPLIT) {
+            const long tiles = total / a.split_k;
+            if (a.split_k < 2 || a.split_k > 0xFFFF || tiles > StreamK::MAX_GRID || (long)a.split_k * BM * BN * 4 >= (1L << 32)) return hipErrorInvalidValue;
+            if constexpr (WITH_EPI) { if (a.epi == 1) return launch_tr<BM, BN, WM, WN, 5, 1, NSTAGE>(a, grid, stream); }
+            return a.epi == 0 ? launch_tr<BM, BN, WM, WN, 5, 0, NSTAGE>(a, grid, stream) : hipErrorInvalidValue;
+        } else {
+            return hipErrorInvalidValue;
+        }
+    }
     if (mode == 4) {
         // K split summed by the last workgroup of every tile: one counter per tile in the workspace's head
         const long tiles = total / a.split_k;
-        if (a.epi != 0 || a.split_k < 2 || a.split_k > 0xFFFF || tiles > StreamK::MAX_GRID || (long)a.split_k * BM * BN * 4 >= (1L << 32)) return hipErrorInvalidValue;
-        return launch_tr<BM, BN, WM, WN, 4, 0, NSTAGE>(a, grid, stream);
+        if (a.split_k < 2 || a.split_k > 0xFFFF || tiles > StreamK::MAX_GRID || (long)a.split_k * BM * BN * 4 >= (1L << 32)) return hipErrorInvalidValue;
+        if constexpr (WITH_EPI) { if (a.epi == 1) return launch_tr<BM, BN, WM, WN, 4, 1, NSTAGE>(a, grid, stream); }
+        return a.epi == 0 ? launch_tr<BM, BN, WM, WN, 4, 0, NSTAGE>(a, grid, stream) : hipErrorInvalidValue;
     }
     if (a.epi != 0) {
-        // the fused silu-mul epilogue exists for the 256x256 tile, dense or grouped, without K split
+        // (with the reduce launch of a K split the planes are plain sums and the reduce kernel applies the epilogue)
         if constexpr (WITH_EPI) {
-            if (a.epi != 1 || mode == 1) return hipErrorInvalidValue;
+            if (a.epi != 1) return hipErrorInvalidValue;
+            if (mode == 1) return launch_tr<BM, BN, WM, WN, 1, 0, NSTAGE>(a, grid, stream);
             if (mode == 2) return launch_tr<BM, BN, WM, WN, 2, 1, NSTAGE>(a, grid, stream);
             return launch_tr<BM, BN, WM, WN, 0, 1, NSTAGE>(a, grid, stream);
         } else {

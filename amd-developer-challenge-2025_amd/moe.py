@@ -11,7 +11,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
-from .submission import _check_operands, _is_kmajor, _stream_ptr
+from .submission import _PLANS_MAX, _check_operands, _grouped_workspace, _is_kmajor, _plan_cache, _stream_ptr, _workspace
 
 
 _route_ws = {}     # (device index, stream) -> uint8 tensor: the routing kernels' scratch, grown on demand, reused across
@@ -109,9 +109,21 @@ def gate_up_silu(data):
     # dtypes, devices, shapes and K-major strides of a, a_scale and h ([rows, n/2]) as for the plain GEMM's c
     _check_operands(a, b, a_scale, b_scale, h, rows, n // 2, k)
     with torch.cuda.device(a.device):
-        _lib.check(_lib.load().fp8bs_gemm_silu_mul(
-            a.data_ptr(), b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(), h.data_ptr(),
-            row_offsets.data_ptr() if grouped else None, num_experts, rows, n, k, _stream_ptr(a.device)))
+        stream = _stream_ptr(a.device)
+        if grouped:
+            ws_ptr, ws_len = _grouped_workspace(a.device, stream, num_experts, rows, n, k)
+        else:
+            need = _plan_cache.get(("silu", rows, n, k))
+            if need is None:
+                if len(_plan_cache) >= _PLANS_MAX:
+                    _plan_cache.clear()
+                need = _plan_cache[("silu", rows, n, k)] = int(_lib.load().fp8bs_silu_mul_workspace_bytes(rows, n, k))
+            ws = _workspace(a.device, need, stream) if need else None
+            ws_ptr, ws_len = (ws.data_ptr(), ws.numel()) if need else (None, 0)
+        fast = _lib.pycall()
+        call = fast.gemm_silu_mul_ws if fast is not None else _lib.load().fp8bs_gemm_silu_mul_ws
+        _lib.check(call(a.data_ptr(), b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(), h.data_ptr(),
+                        row_offsets.data_ptr() if grouped else None, num_experts, rows, n, k, 0, 0, ws_ptr, ws_len, stream))
     return h
 
 

@@ -50,7 +50,8 @@ def _is_kmajor(t: torch.Tensor) -> bool:
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-_plan_cache = {}   # (m, n, k) -> workspace bytes the planner asks for
+_plan_cache = {}   # (m, n, k) and ("grouped", experts, rows, n, k) -> workspace bytes the planner asks for
+_PLANS_MAX = 4096
 
 # Operands that passed the checks once: a caller that hands over the same tensor objects again (a benchmark
 # loop, a layer called every step) skips the dtype / device / K-major checks, which cost more host time than a
@@ -74,19 +75,33 @@ def _gemm_ex_fn():
     return fast.gemm_ex if fast is not None else _lib.load().fp8bs_gemm_ex
 
 
-def _grouped_ex_fn():
+def _grouped_ws_fn():
     fast = _lib.pycall()
-    return fast.gemm_grouped_ex if fast is not None else _lib.load().fp8bs_gemm_grouped_ex
+    return fast.gemm_grouped_ws if fast is not None else _lib.load().fp8bs_gemm_grouped_ws
 
 
-_gemm_ex = _grouped_ex = None
+_gemm_ex = _grouped_ws = None
 
 
 def _bind():
     """Resolve the two call targets once (the CPython binding if built, else ctypes)."""
-    global _gemm_ex, _grouped_ex
-    _gemm_ex, _grouped_ex = _gemm_ex_fn(), _grouped_ex_fn()
-    return _gemm_ex, _grouped_ex
+    global _gemm_ex, _grouped_ws
+    _gemm_ex, _grouped_ws = _gemm_ex_fn(), _grouped_ws_fn()
+    return _gemm_ex, _grouped_ws
+
+
+def _grouped_workspace(device, stream, num_experts, rows, n, k):
+    """(address, bytes) of the workspace a grouped call can use, (None, 0) if it would not use any."""
+    key = ("grouped", num_experts, rows, n, k)
+    need = _plan_cache.get(key)
+    if need is None:
+        if len(_plan_cache) >= _PLANS_MAX:
+            _plan_cache.clear()
+        need = _plan_cache[key] = int(_lib.load().fp8bs_grouped_workspace_bytes(num_experts, rows, n, k))
+    if not need:
+        return None, 0
+    ws = _workspace(device, need, stream)
+    return ws.data_ptr(), ws.numel()
 
 
 def _stream_ptr(device: torch.device) -> int:
@@ -172,6 +187,8 @@ def custom_kernel(data, variant: int = 0, split_k: int = 0):
         need = _plan_cache.get((m, n, k))
         if need is None:
             need = workspace_bytes(m, n, k) if (m > 0 and n > 0 and k > 0) else 0
+            if len(_plan_cache) >= _PLANS_MAX:
+                _plan_cache.clear()
             _plan_cache[(m, n, k)] = need
         _remember(key, data, m, n, k, need, a.device.index)
     else:
@@ -205,7 +222,7 @@ def grouped_kernel(data, variant: int = 0):
     [E, ceil(n/128), k/128] with stride (nb*kb, 1, nb).  Fills and returns ``c``; no host sync.
     """
     a, b, a_scale, b_scale, row_offsets, c = data
-    grouped_ex = _grouped_ex or _bind()[1]
+    grouped_ws = _grouped_ws or _bind()[1]
     key = ("grouped", id(a), id(b), id(a_scale), id(b_scale), id(row_offsets), id(c))
     hit = _checked.get(key)
     if hit is not None:
@@ -213,7 +230,9 @@ def grouped_kernel(data, variant: int = 0):
         now = tuple(t.data_ptr() for t in data)
         if all(r() is t for r, t in zip(refs, data)) and now == ptrs and tuple(t.shape for t in data) == shapes \
                 and tuple(t.stride() for t in data) == strides and dev_index == torch.cuda.current_device():
-            st = grouped_ex(now[0], now[1], now[2], now[3], now[5], now[4], num_experts, rows, n, k, variant, _stream_ptr(a.device))
+            stream = _stream_ptr(a.device)
+            ws_ptr, ws_len = _grouped_workspace(a.device, stream, num_experts, rows, n, k) if variant == 0 else (None, 0)
+            st = grouped_ws(now[0], now[1], now[2], now[3], now[5], now[4], num_experts, rows, n, k, variant, 0, ws_ptr, ws_len, stream)
             if st:
                 _lib.check(st)
             return c
@@ -231,7 +250,9 @@ def grouped_kernel(data, variant: int = 0):
         raise ValueError("row_offsets must be an int32 tensor with num_experts+1 entries on the operands' GPU")
     _remember(key, data, rows, n, k, num_experts, a.device.index)
     with torch.cuda.device(a.device):
-        st = grouped_ex(a.data_ptr(), b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(),
-                        c.data_ptr(), row_offsets.data_ptr(), num_experts, rows, n, k, variant, _stream_ptr(a.device))
+        stream = _stream_ptr(a.device)
+        ws_ptr, ws_len = _grouped_workspace(a.device, stream, num_experts, rows, n, k) if variant == 0 else (None, 0)
+        st = grouped_ws(a.data_ptr(), b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(), c.data_ptr(), row_offsets.data_ptr(),
+                        num_experts, rows, n, k, variant, 0, ws_ptr, ws_len, stream)
     _lib.check(st)
     return c

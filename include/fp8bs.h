@@ -184,11 +184,24 @@ int fp8bs_gemm_grouped(const void* a, const void* b, const float* a_scale, const
 
 /* Same with the tile forced: one of the FP8BS_VARIANT_T* tiles or FP8BS_VARIANT_GENERIC (the streaming
  * variants have no grouped mode: FP8BS_ERR_BAD_VARIANT).  FP8BS_VARIANT_AUTO reproduces
- * fp8bs_gemm_grouped (the 256x256 tile, or the 64x256 three-stage tile when total_rows <= 32 * num_experts, for any n
- * and any operand alignment; the scalar kernel only for k = 0). */
+ * fp8bs_gemm_grouped (the tile that a cost model of the expected row counts picks, for any n and any operand alignment;
+ * the scalar kernel only for k = 0). */
 int fp8bs_gemm_grouped_ex(const void* a, const void* b, const float* a_scale, const float* b_scale,
                           void* c, const int32_t* row_offsets, int num_experts, int total_rows,
                           int n, int k, int variant, void* stream);
+
+/* The same with a workspace, which lets the library split K where the experts' tiles are few (one launch: partial tiles
+ * in the workspace, summed in ascending K by the last workgroup to finish a tile, as in fp8bs_gemm_ex with
+ * FP8BS_SPLIT_SUM_IN_KERNEL).  variant = FP8BS_VARIANT_AUTO and split_k = 0 let the library choose; without a workspace of
+ * fp8bs_grouped_workspace_bytes(...) bytes it chooses what needs none.  A forced split_k > 1 takes a tile that has the
+ * form (FP8BS_VARIANT_T64x256S3 in both forms, form 1 of FP8BS_VARIANT_T64x128; else FP8BS_ERR_BAD_VARIANT).  Contents of
+ * the workspace unspecified on entry, one call at a time per workspace. */
+int fp8bs_gemm_grouped_ws(const void* a, const void* b, const float* a_scale, const float* b_scale,
+                          void* c, const int32_t* row_offsets, int num_experts, int total_rows,
+                          int n, int k, int variant, int split_k, void* ws, size_t ws_bytes, void* stream);
+
+/* Bytes of workspace that a grouped call, plain or with the silu-mul epilogue, can use (0: it would not use any). */
+size_t fp8bs_grouped_workspace_bytes(int num_experts, int total_rows, int n, int k);
 
 /* ---- Quantisers (the step in front of the GEMM) -------------------------------------------------
  * The reference has no counterpart: its operands arrive already quantised from the harness
@@ -262,6 +275,14 @@ int fp8bs_moe_route(const int32_t* top_idx, int tokens, int experts, int topk, i
  * row_offsets NULL: dense (one weight matrix); else grouped as fp8bs_gemm_grouped. */
 int fp8bs_gemm_silu_mul(const void* a, const void* b, const float* a_scale, const float* b_scale, void* h,
                         const int32_t* row_offsets, int num_experts, int rows, int n, int k, void* stream);
+
+/* The same with a workspace for K splits (dense: fp8bs_silu_mul_workspace_bytes(rows, n, k) bytes, with row_offsets
+ * fp8bs_grouped_workspace_bytes(...); smaller or NULL: what needs none) and the tile and the split selectable
+ * (FP8BS_VARIANT_AUTO and 0 reproduce the library's choice; a tile without the epilogue: FP8BS_ERR_BAD_VARIANT). */
+int fp8bs_gemm_silu_mul_ws(const void* a, const void* b, const float* a_scale, const float* b_scale, void* h,
+                           const int32_t* row_offsets, int num_experts, int rows, int n, int k,
+                           int variant, int split_k, void* ws, size_t ws_bytes, void* stream);
+size_t fp8bs_silu_mul_workspace_bytes(int rows, int n, int k);
 
 /* Weighted un-permute: out[t][:] = sum_j weights[t][j] * y[slot_of[t][j]][:]  (y bf16 [rows][d], out bf16
  * [tokens][d], d % 8 == 0, y and out 16-byte aligned; fp32 accumulation in the order j = 0..topk-1, one rounding; a slot outside

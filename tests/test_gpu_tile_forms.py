@@ -59,6 +59,89 @@ def test_grouped(pkg, oracle, dev, tokens, n, k, experts, topk):
         assert ok, "tile %#x: %d elements outside the bar (max abs err %g)" % (tile, nbad, maxerr)
 
 
+def _grouped_ws(lib, data, variant, split, ws, silu_out=None):
+    a, b, sa, sb, ro, c = data
+    out = c if silu_out is None else silu_out
+    fn = lib.fp8bs_gemm_grouped_ws if silu_out is None else lib.fp8bs_gemm_silu_mul_ws
+    st = fn(a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), out.data_ptr(), ro.data_ptr(), b.shape[0], a.shape[0], b.shape[1], b.shape[2],
+            variant, split, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
+    assert st == 0, lib.fp8bs_strerror(st)
+    return out
+
+
+@pytest.mark.parametrize("tokens,n,k,experts,topk", [(1, 64, 256, 8, 2), (37, 200, 384, 5, 2), (150, 518, 640, 8, 3), (90, 300, 1152, 4, 4)])
+def test_grouped_k_split(pkg, oracle, dev, tokens, n, k, experts, topk):
+    """The grouped walk in K partitions, plain and with the silu-mul epilogue: every tile that has the form gives the same
+    bits (whatever the workspace holds), plain ones within the oracle's bar; replays of a captured launch start clean."""
+    lib = pkg._lib.load()
+    cpu = pkg.inputs.make_grouped(pkg.inputs.CONFIGS[4], tokens=tokens, n=n, k=k, experts=experts, topk=topk)
+    ref, data = oracle.ref_grouped(cpu), _to(cpu, dev)
+    ws = torch.randint(0, 256, (64 << 20,), dtype=torch.uint8, device=dev)
+    rows = data[0].shape[0]
+    for split in (2, 3, 7):
+        if split > k // 128:
+            continue
+        want = want_h = None
+        for tile in (12, FORM(12, 1), FORM(4, 1)):
+            what = "tile %#x split %d" % (tile, split)
+            out = _grouped_ws(lib, data[:5] + (torch.full_like(data[5], float("nan")),), tile, split, ws)
+            h = _grouped_ws(lib, data, tile, split, ws, torch.full((rows, n // 2), float("nan"), dtype=torch.bfloat16, device=dev))
+            ok, nbad, maxerr = oracle.within_tolerance(out, ref, RTOL, ATOL)
+            assert ok, "%s: %d elements outside the bar (max abs err %g)" % (what, nbad, maxerr)
+            # (the epilogue works on the unrounded sums: its own rounding, and the two bf16 roundings in this reference)
+            g = out.float()
+            href = torch.nn.functional.silu(g[:, 0::2]) * g[:, 1::2]
+            assert bool(((h.float() - href).abs() <= ATOL + 2 * RTOL * href.abs()).all()), what
+            assert want is None or torch.equal(out.view(torch.int16), want.view(torch.int16)), what
+            assert want_h is None or torch.equal(h.view(torch.int16), want_h.view(torch.int16)), what
+            want, want_h = out, h
+    graph = torch.cuda.CUDAGraph()
+    out = torch.empty_like(data[5])
+    _grouped_ws(lib, data[:5] + (out,), 12, 2, ws)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        _grouped_ws(lib, data[:5] + (out,), 12, 2, ws)
+    first = _grouped_ws(lib, data[:5] + (torch.empty_like(out),), 12, 2, ws)
+    for _ in range(3):
+        out.fill_(5.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), first.view(torch.int16))
+        pkg.grouped_kernel(data)
+        torch.cuda.synchronize()
+    need = ws.numel()
+    for tile, split in ((2, 2), (3, 2)):                              # tiles without the form
+        a, b, sa, sb, ro, c = data
+        assert lib.fp8bs_gemm_grouped_ws(a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), c.data_ptr(), ro.data_ptr(), experts, rows, n, k,
+                                         tile, split, ws.data_ptr(), need, None) == 7
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 2, 128), (65, 130, 384), (250, 512, 1024), (127, 262, 640), (64, 1030, 896), (300, 96, 512)])
+def test_dense_silu_mul_on_every_tile_and_split(pkg, dev, m, n, k):
+    """The epilogue on every tile that has it, unsplit, summed in the kernel and in the reduce kernel: the bits of the
+    256x256 tile's with the same K split."""
+    lib = pkg._lib.load()
+    flag = pkg._lib.SPLIT_SUM_IN_KERNEL
+    a, b, sa, sb, _ = _to(pkg.inputs.make_dense(pkg.inputs.CONFIGS[2], m=m, n=n, k=k), dev)
+    ws = torch.empty(64 << 20, dtype=torch.uint8, device=dev)
+
+    def run(tile, split):
+        h = torch.full((m, n // 2), float("nan"), dtype=torch.bfloat16, device=dev)
+        st = lib.fp8bs_gemm_silu_mul_ws(a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), h.data_ptr(), None, 0, m, n, k, tile, split,
+                                        ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
+        assert st == 0, lib.fp8bs_strerror(st)
+        return h
+    for split in (1, 2, 3, 5):
+        if split > k // 128:
+            continue
+        want = run(2, split)
+        for tile in (10, 4, FORM(4, 1), 12, FORM(12, 1)):
+            for form in (0, flag) if split > 1 else (0,):
+                assert torch.equal(run(tile, split | form).view(torch.int16), want.view(torch.int16)), "tile %#x split %#x" % (tile, split | form)
+    assert lib.fp8bs_gemm_silu_mul_ws(a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), a.data_ptr(), None, 0, m, n, k, 11, 1,
+                                      ws.data_ptr(), ws.numel(), None) == 7          # a tile without the epilogue
+
+
 def test_second_forms_are_named_and_planned(pkg, dev):
     """The plan says which form it takes, and a form that a variant does not have is refused."""
     assert (pkg.plan(512, 2048, 1024).variant, pkg.plan(512, 2048, 1024).form, pkg.plan(512, 2048, 1024).tile_n) == (4, 1, 64)
