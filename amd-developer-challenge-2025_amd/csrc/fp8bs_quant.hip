@@ -11,11 +11,14 @@
 // Rule, bit for bit: scale = max(max|x| / 448, 1e-12) in fp32, q = round-to-nearest-even e4m3fn of
 // clamp(x / scale, -448, 448) with a correctly rounded fp32 division.
 //
-// One workgroup = 128 rows x 128 k (one K block).  Every lane loads four k of four rows (16-byte
-// loads along k, 32 lanes cover a row's block), the per-row maxima are reduced across those 32 lanes,
-// the four rows' bytes are transposed 4x4 in registers (v_perm_b32) so that a dword holds four
-// consecutive rows of one k, and the tile is staged in LDS ([128 k][128 rows], rows padded to 132
-// bytes) so that the global stores are 16 bytes per lane, 128 contiguous bytes per k row.
+// One workgroup = 32, 64 or 128 rows x 128 k (one K block).  Every lane loads four k of four rows (8- or 16-byte
+// loads along k, 32 lanes cover a row's block), the per-row maxima are reduced across those 32 lanes with each lane of a
+// quad ending up with one of the four rows, whose scale and reciprocal it works out for the other three; the four rows'
+// bytes are transposed 4x4 in registers (v_perm_b32) so that a dword holds four consecutive rows of one k, and the tile is
+// staged in LDS ([128 k][rows], padded by 4 bytes) so that the global stores are 16 bytes per lane, on any byte.
+// Bound by HBM where the matrix is large (4096 x 7168 bf16: 19.9 us, 88 MB, 4.4 TB/s; a 1 GiB copy runs at 5.1), by the
+// vector ALU where the rows are gathered: about 9 instructions per value.  With the scale worked out by all 32 lanes of
+// a row, two remainder corrections for bf16, a clamp and a sign repair it took 18 (4096 -> 32768 x 7168: 116 us, now 88).
 // An optional row map gathers input rows (out row i = in row row_map[i]): the expert-contiguous
 // permutation of MoE tokens (2-amd-moe/3-amd-fp8-moe-hip-myhgemm.py:174-191 does it as a copy of its
 // own) then costs nothing extra.
@@ -42,7 +45,13 @@ struct QuantArgs {
     int nb;                   // per-block mode: ceil(rows/128)
 };
 
-static constexpr int TM = 128, TK = 128, LD = 132;   // LDS row pitch in bytes (33 dwords: spreads banks)
+static constexpr int TK = 128;
+
+// accesses on any byte
+typedef v4i v4i_any __attribute__((aligned(1)));
+typedef v2i v2i_any __attribute__((aligned(1)));
+typedef uint32_t u32_any __attribute__((aligned(1)));
+typedef uint16_t u16_any __attribute__((aligned(1)));
 
 __device__ __forceinline__ v4f cvt4(v4i r, const float*) { return __builtin_bit_cast(v4f, r); }
 __device__ __forceinline__ v4f cvt4(v2i r, const uint16_t*) {      // four bf16
@@ -61,41 +70,48 @@ __device__ __forceinline__ v4f load4(__amdgpu_buffer_rsrc_t rsrc, uint32_t byte_
     return cvt4(__builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rsrc, byte_off, 0, 0)), tag);
 }
 
-// max over the 32 lanes that share a row, on the bit patterns of |x|: for non-negative floats the
-// integer order is the float order, and every NaN pattern is above every number, so a NaN in the row
-// comes out as the maximum (torch.amax propagates NaN the same way).  Steps 1, 2 (quad permutes), 4, 8
-// (mirrors: all lanes of a reduced group already agree) are DPP modifiers, step 16 a swizzle.
 __device__ __forceinline__ uint32_t umax(uint32_t a, uint32_t b) { return a > b ? a : b; }
-__device__ __forceinline__ uint32_t rowmax32(uint32_t v) {
-    v = umax(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true));    // quad_perm [1,0,3,2]
-    v = umax(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true));    // quad_perm [2,3,0,1]
-    v = umax(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, true));   // row_half_mirror
-    v = umax(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x140, 0xF, 0xF, true));   // row_mirror
-    v = umax(v, (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, 0x401F));               // lane ^ 16
-    return v;
+template <int CTRL> __device__ __forceinline__ uint32_t dpp(uint32_t v) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true); }
+// Max over the 32 lanes that share four rows, m[r] being the lane's own of row r; every lane gets the one of row (lane & 3).
+// Steps 1 and 2 over a quad on all four rows, then 4, 8 (rotations by 4 and by 8, which keep lane & 3) and 16 on one.  On the bit
+// patterns of |x|: for non-negative floats the integer order is the float order, and every NaN pattern is above every number,
+// so a NaN in the row comes out as the maximum (torch.amax propagates NaN the same way).
+__device__ __forceinline__ uint32_t rowmax32(const uint32_t m[4], int lane) {
+    uint32_t q[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        q[r] = umax(m[r], dpp<0xB1>(m[r]));               // quad_perm [1,0,3,2]
+        q[r] = umax(q[r], dpp<0x4E>(q[r]));               // quad_perm [2,3,0,1]
+    }
+    const uint32_t lo = (lane & 1) ? q[1] : q[0], hi = (lane & 1) ? q[3] : q[2];
+    uint32_t v = (lane & 2) ? hi : lo;
+    v = umax(v, dpp<0x124>(v));                           // row_ror:4
+    v = umax(v, dpp<0x128>(v));                           // row_ror:8
+    return umax(v, (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, 0x401F));               // lane ^ 16
 }
 
 // Correctly rounded x / s for finite s >= 1e-12 and |x / s| < 2^96: the arithmetic of the IEEE
-// division sequence (reciprocal refined once, quotient corrected twice, all by fused multiply-add)
+// division sequence (reciprocal refined once, quotient corrected by its remainder, all by fused multiply-add)
 // without its range scaling, which only acts on quotients or operands at the ends of the exponent
 // range; there the result is a zero after conversion to e4m3fn either way.  `y` is refine_rcp(s).
+// STEPS corrections: two in general; one where x and the block's maximum are bf16 - 8-bit significands, for all
+// 128 x 128 of which it was checked to give the correctly rounded quotient, for the reciprocal rounded correctly and for its
+// neighbours on both sides (tests/test_quant_division.py).  The remainder is taken as s*q - x, so that -0 stays -0.
 __device__ __forceinline__ float refine_rcp(float s) {
     float y = __builtin_amdgcn_rcpf(s);
     float e = __builtin_fmaf(-s, y, 1.0f);
     return __builtin_fmaf(e, y, y);
 }
-__device__ __forceinline__ float div_by(float x, float s, float y) {
+template <int STEPS> __device__ __forceinline__ float div_by(float x, float s, float y) {
     float q = x * y;
-    float r = __builtin_fmaf(-s, q, x);
-    q = __builtin_fmaf(r, y, q);
-    r = __builtin_fmaf(-s, q, x);
-    q = __builtin_fmaf(r, y, q);
-    return __builtin_copysignf(q, x);          // keeps -0 (the residuals above turn it into +0)
+#pragma unroll
+    for (int i = 0; i < STEPS; i++) q = __builtin_fmaf(-__builtin_fmaf(s, q, -x), y, q);
+    return q;
 }
 // scale of a block from the bit pattern of its max |x|
 __device__ __forceinline__ float scale_of(uint32_t amax_bits) {
     const float amax = __builtin_bit_cast(float, amax_bits);
-    float s = div_by(amax, 448.f, refine_rcp(448.f));
+    float s = div_by<2>(amax, 448.f, refine_rcp(448.f));
     s = s < 1e-12f ? 1e-12f : s;
     return amax_bits >= 0x7F800000u ? amax : s;            // inf stays inf, NaN stays NaN
 }
@@ -112,28 +128,37 @@ __device__ __forceinline__ uint32_t cvt4_e4m3fn(v4f v) {
     return (uint32_t)w;
 }
 
+// bits of the largest |x| of the lane's four values, and those values widened
+__device__ __forceinline__ uint32_t absmax4(v4f x) {
+    const v4i b = __builtin_bit_cast(v4i, x) & 0x7FFFFFFF;
+    return umax(umax((uint32_t)b[0], (uint32_t)b[1]), umax((uint32_t)b[2], (uint32_t)b[3]));
+}
+
 // PER_BLOCK false: one scale per row and K block (activations); true: one per 128x128 block (weights)
-template <typename T, bool PER_BLOCK, bool HAS_MAP>
+// ROWS: rows of a workgroup, a multiple of 32 (PER_BLOCK: 128)
+template <typename T, bool PER_BLOCK, bool HAS_MAP, int ROWS>
 __global__ __launch_bounds__(256)
 void quantize_kernel(const QuantArgs p) {
+    constexpr int ITERS = ROWS / 32, LD = ROWS + 4;      // LDS row pitch in bytes (an odd number of dwords: spreads banks)
+    static_assert(!PER_BLOCK || ROWS == 128, "a block's maximum is taken over one workgroup");
     __shared__ __attribute__((aligned(16))) unsigned char tile[TK * LD];
-    __shared__ float row_scale[TM];
+    __shared__ float row_scale[ROWS];
     __shared__ uint32_t wave_max[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int g = lane >> 5, l = lane & 31;
-    const int kb = blockIdx.x, m0 = blockIdx.y * TM;
+    const int kb = blockIdx.x, m0 = blockIdx.y * ROWS;
     __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
         (void*)p.x, 0, (uint32_t)((size_t)p.src_rows * (size_t)p.ldx * sizeof(T)), 0x00020000);
 
     // ---- load: iteration it, row group rg = it*8 + wave*2 + g holds rows 4rg .. 4rg+3 ----
-    v4f v[4][4];
-    uint32_t rmax[4][4];
+    v4f v[ITERS][4];
+    uint32_t rmax[ITERS];                     // of row 4rg + (lane & 3)
     const uint32_t col_off = (uint32_t)((kb * TK + 4 * l) * sizeof(T));
     const uint32_t row_pitch = (uint32_t)(p.ldx * sizeof(T));
-    int src[4][4];
+    int src[ITERS][4];
     // all row-map entries first, then all data loads: neither waits for the other one by one
 #pragma unroll
-    for (int it = 0; it < 4; it++)
+    for (int it = 0; it < ITERS; it++)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int row = m0 + 4 * (it * 8 + wave * 2 + g) + r;
@@ -141,7 +166,7 @@ void quantize_kernel(const QuantArgs p) {
             else src[it][r] = row;
         }
 #pragma unroll
-    for (int it = 0; it < 4; it++)
+    for (int it = 0; it < ITERS; it++)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int row = m0 + 4 * (it * 8 + wave * 2 + g) + r;
@@ -151,19 +176,17 @@ void quantize_kernel(const QuantArgs p) {
         }
     // ---- per-row max |x| ----
 #pragma unroll
-    for (int it = 0; it < 4; it++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const v4i b = __builtin_bit_cast(v4i, v[it][r]) & 0x7FFFFFFF;
-            rmax[it][r] = rowmax32(umax(umax((uint32_t)b[0], (uint32_t)b[1]), umax((uint32_t)b[2], (uint32_t)b[3])));
-        }
+    for (int it = 0; it < ITERS; it++) {
+        const uint32_t m[4] = {absmax4(v[it][0]), absmax4(v[it][1]), absmax4(v[it][2]), absmax4(v[it][3])};
+        rmax[it] = rowmax32(m, lane);
+    }
     float bscale = 0.f;
     if (PER_BLOCK) {
-        uint32_t mx = 0;
+        uint32_t mx = rmax[0];
 #pragma unroll
-        for (int it = 0; it < 4; it++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) mx = umax(mx, rmax[it][r]);
+        for (int it = 1; it < ITERS; it++) mx = umax(mx, rmax[it]);
+        mx = umax(mx, dpp<0xB1>(mx));
+        mx = umax(mx, dpp<0x4E>(mx));
         mx = umax(mx, (uint32_t)__shfl_xor((int)mx, 32, 64));
         if (lane == 0) wave_max[wave] = mx;
         __syncthreads();
@@ -173,29 +196,38 @@ void quantize_kernel(const QuantArgs p) {
     // ---- quantise, transpose 4x4 bytes, stage in LDS ----
     const float bscale_rcp = refine_rcp(bscale);
 #pragma unroll
-    for (int it = 0; it < 4; it++) {
+    for (int it = 0; it < ITERS; it++) {
         const int rg = it * 8 + wave * 2 + g;
         uint32_t rw[4];
+        // the lane's own row (lane & 3): its scale and reciprocal are worked out once and passed around the quad
+        const float own = PER_BLOCK ? bscale : scale_of(rmax[it]);
+        const float own_rcp = PER_BLOCK ? bscale_rcp : refine_rcp(own);
+        if (!PER_BLOCK && l < 4) row_scale[4 * rg + l] = own;
+        const bool special = __builtin_amdgcn_ballot_w64(__builtin_bit_cast(uint32_t, own) >= 0x7F800000u) != 0;
+        auto row_of = [&](float x, int r) -> float {
+            const uint32_t u = __builtin_bit_cast(uint32_t, x);
+            return __builtin_bit_cast(float, PER_BLOCK ? u : r == 0 ? dpp<0x00>(u) : r == 1 ? dpp<0x55>(u) : r == 2 ? dpp<0xAA>(u) : dpp<0xFF>(u));
+        };
+        if (__builtin_expect(special, 0)) {
+            // an inf or NaN in some row: the plain division has the IEEE special cases
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            float s, y;
-            if (PER_BLOCK) { s = bscale; y = bscale_rcp; }
-            else {
-                s = scale_of(rmax[it][r]);
-                y = refine_rcp(s);
-                if (l == 0) row_scale[4 * rg + r] = s;
+            for (int r = 0; r < 4; r++) {
+                const float s = row_of(own, r);
+                v4f qf;
+#pragma unroll
+                for (int j = 0; j < 4; j++) qf[j] = clamp448(v[it][r][j] / s);
+                rw[r] = cvt4_e4m3fn(qf);
             }
-            const v4f a = v[it][r];
-            v4f qf;
-            if (__builtin_expect(__builtin_bit_cast(uint32_t, s) >= 0x7F800000u, 0)) {
-                // an inf or NaN in the block: the plain division has the IEEE special cases
+        } else {
+            // no clamp: |x| <= max |x| <= 448 s (1 + 2^-24), and the quotient one step above 448 that this allows rounds to 448
 #pragma unroll
-                for (int j = 0; j < 4; j++) qf[j] = clamp448(a[j] / s);
-            } else {
+            for (int r = 0; r < 4; r++) {
+                const float s = row_of(own, r), y = row_of(own_rcp, r);
+                v4f qf;
 #pragma unroll
-                for (int j = 0; j < 4; j++) qf[j] = __builtin_amdgcn_fmed3f(div_by(a[j], s, y), -448.f, 448.f);
+                for (int j = 0; j < 4; j++) qf[j] = div_by<sizeof(T) == 2 ? 1 : 2>(v[it][r][j], s, y);
+                rw[r] = cvt4_e4m3fn(qf);
             }
-            rw[r] = cvt4_e4m3fn(qf);
         }
         // rw[r] = bytes (k0..k3) of row r  ->  c[j] = bytes (row0..row3) of k j
         const uint32_t lo01 = __builtin_amdgcn_perm(rw[1], rw[0], 0x05010400u), hi01 = __builtin_amdgcn_perm(rw[1], rw[0], 0x07030602u);
@@ -209,34 +241,59 @@ void quantize_kernel(const QuantArgs p) {
         *(uint32_t*)(t + 3 * LD) = c3;
     }
     __syncthreads();
-    // ---- scales of the 128 rows: 512 contiguous bytes ----
-    if (!PER_BLOCK && tid < TM && m0 + tid < p.rows) p.scale[(size_t)kb * p.rows + m0 + tid] = row_scale[tid];
-    // ---- store: 1024 chunks of 16 rows x 1 k, 4 per thread; 8 consecutive lanes write one k row ----
-    const bool wide = (p.rows & 15) == 0;
+    // ---- scales of the rows, contiguous ----
+    if (!PER_BLOCK && tid < ROWS && m0 + tid < p.rows) p.scale[(size_t)kb * p.rows + m0 + tid] = row_scale[tid];
+    // ---- store: chunks of 16 rows x 1 k; ROWS/16 consecutive lanes write one k row ----
+    // k rows start on any byte where rows is not a multiple of 16: 16-byte stores take that, and the chunk that holds
+    // the last rows leaves in pieces of 8, 4, 2 and 1 bytes (4095 x 7168 bf16: 21.5 us, byte by byte 63.9; 4096 rows 19.9).
+    constexpr int CHUNKS = ROWS / 16;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < TK * CHUNKS / 256; i++) {
         const int id = i * 256 + tid;
-        const int krow = id >> 3, c = id & 7;
+        const int krow = id / CHUNKS, c = id % CHUNKS;
         const unsigned char* s = tile + krow * LD + 16 * c;
         const int row = m0 + 16 * c;
         if (row >= p.rows) continue;
         uint8_t* dst = p.q + ((size_t)kb * TK + krow) * (size_t)p.rows + row;
-        const uint32_t w0 = *(const uint32_t*)s, w1 = *(const uint32_t*)(s + 4), w2 = *(const uint32_t*)(s + 8), w3 = *(const uint32_t*)(s + 12);
-        if (wide) {
-            *(v4i*)dst = (v4i){(int)w0, (int)w1, (int)w2, (int)w3};
+        const uint32_t w[4] = {*(const uint32_t*)s, *(const uint32_t*)(s + 4), *(const uint32_t*)(s + 8), *(const uint32_t*)(s + 12)};
+        const int left = p.rows - row;
+        if (left >= 16) {
+            *(v4i_any*)dst = (v4i){(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
         } else {
-            const uint32_t w[4] = {w0, w1, w2, w3};
-            for (int b = 0; b < 16 && row + b < p.rows; b++) dst[b] = (uint8_t)(w[b >> 2] >> (8 * (b & 3)));
+            if (left & 8) *(v2i_any*)dst = (v2i){(int)w[0], (int)w[1]};
+            const uint32_t w4 = (left & 8) ? w[2] : w[0], w2 = (left & 4) ? ((left & 8) ? w[3] : w[1]) : w4;
+            if (left & 4) *(u32_any*)(dst + (left & 8)) = w4;
+            if (left & 2) *(u16_any*)(dst + (left & 12)) = (uint16_t)w2;
+            if (left & 1) dst[left & 14] = (uint8_t)((left & 2) ? w2 >> 16 : w2);
         }
     }
 }
 
+template <typename T, bool PER_BLOCK, int ROWS>
+static hipError_t launch_quant_rows(const QuantArgs& a, hipStream_t stream) {
+    dim3 grid((unsigned)(a.k / TK), (unsigned)((a.rows + ROWS - 1) / ROWS));
+    if (a.row_map) hipLaunchKernelGGL((quantize_kernel<T, PER_BLOCK, true, ROWS>), grid, dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL((quantize_kernel<T, PER_BLOCK, false, ROWS>), grid, dim3(256), 0, stream, a);
+    return hipGetLastError();
+}
+
+// Rows of a workgroup, us measured with 128 / 64 / 32 of them (bf16, inputs from HBM): few values finish soonest in small
+// workgroups, many of them short chains (64 x 7168 5.2 / 2.8 / 2.4, 4004 x 1024 5.2 / 5.0 / 4.5, 16384 x 512 7.3 / 6.7 / 8.1);
+// large matrices want 128 bytes per k row in one store (4096 x 7168 19.9 / 20.6 / 22.5, 32768 x 2048 41.9 / 43.5 / 44.3; fp32,
+// whose loads weigh more, 32.5 / 32.0 / 33.4 and 66.0 / 64.0 / 61.4).  Gathered rows come from the caches and are bound by the
+// vector ALU: 2000 -> 4000 x 7168 14.0 / 13.5 / 13.2, 4096 -> 32768 x 7168 88 / 99 / 132, and with rows of the output that do not
+// start on 16 bytes, 4095 -> 32760, 116 / 115 / 100.
 template <typename T, bool PER_BLOCK>
 static hipError_t launch_quant(const QuantArgs& a, hipStream_t stream) {
-    dim3 grid((unsigned)(a.k / TK), (unsigned)((a.rows + TM - 1) / TM));
-    if (a.row_map) hipLaunchKernelGGL((quantize_kernel<T, PER_BLOCK, true>), grid, dim3(256), 0, stream, a);
-    else hipLaunchKernelGGL((quantize_kernel<T, PER_BLOCK, false>), grid, dim3(256), 0, stream, a);
-    return hipGetLastError();
+    if constexpr (PER_BLOCK) {
+        return launch_quant_rows<T, true, 128>(a, stream);
+    } else {
+        const size_t values = (size_t)a.rows * (size_t)a.k;
+        const bool large = values >= (24u << 20);
+        if (a.row_map) return large && (a.rows & 15) == 0 ? launch_quant_rows<T, false, 128>(a, stream) : launch_quant_rows<T, false, 32>(a, stream);
+        if (large && sizeof(T) == 2) return launch_quant_rows<T, false, 128>(a, stream);
+        return values >= (6u << 20) ? launch_quant_rows<T, false, 64>(a, stream) : launch_quant_rows<T, false, 32>(a, stream);
+    }
 }
 
 // e4m3fnuz (gfx942: bias 8, max 240, NaN = 0x80, no -0) -> e4m3fn (bias 7) with the same value.
