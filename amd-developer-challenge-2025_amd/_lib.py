@@ -5,6 +5,7 @@ loudly, so a GPU run can never silently take another path.
 """
 import ctypes
 import os
+import types
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libfp8bs.so")
@@ -110,7 +111,7 @@ _pycall = False
 
 
 def pycall():
-    """The CPython binding of fp8bs_gemm_ex / fp8bs_gemm_grouped_ex (csrc/fp8bs_pycall.c: the same library
+    """The CPython binding of the compute entry points (csrc/fp8bs_pycall.c: the same library
     functions without ctypes' per-argument marshalling), or None where it has not been built or cannot be
     imported (one warning); callers then use the ctypes functions of load().  Either way the work is done by libfp8bs.so, which has no substitute."""
     global _pycall
@@ -131,6 +132,23 @@ def pycall():
                 import warnings
                 warnings.warn("_fp8bs_pycall.so cannot be imported (%s); binding libfp8bs.so through ctypes instead" % ex)
     return _pycall
+
+
+_CALLS = ("gemm_ex", "gemm_grouped_ws", "gemm_silu_mul_ws", "quantize_a", "quantize_b", "gather_a", "moe_topk", "moe_route", "moe_combine")
+_calls = None
+
+
+def calls():
+    """The compute entry points by name without their prefix (calls().gemm_ex(...) -> status): the CPython binding
+    where it is built, else the library's functions through ctypes."""
+    global _calls
+    if _calls is None:
+        mod = pycall()
+        if mod is None or any(not hasattr(mod, name) for name in _CALLS):
+            lib = load()
+            mod = types.SimpleNamespace(**{name: getattr(lib, "fp8bs_" + name) for name in _CALLS})
+        _calls = mod
+    return _calls
 
 
 def check(status: int) -> None:

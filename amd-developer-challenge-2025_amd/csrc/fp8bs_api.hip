@@ -244,11 +244,37 @@ void choose_skinny(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may
     fill_plan(m, n, k, FP8BS_VARIANT_T64x256S3, best_s, out, 0, best_fused);
 }
 
+// What the planners below return for a shape is kept, 64 shapes a thread: the cost models take 0.4-0.8 us of host time
+// (all tiles and splits), in a call whose launch takes 3.  Every argument is in the key, so an entry never goes stale.
+template <typename P>
+struct PlanMemo {
+    struct Entry { int key[6]; P plan; };
+    Entry entries[64] = {};                   // no key is all zeros: experts or CUs are at least 1
+    template <typename F>
+    const P& get(const int (&key)[6], F&& make) {
+        uint32_t h = 0;
+        for (int v : key) h = (h ^ (uint32_t)v) * 0x9E3779B1u;
+        Entry& e = entries[h >> 26];
+        bool same = true;
+        for (int i = 0; i < 6; i++) same &= e.key[i] == key[i];
+        if (!same) {
+            make(&e.plan);
+            for (int i = 0; i < 6; i++) e.key[i] = key[i];
+        }
+        return e.plan;
+    }
+};
+
 // Shape-family rule.  A few rows against a large b -> the 64 x 256 three-stage tile.  Everything else -> the
 // tile and K split that the cost model of the tiled kernel picks.
 void choose(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_split = true, bool epi = false) {
-    if (skinny_shape(m, n, k)) choose_skinny(m, n, k, num_cus, out, may_split);
-    else choose_tiled(m, n, k, num_cus, out, may_split, epi);
+    static thread_local PlanMemo<fp8bs_plan_t> memo;
+    if (num_cus <= 0) num_cus = 256;
+    *out = memo.get({m, n, k, num_cus, may_split, epi}, [&](fp8bs_plan_t* plan) {
+        *plan = {};
+        if (skinny_shape(m, n, k)) choose_skinny(m, n, k, num_cus, plan, may_split);
+        else choose_tiled(m, n, k, num_cus, plan, may_split, epi);
+    });
 }
 
 // Order of the tiles of a grouped call (the row counts themselves are on the device).  With a tile or more of
@@ -284,8 +310,7 @@ bool can_split_grouped(const GroupedPlan& p, int experts, int rows, int n, int k
 // costs 2.2 % against the best of each shape in the geometric mean and takes 17 % off the rule it replaced (the 256x256
 // tile above 32 rows per expert on average, 64x256 below): 194 tokens to 4 of 16 experts, 1299 x 5760: 90.8 -> 49.2 us;
 // 801 to 4 of 8, 840 x 1664: 23.2 -> 15.0; 35 to 4 of 8, 1375 x 5504: 43.6 -> 22.8.
-GroupedPlan choose_grouped(int experts, int rows, int n, int k, int num_cus, bool may_split) {
-    if (num_cus <= 0) num_cus = 256;
+GroupedPlan make_grouped_plan(int experts, int rows, int n, int k, int num_cus, bool may_split) {
     struct Cand { int tile; int rmax; double t_full, t_few, t_power, t_fixed, shared, bw; };
     const Cand cands[5] = {
         {FP8BS_VARIANT_T256x256, 1, 2.010, 1.259, 1.681, 6.01, 1.0, 5.18},
@@ -327,6 +352,11 @@ GroupedPlan choose_grouped(int experts, int rows, int n, int k, int num_cus, boo
         }
     }
     return best;
+}
+GroupedPlan choose_grouped(int experts, int rows, int n, int k, int num_cus, bool may_split) {
+    static thread_local PlanMemo<GroupedPlan> memo;
+    if (num_cus <= 0) num_cus = 256;
+    return memo.get({experts, rows, n, k, num_cus, may_split}, [&](GroupedPlan* plan) { *plan = make_grouped_plan(experts, rows, n, k, num_cus, may_split); });
 }
 
 // The value a flag takes in one call that deals K blocks: never zero, different from call to call (and, through

@@ -1,4 +1,4 @@
-/* CPython binding of the GEMM entry points of libfp8bs.so (include/fp8bs.h), for callers that issue many
+/* CPython binding of the compute entry points of libfp8bs.so (include/fp8bs.h), for callers that issue many
  * small calls from Python: ctypes spends ~1.2 us marshalling the 13 arguments of fp8bs_gemm_ex, this module
  * ~0.15 us.  Pointers and the stream arrive as Python ints (tensor.data_ptr(), the raw hipStream_t) or None;
  * the status code is returned as an int.  Nothing else lives here: checks, planning and launches are the
@@ -71,11 +71,68 @@ static PyObject* call_grouped(grouped_fn fn, PyObject* const* args, Py_ssize_t n
 static PyObject* py_gemm_grouped_ws(PyObject* self, PyObject* const* args, Py_ssize_t nargs) { (void)self; return call_grouped(fp8bs_gemm_grouped_ws, args, nargs); }
 static PyObject* py_gemm_silu_mul_ws(PyObject* self, PyObject* const* args, Py_ssize_t nargs) { (void)self; return call_grouped(fp8bs_gemm_silu_mul_ws, args, nargs); }
 
+/* The quantisers and the routing kernels: arguments as `format` says, 'p' an address or None, 'i' an int, 'l' an int64, 'z' a size_t */
+typedef union { void* p; int i; int64_t l; size_t z; } arg;
+static int unpack(PyObject* const* args, Py_ssize_t nargs, const char* format, arg* out) {
+    Py_ssize_t n = 0;
+    for (; format[n]; n++) {
+        if (n >= nargs) break;
+        if (format[n] == 'p') { if (as_pointer(args[n], &out[n].p) < 0) return -1; }
+        else if (format[n] == 'i') { if (as_int(args[n], &out[n].i) < 0) return -1; }
+        else if (format[n] == 'l') { out[n].l = PyLong_AsLongLong(args[n]); if (out[n].l == -1 && PyErr_Occurred()) return -1; }
+        else { out[n].z = PyLong_AsSize_t(args[n]); if (out[n].z == (size_t)-1 && PyErr_Occurred()) return -1; }
+    }
+    if (format[n] || n != nargs) { PyErr_SetString(PyExc_TypeError, "wrong number of arguments"); return -1; }
+    return 0;
+}
+static PyObject* py_quantize_a(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+    (void)self;
+    arg v[10];
+    if (unpack(args, nargs, "pilpippiip", v) < 0) return NULL;
+    return PyLong_FromLong(fp8bs_quantize_a(v[0].p, v[1].i, v[2].l, (const int32_t*)v[3].p, v[4].i, v[5].p, (float*)v[6].p, v[7].i, v[8].i, v[9].p));
+}
+static PyObject* py_quantize_b(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+    (void)self;
+    arg v[8];
+    if (unpack(args, nargs, "pilppiip", v) < 0) return NULL;
+    return PyLong_FromLong(fp8bs_quantize_b(v[0].p, v[1].i, v[2].l, v[3].p, (float*)v[4].p, v[5].i, v[6].i, v[7].p));
+}
+static PyObject* py_gather_a(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+    (void)self;
+    arg v[9];
+    if (unpack(args, nargs, "ppipppiip", v) < 0) return NULL;
+    return PyLong_FromLong(fp8bs_gather_a(v[0].p, (const float*)v[1].p, v[2].i, (const int32_t*)v[3].p, v[4].p, (float*)v[5].p, v[6].i, v[7].i, v[8].p));
+}
+static PyObject* py_moe_topk(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+    (void)self;
+    arg v[6];
+    if (unpack(args, nargs, "piiipp", v) < 0) return NULL;
+    return PyLong_FromLong(fp8bs_moe_topk((const float*)v[0].p, v[1].i, v[2].i, v[3].i, (int32_t*)v[4].p, v[5].p));
+}
+static PyObject* py_moe_route(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+    (void)self;
+    arg v[10];
+    if (unpack(args, nargs, "piiippppzp", v) < 0) return NULL;
+    return PyLong_FromLong(fp8bs_moe_route((const int32_t*)v[0].p, v[1].i, v[2].i, v[3].i, (int32_t*)v[4].p, (int32_t*)v[5].p, (int32_t*)v[6].p, v[7].p, v[8].z, v[9].p));
+}
+static PyObject* py_moe_combine(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+    (void)self;
+    arg v[9];
+    if (unpack(args, nargs, "pipppiiip", v) < 0) return NULL;
+    return PyLong_FromLong(fp8bs_moe_combine(v[0].p, v[1].i, (const int32_t*)v[2].p, (const float*)v[3].p, v[4].p, v[5].i, v[6].i, v[7].i, v[8].p));
+}
+
 static PyMethodDef methods[] = {
     {"gemm_ex", (PyCFunction)(void (*)(void))py_gemm_ex, METH_FASTCALL, "fp8bs_gemm_ex with addresses as ints; returns the status code"},
     {"gemm_grouped_ex", (PyCFunction)(void (*)(void))py_gemm_grouped_ex, METH_FASTCALL, "fp8bs_gemm_grouped_ex with addresses as ints; returns the status code"},
     {"gemm_grouped_ws", (PyCFunction)(void (*)(void))py_gemm_grouped_ws, METH_FASTCALL, "fp8bs_gemm_grouped_ws with addresses as ints; returns the status code"},
     {"gemm_silu_mul_ws", (PyCFunction)(void (*)(void))py_gemm_silu_mul_ws, METH_FASTCALL, "fp8bs_gemm_silu_mul_ws with addresses as ints; returns the status code"},
+    {"quantize_a", (PyCFunction)(void (*)(void))py_quantize_a, METH_FASTCALL, "fp8bs_quantize_a with addresses as ints; returns the status code"},
+    {"quantize_b", (PyCFunction)(void (*)(void))py_quantize_b, METH_FASTCALL, "fp8bs_quantize_b with addresses as ints; returns the status code"},
+    {"gather_a", (PyCFunction)(void (*)(void))py_gather_a, METH_FASTCALL, "fp8bs_gather_a with addresses as ints; returns the status code"},
+    {"moe_topk", (PyCFunction)(void (*)(void))py_moe_topk, METH_FASTCALL, "fp8bs_moe_topk with addresses as ints; returns the status code"},
+    {"moe_route", (PyCFunction)(void (*)(void))py_moe_route, METH_FASTCALL, "fp8bs_moe_route with addresses as ints; returns the status code"},
+    {"moe_combine", (PyCFunction)(void (*)(void))py_moe_combine, METH_FASTCALL, "fp8bs_moe_combine with addresses as ints; returns the status code"},
     {NULL, NULL, 0, NULL},
 };
 

@@ -11,7 +11,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
-from .submission import _PLANS_MAX, _check_operands, _grouped_workspace, _is_kmajor, _plan_cache, _stream_ptr, _workspace
+from .submission import _PLANS_MAX, _call, _check_operands, _experts_kmajor, _grouped_workspace, _is_kmajor, _plan_cache, _stream_ptr, _workspace
 
 
 _route_ws = {}     # (device index, stream) -> uint8 tensor: the routing kernels' scratch, grown on demand, reused across
@@ -28,8 +28,7 @@ def topk(scores: torch.Tensor, k: int, out: Optional[torch.Tensor] = None) -> to
         out = torch.empty(t, k, dtype=torch.int32, device=scores.device)
     elif out.dtype != torch.int32 or tuple(out.shape) != (t, k) or out.device != scores.device or not out.is_contiguous():
         raise ValueError("out must be a contiguous int32 [tokens, k] tensor on the scores' device")
-    with torch.cuda.device(scores.device):
-        _lib.check(_lib.load().fp8bs_moe_topk(scores.data_ptr(), t, e, k, out.data_ptr(), _stream_ptr(scores.device)))
+    _call(_lib.calls().moe_topk, scores.device, scores.data_ptr(), t, e, k, out.data_ptr())
     return out
 
 
@@ -56,21 +55,22 @@ def route(top_idx: torch.Tensor, experts: int, out: Optional[Tuple[torch.Tensor,
         for name, x, shape in (("row_offsets", row_offsets, (experts + 1,)), ("row_map", row_map, (t * k,)), ("slot_of", slot_of, (t, k))):
             if x.dtype != torch.int32 or tuple(x.shape) != shape or x.device != dev or not x.is_contiguous():
                 raise ValueError("out: %s must be a contiguous int32 tensor of shape %s on top_idx's device" % (name, shape))
-    lib = _lib.load()
-    need = lib.fp8bs_moe_route_workspace_bytes(t, experts)
-    with torch.cuda.device(dev):
-        stream = _stream_ptr(dev)
-        key = (dev.index, stream)
-        ws = _route_ws.get(key)
-        if ws is None or ws.numel() < need:
-            # A buffer that is outgrown stays alive until this stream's earlier kernels are done with it: the caching
-            # allocator hands a freed block only to later work of the stream it was allocated on.
-            if ws is None and len(_route_ws) >= 16:      # streams come and go: keep the table bounded (oldest entry out)
-                _route_ws.pop(next(iter(_route_ws)))
-            ws = torch.empty(max(need, 4096), dtype=torch.uint8, device=dev)
-            _route_ws[key] = ws
-        _lib.check(lib.fp8bs_moe_route(top_idx.data_ptr(), t, experts, k, row_offsets.data_ptr(), row_map.data_ptr(),
-                                       slot_of.data_ptr(), ws.data_ptr(), ws.numel(), stream))
+    need = _plan_cache.get(("route", t, experts))
+    if need is None:
+        if len(_plan_cache) >= _PLANS_MAX:
+            _plan_cache.clear()
+        need = _plan_cache[("route", t, experts)] = _lib.load().fp8bs_moe_route_workspace_bytes(t, experts)
+    key = (dev.index, _stream_ptr(dev))
+    ws = _route_ws.get(key)
+    if ws is None or ws.numel() < need:
+        # A buffer that is outgrown stays alive until this stream's earlier kernels are done with it: the caching
+        # allocator hands a freed block only to later work of the stream it was allocated on.
+        if ws is None and len(_route_ws) >= 16:      # streams come and go: keep the table bounded (oldest entry out)
+            _route_ws.pop(next(iter(_route_ws)))
+        ws = torch.empty(max(need, 4096), dtype=torch.uint8, device=dev)
+        _route_ws[key] = ws
+    _call(_lib.calls().moe_route, dev, top_idx.data_ptr(), t, experts, k, row_offsets.data_ptr(), row_map.data_ptr(),
+          slot_of.data_ptr(), ws.data_ptr(), ws.numel())
     return row_offsets, row_map, slot_of
 
 
@@ -95,35 +95,33 @@ def gate_up_silu(data):
         raise ValueError("n must be even: gate and up rows come in pairs")
     nb, kb = (n + 127) // 128, k // 128
     if grouped:
-        if tuple(b.shape) != (num_experts, n, k) or tuple(b_scale.shape) != (num_experts, nb, kb):
+        if b.shape != (num_experts, n, k) or b_scale.shape != (num_experts, nb, kb):
             raise ValueError("b / b_scale shapes do not match [E, n, k] / [E, ceil(n/128), k/128]")
-        if not b.transpose(1, 2).is_contiguous() or not b_scale.transpose(1, 2).is_contiguous():
+        if not _experts_kmajor(b) or not _experts_kmajor(b_scale):
             raise ValueError("every expert of b and b_scale must be K-major")
-        if row_offsets.dtype != torch.int32 or tuple(row_offsets.shape) != (num_experts + 1,) or row_offsets.device != a.device:
+        if row_offsets.dtype != torch.int32 or row_offsets.shape != (num_experts + 1,) or row_offsets.device != a.device:
             raise ValueError("row_offsets must be an int32 tensor with num_experts+1 entries on the operands' GPU")
     else:
-        if tuple(b.shape) != (n, k) or tuple(b_scale.shape) != (nb, kb):
+        if b.shape != (n, k) or b_scale.shape != (nb, kb):
             raise ValueError("b / b_scale shapes do not match [n, k] / [ceil(n/128), k/128]")
         if not _is_kmajor(b) or not _is_kmajor(b_scale):
             raise ValueError("b and b_scale must be K-major")
     # dtypes, devices, shapes and K-major strides of a, a_scale and h ([rows, n/2]) as for the plain GEMM's c
     _check_operands(a, b, a_scale, b_scale, h, rows, n // 2, k)
-    with torch.cuda.device(a.device):
-        stream = _stream_ptr(a.device)
-        if grouped:
-            ws_ptr, ws_len = _grouped_workspace(a.device, stream, num_experts, rows, n, k)
-        else:
-            need = _plan_cache.get(("silu", rows, n, k))
-            if need is None:
-                if len(_plan_cache) >= _PLANS_MAX:
-                    _plan_cache.clear()
+    dev = a.device
+    if grouped:
+        ws_ptr, ws_len = _grouped_workspace(dev, _stream_ptr(dev), num_experts, rows, n, k)
+    else:
+        need = _plan_cache.get(("silu", rows, n, k))
+        if need is None:
+            if len(_plan_cache) >= _PLANS_MAX:
+                _plan_cache.clear()
+            with torch.cuda.device(dev):             # planned for the CU count of the device it runs on
                 need = _plan_cache[("silu", rows, n, k)] = int(_lib.load().fp8bs_silu_mul_workspace_bytes(rows, n, k))
-            ws = _workspace(a.device, need, stream) if need else None
-            ws_ptr, ws_len = (ws.data_ptr(), ws.numel()) if need else (None, 0)
-        fast = _lib.pycall()
-        call = fast.gemm_silu_mul_ws if fast is not None else _lib.load().fp8bs_gemm_silu_mul_ws
-        _lib.check(call(a.data_ptr(), b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(), h.data_ptr(),
-                        row_offsets.data_ptr() if grouped else None, num_experts, rows, n, k, 0, 0, ws_ptr, ws_len, stream))
+        ws = _workspace(dev, need, _stream_ptr(dev)) if need else None
+        ws_ptr, ws_len = (ws.data_ptr(), ws.numel()) if need else (None, 0)
+    _call(_lib.calls().gemm_silu_mul_ws, dev, a.data_ptr(), b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(), h.data_ptr(),
+          row_offsets.data_ptr() if grouped else None, num_experts, rows, n, k, 0, 0, ws_ptr, ws_len)
     return h
 
 
@@ -140,7 +138,5 @@ def combine(y: torch.Tensor, slot_of: torch.Tensor, weights: torch.Tensor) -> to
     t, k = slot_of.shape
     d = y.shape[1]
     out = torch.empty(t, d, dtype=torch.bfloat16, device=y.device)
-    with torch.cuda.device(y.device):
-        _lib.check(_lib.load().fp8bs_moe_combine(y.data_ptr(), y.shape[0], slot_of.data_ptr(), weights.data_ptr(), out.data_ptr(),
-                                                 t, k, d, _stream_ptr(y.device)))
+    _call(_lib.calls().moe_combine, y.device, y.data_ptr(), y.shape[0], slot_of.data_ptr(), weights.data_ptr(), out.data_ptr(), t, k, d)
     return out

@@ -11,6 +11,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
+from .submission import _call
 
 _DTYPES = {torch.float32: 0, torch.bfloat16: 1}
 
@@ -20,10 +21,16 @@ def _check_input(x: torch.Tensor, name: str) -> None:
         raise TypeError("%s must be float32 or bfloat16, got %s" % (name, x.dtype))
     if x.dim() != 2 or not x.is_cuda:
         raise ValueError("%s must be a 2-D tensor on the GPU" % name)
-    if x.shape[1] % 128 != 0:
-        raise ValueError("%s: K = %d is not a multiple of 128" % (name, x.shape[1]))
-    if x.shape[1] > 0 and x.stride(1) != 1:
+    k = x.shape[1]
+    if k % 128 != 0:
+        raise ValueError("%s: K = %d is not a multiple of 128" % (name, k))
+    if k > 0 and x.stride(1) != 1:
         raise ValueError("%s must be row-major (stride 1 along K), got strides %s" % (name, tuple(x.stride())))
+
+
+def _k_major(rows: int, k: int, dtype: torch.dtype, device: torch.device) -> torch.Tensor:
+    """An uninitialised [rows, k] tensor whose storage is [k][rows]."""
+    return torch.empty_strided((rows, k), (1, rows or 1), dtype=dtype, device=device)
 
 
 def quantize_a(x: torch.Tensor, row_map: Optional[torch.Tensor] = None, fused: Optional[bool] = None) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -49,30 +56,22 @@ def quantize_a(x: torch.Tensor, row_map: Optional[torch.Tensor] = None, fused: O
             return gather_a(*quantize_a(x), row_map)
     else:
         m = t
-    a_store = torch.empty(k, m, dtype=torch.float8_e4m3fn, device=x.device)
-    s_store = torch.empty(k // 128, m, dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
-        stream = torch.cuda.current_stream().cuda_stream
-        _lib.check(_lib.load().fp8bs_quantize_a(
-            x.data_ptr(), _DTYPES[x.dtype], x.stride(0) if t > 1 else max(k, 1),
-            row_map.data_ptr() if row_map is not None else None, t,
-            a_store.data_ptr(), s_store.data_ptr(), m, k, stream))
-    return a_store.t(), s_store.t()
+    dev = x.device
+    a, a_scale = _k_major(m, k, torch.float8_e4m3fn, dev), _k_major(m, k // 128, torch.float32, dev)
+    _call(_lib.calls().quantize_a, dev, x.data_ptr(), _DTYPES[x.dtype], x.stride(0) if t > 1 else max(k, 1),
+          row_map.data_ptr() if row_map is not None else None, t, a.data_ptr(), a_scale.data_ptr(), m, k)
+    return a, a_scale
 
 
 def quantize_b(w: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """w [N, K] -> (b e4m3fn [N, K] stride (1, N), b_scale fp32 [ceil(N/128), K/128] stride (1, NB))."""
     _check_input(w, "w")
     n, k = w.shape
-    nb = (n + 127) // 128
-    b_store = torch.empty(k, n, dtype=torch.float8_e4m3fn, device=w.device)
-    s_store = torch.empty(k // 128, nb, dtype=torch.float32, device=w.device)
-    with torch.cuda.device(w.device):
-        stream = torch.cuda.current_stream().cuda_stream
-        _lib.check(_lib.load().fp8bs_quantize_b(
-            w.data_ptr(), _DTYPES[w.dtype], w.stride(0) if n > 1 else max(k, 1),
-            b_store.data_ptr(), s_store.data_ptr(), n, k, stream))
-    return b_store.t(), s_store.t()
+    dev = w.device
+    b, b_scale = _k_major(n, k, torch.float8_e4m3fn, dev), _k_major((n + 127) // 128, k // 128, torch.float32, dev)
+    _call(_lib.calls().quantize_b, dev, w.data_ptr(), _DTYPES[w.dtype], w.stride(0) if n > 1 else max(k, 1),
+          b.data_ptr(), b_scale.data_ptr(), n, k)
+    return b, b_scale
 
 
 def gather_a(a: torch.Tensor, a_scale: torch.Tensor, row_map: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -93,10 +92,7 @@ def gather_a(a: torch.Tensor, a_scale: torch.Tensor, row_map: torch.Tensor) -> T
     if row_map.dtype != torch.int32 or row_map.dim() != 1 or row_map.device != a.device or not row_map.is_contiguous():
         raise ValueError("row_map must be a contiguous int32 vector on a's device")
     m = row_map.numel()
-    a_store = torch.empty(k, m, dtype=torch.float8_e4m3fn, device=a.device)
-    s_store = torch.empty(k // 128, m, dtype=torch.float32, device=a.device)
-    with torch.cuda.device(a.device):
-        _lib.check(_lib.load().fp8bs_gather_a(a.data_ptr(), a_scale.data_ptr(), t, row_map.data_ptr(),
-                                              a_store.data_ptr(), s_store.data_ptr(), m, k,
-                                              torch.cuda.current_stream().cuda_stream))
-    return a_store.t(), s_store.t()
+    dev = a.device
+    out, out_scale = _k_major(m, k, torch.float8_e4m3fn, dev), _k_major(m, k // 128, torch.float32, dev)
+    _call(_lib.calls().gather_a, dev, a.data_ptr(), a_scale.data_ptr(), t, row_map.data_ptr(), out.data_ptr(), out_scale.data_ptr(), m, k)
+    return out, out_scale

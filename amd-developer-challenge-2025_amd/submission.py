@@ -50,7 +50,7 @@ def _is_kmajor(t: torch.Tensor) -> bool:
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-_plan_cache = {}   # (m, n, k) and ("grouped", experts, rows, n, k) -> workspace bytes the planner asks for
+_plan_cache = {}   # (m, n, k) and ("grouped" | "silu" | "route", sizes ...) -> workspace bytes the call asks for
 _PLANS_MAX = 4096
 
 # Operands that passed the checks once: a caller that hands over the same tensor objects again (a benchmark
@@ -69,27 +69,6 @@ def _remember(key, data, *rest):
                      tuple(t.stride() for t in data)) + rest
 
 
-def _gemm_ex_fn():
-    """fp8bs_gemm_ex through the CPython binding when it is built, else through ctypes (same library function)."""
-    fast = _lib.pycall()
-    return fast.gemm_ex if fast is not None else _lib.load().fp8bs_gemm_ex
-
-
-def _grouped_ws_fn():
-    fast = _lib.pycall()
-    return fast.gemm_grouped_ws if fast is not None else _lib.load().fp8bs_gemm_grouped_ws
-
-
-_gemm_ex = _grouped_ws = None
-
-
-def _bind():
-    """Resolve the two call targets once (the CPython binding if built, else ctypes)."""
-    global _gemm_ex, _grouped_ws
-    _gemm_ex, _grouped_ws = _gemm_ex_fn(), _grouped_ws_fn()
-    return _gemm_ex, _grouped_ws
-
-
 def _grouped_workspace(device, stream, num_experts, rows, n, k):
     """(address, bytes) of the workspace a grouped call can use, (None, 0) if it would not use any."""
     key = ("grouped", num_experts, rows, n, k)
@@ -97,7 +76,8 @@ def _grouped_workspace(device, stream, num_experts, rows, n, k):
     if need is None:
         if len(_plan_cache) >= _PLANS_MAX:
             _plan_cache.clear()
-        need = _plan_cache[key] = int(_lib.load().fp8bs_grouped_workspace_bytes(num_experts, rows, n, k))
+        with torch.cuda.device(device):              # planned for the CU count of the device it runs on
+            need = _plan_cache[key] = int(_lib.load().fp8bs_grouped_workspace_bytes(num_experts, rows, n, k))
     if not need:
         return None, 0
     ws = _workspace(device, need, stream)
@@ -111,7 +91,36 @@ def _stream_ptr(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+def _call(fn, device: torch.device, *args) -> None:
+    """fn(*args, stream) on torch's current stream of `device`; the library launches on the current device.
+    Entering torch.cuda.device costs 1.2 us, asking for the stream through torch.cuda 2.6: with ctypes' marshalling they
+    were half of a quantiser call's 12.9 us of host time (now 7.4, of which 3 are the launch and 2 the two allocations)."""
+    if torch.cuda.current_device() == device.index:
+        st = fn(*args, _stream_ptr(device))
+    else:
+        with torch.cuda.device(device):
+            st = fn(*args, _stream_ptr(device))
+    if st:
+        _lib.check(st)
+
+
+_F8, _F32, _BF16 = torch.float8_e4m3fn, torch.float32, torch.bfloat16
+
+
+def _experts_kmajor(t: torch.Tensor) -> bool:
+    """True if every expert of the 3-D tensor is K-major and they lie one behind the other."""
+    e, r, c = t.shape
+    return t.stride() == (r * c, 1, r) or t.transpose(1, 2).is_contiguous()
+
+
 def _check_operands(a, b, a_scale, b_scale, c, rows, n, k):
+    dev = a.get_device()
+    if a.dtype is _F8 and b.dtype is _F8 and a_scale.dtype is _F32 and b_scale.dtype is _F32 and c.dtype is _BF16 \
+            and k % 128 == 0 and a.shape == (rows, k) and a_scale.shape == (rows, k // 128) and c.shape == (rows, n) \
+            and a.stride() == (1, rows) and a_scale.stride() == (1, rows) and c.is_contiguous() and dev >= 0 \
+            and b.get_device() == dev and a_scale.get_device() == dev and b_scale.get_device() == dev and c.get_device() == dev:
+        return
+    # not the usual layout: a dimension of size 1 or 0, or something to refuse
     if a.dtype != torch.float8_e4m3fn or b.dtype != torch.float8_e4m3fn:
         raise TypeError("a and b must be torch.float8_e4m3fn")
     if a_scale.dtype != torch.float32 or b_scale.dtype != torch.float32:
@@ -153,7 +162,7 @@ def custom_kernel(data, variant: int = 0, split_k: int = 0):
     dealt to the workgroups); the defaults let the library's planner decide.
     """
     a, b, a_scale, b_scale, c = data
-    gemm_ex = _gemm_ex or _bind()[0]
+    gemm_ex = _lib.calls().gemm_ex
     key = None
     if variant == 0 and split_k == 0:
         key = (id(a), id(b), id(a_scale), id(b_scale), id(c))
@@ -179,7 +188,7 @@ def custom_kernel(data, variant: int = 0, split_k: int = 0):
     n = b.shape[0]
     _check_operands(a, b, a_scale, b_scale, c, m, n, k)
     nb = (n + 127) // 128
-    if b.shape[1] != k or tuple(b_scale.shape) != (nb, k // 128):
+    if b.shape != (n, k) or b_scale.shape != (nb, k // 128):
         raise ValueError("b / b_scale shapes do not match [n, k] / [ceil(n/128), k/128]")
     if not _is_kmajor(b) or not _is_kmajor(b_scale):
         raise ValueError("b and b_scale must be K-major (stride (1, n) / (1, ceil(n/128)))")
@@ -198,16 +207,13 @@ def custom_kernel(data, variant: int = 0, split_k: int = 0):
         if split_k > 0 and split_k & _lib.SPLIT_SUM_IN_KERNEL:
             # summed in the kernel: a header and split_k fp32 tiles per tile (the largest tile is 256 x 256)
             need = 16384 + (split_k & ~_lib.SPLIT_SUM_IN_KERNEL) * (m + 255) * (n + 255) * 4
-    # kernels are launched on the device the pointers live on: the library uses the current device
-    with torch.cuda.device(a.device):
-        stream = _stream_ptr(a.device)
-        ws_ptr, ws_len = None, 0
-        if need:
-            ws = _workspace(a.device, need, stream)
-            ws_ptr, ws_len = ws.data_ptr(), ws.numel()
-        st = gemm_ex(a.data_ptr(), b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(),
-                     c.data_ptr(), ws_ptr, ws_len, m, n, k, variant, split_k, stream)
-    _lib.check(st)
+    dev = a.device
+    ws_ptr, ws_len = None, 0
+    if need:
+        ws = _workspace(dev, need, _stream_ptr(dev))
+        ws_ptr, ws_len = ws.data_ptr(), ws.numel()
+    _call(gemm_ex, dev, a.data_ptr(), b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(),
+          c.data_ptr(), ws_ptr, ws_len, m, n, k, variant, split_k)
     return c
 
 
@@ -222,37 +228,20 @@ def grouped_kernel(data, variant: int = 0):
     [E, ceil(n/128), k/128] with stride (nb*kb, 1, nb).  Fills and returns ``c``; no host sync.
     """
     a, b, a_scale, b_scale, row_offsets, c = data
-    grouped_ws = _grouped_ws or _bind()[1]
-    key = ("grouped", id(a), id(b), id(a_scale), id(b_scale), id(row_offsets), id(c))
-    hit = _checked.get(key)
-    if hit is not None:
-        refs, ptrs, shapes, strides, rows, n, k, num_experts, dev_index = hit
-        now = tuple(t.data_ptr() for t in data)
-        if all(r() is t for r, t in zip(refs, data)) and now == ptrs and tuple(t.shape for t in data) == shapes \
-                and tuple(t.stride() for t in data) == strides and dev_index == torch.cuda.current_device():
-            stream = _stream_ptr(a.device)
-            ws_ptr, ws_len = _grouped_workspace(a.device, stream, num_experts, rows, n, k) if variant == 0 else (None, 0)
-            st = grouped_ws(now[0], now[1], now[2], now[3], now[5], now[4], num_experts, rows, n, k, variant, 0, ws_ptr, ws_len, stream)
-            if st:
-                _lib.check(st)
-            return c
     rows, k = a.shape
     if b.dim() != 3:
         raise ValueError("b must be [E, n, k]")
     num_experts, n = b.shape[0], b.shape[1]
     _check_operands(a, b, a_scale, b_scale, c, rows, n, k)
     nb, kb = (n + 127) // 128, k // 128
-    if tuple(b.shape) != (num_experts, n, k) or tuple(b_scale.shape) != (num_experts, nb, kb):
+    if b.shape != (num_experts, n, k) or b_scale.shape != (num_experts, nb, kb):
         raise ValueError("b / b_scale shapes do not match [E, n, k] / [E, ceil(n/128), k/128]")
-    if not b.transpose(1, 2).is_contiguous() or not b_scale.transpose(1, 2).is_contiguous():
+    if not _experts_kmajor(b) or not _experts_kmajor(b_scale):
         raise ValueError("every expert of b and b_scale must be K-major")
-    if row_offsets.dtype != torch.int32 or tuple(row_offsets.shape) != (num_experts + 1,) or row_offsets.device != a.device:
+    if row_offsets.dtype != torch.int32 or row_offsets.shape != (num_experts + 1,) or row_offsets.device != a.device:
         raise ValueError("row_offsets must be an int32 tensor with num_experts+1 entries on the operands' GPU")
-    _remember(key, data, rows, n, k, num_experts, a.device.index)
-    with torch.cuda.device(a.device):
-        stream = _stream_ptr(a.device)
-        ws_ptr, ws_len = _grouped_workspace(a.device, stream, num_experts, rows, n, k) if variant == 0 else (None, 0)
-        st = grouped_ws(a.data_ptr(), b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(), c.data_ptr(), row_offsets.data_ptr(),
-                        num_experts, rows, n, k, variant, 0, ws_ptr, ws_len, stream)
-    _lib.check(st)
+    dev = a.device
+    ws_ptr, ws_len = _grouped_workspace(dev, _stream_ptr(dev), num_experts, rows, n, k) if variant == 0 else (None, 0)
+    _call(_lib.calls().gemm_grouped_ws, dev, a.data_ptr(), b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(), c.data_ptr(),
+          row_offsets.data_ptr(), num_experts, rows, n, k, variant, 0, ws_ptr, ws_len)
     return c
