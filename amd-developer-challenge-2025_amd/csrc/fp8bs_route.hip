@@ -10,7 +10,7 @@
 //   host read of the counts      :230-234           hipDeviceSynchronize + loop, to size the next launch
 // Here the positions are deterministic: rows of an expert are ordered by token id (then choice), which
 // is what a stable sort by expert gives and what inputs.make_grouped builds.  Counting is done per block
-// of 256 tokens in LDS (integer atomics: the totals do not depend on the order), a one-block scan turns
+// of 256 tokens in LDS (integer atomics: the totals do not depend on the order), a scan turns
 // the per-block counts into bases and the expert totals into row_offsets[E+1] (total appended), and a
 // third kernel ranks every choice inside its block from LDS bitmaps and writes
 //   row_map[row] = token   (the gather list fp8bs_quantize_a takes)   and   slot_of[token][choice] = row.
@@ -26,11 +26,37 @@ static constexpr int RB = 256;            // tokens per block
 static constexpr int MAX_EXPERTS = 1024;  // LDS: 32 bytes of bitmap per expert
 static constexpr int MAX_TOPK = 16;       // a token's choices are held in registers
 
+// A token's entries of top_idx or slot_of are moved 16 bytes at a time where they lie so: one at a time the lanes of a
+// wave touch 64 places per instruction, topk times.
+typedef int v4i __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ bool four_wide(int topk, const int32_t* p) { return (topk & 3) == 0 && ((uintptr_t)p & 15) == 0; }
+
+__device__ __forceinline__ void store_slots(int32_t* __restrict__ slot_of, int t, int topk, const int (&dest)[MAX_TOPK]) {
+    if (four_wide(topk, slot_of)) {
+#pragma unroll
+        for (int j = 0; j < MAX_TOPK; j += 4)
+            if (j < topk) *(v4i*)(slot_of + (size_t)t * topk + j) = (v4i){dest[j], dest[j + 1], dest[j + 2], dest[j + 3]};
+    } else {
+#pragma unroll
+        for (int j = 0; j < MAX_TOPK; j++)
+            if (j < topk) slot_of[(size_t)t * topk + j] = dest[j];
+    }
+}
+
 // the choices of token t, all loads in flight at once; absent entries are -1; an expert repeated by the
 // token is kept at its first occurrence only (later ones become -1 as well)
 __device__ __forceinline__ void load_choices(const int32_t* __restrict__ top_idx, int t, int tokens, int experts, int topk, int (&ch)[MAX_TOPK]) {
+    if (four_wide(topk, top_idx)) {
 #pragma unroll
-    for (int j = 0; j < MAX_TOPK; j++) ch[j] = (t < tokens && j < topk) ? top_idx[(size_t)t * topk + j] : -1;
+        for (int j = 0; j < MAX_TOPK; j += 4) {
+            const v4i v = (t < tokens && j < topk) ? *(const v4i*)(top_idx + (size_t)t * topk + j) : (v4i){-1, -1, -1, -1};
+#pragma unroll
+            for (int i = 0; i < 4; i++) ch[j + i] = v[i];
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < MAX_TOPK; j++) ch[j] = (t < tokens && j < topk) ? top_idx[(size_t)t * topk + j] : -1;
+    }
 #pragma unroll
     for (int j = 0; j < MAX_TOPK; j++) {
         bool keep = ch[j] >= 0 && ch[j] < experts;
@@ -101,6 +127,18 @@ void moe_topk64_kernel(const float* __restrict__ scores, int tokens, int experts
     }
 }
 
+// inclusive prefix over groups of WIDTH consecutive lanes
+template <int WIDTH>
+__device__ __forceinline__ int inclusive_scan(int v) {
+    const int l = threadIdx.x & (WIDTH - 1);
+#pragma unroll
+    for (int off = 1; off < WIDTH; off <<= 1) {
+        const int u = __shfl_up(v, off, WIDTH);
+        v += l >= off ? u : 0;
+    }
+    return v;
+}
+
 // block_counts[b][e] = number of choices of expert e among the tokens of block b
 __global__ __launch_bounds__(RB)
 void route_count_kernel(const int32_t* __restrict__ top_idx, int tokens, int experts, int topk, int32_t* __restrict__ block_counts) {
@@ -150,7 +188,7 @@ void route_assign_kernel(const int32_t* __restrict__ top_idx, int tokens, int ex
                          int32_t* __restrict__ row_map, int32_t* __restrict__ slot_of) {
     __shared__ uint32_t bits[MAX_EXPERTS * (RB / 32)];
     __shared__ int first_row[MAX_EXPERTS];       // first row of this block's tokens inside expert e's segment
-    __shared__ int part[RB];
+    __shared__ int part[RB / 64];
     __shared__ int tot_s[SCAN_HERE ? MAX_EXPERTS : 1], base_s[SCAN_HERE ? MAX_EXPERTS : 1];
     int row_offsets_total;                       // row_offsets[experts]: rows that belong to some expert
     for (int i = threadIdx.x; i < experts * (RB / 32); i += RB) bits[i] = 0;
@@ -175,15 +213,16 @@ void route_assign_kernel(const int32_t* __restrict__ top_idx, int tokens, int ex
             tot[i] = e < experts ? tot_s[e] : 0;
             base[i] = e < experts ? base_s[e] : 0;
         }
-        part[threadIdx.x] = tot[0] + tot[1] + tot[2] + tot[3];
+        const int own = tot[0] + tot[1] + tot[2] + tot[3];
+        const int incl = inclusive_scan<64>(own);
+        if ((threadIdx.x & 63) == 63) part[threadIdx.x >> 6] = incl;
         __syncthreads();
-        for (int off = 1; off < RB; off <<= 1) {           // inclusive scan of the 256 partial sums
-            const int v = threadIdx.x >= off ? part[threadIdx.x - off] : 0;
-            __syncthreads();
-            part[threadIdx.x] += v;
-            __syncthreads();
+        int run = incl - own, all = 0;
+#pragma unroll
+        for (int i = 0; i < RB / 64; i++) {
+            if (i < (int)(threadIdx.x >> 6)) run += part[i];
+            all += part[i];
         }
-        int run = part[threadIdx.x] - (tot[0] + tot[1] + tot[2] + tot[3]);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int e = 4 * threadIdx.x + i;
@@ -193,8 +232,8 @@ void route_assign_kernel(const int32_t* __restrict__ top_idx, int tokens, int ex
             }
             run += tot[i];
         }
-        if (blockIdx.x == 0 && threadIdx.x == RB - 1) row_offsets[experts] = part[RB - 1];
-        row_offsets_total = part[RB - 1];
+        if (blockIdx.x == 0 && threadIdx.x == 0) row_offsets[experts] = all;
+        row_offsets_total = all;
     } else {
         for (int e = threadIdx.x; e < experts; e += RB) first_row[e] = row_offsets[e] + block_base[(size_t)blockIdx.x * experts + e];
         row_offsets_total = row_offsets[experts];
@@ -211,51 +250,122 @@ void route_assign_kernel(const int32_t* __restrict__ top_idx, int tokens, int ex
     // rows beyond the last expert's (they exist only if some choices were outside [0, experts)) map to no token
     for (int r = row_offsets_total + blockIdx.x * RB + threadIdx.x; r < tokens * topk; r += gridDim.x * RB) row_map[r] = -1;
     if (t >= tokens) return;
+    int dest[MAX_TOPK];
 #pragma unroll
     for (int j = 0; j < MAX_TOPK; j++) {
-        if (j < topk) {
-            int dest = -1;
-            if (ch[j] >= 0) {
-                const uint32_t* bm = bits + ch[j] * (RB / 32);
-                int rank = __builtin_popcount(bm[w] & ((1u << bit) - 1u));
+        dest[j] = -1;
+        if (ch[j] >= 0) {
+            const uint32_t* bm = bits + ch[j] * (RB / 32);
+            int rank = __builtin_popcount(bm[w] & ((1u << bit) - 1u));
 #pragma unroll
-                for (int x = 0; x < RB / 32; x++) rank += x < w ? __builtin_popcount(bm[x]) : 0;
-                dest = first_row[ch[j]] + rank;
-                row_map[dest] = t;
-            }
-            if (slot_of) slot_of[(size_t)t * topk + j] = dest;
+            for (int x = 0; x < RB / 32; x++) rank += x < w ? __builtin_popcount(bm[x]) : 0;
+            dest[j] = first_row[ch[j]] + rank;
+            row_map[dest[j]] = t;
         }
     }
+    if (slot_of) store_slots(slot_of, t, topk, dest);
+}
+
+// The whole of route in one workgroup of T threads, one per token: up to T tokens and ONE_BITS / T experts of them.
+// One bit per (expert, token); T/32 lanes share an expert, so its words' prefix and its total are one short scan, the
+// experts' prefix another, and a token's rank is a table entry and one popcount.  Bound by latency: two launches, a table
+// of counts written and read back, and 16 barriers of a scan in LDS before.  us on the GPU, before -> after: 64 tokens to 8
+// of 32 experts 10.2 -> 5.0, 256 to 8 12.4 -> 5.4, 700 to 8 12.9 -> 10.2, 1024 to 2 of 8 9.4 -> 7.2.  One CU's scattered
+// stores are what it costs with more rows, so a token's slots leave 16 bytes at a time and row_map in whole lines.
+static constexpr int ONE_BITS = 8192 * 32;
+template <int T>
+__global__ __launch_bounds__(T)
+void route_one_kernel(const int32_t* __restrict__ top_idx, int tokens, int experts, int topk,
+                      int32_t* __restrict__ row_offsets, int32_t* __restrict__ row_map, int32_t* __restrict__ slot_of) {
+    constexpr int W = T / 32;
+    __shared__ uint32_t bits[ONE_BITS / 32];
+    __shared__ uint16_t before[ONE_BITS / 32];   // of an expert's word: its tokens in earlier words
+    __shared__ int first_row[ONE_BITS / T];      // first the expert's total
+    __shared__ int all_rows;
+    const int tid = threadIdx.x;
+    int ch[MAX_TOPK];
+    load_choices(top_idx, tid, tokens, experts, topk, ch);
+    for (int i = tid; i < experts * W; i += T) bits[i] = 0;
+    __syncthreads();
+    const int w = tid >> 5, bit = tid & 31;
+#pragma unroll
+    for (int j = 0; j < MAX_TOPK; j++)
+        if (ch[j] >= 0) atomicOr(&bits[ch[j] * W + w], 1u << bit);
+    __syncthreads();
+    for (int i = tid; i < experts * W; i += T) {
+        const int c = __builtin_popcount(bits[i]), incl = inclusive_scan<W>(c);
+        before[i] = (uint16_t)(incl - c);
+        if ((i & (W - 1)) == W - 1) first_row[i / W] = incl;
+    }
+    __syncthreads();
+    if (tid < 64) {
+        int base = 0;
+        for (int e0 = 0; e0 < experts; e0 += 64) {
+            const int e = e0 + tid;
+            const int c = e < experts ? first_row[e] : 0, incl = inclusive_scan<64>(c);
+            if (e < experts) {
+                first_row[e] = base + incl - c;
+                row_offsets[e] = base + incl - c;
+            }
+            base += __shfl(incl, 63, 64);
+        }
+        if (tid == 0) { row_offsets[experts] = base; all_rows = base; }
+    }
+    __syncthreads();
+    int dest[MAX_TOPK];
+#pragma unroll
+    for (int j = 0; j < MAX_TOPK; j++) {
+        dest[j] = -1;
+        if (ch[j] >= 0) {
+            const int at = ch[j] * W + w;
+            dest[j] = first_row[ch[j]] + before[at] + __builtin_popcount(bits[at] & ((1u << bit) - 1u));
+        }
+    }
+    if (slot_of && tid < tokens) store_slots(slot_of, tid, topk, dest);
+    // row_map is put in order in LDS, where the bitmaps were, and leaves in whole lines
+    uint16_t* map = (uint16_t*)bits;
+    static_assert(sizeof(bits) >= T * MAX_TOPK * sizeof(uint16_t), "one entry per choice");
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < MAX_TOPK; j++)
+        if (dest[j] >= 0) map[dest[j]] = (uint16_t)tid;
+    __syncthreads();
+    // rows beyond the last expert's (they exist only if some choices were outside [0, experts)) map to no token
+    for (int r = tid; r < tokens * topk; r += T) row_map[r] = r < all_rows ? (int)map[r] : -1;
 }
 
 // out[t][d] = sum_j weights[t][j] * y[slot_of[t][j]][d], fp32 accumulation in the order j = 0..topk-1,
 // one rounding to bf16 (role of pack_output, 2-amd-moe/amd-moe-submission.py:239-301, which accumulates
-// in fp16).  One block per token, 8 columns (16 bytes) per thread and step; entries whose slot is not a
-// row of y (-1 or beyond) are skipped.
-typedef int cv4i __attribute__((ext_vector_type(4)));
-__global__ __launch_bounds__(RB)
+// in fp16).  8 columns (16 bytes) per thread and step; entries whose slot is not a row of y (-1 or beyond) are skipped.
+// Bound by HBM with many tokens (4096 x 8 x 7168: 96 us, 5.5 TB/s): one block of 256 threads per token, four choices at a
+// time.  With up to 1024 tokens a block per 1024 columns and eight choices at a time: one block per token walked its
+// columns and choices in eight round trips to memory (x 8 x 7168, us before -> after: 1 token 6.5 -> 2.9, 64 6.8 -> 3.4, 256
+// 9.8 -> 5.4, 1024 24.4 -> 22.7; 2048 47.4 -> 48.6, left as it was, and so is d <= 2048, one step of a block: 64 x 2 x 1024 2.4
+// against 2.7).
+template <int T, int NJ>
+__global__ __launch_bounds__(T)
 void moe_combine_kernel(const uint16_t* __restrict__ y, const int32_t* __restrict__ slot_of, const float* __restrict__ weights,
                         uint16_t* __restrict__ out, int rows, int topk, int d) {
     const int t = blockIdx.x;
-    for (int c = threadIdx.x * 8; c < d; c += RB * 8) {
+    for (uint32_t c = (blockIdx.y * T + threadIdx.x) * 8u; c < (uint32_t)d; c += gridDim.y * T * 8u) {
         float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        // four rows at a time, all four loads issued before the first is used (one after the other a step costs
+        // NJ rows at a time, all their loads issued before the first is used (one after the other a step costs
         // one memory latency per choice); a choice that is skipped enters as weight 0 times zeros, which leaves
         // the sum as it is
-        for (int j0 = 0; j0 < topk; j0 += 4) {
-            cv4i v[4];
-            float w[4];
+        for (int j0 = 0; j0 < topk; j0 += NJ) {
+            v4i v[NJ];
+            float w[NJ];
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
+            for (int i = 0; i < NJ; i++) {
                 const int j = j0 + i;
                 const int slot = j < topk ? slot_of[(size_t)t * topk + j] : -1;
                 const bool ok = slot >= 0 && slot < rows;
                 w[i] = ok ? weights[(size_t)t * topk + j] : 0.f;
-                v[i] = (cv4i){0, 0, 0, 0};
-                if (ok) v[i] = __builtin_nontemporal_load((const cv4i*)(y + (size_t)slot * d + c));
+                v[i] = (v4i){0, 0, 0, 0};
+                if (ok) v[i] = __builtin_nontemporal_load((const v4i*)(y + (size_t)slot * d + c));
             }
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
+            for (int i = 0; i < NJ; i++) {
 #pragma unroll
                 for (int x = 0; x < 4; x++) {
                     acc[2 * x] = __builtin_fmaf(w[i], __builtin_bit_cast(float, (uint32_t)v[i][x] << 16), acc[2 * x]);
@@ -263,7 +373,7 @@ void moe_combine_kernel(const uint16_t* __restrict__ y, const int32_t* __restric
                 }
             }
         }
-        cv4i o;
+        v4i o;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             typedef float cv2f __attribute__((ext_vector_type(2)));
@@ -271,7 +381,7 @@ void moe_combine_kernel(const uint16_t* __restrict__ y, const int32_t* __restric
             cv2f f = {acc[2 * i], acc[2 * i + 1]};
             o[i] = (int)__builtin_bit_cast(uint32_t, __builtin_convertvector(f, cv2bf));
         }
-        *(cv4i*)(out + (size_t)t * d + c) = o;
+        *(v4i*)(out + (size_t)t * d + c) = o;
     }
 }
 
@@ -309,6 +419,16 @@ extern "C" int fp8bs_moe_route(const int32_t* top_idx, int tokens, int experts, 
     }
     if (!top_idx || !row_map) return FP8BS_ERR_NULL_POINTER;
     if (!ws || ws_bytes < fp8bs_moe_route_workspace_bytes(tokens, experts)) return FP8BS_ERR_WORKSPACE;
+    // One workgroup where its LDS holds a bit per token and expert, and up to 8192 rows: 1024 tokens to 8 experts each
+    // take 12.3 us in it and 11.0 in two kernels over several CUs, with 16 each it would be twice that.
+    if (tokens <= 256 && experts <= fp8bs::ONE_BITS / 256) {
+        hipLaunchKernelGGL(fp8bs::route_one_kernel<256>, dim3(1), dim3(256), 0, s, top_idx, tokens, experts, topk, row_offsets, row_map, slot_of);
+        return hipGetLastError() == hipSuccess ? FP8BS_OK : FP8BS_ERR_LAUNCH;
+    }
+    if (tokens <= 1024 && experts <= fp8bs::ONE_BITS / 1024 && tokens * topk < 8192) {
+        hipLaunchKernelGGL(fp8bs::route_one_kernel<1024>, dim3(1), dim3(1024), 0, s, top_idx, tokens, experts, topk, row_offsets, row_map, slot_of);
+        return hipGetLastError() == hipSuccess ? FP8BS_OK : FP8BS_ERR_LAUNCH;
+    }
     hipLaunchKernelGGL(fp8bs::route_count_kernel, dim3(nblocks), dim3(fp8bs::RB), 0, s, top_idx, tokens, experts, topk, (int32_t*)ws);
     if (hipGetLastError() != hipSuccess) return FP8BS_ERR_LAUNCH;
     if (nblocks <= 64) {
@@ -330,7 +450,12 @@ extern "C" int fp8bs_moe_combine(const void* y, int rows, const int32_t* slot_of
     if (tokens == 0 || d == 0) return FP8BS_OK;
     if (!y || !slot_of || !weights || !out) return FP8BS_ERR_NULL_POINTER;
     if ((((uintptr_t)y | (uintptr_t)out) & 15) != 0) return FP8BS_ERR_BAD_SHAPE;      // 16-byte row accesses
-    hipLaunchKernelGGL(fp8bs::moe_combine_kernel, dim3(tokens), dim3(fp8bs::RB), 0, (hipStream_t)stream,
-                       (const uint16_t*)y, slot_of, weights, (uint16_t*)out, rows, topk, d);
+    const int chunks = (d + 1023) / 1024;
+    if (d > 2048 && tokens <= 1024)
+        hipLaunchKernelGGL((fp8bs::moe_combine_kernel<128, 8>), dim3(tokens, chunks < 65535 ? chunks : 65535), dim3(128), 0, (hipStream_t)stream,
+                           (const uint16_t*)y, slot_of, weights, (uint16_t*)out, rows, topk, d);
+    else
+        hipLaunchKernelGGL((fp8bs::moe_combine_kernel<fp8bs::RB, 4>), dim3(tokens), dim3(fp8bs::RB), 0, (hipStream_t)stream,
+                           (const uint16_t*)y, slot_of, weights, (uint16_t*)out, rows, topk, d);
     return hipGetLastError() == hipSuccess ? FP8BS_OK : FP8BS_ERR_LAUNCH;
 }

@@ -92,6 +92,12 @@ def test_combine(moe, oracle, mo, dev, tokens, k, d):
     _within(oracle, out.cpu(), mo.combine_ref(y, slot, w), "combine")
 
 
+@pytest.mark.parametrize("tokens,k,d", [(3, 8, 2048), (5, 9, 2056), (2, 1, 3080), (7, 16, 8200), (1500, 2, 4096)])
+def test_combine_on_both_sides_of_2048_columns(moe, oracle, mo, dev, tokens, k, d):
+    """Wider rows go to several workgroups, eight choices at a time: widths off its 1024-column chunks, more choices than eight."""
+    test_combine(moe, oracle, mo, dev, tokens, k, d)
+
+
 def test_expert_ffn_chain(pkg, moe, quant, oracle, mo, ro, dev):
     """scores -> top-k -> route -> quantise+gather -> gate/up GEMM with fused silu-mul -> quantise ->
     down GEMM -> weighted un-permute, against the same chain built from the oracles on the host."""

@@ -105,6 +105,26 @@ def test_route_bit_exact(moe, ro, dev, tokens, experts, k):
     assert np.array_equal(slot_of.cpu().numpy(), ws)
 
 
+@pytest.mark.parametrize("tokens,experts,k", [(1, 1, 1), (256, 1024, 16), (257, 256, 4), (511, 32, 16), (512, 32, 16), (1023, 256, 8), (1024, 256, 8), (1024, 64, 7), (1024, 257, 4), (1025, 8, 4)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_route_in_one_workgroup_and_on_both_sides_of_its_limits(moe, ro, dev, tokens, experts, k, offset):
+    """Up to 256 or 1024 tokens in one workgroup, up to 1024 or 256 experts, less than 8192 rows; entries and slots on the
+    16-byte grid and off it; some entries are repeated or outside the experts."""
+    rng = np.random.default_rng(tokens * 31 + experts)
+    k = min(k, experts)
+    top = np.stack([rng.permutation(experts)[:k] for _ in range(tokens)]).astype(np.int32)
+    if k > 1:
+        top[::7, 1] = top[::7, 0]
+        top[::11, k - 1] = experts
+    flat = torch.full((tokens * k + offset,), -7, dtype=torch.int32, device=dev)
+    flat[offset:] = torch.from_numpy(top.ravel()).to(dev)
+    slots = torch.full((tokens * k + offset,), -9, dtype=torch.int32, device=dev)
+    out = (torch.full((experts + 1,), -9, dtype=torch.int32, device=dev), torch.full((tokens * k,), -9, dtype=torch.int32, device=dev), slots[offset:].view(tokens, k))
+    moe.route(flat[offset:].view(tokens, k), experts, out=out)
+    for got, want in zip(out, ro.route_ref(top, experts)):
+        assert np.array_equal(got.cpu().numpy(), want)
+
+
 def test_route_ignores_bad_and_repeated_entries(moe, ro, dev):
     rng = np.random.default_rng(9)
     top = np.stack([rng.permutation(6)[:3] for _ in range(700)]).astype(np.int32)
