@@ -73,7 +73,9 @@ inline int device_cus() {
 
 // Upper bound on the m-tile slots of a grouped call of `rows` rows: an expert of r rows starts up to 15 rows into its first
 // tile and has ceil((r + 15) / bm) <= 1 + r / (bm - 14) of them, and no more experts have rows than there are rows.
-inline long grouped_slots_bound(long rows, long experts, int bm) { return (rows < experts ? rows : experts) + rows / (bm - 14); }
+// (For row_offsets that do not descend; the kernel cuts the slots of any others here where it sums K partitions, whose
+// counters and partial tiles are laid out for this many.)
+__host__ __device__ inline long grouped_slots_bound(long rows, long experts, int bm) { return (rows < experts ? rows : experts) + rows / (bm - 14); }
 
 // mode: 0 dense bf16, 1 dense split-K partials, 2 grouped, 3 K blocks dealt, 4 dense split-K summed in the kernel, 5 grouped likewise.  tile: FP8BS_VARIANT_* (not AUTO) + 256 * form.
 hipError_t launch_gemm(int tile, int mode, const GemmArgs& args, hipStream_t stream);

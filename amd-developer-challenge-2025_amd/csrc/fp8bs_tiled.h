@@ -309,6 +309,10 @@ void gemm_tr_kernel(const GemmArgs p) {
                 total_slots += (hi > lo) ? (hi - (lo & ~15) + BM - 1) / BM : 0;
             }
         }
+        if constexpr (MODE == 5) {             // a malformed table must not reach beyond the workspace either
+            const int bound = (int)grouped_slots_bound(p.m, p.num_experts, BM);
+            total_slots = total_slots < bound ? total_slots : bound;
+        }
     }
     [[maybe_unused]] const int sk_self = xcd_virtual_id(blockIdx.x, gridDim.x);
     auto pick_tile = [&](int it) -> Tile {

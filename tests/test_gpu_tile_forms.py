@@ -150,3 +150,17 @@ def test_second_forms_are_named_and_planned(pkg, dev):
     for tile in (FORM(2, 1), FORM(4, 2), FORM(13, 0)):
         with pytest.raises(RuntimeError):
             pkg.custom_kernel(data, variant=tile, split_k=1)
+
+
+def test_grouped_split_keeps_to_its_workspace_with_a_malformed_table(pkg, dev):
+    """Row offsets that descend claim more tiles than the rows can give: the partial tiles stay inside the workspace."""
+    lib = pkg._lib.load()
+    experts, n, k = 6, 256, 512
+    data = _to(pkg.inputs.make_grouped(pkg.inputs.CONFIGS[4], tokens=96, n=n, k=k, experts=experts, topk=2), dev)
+    rows = data[0].shape[0]
+    table = torch.tensor([0, rows, 0, rows, 0, rows, 0], dtype=torch.int32, device=dev)
+    for tile, bm, bn in ((12, 64, 256), (FORM(12, 1), 128, 128), (FORM(4, 1), 64, 64)):
+        need = 16384 + (experts + rows // (bm - 14)) * (n // bn) * 2 * bm * bn * 4        # a header and two partial tiles per tile
+        ws = torch.full((need + (8 << 20),), 0xA5, dtype=torch.uint8, device=dev)
+        _grouped_ws(lib, data[:4] + (table, torch.empty_like(data[5])), tile, 2, ws[:need])
+        assert bool((ws[need:] == 0xA5).all()), "tile %#x" % tile
