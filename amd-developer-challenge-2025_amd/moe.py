@@ -61,7 +61,8 @@ def route(top_idx: torch.Tensor, experts: int, out: Optional[Tuple[torch.Tensor,
             _plan_cache.clear()
         need = _plan_cache[("route", t, experts)] = _lib.load().fp8bs_moe_route_workspace_bytes(t, experts)
     key = (dev.index, _stream_ptr(dev))
-    ws = _route_ws.get(key)
+    capturing = torch.cuda.is_current_stream_capturing()     # then from the graph's memory pool, see submission._workspace
+    ws = torch.empty(need, dtype=torch.uint8, device=dev) if capturing else _route_ws.get(key)
     if ws is None or ws.numel() < need:
         # A buffer that is outgrown stays alive until this stream's earlier kernels are done with it: the caching
         # allocator hands a freed block only to later work of the stream it was allocated on.

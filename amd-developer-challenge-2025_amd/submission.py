@@ -28,7 +28,10 @@ _workspaces = {}   # (device index, stream) -> uint8 tensor, grown on demand, re
 
 def _workspace(device: torch.device, nbytes: int, stream: int = 0) -> torch.Tensor:
     """The K split's partial planes: one buffer per device and stream, so that calls that overlap on two
-    streams do not write each other's planes."""
+    streams do not write each other's planes.  A call that is being captured takes a buffer of its own from the graph's
+    memory pool, which lives as long as the graph: one of the table could be outgrown, and freed, before a replay."""
+    if torch.cuda.is_current_stream_capturing():
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
     key = (device.index, stream)
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:

@@ -164,3 +164,39 @@ def test_grouped_split_keeps_to_its_workspace_with_a_malformed_table(pkg, dev):
         ws = torch.full((need + (8 << 20),), 0xA5, dtype=torch.uint8, device=dev)
         _grouped_ws(lib, data[:4] + (table, torch.empty_like(data[5])), tile, 2, ws[:need])
         assert bool((ws[need:] == 0xA5).all()), "tile %#x" % tile
+
+
+def test_captured_calls_keep_no_buffer_of_the_table(pkg, dev):
+    """A captured K split works in memory of its graph: a larger call, which outgrows the tables' buffers, and the caching
+    allocator's reuse of them leave the replays as they were."""
+    sub = __import__("importlib").import_module(pkg.__name__ + ".submission")
+    moe = __import__("importlib").import_module(pkg.__name__ + ".moe")
+    grouped = _to(pkg.inputs.make_grouped(pkg.inputs.CONFIGS[4], tokens=8, n=512, k=7168, experts=8, topk=2), dev)
+    dense = _to(pkg.inputs.make_dense(pkg.inputs.CONFIGS[2], m=64, n=512, k=7168), dev)
+    idx = torch.stack([torch.randperm(16)[:4] for _ in range(2048)]).to(torch.int32).to(dev)
+    assert pkg.plan(64, 512, 7168).workspace_bytes > 0
+    assert pkg._lib.load().fp8bs_grouped_workspace_bytes(8, grouped[0].shape[0], 512, 7168) > 0
+
+    def calls():
+        pkg.custom_kernel(dense)
+        pkg.grouped_kernel(grouped)
+        return (dense[4], grouped[5]) + tuple(moe.route(idx, 16))
+    want = [t.clone() for t in calls()]
+    torch.cuda.synchronize()
+    before = {k: v.data_ptr() for k, v in sub._workspaces.items()}, {k: v.data_ptr() for k, v in moe._route_ws.items()}
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = calls()
+    assert before == ({k: v.data_ptr() for k, v in sub._workspaces.items()}, {k: v.data_ptr() for k, v in moe._route_ws.items()})
+    for _ in range(3):
+        for t in out:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for t, w in zip(out, want):
+            assert torch.equal(t.view(torch.int16), w.view(torch.int16))
+        sub._workspaces.clear()
+        moe._route_ws.clear()
+        pkg.custom_kernel(dense, split_k=7)
+        torch.full((32 << 20,), 255, dtype=torch.uint8, device=dev)
+        torch.cuda.synchronize()
