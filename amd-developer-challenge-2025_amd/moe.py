@@ -60,16 +60,7 @@ def route(top_idx: torch.Tensor, experts: int, out: Optional[Tuple[torch.Tensor,
         if len(_plan_cache) >= _PLANS_MAX:
             _plan_cache.clear()
         need = _plan_cache[("route", t, experts)] = _lib.load().fp8bs_moe_route_workspace_bytes(t, experts)
-    key = (dev.index, _stream_ptr(dev))
-    capturing = torch.cuda.is_current_stream_capturing()     # then from the graph's memory pool, see submission._workspace
-    ws = torch.empty(need, dtype=torch.uint8, device=dev) if capturing else _route_ws.get(key)
-    if ws is None or ws.numel() < need:
-        # A buffer that is outgrown stays alive until this stream's earlier kernels are done with it: the caching
-        # allocator hands a freed block only to later work of the stream it was allocated on.
-        if ws is None and len(_route_ws) >= 16:      # streams come and go: keep the table bounded (oldest entry out)
-            _route_ws.pop(next(iter(_route_ws)))
-        ws = torch.empty(max(need, 4096), dtype=torch.uint8, device=dev)
-        _route_ws[key] = ws
+    ws = _workspace(dev, need, _stream_ptr(dev), _route_ws, 4096)
     _call(_lib.calls().moe_route, dev, top_idx.data_ptr(), t, experts, k, row_offsets.data_ptr(), row_map.data_ptr(),
           slot_of.data_ptr(), ws.data_ptr(), ws.numel())
     return row_offsets, row_map, slot_of

@@ -184,9 +184,11 @@ def test_captured_calls_keep_no_buffer_of_the_table(pkg, dev):
     want = [t.clone() for t in calls()]
     torch.cuda.synchronize()
     before = {k: v.data_ptr() for k, v in sub._workspaces.items()}, {k: v.data_ptr() for k, v in moe._route_ws.items()}
+    held = sum(map(len, sub._held.values()))
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         out = calls()
+    assert held == sum(map(len, sub._held.values()))
     assert before == ({k: v.data_ptr() for k, v in sub._workspaces.items()}, {k: v.data_ptr() for k, v in moe._route_ws.items()})
     for _ in range(3):
         for t in out:
@@ -200,3 +202,51 @@ def test_captured_calls_keep_no_buffer_of_the_table(pkg, dev):
         pkg.custom_kernel(dense, split_k=7)
         torch.full((32 << 20,), 255, dtype=torch.uint8, device=dev)
         torch.cuda.synchronize()
+
+
+def test_a_capture_begun_with_hip_itself(pkg, dev):
+    """No memory pool belongs to such a graph: its replays stay right when larger calls outgrow the stream's buffers and the
+    allocator hands out what was freed, with eager work between them."""
+    import ctypes
+    moe = __import__("importlib").import_module(pkg.__name__ + ".moe")
+    hip = ctypes.CDLL("libamdhip64.so")
+    def ok(status):
+        assert status == 0, "HIP status %d" % status
+    dense = _to(pkg.inputs.make_dense(pkg.inputs.CONFIGS[2], m=64, n=512, k=7168), dev)
+    idx = torch.stack([torch.randperm(16)[:4] for _ in range(2048)]).to(torch.int32).to(dev)
+    out = (torch.empty(17, dtype=torch.int32, device=dev), torch.empty(8192, dtype=torch.int32, device=dev), torch.empty(2048, 4, dtype=torch.int32, device=dev))
+    assert pkg.plan(64, 512, 7168).workspace_bytes > 0
+
+    def calls():
+        pkg.custom_kernel(dense)
+        moe.route(idx, 16, out=out)
+    side = torch.cuda.Stream()
+    graph, program = ctypes.c_void_p(), ctypes.c_void_p()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        calls()
+        torch.cuda.synchronize()
+        want = [t.clone() for t in (dense[4],) + out]
+        torch.cuda.synchronize()
+        stream = ctypes.c_void_p(side.cuda_stream)
+        ok(hip.hipStreamBeginCapture(stream, 2))                     # relaxed
+        try:
+            calls()
+        finally:
+            ok(hip.hipStreamEndCapture(stream, ctypes.byref(graph)))
+        ok(hip.hipGraphInstantiate(ctypes.byref(program), graph, None, None, 0))
+        for _ in range(3):
+            for t in (dense[4],) + out:
+                t.zero_()
+            ok(hip.hipGraphLaunch(program, stream))
+            torch.cuda.synchronize()
+            for t, w in zip((dense[4],) + out, want):
+                assert torch.equal(t, w)
+            pkg.custom_kernel(dense, split_k=56)
+            moe.route(idx.repeat(64, 1), 16)
+            kept = [torch.full((size,), 255, dtype=torch.uint8, device=dev) for size in (1 << 20, 2 << 20, 4 << 20, 8 << 20)]
+            ok(hip.hipGraphLaunch(program, stream))
+            torch.cuda.synchronize()
+            assert all(bool((t == 255).all()) for t in kept)         # nothing was written to memory that is another's now
+        ok(hip.hipGraphExecDestroy(program))
+        ok(hip.hipGraphDestroy(graph))
