@@ -501,7 +501,7 @@ static int dense_call(const void* a, const void* b, const float* a_scale, const 
         if (is_streaming_variant(variant) && !simple) return FP8BS_ERR_BAD_VARIANT;
         if (is_streaming_variant(variant) && variant != FP8BS_VARIANT_SKINNY64x144 && (m % 4) != 0) return FP8BS_ERR_BAD_VARIANT;   // only the planner's width repairs a
         if (split_k < 0) {
-            if (is_streaming_variant(variant) || variant == FP8BS_VARIANT_GENERIC) return FP8BS_ERR_BAD_VARIANT;   // K blocks are dealt by the tiled kernel only
+            if (is_streaming_variant(variant) || variant == FP8BS_VARIANT_GENERIC || form_of(tile) != 0) return FP8BS_ERR_BAD_VARIANT;   // K blocks are dealt by the tiled kernel's first forms only
             fill_plan(m, n, k, variant, 1, &plan, streamk_grid(variant, m, n, k, cus));
         } else {
             const bool in_kernel = split_k > 0 && (split_k & FP8BS_SPLIT_SUM_IN_KERNEL) != 0;

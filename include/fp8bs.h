@@ -136,8 +136,8 @@ int fp8bs_gemm(const void* a, const void* b, const float* a_scale, const float* 
  * (FP8BS_ERR_WORKSPACE if smaller), contents unspecified on entry (a counter carries the call's own tag, so
  * whatever an earlier use left there counts as zero), one call at a time per workspace.
  * split_k < 0: another one-launch form, K BLOCKS instead of tiles dealt to
- * the workgroups (one per place on the chip, G = min(places, tiles * K/128); the tiled variants only, else
- * FP8BS_ERR_BAD_VARIANT); a workgroup whose run of K blocks ends inside a tile leaves an fp32 partial tile in the
+ * the workgroups (one per place on the chip, G = min(places, tiles * K/128); the tiled variants in
+ * their first form only, else FP8BS_ERR_BAD_VARIANT); a workgroup whose run of K blocks ends inside a tile leaves an fp32 partial tile in the
  * workspace and raises a flag there, the workgroup that holds the tile's last K block waits for the flags (a
  * bounded number of polls), adds the partial tiles in ascending K to its own accumulators - a fixed order, so the
  * result is the same from run to run - and writes c.  Workspace: 16384 + G * tile_m * tile_n * 4 bytes
