@@ -34,8 +34,20 @@ class Plan(ctypes.Structure):
     ]
 
 
+SECOND_FORM_NAMES = {4: "t64x64s4", 12: "t128x128s4"}
 SPLIT_SUM_IN_KERNEL = 1 << 30        # FP8BS_SPLIT_SUM_IN_KERNEL
-MIN_VERSION = 300                    # fp8bs_version() of the first library whose fp8bs_plan_t has sum_in_kernel
+MIN_VERSION = 400                    # fp8bs_version() of the first library whose fp8bs_plan_t has form
+
+
+def planned_variant(plan: Plan) -> int:
+    """The variant argument that forces the planned tile, whichever form it is (FP8BS_VARIANT_FORM)."""
+    return plan.variant | (plan.form + 1) << 8
+
+
+def tile_name(variant: int) -> str:
+    """Name of a variant argument, plain or with a form."""
+    names = SECOND_FORM_NAMES if variant >> 8 == 2 else VARIANT_NAMES
+    return names.get(variant & 255, "variant %d" % variant)
 
 
 _lib = None
@@ -55,7 +67,7 @@ def load() -> ctypes.CDLL:
     lib.fp8bs_version.restype = i32
     lib.fp8bs_version.argtypes = []
     if lib.fp8bs_version() < MIN_VERSION:
-        # an older build fills a shorter fp8bs_plan_t than the Plan mirrored here
+        # an older build fills another fp8bs_plan_t than the Plan mirrored here
         raise RuntimeError("%s is version %d, this package needs %d or later: rebuild it with "
                            "`python amd-developer-challenge-2025_amd/build.py`" % (LIB_PATH, lib.fp8bs_version(), MIN_VERSION))
     lib.fp8bs_strerror.restype = ctypes.c_char_p

@@ -428,7 +428,7 @@ static int scratch_address(void** out, hipStream_t stream) {
 
 extern "C" {
 
-int fp8bs_version(void) { return 300; }      // 0.3.0: fp8bs_plan_t grew (sum_in_kernel)
+int fp8bs_version(void) { return 400; }      // 0.4.0: a plan is (variant, form): fp8bs_plan_t::form in the place of a reserved word
 
 const char* fp8bs_strerror(int status) {
     switch (status) {

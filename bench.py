@@ -291,7 +291,7 @@ def main():
         nsets = min(8, -(-3 * 256 * 2 ** 20 // by)) if hbm else 1
         sets = [gpu_dense_inputs(pkg, cfg, dev, cfg.seed + 100 * s) for s in range(nsets)]
         us, us_min = time_calls(lambda i: pkg.custom_kernel(sets[i % nsets], variant=variant, split_k=split), args.steps, args.warmup)
-        print(json.dumps({"only": {"config": cfg.name, "variant": pkg._lib.VARIANT_NAMES.get(variant, str(variant)), "split_k": split,
+        print(json.dumps({"only": {"config": cfg.name, "variant": pkg._lib.tile_name(variant), "split_k": split,
                                    "input_sets": nsets, "us": round(us, 2), "us_min": round(us_min, 2),
                                    "frac": round(by / us * 1e-3 / PEAK_HBM_GBS if hbm else fl / us * 1e-6 / PEAK_FP8_TFLOPS, 4),
                                    "bound": "hbm" if hbm else "mfma"}}))
@@ -343,7 +343,7 @@ def main():
     plan = pkg.plan(cfg2.m, cfg2.n, cfg2.k)
     traffic, prof = profiled_traffic()
     # only when the planned kernel is the profiled one do the profile's figures belong on this line
-    if pkg._lib.VARIANT_NAMES.get(plan.variant) != "t256x256" or plan.split_k != 1 or plan.stream_k != 0:
+    if pkg._lib.tile_name(pkg._lib.planned_variant(plan)) != "t256x256" or plan.split_k != 1 or plan.stream_k != 0:
         traffic, prof = None, {}
 
     result = {
@@ -352,7 +352,7 @@ def main():
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "fp8_e4m3fn x fp8_e4m3fn -> f32 -> bf16",
         "data": "synthetic",
         "config": {"workload": "cfg2: M=N=K=4096, A 1x128 / B 128x128 fp32 block scales, bf16 out, seed %d" % cfg2.seed,
-                   "variant": pkg._lib.VARIANT_NAMES.get(plan.variant, "variant %d" % plan.variant), "split_k": plan.split_k, "grid": plan.grid_x,
+                   "variant": pkg._lib.tile_name(pkg._lib.planned_variant(plan)), "split_k": plan.split_k, "grid": plan.grid_x,
                    "preheat_calls": preheated},
         "roofline": {"bound": "mfma", "achieved": round(achieved, 2), "peak": PEAK_FP8_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(achieved / PEAK_FP8_TFLOPS, 4), "traffic": traffic,

@@ -85,7 +85,9 @@ typedef struct fp8bs_plan_t {
     int32_t sum_in_kernel;  /* 1 (with split_k > 1): one launch - the workgroups of a tile's K partitions leave fp32
                                partial tiles in the workspace and the last one to finish adds them in ascending K and
                                writes c; 0: partial planes and a reduce kernel (two launches)      */
-    int32_t form;           /* form of the variant (0 unless the variant has two)  */
+    int32_t form;           /* form of the variant (0 unless the variant has two); a plan is run again by forcing
+                               FP8BS_VARIANT_FORM(variant, form), the variant alone names its first form, another
+                               tile with another workspace need where form is 1                    */
     uint64_t workspace_bytes;
 } fp8bs_plan_t;
 

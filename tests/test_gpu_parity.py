@@ -186,14 +186,14 @@ def test_seeded_random_shapes_through_the_planner(pkg, oracle, dev):
         cpu = pkg.inputs.make_dense(cfg, m=m, n=n, k=k)
         ref = oracle.ref_kernel(cpu)
         plan = pkg.plan(m, n, k)
-        seen.add((plan.variant, plan.split_k > 1))
+        seen.add(((plan.variant, plan.form), plan.split_k > 1))
         out = pkg.custom_kernel(_to(cpu, dev))
-        _check(oracle, out, ref, "shape %dx%dx%d planned variant %d split %d" % (m, n, k, plan.variant, plan.split_k))
+        _check(oracle, out, ref, "shape %dx%dx%d planned variant %d form %d split %d" % (m, n, k, plan.variant, plan.form, plan.split_k))
         split = int(rng.integers(2, 6))
         if plan.variant in (6, 7, 8) and m % 4:
             continue                                              # the streaming kernels cannot be forced on such an m
-        out = pkg.custom_kernel(_to(cpu, dev), variant=plan.variant, split_k=split)
-        _check(oracle, out, ref, "shape %dx%dx%d variant %d forced split %d" % (m, n, k, plan.variant, split))
+        out = pkg.custom_kernel(_to(cpu, dev), variant=pkg._lib.planned_variant(plan), split_k=split)
+        _check(oracle, out, ref, "shape %dx%dx%d variant %d form %d forced split %d" % (m, n, k, plan.variant, plan.form, split))
     assert len({v for v, _ in seen}) >= 3 and any(s for _, s in seen), "the draw should reach several tiles and a K split: %s" % sorted(seen)
 
 

@@ -14,3 +14,19 @@ def test_dealt_k_blocks_are_refused_for_a_second_form(pkg):
         assert lib.fp8bs_gemm_ex(ONE, ONE, ONE, ONE, ONE, None, 0, 256, 512, 1024, FORM(variant, 1), -1, None) == BAD_VARIANT
         assert lib.fp8bs_gemm_ex(ONE, ONE, ONE, ONE, ONE, None, 0, 256, 512, 1024, FORM(variant, 0), -1, None) == WORKSPACE
         assert lib.fp8bs_gemm_ex(ONE, ONE, ONE, ONE, ONE, None, 0, 256, 512, 1024, variant, -1, None) == WORKSPACE
+
+
+def test_a_plan_is_run_again_and_named_with_its_form(pkg):
+    """The variant alone names its first form: another tile, with another name and another workspace need."""
+    lib, second = pkg._lib.load(), 0
+    for m, n, k in [(512, 2048, 1024), (1024, 1536, 7168), (2048, 1152, 4096), (640, 1536, 7168), (64, 18432, 7168), (4096, 4096, 4096), (4096, 2112, 7168)]:
+        p = pkg.plan(m, n, k)
+        again = pkg._lib.planned_variant(p)
+        assert "%dx%d" % (p.tile_m, p.tile_n) in pkg._lib.tile_name(again)
+        second += p.form
+        if p.sum_in_kernel:
+            split = p.split_k | pkg._lib.SPLIT_SUM_IN_KERNEL
+            assert lib.fp8bs_gemm_ex(ONE, ONE, ONE, ONE, ONE, ONE, p.workspace_bytes - 4, m, n, k, again, split, None) == WORKSPACE
+    assert second >= 2
+    assert [pkg._lib.tile_name(v) for v in (0, 2, 12, FORM(12, 0), FORM(12, 1), 4, FORM(4, 1))] == ["auto", "t256x256", "t64x256s3", "t64x256s3", "t128x128s4", "t64x128", "t64x64s4"]
+    assert lib.fp8bs_version() >= 400
