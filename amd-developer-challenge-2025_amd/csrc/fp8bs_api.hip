@@ -310,7 +310,8 @@ bool can_split_grouped(const GroupedPlan& p, int experts, int rows, int n, int k
 // costs 2.2 % against the best of each shape in the geometric mean and takes 17 % off the rule it replaced (the 256x256
 // tile above 32 rows per expert on average, 64x256 below): 194 tokens to 4 of 16 experts, 1299 x 5760: 90.8 -> 49.2 us;
 // 801 to 4 of 8, 840 x 1664: 23.2 -> 15.0; 35 to 4 of 8, 1375 x 5504: 43.6 -> 22.8.
-GroupedPlan make_grouped_plan(int experts, int rows, int n, int k, int num_cus, bool may_split) {
+// split 0: as many partitions as finish soonest; else that many, {.., 1} if no tile can.
+GroupedPlan make_grouped_plan(int experts, int rows, int n, int k, int num_cus, int split) {
     struct Cand { int tile; int rmax; double t_full, t_few, t_power, t_fixed, shared, bw; };
     const Cand cands[5] = {
         {FP8BS_VARIANT_T256x256, 1, 2.010, 1.259, 1.681, 6.01, 1.0, 5.18},
@@ -333,10 +334,11 @@ GroupedPlan make_grouped_plan(int experts, int rows, int n, int k, int num_cus, 
         double fill = (average / slots + 24.0) / vi.bm;
         if (fill > 1.0) fill = 1.0;
         const double t_alone = c.t_few + (c.t_full - c.t_few) * fill;
-        for (int s = 1; s <= 4; s++) {
+        for (int s = split ? split : 1; s <= (split ? split : 4); s++) {
             const GroupedPlan p{c.tile, s};
+            if (s > 1 && !can_split_grouped(p, experts, rows, n, k)) break;
             // (partial tiles of 64 MB at most: beyond that a call has tiles enough without a split)
-            if (s > 1 && (!may_split || kbt / s < 2 || !can_split_grouped(p, experts, rows, n, k) || grouped_bytes(p, experts, rows, n) > (64u << 20))) break;
+            if (s > 1 && !split && (kbt / s < 2 || grouped_bytes(p, experts, rows, n) > (64u << 20))) break;
             const double wgs = active * slots * (double)cdiv(n, vi.bn) * s, per_round = (double)num_cus * c.rmax, kb = (double)cdiv(kbt, s);
             auto t_block = [&](double w) {
                 double t = t_alone * (w > num_cus && c.rmax > 1 ? c.shared : 1.0);
@@ -353,10 +355,10 @@ GroupedPlan make_grouped_plan(int experts, int rows, int n, int k, int num_cus, 
     }
     return best;
 }
-GroupedPlan choose_grouped(int experts, int rows, int n, int k, int num_cus, bool may_split) {
+GroupedPlan choose_grouped(int experts, int rows, int n, int k, int num_cus, int split) {
     static thread_local PlanMemo<GroupedPlan> memo;
     if (num_cus <= 0) num_cus = 256;
-    return memo.get({experts, rows, n, k, num_cus, may_split}, [&](GroupedPlan* plan) { *plan = make_grouped_plan(experts, rows, n, k, num_cus, may_split); });
+    return memo.get({experts, rows, n, k, num_cus, split}, [&](GroupedPlan* plan) { *plan = make_grouped_plan(experts, rows, n, k, num_cus, split); });
 }
 
 // The value a flag takes in one call that deals K blocks: never zero, different from call to call (and, through
@@ -575,6 +577,8 @@ static int grouped_call(const void* a, const void* b, const float* a_scale, cons
                         int num_experts, int rows, int n, int k, int variant, int split_k, int epi, void* ws, size_t ws_bytes, void* stream) {
     if (num_experts <= 0) return FP8BS_ERR_BAD_OFFSETS;
     if (!row_offsets) return FP8BS_ERR_NULL_POINTER;
+    if (split_k < 0) return FP8BS_ERR_BAD_VARIANT;               // K blocks are dealt in dense calls only
+    split_k &= ~FP8BS_SPLIT_SUM_IN_KERNEL;                       // the only form a grouped split has
     int st = check_common(a, b, a_scale, b_scale, c, rows, n, k);
     if (st != FP8BS_OK) return st;
     if (rows == 0 || n == 0) return FP8BS_OK;
@@ -593,8 +597,12 @@ static int grouped_call(const void* a, const void* b, const float* a_scale, cons
     GroupedPlan plan{forced_tile(variant), split_k > 1 ? split_k : 1};
     if (k == 0 && variant == FP8BS_VARIANT_AUTO) plan = {FP8BS_VARIANT_GENERIC, 1};
     else if (variant == FP8BS_VARIANT_AUTO) {
-        plan = choose_grouped(num_experts, rows, n, k, fp8bs::device_cus(), true);
-        if (plan.split > 1 && (!ws || ws_bytes < grouped_bytes(plan, num_experts, rows, n))) plan = choose_grouped(num_experts, rows, n, k, fp8bs::device_cus(), false);
+        plan = choose_grouped(num_experts, rows, n, k, fp8bs::device_cus(), split_k);
+        if (split_k > 1 && plan.split != split_k) return FP8BS_ERR_BAD_VARIANT;      // no tile takes this split of this call
+        if (plan.split > 1 && (!ws || ws_bytes < grouped_bytes(plan, num_experts, rows, n))) {
+            if (split_k > 1) return FP8BS_ERR_WORKSPACE;
+            plan = choose_grouped(num_experts, rows, n, k, fp8bs::device_cus(), 1);
+        }
     } else {
         VariantInfo vi{};
         if (!variant_info(plan.tile, &vi) || is_streaming_variant(plan.tile)) return FP8BS_ERR_BAD_VARIANT;   // no grouped mode in the streaming kernels
@@ -612,7 +620,7 @@ static int grouped_call(const void* a, const void* b, const float* a_scale, cons
 
 size_t fp8bs_grouped_workspace_bytes(int num_experts, int total_rows, int n, int k) {
     if (num_experts <= 0 || total_rows <= 0 || n <= 0 || k <= 0 || (k % KBLK) != 0) return 0;
-    return (size_t)grouped_bytes(choose_grouped(num_experts, total_rows, n, k, fp8bs::device_cus(), true), num_experts, total_rows, n);
+    return (size_t)grouped_bytes(choose_grouped(num_experts, total_rows, n, k, fp8bs::device_cus(), 0), num_experts, total_rows, n);
 }
 
 size_t fp8bs_silu_mul_workspace_bytes(int rows, int n, int k) {
@@ -647,7 +655,7 @@ int fp8bs_gemm_silu_mul_ws(const void* a, const void* b, const float* a_scale, c
     if (split_k < 0) return FP8BS_ERR_BAD_VARIANT;               // K blocks are dealt without an epilogue only
     // any even n and any operand alignment: rows of h that do not keep 16-byte stores aligned are stored in pieces
     if (row_offsets)
-        return grouped_call(a, b, a_scale, b_scale, h, row_offsets, num_experts, rows, n, k, variant, split_k & ~FP8BS_SPLIT_SUM_IN_KERNEL, 1, ws, ws_bytes, stream);
+        return grouped_call(a, b, a_scale, b_scale, h, row_offsets, num_experts, rows, n, k, variant, split_k, 1, ws, ws_bytes, stream);
     return dense_call(a, b, a_scale, b_scale, h, ws, ws_bytes, rows, n, k, variant, split_k, 1, stream);
 }
 

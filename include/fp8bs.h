@@ -196,8 +196,12 @@ int fp8bs_gemm_grouped_ex(const void* a, const void* b, const float* a_scale, co
  * in the workspace, summed in ascending K by the last workgroup to finish a tile, as in fp8bs_gemm_ex with
  * FP8BS_SPLIT_SUM_IN_KERNEL).  variant = FP8BS_VARIANT_AUTO and split_k = 0 let the library choose; without a workspace of
  * fp8bs_grouped_workspace_bytes(...) bytes it chooses what needs none.  A forced split_k > 1 takes a tile that has the
- * form (FP8BS_VARIANT_T64x256S3 in both forms, form 1 of FP8BS_VARIANT_T64x128; else FP8BS_ERR_BAD_VARIANT).  Contents of
- * the workspace unspecified on entry, one call at a time per workspace. */
+ * form (FP8BS_VARIANT_T64x256S3 in both forms, form 1 of FP8BS_VARIANT_T64x128; else FP8BS_ERR_BAD_VARIANT), with
+ * FP8BS_VARIANT_AUTO the one of them that the model picks; split_k = 1 takes none, split_k < 0 is FP8BS_ERR_BAD_VARIANT.
+ * A forced split needs 16384 + tiles * split_k * tile_m * tile_n * 4 bytes, tiles = (min(total_rows, num_experts) +
+ * total_rows / (tile_m - 14)) * ceil(n / tile_n) (FP8BS_ERR_WORKSPACE if there are fewer; FP8BS_ERR_BAD_VARIANT with more
+ * than 2016 tiles, more than 255 partitions or more than K has blocks).  Contents of the workspace unspecified on entry,
+ * one call at a time per workspace. */
 int fp8bs_gemm_grouped_ws(const void* a, const void* b, const float* a_scale, const float* b_scale,
                           void* c, const int32_t* row_offsets, int num_experts, int total_rows,
                           int n, int k, int variant, int split_k, void* ws, size_t ws_bytes, void* stream);

@@ -250,3 +250,14 @@ def test_a_capture_begun_with_hip_itself(pkg, dev):
             assert all(bool((t == 255).all()) for t in kept)         # nothing was written to memory that is another's now
         ok(hip.hipGraphExecDestroy(program))
         ok(hip.hipGraphDestroy(graph))
+
+
+def test_grouped_split_with_the_tile_left_to_the_library(pkg, dev):
+    """A split given with FP8BS_VARIANT_AUTO is the split that runs: the bits of the tiles that have the form, with as many."""
+    lib = pkg._lib.load()
+    data = _to(pkg.inputs.make_grouped(pkg.inputs.CONFIGS[4], tokens=37, n=518, k=1152, experts=5, topk=2), dev)
+    ws = torch.randint(0, 256, (64 << 20,), dtype=torch.uint8, device=dev)
+    fresh = lambda: data[:5] + (torch.full_like(data[5], float("nan")),)
+    for split in (1, 2, 3, 9):
+        want = _grouped_ws(lib, fresh(), 12, split, ws)
+        assert torch.equal(_grouped_ws(lib, fresh(), 0, split, ws).view(torch.int16), want.view(torch.int16)), split

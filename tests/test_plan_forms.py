@@ -30,3 +30,16 @@ def test_a_plan_is_run_again_and_named_with_its_form(pkg):
     assert second >= 2
     assert [pkg._lib.tile_name(v) for v in (0, 2, 12, FORM(12, 0), FORM(12, 1), 4, FORM(4, 1))] == ["auto", "t256x256", "t64x256s3", "t64x256s3", "t128x128s4", "t64x128", "t64x64s4"]
     assert lib.fp8bs_version() >= 400
+
+
+def test_a_forced_grouped_split_is_honoured_or_refused(pkg):
+    """Also with the tile left to the library, as in a dense call: a split that cannot be done, or not with this workspace,
+    is an error and not another split."""
+    lib = pkg._lib.load()
+    for fn in (lib.fp8bs_gemm_grouped_ws, lib.fp8bs_gemm_silu_mul_ws):
+        call = lambda variant, split, k=1024: fn(ONE, ONE, ONE, ONE, ONE, ONE, 4, 64, 256, k, variant, split, None, 0, None)
+        for variant in (0, 12, FORM(4, 1)):
+            assert call(variant, 2) == WORKSPACE and call(variant, 2 | pkg._lib.SPLIT_SUM_IN_KERNEL) == WORKSPACE
+            assert call(variant, 9) == BAD_VARIANT                          # more partitions than K blocks
+            assert call(variant, -1) == BAD_VARIANT
+        assert call(2, 2) == BAD_VARIANT                                    # a tile without the form
