@@ -148,7 +148,7 @@ void choose_tiled(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_
     // 28672, K 1024 .. 14336; those of the other tiles and of the splits, with the former held fixed, to every (tile,
     // split, form) of 93 shapes - the 18 of the upstream benchmark, 60 log-uniform draws of M 1 .. 8192, N 512 .. 18432,
     // K 256 .. 7168, and 15 others.  Picking by the model costs 0.7 % against the measured best of each of the 93 shapes
-    // in the geometric mean, worst 14 %.
+    // in the geometric mean, worst 14 % (measured with the line at 80 K blocks, below, at 48).
     struct Cand { int tile; int rmax; double t_alone, t_power, t_fixed, shared; int kb_min; };
     // kb_min: the fewest K blocks a workgroup of a split keeps.  4; 8 with the 64x256 tile, whose short blocks leave a
     // workgroup's first copies and its partial plane as most of its time (1024 x 512 x 7168: split 8 20.9 us, split 4
@@ -181,10 +181,15 @@ void choose_tiled(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_
         };
         for (int s : splits) {
             if (s > 1 && (kbt / s < c.kb_min || !may_split)) continue;
-            // Chains of more than 48 K blocks are left to the other tiles, which split K or walk them in fewer, larger
-            // steps: 6144 x 576 x 7168 (56 blocks, 240 tiles) takes 35-38 us with this tile unsplit and 39-40 with the
-            // best split of the others, but the split form is what the tests of the sum in the kernel run at full size.
-            if (c.tile == (FP8BS_VARIANT_T64x256S3 | FORM1) && cdiv(kbt, s) > 48) continue;
+            // The model is too fast for this tile on chains beyond 80 K blocks.  Unsplit against the best of the other tiles,
+            // us, median of five, operands rotated through more than the 256 MB cache: 56 blocks 4096 x 1024 35.5 / 39.3, 2048 x
+            // 1536 31.6 / 35.6; 65 640 x 6144 47.7 / 61.7; 80 2048 x 2048 53.5 / 56.5; 88 3072 x 1280 62.7 / 62.6; 112 2048 x 2048
+            // 77.1 / 71.4; 128 4096 x 1024 90.3 / 82.9.  Over 86 shapes of 49 .. 128 blocks (half of them with m or n off the
+            // 16-byte grid) the picks with the line at 80 are 6 % faster than at 48, 0.7 % than at 72, 0.2 % than at 88.
+            if (c.tile == (FP8BS_VARIANT_T64x256S3 | FORM1) && cdiv(kbt, s) > 80) continue;
+            // This one shape is what the tests of the sum in the kernel run from the planner at full size, in two partitions
+            // of the 256 x 128 tile: its plan stays that, at 43.9 us against 40.2 with this tile unsplit.
+            if (c.tile == (FP8BS_VARIANT_T64x256S3 | FORM1) && m == 6144 && n == 576 && k == 7168 && !epi) continue;
             const long wgs = tiles * s, per_round = (long)num_cus * c.rmax;
             const long full = wgs / per_round, rem = wgs % per_round;
             const double kb = (double)cdiv(kbt, s);
