@@ -43,6 +43,7 @@ struct QuantArgs {
     int64_t ldx;              // elements between input rows
     int rows, k, src_rows;    // output rows, K, rows of the input matrix (row_map targets)
     int nb;                   // per-block mode: ceil(rows/128)
+    int row0;                 // first row of this launch
 };
 
 static constexpr int TK = 128;
@@ -146,7 +147,7 @@ void quantize_kernel(const QuantArgs p) {
     __shared__ uint32_t wave_max[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int g = lane >> 5, l = lane & 31;
-    const int kb = blockIdx.x, m0 = blockIdx.y * ROWS;
+    const int kb = blockIdx.x, m0 = p.row0 + blockIdx.y * ROWS;
     __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
         (void*)p.x, 0, (uint32_t)((size_t)p.src_rows * (size_t)p.ldx * sizeof(T)), 0x00020000);
 
@@ -191,7 +192,7 @@ void quantize_kernel(const QuantArgs p) {
         if (lane == 0) wave_max[wave] = mx;
         __syncthreads();
         bscale = scale_of(umax(umax(wave_max[0], wave_max[1]), umax(wave_max[2], wave_max[3])));
-        if (tid == 0) p.scale[(size_t)kb * p.nb + blockIdx.y] = bscale;
+        if (tid == 0) p.scale[(size_t)kb * p.nb + m0 / ROWS] = bscale;
     }
     // ---- quantise, transpose 4x4 bytes, stage in LDS ----
     const float bscale_rcp = refine_rcp(bscale);
@@ -270,11 +271,18 @@ void quantize_kernel(const QuantArgs p) {
 }
 
 template <typename T, bool PER_BLOCK, int ROWS>
-static hipError_t launch_quant_rows(const QuantArgs& a, hipStream_t stream) {
-    dim3 grid((unsigned)(a.k / TK), (unsigned)((a.rows + ROWS - 1) / ROWS));
-    if (a.row_map) hipLaunchKernelGGL((quantize_kernel<T, PER_BLOCK, true, ROWS>), grid, dim3(256), 0, stream, a);
-    else hipLaunchKernelGGL((quantize_kernel<T, PER_BLOCK, false, ROWS>), grid, dim3(256), 0, stream, a);
-    return hipGetLastError();
+static hipError_t launch_quant_rows(QuantArgs a, hipStream_t stream) {
+    // a grid has 65535 places in y: one launch per that many workgroups of rows (rows * k < 2^32 keeps rows below 2^25)
+    constexpr int MAX_Y = 65535;
+    for (a.row0 = 0; a.row0 < a.rows; a.row0 += MAX_Y * ROWS) {
+        const int groups = (a.rows - a.row0 + ROWS - 1) / ROWS;
+        dim3 grid((unsigned)(a.k / TK), (unsigned)(groups < MAX_Y ? groups : MAX_Y));
+        if (a.row_map) hipLaunchKernelGGL((quantize_kernel<T, PER_BLOCK, true, ROWS>), grid, dim3(256), 0, stream, a);
+        else hipLaunchKernelGGL((quantize_kernel<T, PER_BLOCK, false, ROWS>), grid, dim3(256), 0, stream, a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 // Rows of a workgroup, us measured with 128 / 64 / 32 of them (bf16, inputs from HBM): few values finish soonest in small
@@ -478,7 +486,7 @@ int quantize_common(const void* x, int dtype, int64_t ldx, const int32_t* row_ma
     if (((uintptr_t)x & 15) != 0 || ((ldx * esz) & (dtype == FP8BS_DTYPE_F32 ? 15 : 7)) != 0) return FP8BS_ERR_BAD_SHAPE;
     if ((size_t)rows * (size_t)k > 0xFFFFFFFFull) return FP8BS_ERR_TOO_LARGE;
     if ((size_t)(row_map ? src_rows : rows) * (size_t)ldx * (size_t)esz > 0xFFFFFFFFull) return FP8BS_ERR_TOO_LARGE;   // buffer addressing
-    fp8bs::QuantArgs a{x, row_map, (uint8_t*)q, scale, ldx, rows, k, row_map ? src_rows : rows, (rows + 127) / 128};
+    fp8bs::QuantArgs a{x, row_map, (uint8_t*)q, scale, ldx, rows, k, row_map ? src_rows : rows, (rows + 127) / 128, 0};
     hipStream_t s = (hipStream_t)stream;
     hipError_t e;
     if (dtype == FP8BS_DTYPE_F32) e = per_block ? fp8bs::launch_quant<float, true>(a, s) : fp8bs::launch_quant<float, false>(a, s);

@@ -1,0 +1,80 @@
+"""Launches of very tall matrices stay inside the documented grid limit of 65535 in y and still cover every row.
+
+On the CPU the launches are recorded instead of made: a small library loaded ahead of the HIP runtime takes the launch
+configuration that hipcc's host code hands over, and declines.  No pointer is dereferenced."""
+import importlib
+import json
+import subprocess
+import sys
+
+import pytest
+import torch
+
+SHIM = r"""
+#include <stdint.h>
+#include <stdio.h>
+typedef struct { uint32_t x, y, z; } grid3;
+int __hipPushCallConfiguration(grid3 g, grid3 b, size_t lds, void* stream) {
+    (void)lds; (void)stream;
+    printf("[%u, %u, %u, %u]\n", g.x, g.y, g.z, b.x); fflush(stdout);
+    return 1;
+}
+int hipGetLastError(void) { return 0; }
+"""
+CALL = r"""
+import ctypes, sys
+ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+lib = ctypes.CDLL(sys.argv[2])
+one = ctypes.c_void_p(1 << 20)
+fn, dtype, gathered, rows, k = sys.argv[3], int(sys.argv[4]), int(sys.argv[5]), int(sys.argv[6]), int(sys.argv[7])
+if fn == "a":
+    st = lib.fp8bs_quantize_a(one, dtype, ctypes.c_int64(k), one if gathered else None, 1000 if gathered else rows, one, one, rows, k, None)
+else:
+    st = lib.fp8bs_quantize_b(one, dtype, ctypes.c_int64(k), one, one, rows, k, None)
+assert st == 0, st
+"""
+
+
+@pytest.fixture(scope="module")
+def shim(tmp_path_factory):
+    d = tmp_path_factory.mktemp("shim")
+    (d / "shim.c").write_text(SHIM)
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", str(d / "shim.so"), str(d / "shim.c")], check=True)
+    return str(d / "shim.so")
+
+
+@pytest.mark.parametrize("fn,dtype,gathered,rows,k", [("a", 1, 1, 65535 * 32, 128), ("a", 1, 1, 65535 * 32 + 1, 128), ("a", 1, 1, 16000001, 256), ("a", 0, 0, 65535 * 64 + 1, 128),
+                                                      ("a", 0, 0, 8388607, 128), ("a", 1, 0, 16777215, 128), ("b", 1, 0, 65535 * 128, 128), ("b", 1, 0, 65535 * 128 + 1, 128),
+                                                      ("a", 1, 0, 300, 256), ("b", 0, 0, 129, 128)])
+def test_rows_beyond_the_grid_limit(pkg, shim, fn, dtype, gathered, rows, k):
+    out = subprocess.run([sys.executable, "-c", CALL, shim, pkg._lib.LIB_PATH, fn, str(dtype), str(gathered), str(rows), str(k)],
+                         check=True, stdout=subprocess.PIPE, text=True, timeout=100).stdout
+    grids = [json.loads(line) for line in out.splitlines()]
+    assert grids and all(g[0] == k // 128 and 1 <= g[1] <= 65535 and g[2] == 1 and g[3] == 256 for g in grids), grids
+    assert sum(g[1] for g in grids) in [-(-rows // r) for r in ((128,) if fn == "b" else (32, 64, 128))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,rows", [("gathered", 65535 * 32 + 33), ("f32", 65535 * 64 + 70), ("b", 65535 * 128 + 200)])
+def test_values_on_both_sides_of_the_grid_limit(kind, rows):
+    """The rows of the second launch: the bytes and scales of the same rows quantised on their own."""
+    quant = importlib.import_module("amd-developer-challenge-2025_amd.quant")
+    dev = torch.device("cuda:0")
+    base = torch.randn(1024, 128, generator=torch.Generator().manual_seed(3)) * torch.logspace(-3, 3, 1024)[:, None]
+    base = base.to(torch.float32 if kind == "f32" else torch.bfloat16).to(dev)
+    if kind == "gathered":
+        rmap = (torch.arange(rows, dtype=torch.int64, device=dev) * 7 % 1024).to(torch.int32)
+        q, s = quant.quantize_a(base, rmap, fused=True)
+    else:
+        rmap = torch.arange(rows, device=dev) % 1024
+        q, s = (quant.quantize_b if kind == "b" else quant.quantize_a)(base.repeat(-(-rows // 1024), 1)[:rows])
+    at = rmap.long()
+    if kind == "b":
+        wq, ws = quant.quantize_b(base)
+        whole = rows // 128                                                    # (the last block has other rows, and may have another maximum)
+        assert torch.equal(s[:whole, 0], ws[torch.arange(whole, device=dev) % 8, 0])
+        rows = whole * 128
+    else:
+        wq, ws = quant.quantize_a(base)
+        assert torch.equal(s[:, 0], ws[:, 0][at])
+    assert torch.equal(q.t()[:, :rows].view(torch.uint8), wq.t().view(torch.uint8)[:, at[:rows]])
