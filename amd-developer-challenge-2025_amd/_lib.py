@@ -152,11 +152,17 @@ _calls = None
 
 def calls():
     """The compute entry points by name without their prefix (calls().gemm_ex(...) -> status): the CPython binding
-    where it is built, else the library's functions through ctypes."""
+    where it is built, else (with one warning, where a build older than this file lacks some) the library's functions
+    through ctypes."""
     global _calls
     if _calls is None:
         mod = pycall()
-        if mod is None or any(not hasattr(mod, name) for name in _CALLS):
+        missing = [name for name in _CALLS if mod is not None and not hasattr(mod, name)]
+        if missing:
+            import warnings
+            warnings.warn("_fp8bs_pycall.so lacks %s; binding libfp8bs.so through ctypes instead, which costs host time in every "
+                          "call: rebuild it with `python amd-developer-challenge-2025_amd/build.py`" % ", ".join(missing))
+        if mod is None or missing:
             lib = load()
             mod = types.SimpleNamespace(**{name: getattr(lib, "fp8bs_" + name) for name in _CALLS})
         _calls = mod

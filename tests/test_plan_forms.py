@@ -1,6 +1,10 @@
 """Plans and forced arguments that name one of the two forms of a variant, or a K split: honoured or refused, never
 something else run in their place.  Host checks only: every call here returns before a launch."""
 import ctypes
+import types
+import warnings
+
+import pytest
 
 ONE = ctypes.c_void_p(16)                                    # never dereferenced
 FORM = lambda variant, form: variant | (form + 1) << 8      # FP8BS_VARIANT_FORM
@@ -55,3 +59,17 @@ def test_long_chains_take_the_tile_that_measures_fastest(pkg):
     for m, n, k in [(2048, 2048, 14336), (4096, 1024, 16384)]:
         p = pkg.plan(m, n, k)
         assert (p.tile_m, p.tile_n, p.split_k, p.sum_in_kernel) == (256, 128, 2, 1), (m, n, k)
+
+
+def test_an_incomplete_binding_is_named(pkg, monkeypatch):
+    """A CPython binding built before a function was added to it gives way to ctypes with a warning that says so."""
+    lib_mod, whole = pkg._lib, pkg._lib.pycall()
+    stale = types.SimpleNamespace(**{name: getattr(whole, name) for name in lib_mod._CALLS if name not in ("quantize_a", "moe_route")})
+    monkeypatch.setattr(lib_mod, "_pycall", stale)
+    monkeypatch.setattr(lib_mod, "_calls", None)
+    with pytest.warns(UserWarning, match="quantize_a, moe_route"):
+        calls = lib_mod.calls()
+    assert all(hasattr(calls, name) for name in lib_mod._CALLS)
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert lib_mod.calls() is calls                                     # once
