@@ -53,10 +53,9 @@ def test_one_correction_is_exact_for_bf16(maxima):
                 assert one_step(Fraction(x), s, y) == want, (float(s), x)
 
 
-@pytest.mark.gpu
-def test_every_pair_of_bf16_significands():
-    """Every (maximum, x) pair of significands at ten exponent distances, both signs, and -0: the CPU quantiser's bytes."""
-    quant = importlib.import_module("amd-developer-challenge-2025_amd.quant")
+def _every_pair(exponent):
+    """Every (maximum, x) pair of significands at ten exponent distances, both signs, and -0; the rows of distance `gap` are
+    scaled by 2^(7 gap + exponent)."""
     sig = torch.arange(128, 256, dtype=torch.float32)
     rows = []
     for gap in range(10):
@@ -67,10 +66,21 @@ def test_every_pair_of_bf16_significands():
             lo, hi = x.clone(), x.clone()
             lo[0], hi[127] = a, -a                            # both halves hold the maximum; together they hold every x
             lo[1 + gap] = -0.0
-            rows.append(torch.cat([lo, hi]) * 2.0 ** (7 * gap - 40))
-    x = torch.stack(rows).to(torch.bfloat16)
+            rows.append(torch.cat([lo, hi]) * 2.0 ** (7 * gap + exponent))
+    return torch.stack(rows).to(torch.bfloat16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("exponent", [-40, -30])
+def test_every_pair_of_bf16_significands(exponent):
+    """The CPU quantiser's bytes.  At -30 every scale is max / 448, also at distance 0, where x is within a factor of two of the
+    maximum; at -40 the rows of distance 0 have the smallest scale, 1e-12."""
+    quant = importlib.import_module("amd-developer-challenge-2025_amd.quant")
+    x = _every_pair(exponent)
     q, s = quant.quantize_a(x.cuda())
     rq, rs = inputs.quantize_a(x.float())
+    least = torch.tensor(1e-12, dtype=torch.float32)
+    assert bool((rs[:128] == least).all() if exponent == -40 else (rs > least).all()) and bool((rs[128:] > least).all())
     assert torch.equal(s.cpu(), rs)
     assert torch.equal(q.cpu().view(torch.uint8), rq.view(torch.uint8))
 
