@@ -61,7 +61,7 @@ def build(verbose: bool = False, jobs: int = 0) -> str:
 
 
 def build_pycall(verbose: bool = False) -> str:
-    """The CPython binding of the two GEMM entry points (csrc/fp8bs_pycall.c): host compiler, linked against
+    """The CPython binding of the compute entry points (csrc/fp8bs_pycall.c): host compiler, linked against
     libfp8bs.so next to it.  Replaces ctypes' argument marshalling on the hot call path only."""
     import sysconfig
     cc = os.environ.get("CC", "gcc")

@@ -126,8 +126,8 @@ void fill_plan(int m, int n, int k, int tile, int split_k, fp8bs_plan_t* out, in
 
 // Rows of c (n bf16) that keep 16-byte stores aligned: what the streaming kernels need (forced variants only;
 // the tiled kernels take any m and n in every mode: they repair the last bytes of a and b themselves, store a
-// row's last chunk of c in pieces and write the partial planes of a K split element by element where rows do not
-// end on a group of four).
+// row's last chunk of c in pieces and write the partial planes of a K split with stores that need no more than a float's
+// alignment, element by element only in a row's last group of four where the row ends inside it).
 bool vector_shape(int n) { return (n % 8) == 0; }
 
 // At most 64 rows against a b of 24 MB or more: the call streams b from HBM once and everything else is small.
@@ -205,7 +205,8 @@ void choose_tiled(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_
             const bool fuse = (s == 2 || s == 3) && can_sum_in_kernel(m, n, c.tile, s) && in_kernel < planes;
             if (s > 1) cost += fuse ? in_kernel : planes;
             // calls issued one after another are never faster than the host launches them: the reduce launch of a split
-            // pays only beyond that (2 x 700 x 3200 in eight partitions: done on the GPU after 7.2 us, 9.5 us a call)
+            // pays only beyond that (2 x 700 x 3200 in eight partitions: done on the GPU after 7.2 us, 9.5 us a call).  These are
+            // Python callers' launches; a captured graph or a C program, whose launches cost less, is given the same plan.
             const double host = s > 1 && !fuse ? 7.8 : 4.5;
             if (cost < host) cost = host;
             if (best_tile == 0 || cost < best_cost) { best_tile = c.tile; best_split = s; best_cost = cost; best_fused = fuse; }

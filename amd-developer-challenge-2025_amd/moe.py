@@ -73,6 +73,7 @@ def gate_up_silu(data):
     every expert K-major (or [n, k] K-major with ``row_offsets=None`` for one dense weight); ``h`` is
     bf16 [rows, n/2].  Role of re_silu_mul_kernel (2-amd-moe/amd-moe-submission.py:366-407) fused as in
     2-amd-moe/5-amd-fp8-moe-hip-fuse.py:366-408.  Fills and returns ``h``.
+    A call that splits K keeps its workspace (grouped: up to 64 MiB) for this device and stream, the one `custom_kernel` uses.
     """
     a, b, a_scale, b_scale, row_offsets, h = data
     if a.dim() != 2:

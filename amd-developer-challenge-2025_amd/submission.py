@@ -268,6 +268,7 @@ def grouped_kernel(data, variant: int = 0):
     [row_offsets[e], row_offsets[e+1]) of the expert-contiguous ``a`` ([rows, k], K-major) and ``c``
     ([rows, n]).  ``b`` is [E, n, k] with each expert K-major (stride (n*k, 1, n)); ``b_scale`` is
     [E, ceil(n/128), k/128] with stride (nb*kb, 1, nb).  Fills and returns ``c``; no host sync.
+    A call that splits K keeps a workspace of up to 64 MiB for this device and stream (the one `custom_kernel` uses).
     """
     a, b, a_scale, b_scale, row_offsets, c = data
     rows, k = a.shape
