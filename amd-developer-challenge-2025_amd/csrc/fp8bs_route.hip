@@ -420,12 +420,16 @@ extern "C" int fp8bs_moe_route(const int32_t* top_idx, int tokens, int experts, 
     if (!top_idx || !row_map) return FP8BS_ERR_NULL_POINTER;
     if (!ws || ws_bytes < fp8bs_moe_route_workspace_bytes(tokens, experts)) return FP8BS_ERR_WORKSPACE;
     // One workgroup where its LDS holds a bit per token and expert, and up to 8192 rows: 1024 tokens to 8 experts each
-    // take 12.3 us in it and 11.0 in two kernels over several CUs, with 16 each it would be twice that.
+    // take 12.3 us in it and 11.0 in two kernels over several CUs, with 16 each it would be twice that.  A table of many experts
+    // and many rows is too much for one CU sooner; us a call among others, one workgroup / two kernels (12.5 throughout, the
+    // host's time for two launches): 1024 tokens to 7 of 32, 64, 128, 256 experts 12.4, 13.5, 14.9, 17.0; to 4 of 128, 256 10.8,
+    // 12.7; 700 to 8 of 128, 256 12.3, 14.4; 512 to 8 of 256 12.7.
     if (tokens <= 256 && experts <= fp8bs::ONE_BITS / 256) {
         hipLaunchKernelGGL(fp8bs::route_one_kernel<256>, dim3(1), dim3(256), 0, s, top_idx, tokens, experts, topk, row_offsets, row_map, slot_of);
         return hipGetLastError() == hipSuccess ? FP8BS_OK : FP8BS_ERR_LAUNCH;
     }
-    if (tokens <= 1024 && experts <= fp8bs::ONE_BITS / 1024 && tokens * topk < 8192) {
+    if (tokens <= 1024 && experts <= fp8bs::ONE_BITS / 1024 && tokens * topk < 8192 &&
+        (experts <= 32 || tokens * topk + 12 * experts <= 7100)) {
         hipLaunchKernelGGL(fp8bs::route_one_kernel<1024>, dim3(1), dim3(1024), 0, s, top_idx, tokens, experts, topk, row_offsets, row_map, slot_of);
         return hipGetLastError() == hipSuccess ? FP8BS_OK : FP8BS_ERR_LAUNCH;
     }

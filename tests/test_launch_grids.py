@@ -1,4 +1,5 @@
-"""Launches of very tall matrices stay inside the documented grid limit of 65535 in y and still cover every row.
+"""Launches of very tall matrices stay inside the documented grid limit of 65535 in y and still cover every row; which of two
+kernels a call of the routing functions takes.
 
 On the CPU the launches are recorded instead of made: a small library loaded ahead of the HIP runtime takes the launch
 configuration that hipcc's host code hands over, and declines.  No pointer is dereferenced."""
@@ -29,8 +30,11 @@ one = ctypes.c_void_p(1 << 20)
 fn, dtype, gathered, rows, k = sys.argv[3], int(sys.argv[4]), int(sys.argv[5]), int(sys.argv[6]), int(sys.argv[7])
 if fn == "a":
     st = lib.fp8bs_quantize_a(one, dtype, ctypes.c_int64(k), one if gathered else None, 1000 if gathered else rows, one, one, rows, k, None)
-else:
+elif fn == "b":
     st = lib.fp8bs_quantize_b(one, dtype, ctypes.c_int64(k), one, one, rows, k, None)
+else:
+    tokens, experts, topk = dtype, gathered, rows
+    st = lib.fp8bs_moe_route(one, tokens, experts, topk, one, one, one, one, ctypes.c_size_t(1 << 30), None)
 assert st == 0, st
 """
 
@@ -43,15 +47,28 @@ def shim(tmp_path_factory):
     return str(d / "shim.so")
 
 
+def launches(pkg, shim, *args):
+    out = subprocess.run([sys.executable, "-c", CALL, shim, pkg._lib.LIB_PATH] + [str(a) for a in args],
+                         check=True, stdout=subprocess.PIPE, text=True, timeout=100).stdout
+    return [json.loads(line) for line in out.splitlines()]
+
+
 @pytest.mark.parametrize("fn,dtype,gathered,rows,k", [("a", 1, 1, 65535 * 32, 128), ("a", 1, 1, 65535 * 32 + 1, 128), ("a", 1, 1, 16000001, 256), ("a", 0, 0, 65535 * 64 + 1, 128),
                                                       ("a", 0, 0, 8388607, 128), ("a", 1, 0, 16777215, 128), ("b", 1, 0, 65535 * 128, 128), ("b", 1, 0, 65535 * 128 + 1, 128),
                                                       ("a", 1, 0, 300, 256), ("b", 0, 0, 129, 128)])
 def test_rows_beyond_the_grid_limit(pkg, shim, fn, dtype, gathered, rows, k):
-    out = subprocess.run([sys.executable, "-c", CALL, shim, pkg._lib.LIB_PATH, fn, str(dtype), str(gathered), str(rows), str(k)],
-                         check=True, stdout=subprocess.PIPE, text=True, timeout=100).stdout
-    grids = [json.loads(line) for line in out.splitlines()]
+    grids = launches(pkg, shim, fn, dtype, gathered, rows, k)
     assert grids and all(g[0] == k // 128 and 1 <= g[1] <= 65535 and g[2] == 1 and g[3] == 256 for g in grids), grids
     assert sum(g[1] for g in grids) in [-(-rows // r) for r in ((128,) if fn == "b" else (32, 64, 128))]
+
+
+@pytest.mark.parametrize("tokens,experts,topk,one", [(256, 1024, 16, True), (1024, 32, 7, True), (900, 32, 8, True), (512, 256, 7, True), (700, 128, 7, True),
+                                                      (1024, 256, 2, True), (1024, 256, 7, False), (1024, 128, 7, False), (900, 128, 8, False),
+                                                      (700, 256, 8, False), (1024, 32, 8, False), (1025, 8, 1, False)])
+def test_routing_in_one_workgroup_where_that_is_faster(pkg, shim, tokens, experts, topk, one):
+    """Many rows to many experts leave one workgroup slower than two kernels over several."""
+    threads = [g[3] for g in launches(pkg, shim, "route", tokens, experts, topk, 0)]
+    assert threads == ([256, 256] if not one else [256] if tokens <= 256 else [1024])
 
 
 @pytest.mark.gpu
