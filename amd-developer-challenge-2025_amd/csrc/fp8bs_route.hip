@@ -341,7 +341,8 @@ void route_one_kernel(const int32_t* __restrict__ top_idx, int tokens, int exper
 // time.  With up to 1024 tokens a block per 1024 columns and eight choices at a time: one block per token walked its
 // columns and choices in eight round trips to memory (x 8 x 7168, us before -> after: 1 token 6.5 -> 2.9, 64 6.8 -> 3.4, 256
 // 9.8 -> 5.4, 1024 24.4 -> 22.7; 2048 47.4 -> 48.6, left as it was, and so is d <= 2048, one step of a block: 64 x 2 x 1024 2.4
-// against 2.7).
+// against 2.7).  Up to four choices are half as many round trips, and the line lies at 768 tokens (850 x 3 x 4096 6.9 -> 7.3,
+// 1024 x 4 x 4096 8.2 -> 9.3, 1024 x 1 x 7168 7.7 -> 8.9, 700 x 4 x 7168 10.6 -> 10.4).
 template <int T, int NJ>
 __global__ __launch_bounds__(T)
 void moe_combine_kernel(const uint16_t* __restrict__ y, const int32_t* __restrict__ slot_of, const float* __restrict__ weights,
@@ -455,7 +456,7 @@ extern "C" int fp8bs_moe_combine(const void* y, int rows, const int32_t* slot_of
     if (!y || !slot_of || !weights || !out) return FP8BS_ERR_NULL_POINTER;
     if ((((uintptr_t)y | (uintptr_t)out) & 15) != 0) return FP8BS_ERR_BAD_SHAPE;      // 16-byte row accesses
     const int chunks = (d + 1023) / 1024;
-    if (d > 2048 && tokens <= 1024)
+    if (d > 2048 && tokens <= (topk > 4 ? 1024 : 768))
         hipLaunchKernelGGL((fp8bs::moe_combine_kernel<128, 8>), dim3(tokens, chunks < 65535 ? chunks : 65535), dim3(128), 0, (hipStream_t)stream,
                            (const uint16_t*)y, slot_of, weights, (uint16_t*)out, rows, topk, d);
     else

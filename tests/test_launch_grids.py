@@ -32,6 +32,9 @@ if fn == "a":
     st = lib.fp8bs_quantize_a(one, dtype, ctypes.c_int64(k), one if gathered else None, 1000 if gathered else rows, one, one, rows, k, None)
 elif fn == "b":
     st = lib.fp8bs_quantize_b(one, dtype, ctypes.c_int64(k), one, one, rows, k, None)
+elif fn == "combine":
+    tokens, topk, d = dtype, gathered, rows
+    st = lib.fp8bs_moe_combine(one, tokens * topk, one, one, one, tokens, topk, d, None)
 else:
     tokens, experts, topk = dtype, gathered, rows
     st = lib.fp8bs_moe_route(one, tokens, experts, topk, one, one, one, one, ctypes.c_size_t(1 << 30), None)
@@ -69,6 +72,12 @@ def test_routing_in_one_workgroup_where_that_is_faster(pkg, shim, tokens, expert
     """Many rows to many experts leave one workgroup slower than two kernels over several."""
     threads = [g[3] for g in launches(pkg, shim, "route", tokens, experts, topk, 0)]
     assert threads == ([256, 256] if not one else [256] if tokens <= 256 else [1024])
+
+
+@pytest.mark.parametrize("tokens,topk,d,split", [(1, 8, 7168, True), (768, 1, 7168, True), (1024, 8, 7168, True), (1024, 6, 5120, True), (64, 8, 2056, True),
+                                                 (1024, 1, 7168, False), (1000, 2, 7168, False), (1024, 4, 4096, False), (1025, 8, 7168, False), (64, 8, 2048, False)])
+def test_combining_over_several_workgroups_where_that_is_faster(pkg, shim, tokens, topk, d, split):
+    assert launches(pkg, shim, "combine", tokens, topk, d, 0) == ([[tokens, -(-d // 1024), 1, 128]] if split else [[tokens, 1, 1, 256]])
 
 
 @pytest.mark.gpu
