@@ -33,16 +33,30 @@ def _k_major(rows: int, k: int, dtype: torch.dtype, device: torch.device) -> tor
     return torch.empty_strided((rows, k), (1, rows or 1), dtype=dtype, device=device)
 
 
+def _quantise_then_gather(dtype: torch.dtype, t: int, m: int, k: int, row_map: torch.Tensor) -> bool:
+    """Whether two kernels are faster than one for m gathered rows of t tokens, by measurement (us, one / two): where rows repeat
+    often, the output is large and ``gather_a`` has a fast path that keeps 8 or 16 k rows of the source in LDS (T and M multiples
+    of 4, T <= 8192).  Reading the tokens again costs fp32 twice what it costs bf16, so its lines lie lower.
+
+    bf16, 4096 tokens: to 8 of 7168 values 103 / 85, of 4096 50.6 / 47.2, of 2048 24.4 / 27.5; to 5 of 7168 65.9 / 61.7, of 4096
+    30.5 / 38.7; to 4 of 7168 51.6 / 53.8.  8192 tokens to 8 of 7168 224 / 233, of 1024 24.4 / 32.5; 16384 to 8 of 7168 447 / 831.
+    fp32, 4096 tokens: to 8 of 2048 31.5 / 28.9, of 1024 16.5 / 20.3; to 4 of 7168 83 / 68, of 4096 40.8 / 33.7, of 2048 17.6 /
+    25.4; to 3 of 7168 63.5 / 63.0.  8192 tokens to 8 of 2048 80.7 / 67.9, of 1024 30.7 / 32.8; to 4 of 7168 167 / 166.
+    """
+    if t % 4 or m % 4 or not 0 < t <= 8192 or row_map.data_ptr() % 16:
+        return False
+    if dtype == torch.bfloat16:
+        return t <= 4096 and m > 4 * t and m * k >= 100 << 20
+    return m >= 4 * t and m * k >= (48 if t <= 4096 else 96) << 20
+
+
 def quantize_a(x: torch.Tensor, row_map: Optional[torch.Tensor] = None, fused: Optional[bool] = None) -> Tuple[torch.Tensor, torch.Tensor]:
     """x [T, K] -> (a e4m3fn [M, K] stride (1, M), a_scale fp32 [M, K/128] stride (1, M)).
 
     Without ``row_map`` M = T.  With ``row_map`` (int32 [M] on the GPU) output row i is input row
     ``row_map[i]``: the expert-contiguous gather of routed tokens.  Two routes, the same bytes: the gather fused into the
-    quantiser (one kernel), or every token quantised once and the bytes gathered by ``gather_a`` (two kernels).  The
-    second where the output is large, rows repeat and the gather's fast path applies (T and M multiples of 4, T <= 40960):
-    a layer over 4096 tokens to 8 experts each, 32768 rows x 7168, takes 16 us less with it.  Elsewhere one kernel is faster
-    (64 -> 512 rows x 7168: 3.7 us against 5.5, 2048 -> 16384 x 2048 14.5 against 18, 4095 -> 32760 x 7168 100 against 305).
-    ``fused`` = True / False forces the one-kernel / two-kernel route.
+    quantiser (one kernel), or every token quantised once and the bytes gathered by ``gather_a`` (two kernels), see
+    ``_quantise_then_gather``.  ``fused`` = True / False forces the one-kernel / two-kernel route.
     """
     _check_input(x, "x")
     t, k = x.shape
@@ -51,7 +65,7 @@ def quantize_a(x: torch.Tensor, row_map: Optional[torch.Tensor] = None, fused: O
             raise ValueError("row_map must be a contiguous int32 vector on x's device")
         m = row_map.numel()
         if fused is None:
-            fused = not (m > 4 * t and m * k >= 1 << 26 and t % 4 == 0 and m % 4 == 0 and 0 < t <= 40960)
+            fused = not _quantise_then_gather(x.dtype, t, m, k, row_map)
         if not fused:
             return gather_a(*quantize_a(x), row_map)
     else:

@@ -80,6 +80,28 @@ def test_combining_over_several_workgroups_where_that_is_faster(pkg, shim, token
     assert launches(pkg, shim, "combine", tokens, topk, d, 0) == ([[tokens, -(-d // 1024), 1, 128]] if split else [[tokens, 1, 1, 256]])
 
 
+@pytest.mark.parametrize("dtype,t,m,k,aligned,two", [
+    (torch.bfloat16, 4096, 32768, 7168, True, True), (torch.bfloat16, 4096, 20480, 7168, True, True), (torch.bfloat16, 2048, 16384, 7168, True, True),
+    (torch.bfloat16, 4096, 16384, 7168, True, False), (torch.bfloat16, 4096, 20480, 4096, True, False), (torch.bfloat16, 8192, 65536, 2048, True, False),
+    (torch.bfloat16, 16384, 131072, 1024, True, False), (torch.bfloat16, 4094, 32752, 7168, True, False), (torch.bfloat16, 4096, 32768, 7168, False, False),
+    (torch.float32, 4096, 16384, 7168, True, True), (torch.float32, 4096, 16384, 4096, True, True), (torch.float32, 2048, 8192, 7168, True, True),
+    (torch.float32, 1024, 8192, 7168, True, True), (torch.float32, 8192, 40960, 4096, True, True), (torch.float32, 4096, 8192, 7168, True, False),
+    (torch.float32, 8192, 65536, 1024, True, False), (torch.float32, 16384, 131072, 2048, True, False)])
+def test_the_faster_route_of_a_gathered_quantisation(monkeypatch, dtype, t, m, k, aligned, two):
+    """One kernel that gathers as it quantises, or two: shapes where each is faster by measurement.  The calls stop before the library's."""
+    quant = importlib.import_module("amd-developer-challenge-2025_amd.quant")
+    calls = []
+    monkeypatch.setattr(quant, "_check_input", lambda x, name: None)
+    monkeypatch.setattr(quant, "_call", lambda fn, *args: calls.append("quantise"))
+    monkeypatch.setattr(quant, "gather_a", lambda *args: calls.append("gather"))
+    monkeypatch.setattr(quant, "_k_major", lambda rows, k, dtype, device: torch.empty(0, device="cpu"))
+    x = torch.empty(t, 1, dtype=dtype).expand(t, k)                # sizes and addresses are all that is looked at
+    row_map = torch.empty(m + 8, dtype=torch.int32)
+    row_map = row_map[-row_map.data_ptr() % 16 // 4 + (0 if aligned else 1):][:m]
+    quant.quantize_a(x, row_map)
+    assert calls == (["quantise", "gather"] if two else ["quantise"])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind,rows", [("gathered", 65535 * 32 + 33), ("f32", 65535 * 64 + 70), ("b", 65535 * 128 + 200)])
 def test_values_on_both_sides_of_the_grid_limit(kind, rows):
