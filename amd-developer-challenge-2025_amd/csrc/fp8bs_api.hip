@@ -137,6 +137,14 @@ bool skinny_shape(int m, int n, int k) { return m <= 64 && (double)n * (double)k
 void choose_tiled(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_split, bool epi) {
     if (num_cus <= 0) num_cus = 256;
     int kbt = k / KBLK;
+    // One K block is all first copies and output, which the constants below, fits to two blocks and more, take for too little
+    // with large tiles.  us, 64x64 / 128x128 in four waves / 256x128 / 256x256: 1803 x 576 6.0 / 6.1 / 7.4 / 9.9; 2944 x 171 6.4 /
+    // 6.2 / 7.9 / 10.8; 9106 x 256 7.8 / 6.5 / 7.9 / 10.1; 10880 x 1484 22.7 / 13.5 / 17.2 / 18.0; 8192 x 8192 48.7 / 26.8 / 26.0 / 28.0.
+    // (With the silu-mul epilogue the output is half as large, and 256x128 and 256x256, which the model picks, are the fastest.)
+    if (kbt == 1 && !epi) {
+        fill_plan(m, n, k, cdiv(m, 64) * cdiv(n, 64) <= 2L * num_cus ? FP8BS_VARIANT_T64x128 | FORM1 : FP8BS_VARIANT_T128x128, 1, out);
+        return;
+    }
     // The tile and K split that finish soonest under a cost model in microseconds.  A workgroup advances one K block in
     // max(t_alone x shared, t_power x w / CUs): t_alone is the tile's time per block with one workgroup on a CU, shared
     // the factor with two, t_power what the board's power limit allows when every CU runs one such workgroup - with w

@@ -61,6 +61,13 @@ def test_long_chains_take_the_tile_that_measures_fastest(pkg):
         assert (p.tile_m, p.tile_n, p.split_k, p.sum_in_kernel) == (256, 128, 2, 1), (m, n, k)
 
 
+def test_one_k_block_takes_a_small_tile(pkg):
+    """K = 128 is all first copies and output: 64x64 where the chip holds those tiles at once, else 128x128 in four waves."""
+    for m, n, tile in [(1, 115, 64), (2944, 171, 64), (640, 575, 64), (107, 6464, 64), (13653, 64, 64), (8576, 2624, 128), (10880, 1484, 128), (9106, 256, 128), (8192, 8192, 128)]:
+        p = pkg.plan(m, n, 128)
+        assert (p.tile_m, p.tile_n, p.split_k, p.block_threads) == (tile, tile, 1, 256), (m, n)
+
+
 def test_an_incomplete_binding_is_named(pkg, monkeypatch):
     """A CPython binding built before a function was added to it gives way to ctypes with a warning that says so."""
     lib_mod, whole = pkg._lib, pkg._lib.pycall()
