@@ -36,18 +36,22 @@ def _k_major(rows: int, k: int, dtype: torch.dtype, device: torch.device) -> tor
 def _quantise_then_gather(dtype: torch.dtype, t: int, m: int, k: int, row_map: torch.Tensor) -> bool:
     """Whether two kernels are faster than one for m gathered rows of t tokens, by measurement (us, one / two): where rows repeat
     often, the output is large and ``gather_a`` has a fast path that keeps 8 or 16 k rows of the source in LDS (T and M multiples
-    of 4, T <= 8192).  Reading the tokens again costs fp32 twice what it costs bf16, so its lines lie lower.
+    of 4, T <= 8192; up to 6826 tokens three of its workgroups fit a CU, beyond that two).  Reading the tokens again costs fp32
+    twice what it costs bf16, so its lines lie lower.
 
-    bf16, 4096 tokens: to 8 of 7168 values 103 / 85, of 4096 50.6 / 47.2, of 2048 24.4 / 27.5; to 5 of 7168 65.9 / 61.7, of 4096
-    30.5 / 38.7; to 4 of 7168 51.6 / 53.8.  8192 tokens to 8 of 7168 224 / 233, of 1024 24.4 / 32.5; 16384 to 8 of 7168 447 / 831.
+    bf16, 4096 tokens: to 8 of 7168 values 103 / 85, of 4096 47.4 / 47.7, of 2048 24.4 / 27.5; to 5 of 7168 65.9 / 61.7, of 4096
+    30.5 / 38.7; to 4 of 7168 51.6 / 53.8.  6016 tokens to 8 of 7168 158 / 135, to 6 of 4096 59.3 / 61.8; 6976 to 8 of 7168 184 /
+    189; 8192 to 8 of 7168 224 / 233, of 1024 24.4 / 32.5; 16384 to 8 of 7168 447 / 831.
     fp32, 4096 tokens: to 8 of 2048 31.5 / 28.9, of 1024 16.5 / 20.3; to 4 of 7168 83 / 68, of 4096 40.8 / 33.7, of 2048 17.6 /
-    25.4; to 3 of 7168 63.5 / 63.0.  8192 tokens to 8 of 2048 80.7 / 67.9, of 1024 30.7 / 32.8; to 4 of 7168 167 / 166.
+    25.4; to 3 of 7168 63.5 / 63.0.  6016 tokens to 4 of 2048 28.9 / 28.5; 8192 to 8 of 2048 80.7 / 67.9, of 1024 30.7 / 32.8; to 5
+    of 2048 51.4 / 54.5; to 4 of 7168 167 / 166; 16384 to 8 of 7168 712 / 900.
     """
     if t % 4 or m % 4 or not 0 < t <= 8192 or row_map.data_ptr() % 16:
         return False
+    three_a_cu = t <= 6826
     if dtype == torch.bfloat16:
-        return t <= 4096 and m > 4 * t and m * k >= 100 << 20
-    return m >= 4 * t and m * k >= (48 if t <= 4096 else 96) << 20
+        return three_a_cu and m > 4 * t and m * k >= (100 if t <= 4096 else 144) << 20
+    return m >= 4 * t and m * k >= (48 if three_a_cu else 84) << 20
 
 
 def quantize_a(x: torch.Tensor, row_map: Optional[torch.Tensor] = None, fused: Optional[bool] = None) -> Tuple[torch.Tensor, torch.Tensor]:

@@ -82,7 +82,8 @@ def test_combining_over_several_workgroups_where_that_is_faster(pkg, shim, token
 
 @pytest.mark.parametrize("dtype,t,m,k,aligned,two", [
     (torch.bfloat16, 4096, 32768, 7168, True, True), (torch.bfloat16, 4096, 20480, 7168, True, True), (torch.bfloat16, 2048, 16384, 7168, True, True),
-    (torch.bfloat16, 4096, 16384, 7168, True, False), (torch.bfloat16, 4096, 20480, 4096, True, False), (torch.bfloat16, 8192, 65536, 2048, True, False),
+    (torch.bfloat16, 6016, 48128, 4096, True, True), (torch.bfloat16, 6016, 36096, 4096, True, False), (torch.bfloat16, 6976, 55808, 7168, True, False),
+    (torch.float32, 6016, 24064, 4096, True, True), (torch.bfloat16, 4096, 16384, 7168, True, False), (torch.bfloat16, 4096, 20480, 4096, True, False), (torch.bfloat16, 8192, 65536, 2048, True, False),
     (torch.bfloat16, 16384, 131072, 1024, True, False), (torch.bfloat16, 4094, 32752, 7168, True, False), (torch.bfloat16, 4096, 32768, 7168, False, False),
     (torch.float32, 4096, 16384, 7168, True, True), (torch.float32, 4096, 16384, 4096, True, True), (torch.float32, 2048, 8192, 7168, True, True),
     (torch.float32, 1024, 8192, 7168, True, True), (torch.float32, 8192, 40960, 4096, True, True), (torch.float32, 4096, 8192, 7168, True, False),
