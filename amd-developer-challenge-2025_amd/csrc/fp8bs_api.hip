@@ -176,7 +176,7 @@ void choose_tiled(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_
         {FP8BS_VARIANT_T64x256S3 | FORM1, 1, 0.467, 0.531, 4.57, 1.0, 4},
     };
     const int splits[6] = {1, 2, 3, 4, 6, 8};
-    int best_tile = 0, best_split = 1; double best_cost = 0; bool best_fused = false;
+    int best_tile = 0, best_split = 1; double best_cost = 0, best_gpu = 0; bool best_fused = false;
     for (const Cand& c : cands) {
         if (epi && !has_epilogue(c.tile)) continue;
         VariantInfo vi{};
@@ -210,14 +210,18 @@ void choose_tiled(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_
             const double planes = 2.66 + 1.656e-6 * s * (double)m * (double)n;
             const double in_kernel = 2.34 + 0.891e-6 * s * (double)m * (double)n
                                      + 13.2 * (s - 1) * (vi.bm * vi.bn * 4e-6) * (double)cdiv(wgs, num_cus);
-            const bool fuse = (s == 2 || s == 3) && can_sum_in_kernel(m, n, c.tile, s) && in_kernel < planes;
-            if (s > 1) cost += fuse ? in_kernel : planes;
-            // calls issued one after another are never faster than the host launches them: the reduce launch of a split
-            // pays only beyond that (2 x 700 x 3200 in eight partitions: done on the GPU after 7.2 us, 9.5 us a call).  These are
-            // Python callers' launches; a captured graph or a C program, whose launches cost less, is given the same plan.
-            const double host = s > 1 && !fuse ? 7.8 : 4.5;
-            if (cost < host) cost = host;
-            if (best_tile == 0 || cost < best_cost) { best_tile = c.tile; best_split = s; best_cost = cost; best_fused = fuse; }
+            // calls issued one after another are never faster than the host launches them: 5.2 to 6.2 us, or 7.7 to 10.2 with the
+            // reduce launch of a split, by the machine.  The latter stands as 8.5 here: the constants are 0.5 to 1.2 us over
+            // what such small calls take, and at 8.5 neither side loses much on a fast or a slow host (12 x 512 x 1536 unsplit 5.4,
+            // in four partitions and two launches 8.1 and 9.1; 1 x 512 x 3456 in three, one launch, 8.8, in eight 7.7 and 9.1).
+            // These are Python callers' launches; a captured graph or a C program, whose launches cost less, is given the same plan.
+            auto issued = [](double gpu, double host) { return gpu > host ? gpu : host; };
+            const double one = s > 1 ? cost + in_kernel : cost, two = cost + planes;
+            const bool fuse = (s == 2 || s == 3) && can_sum_in_kernel(m, n, c.tile, s) && issued(one, 5.3) < issued(two, 8.5);
+            const double gpu = s == 1 || fuse ? one : two;
+            cost = issued(gpu, s == 1 || fuse ? 5.3 : 8.5);
+            // (among equals, which the host alone makes, the shorter kernel)
+            if (best_tile == 0 || cost < best_cost || (cost == best_cost && gpu < best_gpu)) { best_tile = c.tile; best_split = s; best_cost = cost; best_gpu = gpu; best_fused = fuse; }
         }
     }
     fill_plan(m, n, k, best_tile, best_split, out, 0, best_fused);

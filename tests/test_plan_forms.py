@@ -68,6 +68,16 @@ def test_one_k_block_takes_a_small_tile(pkg):
         assert (p.tile_m, p.tile_n, p.split_k, p.block_threads) == (tile, tile, 1, 256), (m, n)
 
 
+def test_small_products_take_one_launch_where_that_is_faster(pkg):
+    """A second launch costs a caller 2.5 to 4 us: with 12 to 15 K blocks more than the K split behind it saves."""
+    for m, n, k in [(12, 128, 1536), (12, 512, 1536), (8, 576, 1664), (64, 512, 1536), (4, 832, 1792), (21, 576, 1792), (200, 128, 1536)]:
+        p = pkg.plan(m, n, k)
+        assert p.split_k == 1 or p.sum_in_kernel, (m, n, k)
+    for m, n, k in [(1, 512, 7168), (12, 512, 5632), (64, 512, 7168)]:
+        p = pkg.plan(m, n, k)
+        assert p.split_k >= 4 and not p.sum_in_kernel, (m, n, k)
+
+
 def test_an_incomplete_binding_is_named(pkg, monkeypatch):
     """A CPython binding built before a function was added to it gives way to ctypes with a warning that says so."""
     lib_mod, whole = pkg._lib, pkg._lib.pycall()
