@@ -368,6 +368,11 @@ GroupedPlan make_grouped_plan(int experts, int rows, int n, int k, int num_cus, 
             double cost = full * (c.t_fixed + kb * t_block(per_round));
             if (rem > 0.5) cost += c.t_fixed + kb * t_block(rem);
             if (s > 1) cost += 3.56 + 0.757e-6 * s * (double)rows * (double)n;
+            // With more than 32 rows per expert the model flatters the smaller tiles against this one: 640 tokens to 4 of 32 experts,
+            // 3664 x 5376, 128x128 in eight waves 217 us, this 169; 704 to 8 of 32, 2176 x 1280, 39.2 and 35.2; 931 to 8 of 16, 3806 x
+            // 5888, 256x128 278, this 260.  Over 480 further shapes of the same ranges and wider ones any factor from 0.85 to 0.95 brings
+            // the picks from 3.6 to 3.2 % behind the best, and from 37 to 19-25 those more than 5 % behind the rule before the model.
+            if (c.tile == FP8BS_VARIANT_T256x256 && (long)rows > 32L * experts) cost *= 0.92;
             if (best_cost == 0 || cost < best_cost) { best = p; best_cost = cost; }
         }
     }

@@ -16,11 +16,12 @@ SHIM = r"""
 #include <stdio.h>
 typedef struct { uint32_t x, y, z; } grid3;
 int __hipPushCallConfiguration(grid3 g, grid3 b, size_t lds, void* stream) {
-    (void)lds; (void)stream;
-    printf("[%u, %u, %u, %u]\n", g.x, g.y, g.z, b.x); fflush(stdout);
+    (void)stream;
+    printf("[%u, %u, %u, %u, %zu]\n", g.x, g.y, g.z, b.x, lds); fflush(stdout);
     return 1;
 }
 int hipGetLastError(void) { return 0; }
+int hipFuncSetAttribute(const void* f, int attr, int value) { (void)f; (void)attr; (void)value; return 0; }
 """
 CALL = r"""
 import ctypes, sys
@@ -32,6 +33,9 @@ if fn == "a":
     st = lib.fp8bs_quantize_a(one, dtype, ctypes.c_int64(k), one if gathered else None, 1000 if gathered else rows, one, one, rows, k, None)
 elif fn == "b":
     st = lib.fp8bs_quantize_b(one, dtype, ctypes.c_int64(k), one, one, rows, k, None)
+elif fn == "grouped":
+    experts, rows, n, k = dtype, gathered, rows, k
+    st = lib.fp8bs_gemm_grouped(one, one, one, one, one, one, experts, rows, n, k, None)
 elif fn == "combine":
     tokens, topk, d = dtype, gathered, rows
     st = lib.fp8bs_moe_combine(one, tokens * topk, one, one, one, tokens, topk, d, None)
@@ -53,7 +57,7 @@ def shim(tmp_path_factory):
 def launches(pkg, shim, *args):
     out = subprocess.run([sys.executable, "-c", CALL, shim, pkg._lib.LIB_PATH] + [str(a) for a in args],
                          check=True, stdout=subprocess.PIPE, text=True, timeout=100).stdout
-    return [json.loads(line) for line in out.splitlines()]
+    return [json.loads(line)[:5 if args[0] == "grouped" else 4] for line in out.splitlines()]
 
 
 @pytest.mark.parametrize("fn,dtype,gathered,rows,k", [("a", 1, 1, 65535 * 32, 128), ("a", 1, 1, 65535 * 32 + 1, 128), ("a", 1, 1, 16000001, 256), ("a", 0, 0, 65535 * 64 + 1, 128),
@@ -101,6 +105,14 @@ def test_the_faster_route_of_a_gathered_quantisation(monkeypatch, dtype, t, m, k
     row_map = row_map[-row_map.data_ptr() % 16 // 4 + (0 if aligned else 1):][:m]
     quant.quantize_a(x, row_map)
     assert calls == (["quantise", "gather"] if two else ["quantise"])
+
+
+@pytest.mark.parametrize("tokens,experts,topk,n,k,tile", [(640, 32, 4, 3664, 5376, 2), (704, 32, 8, 2176, 1280, 2), (931, 16, 8, 3806, 5888, 2), (2972, 16, 2, 3200, 1408, 2),
+                                                          (4096, 32, 8, 4096, 7168, 2), (704, 16, 4, 512, 1280, 12 | 2 << 8), (32, 32, 8, 4096, 7168, 12)])
+def test_the_tile_of_a_grouped_call(pkg, shim, tokens, experts, topk, n, k, tile):
+    """Shapes on which the tile is the fastest by measurement, known here by its threads and its LDS."""
+    (_, _, _, threads, lds), = launches(pkg, shim, "grouped", experts, tokens * topk, n, k)
+    assert threads == 512 and lds == {2: 2 * (128 * 512 + 1024 + 256), 12: 3 * (128 * 320 + 1024 + 256), 12 | 2 << 8: 4 * (128 * 256 + 1024 + 256)}[tile]
 
 
 @pytest.mark.gpu
