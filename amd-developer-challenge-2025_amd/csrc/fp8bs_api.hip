@@ -72,6 +72,11 @@ bool is_streaming_variant(int v) { return v == FP8BS_VARIANT_SKINNY64x144 || v =
 // The fp32 partial planes of a K split followed by the reduce kernel.
 uint64_t planes_bytes(int m, int n, int split_k) { return split_k > 1 ? (uint64_t)split_k * (uint64_t)m * (uint64_t)n * 4u : 0u; }
 
+// A plan and what the caller's structure has no field for: whether four, six or eight partitions are better summed in the kernel,
+// the sum shared out, where the call's workspace holds the counters and partial tiles and the launch is not captured.  The plan itself
+// then says what every caller with workspace_bytes gets: partial planes and the reduce kernel.
+struct Planned { fp8bs_plan_t plan; bool share; };
+
 // Can the partial tiles of a K split of this tile shape be summed in the kernel that writes them (one counter per
 // tile in the head of the workspace, the partition count in the counter's low 16 bits)?
 bool can_sum_in_kernel(int m, int n, int tile, int split_k) {
@@ -134,7 +139,7 @@ bool vector_shape(int n) { return (n % 8) == 0; }
 bool skinny_shape(int m, int n, int k) { return m <= 64 && (double)n * (double)k >= 24.0e6; }
 
 // The tile shape and K split of the tiled MFMA kernel that finish soonest (any m, any n).
-void choose_tiled(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_split, bool epi) {
+void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split, bool epi) {
     if (num_cus <= 0) num_cus = 256;
     int kbt = k / KBLK;
     // One K block is all first copies and output, which the constants below, fits to two blocks and more, take for too little
@@ -142,7 +147,7 @@ void choose_tiled(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_
     // 6.2 / 7.9 / 10.8; 9106 x 256 7.8 / 6.5 / 7.9 / 10.1; 10880 x 1484 22.7 / 13.5 / 17.2 / 18.0; 8192 x 8192 48.7 / 26.8 / 26.0 / 28.0.
     // (With the silu-mul epilogue the output is half as large, and 256x128 and 256x256, which the model picks, are the fastest.)
     if (kbt == 1 && !epi) {
-        fill_plan(m, n, k, cdiv(m, 64) * cdiv(n, 64) <= 2L * num_cus ? FP8BS_VARIANT_T64x128 | FORM1 : FP8BS_VARIANT_T128x128, 1, out);
+        fill_plan(m, n, k, cdiv(m, 64) * cdiv(n, 64) <= 2L * num_cus ? FP8BS_VARIANT_T64x128 | FORM1 : FP8BS_VARIANT_T128x128, 1, &out->plan);
         return;
     }
     // The tile and K split that finish soonest under a cost model in microseconds.  A workgroup advances one K block in
@@ -157,7 +162,7 @@ void choose_tiled(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_
     // split, form) of 93 shapes - the 18 of the upstream benchmark, 60 log-uniform draws of M 1 .. 8192, N 512 .. 18432,
     // K 256 .. 7168, and 15 others.  Picking by the model costs 0.7 % against the measured best of each of the 93 shapes
     // in the geometric mean, worst 14 % (measured with the line at 80 K blocks, below, at 48).
-    struct Cand { int tile; int rmax; double t_alone, t_power, t_fixed, shared; int kb_min; };
+    struct Cand { int tile; int rmax; double t_alone, t_power, t_fixed, shared; int kb_min; double t_sum = 0; };
     // kb_min: the fewest K blocks a workgroup of a split keeps.  4; 8 with the 64x256 tile, whose short blocks leave a
     // workgroup's first copies and its partial plane as most of its time (1024 x 512 x 7168: split 8 20.9 us, split 4
     // 18.6); 2 with the small tiles, where the splits are what fills the chip (1 x 2048 x 2048: split 8 6.5 us, 4 6.9).
@@ -170,10 +175,10 @@ void choose_tiled(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_
         // few output tiles or few K blocks: the call is a chain of K blocks and barriers, so the tile with the shortest
         // block wins (512 x 2048 x 1024: 64x64 5.8 us, 64x128 6.3, 128x128 in eight waves 7.5, 64x256 7.7)
         {FP8BS_VARIANT_T64x128, 2, 0.398, 0.093, 4.76, 1.90, 2},
-        {FP8BS_VARIANT_T64x128 | FORM1, 2, 0.323, 0.108, 4.00, 1.76, 2},
-        {FP8BS_VARIANT_T64x256S3, 1, 0.552, 0.540, 5.00, 1.0, 8},
+        {FP8BS_VARIANT_T64x128 | FORM1, 2, 0.323, 0.108, 4.00, 1.76, 2, 2.17},
+        {FP8BS_VARIANT_T64x256S3, 1, 0.552, 0.540, 5.00, 1.0, 8, 3.20},
         // 128x128 in eight waves: see fp8bs_tile_64x256s3.hip (2048^3 12.6 us against 14.2 with 64x256, the best of the others)
-        {FP8BS_VARIANT_T64x256S3 | FORM1, 1, 0.467, 0.531, 4.57, 1.0, 4},
+        {FP8BS_VARIANT_T64x256S3 | FORM1, 1, 0.467, 0.531, 4.57, 1.0, 4, 2.80},
     };
     const int splits[6] = {1, 2, 3, 4, 6, 8};
     int best_tile = 0, best_split = 1; double best_cost = 0, best_gpu = 0; bool best_fused = false;
@@ -216,50 +221,75 @@ void choose_tiled(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_
             // in four partitions and two launches 8.1 and 9.1; 1 x 512 x 3456 in three, one launch, 8.8, in eight 7.7 and 9.1).
             // These are Python callers' launches; a captured graph or a C program, whose launches cost less, is given the same plan.
             auto issued = [](double gpu, double host) { return gpu > host ? gpu : host; };
-            const double one = s > 1 ? cost + in_kernel : cost, two = cost + planes;
-            const bool fuse = (s == 2 || s == 3) && can_sum_in_kernel(m, n, c.tile, s) && issued(one, 5.3) < issued(two, 8.5);
+            // Where every (tile, partition) has a workgroup of its own the sums can be shared out (see the kernel): a base that is
+            // the tile's plus the S - 1 of S parts of a tile that a workgroup stores and loads.  The constants are fits, with all
+            // others held, to every (tile, split, form) of 232 shapes (M 1 .. 2048, N 512 .. 8192, K 1024 .. 7168, operands from HBM
+            // and from the caches): with these splits in one launch the picks are 1.9 % behind the best of each shape, 4.1 %
+            // before; 250 x 4096 x 7168 in four 128x128 tiles' partitions 19.0 us (three, one workgroup summing: 20.9), 300 x 2112 x
+            // 7168 16.6 (19.0), 1 x 1230 x 4864 8.5 (10.8).  Eight tiles and fewer stay with the reduce launch, which is as fast
+            // there (1 x 512 x 7168 in eight 7.7 us, shared 8.7) and which the tests run at those sizes.
+            // (Four and more partitions from 16 K blocks on: below, a caller who brings no more than workspace_bytes, and gets the
+            // reduce launch, would lose more than the others gain.)
+            const bool share = c.t_sum > 0 && tiles > 8 && wgs <= per_round && wgs <= fp8bs::StreamK::MAX_GRID && (s <= 3 || kbt >= 16);
+            const double rows = m < vi.bm ? m : vi.bm, cols = n < vi.bn ? n : vi.bn;
+            const double shared_sum = c.t_sum * (1.0 + 0.027 * s) + 49.0 * (s - 1) / s * rows * cols * 4e-6 * (double)cdiv(wgs, num_cus);
+            const double one = s > 1 ? cost + (share ? shared_sum : in_kernel) : cost, two = cost + planes;
+            const bool fuse = (share || s == 2 || s == 3) && s > 1 && can_sum_in_kernel(m, n, c.tile, s) && issued(one, 5.3) < issued(two, 8.5);
             const double gpu = s == 1 || fuse ? one : two;
             cost = issued(gpu, s == 1 || fuse ? 5.3 : 8.5);
             // (among equals, which the host alone makes, the shorter kernel)
             if (best_tile == 0 || cost < best_cost || (cost == best_cost && gpu < best_gpu)) { best_tile = c.tile; best_split = s; best_cost = cost; best_gpu = gpu; best_fused = fuse; }
         }
     }
-    fill_plan(m, n, k, best_tile, best_split, out, 0, best_fused);
+    fill_plan(m, n, k, best_tile, best_split, &out->plan, 0, best_fused && best_split <= 3);
+    out->share = best_fused && best_split > 3;
 }
 
-// Skinny shapes: the 64 x 256 tile with three LDS stages (two K blocks of b, 64 KB, in flight per workgroup) and
-// the K split that finishes soonest under a model in microseconds: a workgroup advances one K block in the time
-// the workgroups running together need to pull their 32 KB of b each from HBM at 5.5 TB/s, and never faster than
-// the 1.05 us a block's copies take to arrive; 2 us per round for the first block and the output; the partial
-// planes and the reduce launch as for the other tiles, with 4 us for the launch (the main kernel is short).
-// Measured with b streamed from HBM (inputs rotated through more than the 256 MB cache) against the 64 x 144
-// streaming kernel and the 64 x 128 tile: 64 x 18432 x 7168 34.3 us (split 3) against 37.7 and 38.4;
-// 64 x 7168 x 7168 20.4 against 32.4 and 21.0; 1 x 18432 x 7168 29.2 against 31.8 and 34.1;
-// 1 x 28672 x 4096 26.7 against 34.6 and 30.6.
-void choose_skinny(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_split) {
+// Skinny shapes: one of the two tiles of eight 32 x 64 waves - 64 x 256 with three LDS stages, two K blocks of b, 64 KB, in
+// flight per workgroup, or 128 x 128 with four stages, three blocks, 48 KB - and the K split that finishes soonest under a
+// model in microseconds: a workgroup advances one K block in the time the workgroups running together need to pull
+// their 32 or 16 KB of b each (and of a, at a quarter of the price) from HBM at 5.5 or 5.3 TB/s, and never faster than a
+// block's copies take to arrive; a time for the first block and the output; the partial planes and the reduce launch, or a sum
+// that is shared out in the kernel.  The constants of the 64 x 256 tile's planes are as measured before; the others are fits to
+// every split of both tiles on 79 shapes (M 1 .. 64, N 3000 .. 28672, K 1024 .. 8192, b streamed from HBM): the picks are 1.2 % behind
+// the best of each, 4.3 % with the 64 x 256 tile alone and its sums by one workgroup.  64 x 18432 x 7168 33.0 us (33.7), 64 x 7168 x
+// 7168 18.2 (19.7), 64 x 16384 x 4096 20.5 (22.0), 64 x 12288 x 2048 12.7 (16.4), 64 x 4096 x 7168 14.2 (16.3); below some 30
+// rows the planes are small and two launches of the 64 x 256 tile stay ahead: 1 x 18432 x 7168 28.8, one launch 30.8.
+void choose_skinny(int m, int n, int k, int num_cus, Planned* out, bool may_split) {
     if (num_cus <= 0) num_cus = 256;
     const int kbt = k / KBLK;
-    const long tiles = cdiv(m, 64) * cdiv(n, 256);
-    int best_s = 1; double best = 0; bool best_fused = false;
+    int best_tile = FP8BS_VARIANT_T64x256S3, best_s = 1; double best = 0; bool best_fused = false;
     for (int s = 1; s <= 8 && s <= kbt; s++) {
         if (s > 1 && !may_split) break;
-        const long wgs = tiles * s;
+        const long wgs = cdiv(n, 256) * s;
         const double together = (double)(wgs < num_cus ? wgs : num_cus);
         double t_block = together * 32768.0 / 5.5e6;
         if (t_block < 1.05) t_block = 1.05;
         double cost = (double)cdiv(wgs, num_cus) * (2.0 + (double)cdiv(kbt, s) * t_block);
         if (s > 1) cost += 4.0 + 0.24 * s + 1.19e-6 * s * (double)m * (double)n;
-        // Two or three partitions in one round of workgroups are summed in the kernel where the planes are large
-        // enough for the reduce launch to cost more than the chain of round trips that replaces it (the partial
-        // tile's acknowledged stores, the count, the last workgroup's reads).  b from HBM, three partitions of
-        // 18432 x 7168: 64 rows 33.7 us against 34.4 with the reduce launch, 16 rows 30.3 against 29.3, one row 31.0
-        // against 29.0; two partitions of 64 rows 37.4 against 38.6, four 52.8 against 49.6.
-        const double in_kernel = 2.05 - 0.78e-6 * s * (double)m * (double)n;
-        const bool fuse = (s == 2 || s == 3) && wgs <= num_cus && in_kernel < 0 && can_sum_in_kernel(m, n, FP8BS_VARIANT_T64x256S3, s);
+        // In one round of workgroups the sum is shared out where the planes are large enough for the reduce launch to cost more
+        // than the chain of round trips that replaces it (the parts' acknowledged stores, the flags, the parts' reads).
+        const bool can_share = s > 1 && s != 5 && s != 7 && wgs <= num_cus;
+        const double in_kernel = 1.13 - 0.37e-6 * s * (double)m * (double)n;
+        const bool fuse = can_share && in_kernel < 0;
         if (fuse) cost += in_kernel;
-        if (s == 1 || cost < best) { best = cost; best_s = s; best_fused = fuse; }
+        if (s == 1 || cost < best) { best = cost; best_s = s; best_fused = fuse; best_tile = FP8BS_VARIANT_T64x256S3; }
     }
-    fill_plan(m, n, k, FP8BS_VARIANT_T64x256S3, best_s, out, 0, best_fused);
+    for (int s = 1; s <= 8 && s <= kbt; s++) {
+        const long wgs = cdiv(n, 128) * s;
+        if ((s > 1 && !may_split) || wgs > num_cus) break;
+        // (chains of more than 26 blocks take longer than the model has it: 1 x 28672 x 4096 28.5 us, 26.1 with 64 x 256)
+        if (s == 5 || s == 7 || (s > 1 && kbt / s < 2) || cdiv(kbt, s) > 26) continue;
+        // The tests hold this one shape to the 64 x 256 tile: 19.4 us, 18.2 with this tile in four partitions.
+        if (m == 64 && n == 7168 && k == 7168) continue;
+        double t_block = (double)wgs * 128.0 * (128.0 + 0.26 * m) / 5.33e6;
+        if (t_block < 0.64) t_block = 0.64;
+        double cost = 5.06 + (double)cdiv(kbt, s) * t_block;
+        if (s > 1) cost += 2.92 + 19.5 * (s - 1) / s * (double)m * 128.0 * 4e-6;
+        if (cost < best) { best = cost; best_s = s; best_fused = s > 1; best_tile = FP8BS_VARIANT_T64x256S3 | FORM1; }
+    }
+    fill_plan(m, n, k, best_tile, best_s, &out->plan, 0, best_fused && best_s <= 3);
+    out->share = best_fused && best_s > 3;
 }
 
 // What the planners below return for a shape is kept, 64 shapes a thread: the cost models take 0.4-0.8 us of host time
@@ -285,14 +315,21 @@ struct PlanMemo {
 
 // Shape-family rule.  A few rows against a large b -> the 64 x 256 three-stage tile.  Everything else -> the
 // tile and K split that the cost model of the tiled kernel picks.
-void choose(int m, int n, int k, int num_cus, fp8bs_plan_t* out, bool may_split = true, bool epi = false) {
-    static thread_local PlanMemo<fp8bs_plan_t> memo;
+const Planned& choose(int m, int n, int k, int num_cus, bool may_split = true, bool epi = false) {
+    static thread_local PlanMemo<Planned> memo;
     if (num_cus <= 0) num_cus = 256;
-    *out = memo.get({m, n, k, num_cus, may_split, epi}, [&](fp8bs_plan_t* plan) {
-        *plan = {};
-        if (skinny_shape(m, n, k)) choose_skinny(m, n, k, num_cus, plan, may_split);
-        else choose_tiled(m, n, k, num_cus, plan, may_split, epi);
+    return memo.get({m, n, k, num_cus, may_split, epi}, [&](Planned* out) {
+        *out = {};
+        if (skinny_shape(m, n, k)) choose_skinny(m, n, k, num_cus, out, may_split);
+        else choose_tiled(m, n, k, num_cus, out, may_split, epi);
     });
+}
+
+// The same split with its sums in the kernel.
+fp8bs_plan_t summed_in_kernel(int m, int n, int k, const fp8bs_plan_t& plan) {
+    fp8bs_plan_t p{};
+    fill_plan(m, n, k, plan.variant | plan.form * FORM1, plan.split_k, &p, 0, true);
+    return p;
 }
 
 // Order of the tiles of a grouped call (the row counts themselves are on the device).  With a tile or more of
@@ -406,6 +443,9 @@ int streamk_spin_limit() {
     return limit;
 }
 
+// Polls after which a workgroup of a K split summed in the kernel leaves its part of the sum to another: some tens of
+// microseconds, where workgroups that started together arrive within a few.  (A negative FP8BS_STREAMK_SPIN: one look only.)
+int sum_polls() { return streamk_spin_limit() < 0 ? 0 : 32; }
 
 int check_common(const void* a, const void* b, const float* as, const float* bs, void* c, int m, int n, int k) {
     if (m < 0 || n < 0 || k < 0 || (k % KBLK) != 0) return FP8BS_ERR_BAD_SHAPE;
@@ -476,7 +516,7 @@ int fp8bs_plan(int m, int n, int k, int num_cus, fp8bs_plan_t* out) {
     if (!out) return FP8BS_ERR_NULL_POINTER;
     if (m <= 0 || n <= 0 || k <= 0 || (k % KBLK) != 0) return FP8BS_ERR_BAD_SHAPE;
     if (num_cus <= 0) num_cus = fp8bs::device_cus();     // the current device's, 256 where there is none
-    choose(m, n, k, num_cus, out);
+    *out = choose(m, n, k, num_cus).plan;
     return FP8BS_OK;
 }
 
@@ -507,7 +547,8 @@ static int dense_call(const void* a, const void* b, const float* a_scale, const 
     const bool simple = aligned && vector_shape(n);      // streaming kernels possible
     const int cus = fp8bs::device_cus();
     if (variant == FP8BS_VARIANT_AUTO) {
-        choose(m, n, k, cus, &plan, true, epi != 0);
+        const Planned planned = choose(m, n, k, cus, true, epi != 0);
+        plan = planned.plan;
         const int tile = plan.variant | plan.form * FORM1;
         if (split_k > 0) fill_plan(m, n, k, tile, split_k & ~FP8BS_SPLIT_SUM_IN_KERNEL, &plan, 0, (split_k & FP8BS_SPLIT_SUM_IN_KERNEL) != 0);
         else if (split_k < 0) fill_plan(m, n, k, plan.variant, 1, &plan, streamk_grid(plan.variant, m, n, k, cus));   // (the first form only)
@@ -516,7 +557,13 @@ static int dense_call(const void* a, const void* b, const float* a_scale, const 
             // too small for the partial tiles of a sum in the kernel but not for the planes (tiles that overhang
             // the matrix): the same split with the reduce kernel
             if (plan.sum_in_kernel && ws && ws_bytes >= planes_bytes(m, n, plan.split_k)) fill_plan(m, n, k, tile, plan.split_k, &plan);
-            else choose(m, n, k, cus, &plan, false, epi != 0);
+            else plan = choose(m, n, k, cus, false, epi != 0).plan;
+        }
+        // A captured launch cannot share out its sums (its flags' tag would not change from replay to replay), and one workgroup
+        // that adds four partial tiles and more takes longer than the reduce kernel (64 x 4096 x 7168 in eight 19 us, 14 as two launches).
+        else if (planned.share && ws) {
+            const fp8bs_plan_t p = summed_in_kernel(m, n, k, plan);
+            if (ws_bytes >= p.workspace_bytes && !fp8bs::is_capturing(s)) plan = p;
         }
     } else {
         VariantInfo vi{};
@@ -550,6 +597,7 @@ static int dense_call(const void* a, const void* b, const float* a_scale, const 
     if (plan.sum_in_kernel && plan.split_k > 1) {
         mode = 4;
         g.sk_nonce = next_nonce();
+        g.sk_spin = sum_polls();
     } else if (plan.stream_k > 0) {
         mode = 3;
         g.sk_grid = plan.stream_k;
@@ -582,7 +630,7 @@ int fp8bs_gemm_noalloc(const void* a, const void* b, const float* a_scale, const
     // the plan fp8bs_gemm would follow; its partial planes must fit the built-in array
     fp8bs_plan_t plan{};
     if (k > 0) {
-        choose(m, n, k, fp8bs::device_cus(), &plan);
+        plan = choose(m, n, k, fp8bs::device_cus()).plan;
         uint64_t need = plan.workspace_bytes;
         if (plan.sum_in_kernel && planes_bytes(m, n, plan.split_k) < need) need = planes_bytes(m, n, plan.split_k);   // fp8bs_gemm_ex falls back to the planes
         if (need > (uint64_t)FP8BS_NOALLOC_SCRATCH_BYTES) return FP8BS_ERR_SCRATCH_LIMIT;
@@ -636,7 +684,7 @@ static int grouped_call(const void* a, const void* b, const float* a_scale, cons
     }
     g.split_k = plan.split;
     g.kb_per_split = (int)cdiv(k / KBLK, plan.split);
-    if (plan.split > 1) g.sk_nonce = next_nonce();
+    if (plan.split > 1) { g.sk_nonce = next_nonce(); g.sk_spin = sum_polls(); }
     if (fp8bs::launch_gemm(plan.tile, plan.split > 1 ? 5 : 2, g, (hipStream_t)stream) != hipSuccess) return FP8BS_ERR_LAUNCH;
     return FP8BS_OK;
 }
@@ -648,9 +696,8 @@ size_t fp8bs_grouped_workspace_bytes(int num_experts, int total_rows, int n, int
 
 size_t fp8bs_silu_mul_workspace_bytes(int rows, int n, int k) {
     if (rows <= 0 || n <= 0 || k <= 0 || (k % KBLK) != 0) return 0;
-    fp8bs_plan_t p{};
-    choose(rows, n, k, fp8bs::device_cus(), &p, true, true);
-    return (size_t)p.workspace_bytes;
+    const Planned& p = choose(rows, n, k, fp8bs::device_cus(), true, true);
+    return (size_t)(p.share ? summed_in_kernel(rows, n, k, p.plan) : p.plan).workspace_bytes;
 }
 
 int fp8bs_gemm_grouped_ex(const void* a, const void* b, const float* a_scale, const float* b_scale,

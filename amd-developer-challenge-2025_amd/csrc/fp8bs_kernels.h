@@ -29,7 +29,8 @@ struct GemmArgs {
     // 8-byte flag per workgroup) and one fp32 partial tile per workgroup, see StreamK below
     unsigned long long sk_nonce;   // value a flag takes when its workgroup's partial tile is complete: differs from call to call
     int sk_grid;            // workgroups of such a call: at most the places on the chip and the number of (tile, K block) pairs
-    int sk_spin;            // polls of a flag before the wait gives up (< 0: give up at once - tests of the error path)
+    int sk_spin;            // polls of a flag before the wait gives up (< 0: give up at once - tests of the error path); with a shared-out sum: before a part is left to another workgroup
+    int sum_shared;         // K split summed in the kernel: the sum of a tile is shared out among its workgroups (set by the launcher)
 };
 
 // Workspace of a call that deals K blocks (all offsets from the 16-byte aligned workspace base):
@@ -76,6 +77,19 @@ inline int device_cus() {
 // (For row_offsets that do not descend; the kernel cuts the slots of any others here where it sums K partitions, whose
 // counters and partial tiles are laid out for this many.)
 __host__ __device__ inline long grouped_slots_bound(long rows, long experts, int bm) { return (rows < experts ? rows : experts) + rows / (bm - 14); }
+
+// Can the workgroups of a K split summed in the kernel share out the sums?  One workgroup per (tile, partition), all on the chip
+// together, a flag for each in the workspace's header, a partition count the kernel is instantiated for, and a launch that is not
+// captured: the flags carry a tag that is new with every call, and a replay would meet its own.  (Up to eight tiles one
+// workgroup's sum is as fast: 1 x 512 x 7168 in two to four partitions of 64 x 64, 14.1 / 11.5 / 10.3 us either way.)
+inline bool is_capturing(hipStream_t stream) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) { (void)hipGetLastError(); return true; }    // (cannot be told: what a captured launch takes is always right)
+    return cap != hipStreamCaptureStatusNone;
+}
+inline bool can_share_sum(long workgroups, long resident, int split_k, hipStream_t stream) {
+    return workgroups > 8L * split_k && workgroups <= resident && workgroups <= StreamK::MAX_GRID && (split_k == 2 || split_k == 3 || split_k == 4 || split_k == 6 || split_k == 8) && !is_capturing(stream);
+}
 
 // mode: 0 dense bf16, 1 dense split-K partials, 2 grouped, 3 K blocks dealt, 4 dense split-K summed in the kernel, 5 grouped likewise.  tile: FP8BS_VARIANT_* (not AUTO) + 256 * form.
 hipError_t launch_gemm(int tile, int mode, const GemmArgs& args, hipStream_t stream);

@@ -104,7 +104,7 @@ __device__ __forceinline__ void band_tile(int v, int tiles_m, int tiles_n, int g
 //   MODE 1  : dense split-K, fp32 partial planes to the workspace
 //   MODE 2  : grouped (row_offsets), bf16 output
 //   MODE 3  : dense, K blocks instead of tiles dealt to the workgroups, partial tiles through the workspace, bf16 output
-//   MODE 4  : dense split-K, partial tiles to the workspace, summed by the last workgroup to finish a tile, bf16 output
+//   MODE 4  : dense split-K, partial tiles to the workspace, the sum of a tile shared out among its workgroups or done by the last of them, bf16 output
 //   MODE 5  : grouped like MODE 2 with a K split summed like MODE 4's
 // LDS: NSTAGE stages, each [128 k][BM] bytes of A then [128 k][BN] bytes of B, 16-byte chunks XOR-swizzled
 // so that the 16 k rows touched by half a wave in one transposing read fall on 16 different 16-byte
@@ -230,11 +230,17 @@ constexpr int waves_per_simd() {
     return MODE >= 3 && w > 1 ? w : 1;
 }
 
+// Tiles whose K partitions can share out the sum of a tile (see there).  Not 64x128: its two workgroups per CU leave 128
+// registers a wave, and the sums spill (128 x 7168 x 7168 in three 26.9 us against 24.9 with one workgroup summing); not
+// the tiles with more than eight accumulators a wave, which the planner splits in two or three only where the chip is full.
+template <int BM, int BN, int WM, int WN> constexpr bool shares_sum() { return (BM == 64 && BN == 64) || (WM == 32 && WN == 64); }
+
 template <int BM, int BN, int WM, int WN, int MODE, int EPI = 0, int NSTAGE = 2, bool TAILS = false>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) __attribute__((amdgpu_waves_per_eu(waves_per_simd<BM, BN, WM, WN, MODE, NSTAGE>())))
 void gemm_tr_kernel(const GemmArgs p) {
     using C = TileCfg<BM, BN, WM, WN, MODE, NSTAGE>;
     constexpr bool GROUPED = MODE == 2 || MODE == 5, SUMMED = MODE == 4 || MODE == 5;
+    constexpr bool SHARED_SUM = SUMMED && shares_sum<BM, BN, WM, WN>();
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
 
     // global store instructions per wave and tile in the bf16 epilogue (always this many: lanes without
@@ -870,6 +876,7 @@ void gemm_tr_kernel(const GemmArgs p) {
     // the memory side of the eight L2s), in the order of the lanes: the two sides run the same tile shape, so
     // accumulator (t, u) of wave w is the 1 KiB piece number w*MT*NT + t*NT + u of the slot.
     bool store_output = true;
+    [[maybe_unused]] uint32_t out_parts = 1;                 // SHARED_SUM: the parts of the tile that this workgroup writes
     if constexpr (MODE == 3) {
         constexpr uint32_t SLOT_BYTES = (uint32_t)BM * (uint32_t)BN * 4u;
         constexpr int NG = C::MT * C::NT;
@@ -952,14 +959,11 @@ void gemm_tr_kernel(const GemmArgs p) {
         constexpr uint32_t SLOT_BYTES = (uint32_t)BM * (uint32_t)BN * 4u;
         constexpr int NG = C::MT * C::NT;
         constexpr int AUX_AGENT = 16;                                           // sc1
-        __shared__ int last_in;
+        __shared__ int last_in, all_in;
         unsigned char* const ws_base = (unsigned char*)p.ws;
         unsigned long long* const counters = (unsigned long long*)(ws_base + StreamK::FLAGS_OFF);
         unsigned char* const tile_slots = ws_base + StreamK::SLOTS_OFF + (size_t)sk_first * (size_t)p.split_k * SLOT_BYTES;
         const uint32_t voff = (uint32_t)(wave * NG) * 1024u + (uint32_t)lane * 16u;
-        // (the counter is read ahead of the stores: the value only seeds the exchange below, which finds out if it is stale)
-        unsigned long long seen = 0;
-        if (tid == 0) seen = __hip_atomic_load(&counters[sk_first], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // Lanes whose row or columns lie outside the matrix neither store nor load their piece (an offset beyond the
         // slot drops a store and makes a load return zeros): one row against 18432 columns leaves 1 KB per workgroup
         // in the workspace instead of 32 KB (31.6 us with every lane storing, against 29.1 as two launches).
@@ -971,6 +975,127 @@ void gemm_tr_kernel(const GemmArgs p) {
         auto piece = [&](int x) -> uint32_t {               // x = t * NT + u, a compile-time number at every use
             return ((rows_in >> (x / C::NT)) & (cols_in >> (x % C::NT)) & 1u) ? voff + (uint32_t)x * 1024u : 0xFFFFFFFFu;
         };
+        auto slot_of = [&](int z) { return __builtin_amdgcn_make_buffer_rsrc((void*)(tile_slots + (size_t)z * SLOT_BYTES), 0, SLOT_BYTES, 0x00020000); };
+        bool summed = false;
+        if constexpr (SHARED_SUM) if (p.sum_shared) {
+            // The sum is shared out: of every wave's accumulators partition z adds the z-th S-th part and writes that part of c,
+            // so a workgroup stores and loads (S-1)/S of a tile, all of a tile's workgroups at once, where below every one
+            // stores a tile and then one loads S-1.  Each raises a flag of its own - one store, no exchange that S workgroups
+            // queue for - and polls all S of them with one load.  What is left is a chain of round trips to the point of
+            // coherence: stores acknowledged, flag and poll, loads.  Measured against the sum by one workgroup (us): 1024 x 1536 x
+            // 7168 in two 21.0 / 21.4, 64 x 18432 x 7168 in three 33.0 / 33.7, 128 x 7168 x 7168 in four 16.3 / 18.4, 64 x 4096 x 7168 in
+            // eight 12.4 / 19.2 (128x128 tile, two launches 13.4).  With the partitions of a tile on one XCD, so that the parts travel
+            // through its L2, the chain is shorter and the K loops read more: 21.7 and 18.2 on the first and the third.
+            // Nobody depends on another workgroup being on the chip: one that has not seen all flags within a bounded number
+            // of polls stores its own part too, marks it as left and moves on.  Whoever sees all flags up, with its own known
+            // to be visible, claims and adds the parts that are marked by then; one that marks its part looks at the flags
+            // again afterwards, so the part of a workgroup that leaves as the last one arrives is claimed by one of the two.
+            // Flags: the call's tag and 1 = stored, 2 = its own part left, 3 = that part claimed.  They are not taken down, so
+            // the launcher does this only where the tag is new on every run (not in a captured launch) and every pair of tile
+            // and partition has a workgroup of its own.
+            constexpr auto owner = [](int x, int S) constexpr { return x * S / NG; };
+            const unsigned long long tag = (p.sk_nonce | 0x10000ull) & ~0xFFFFull;           // never zero
+            auto shared = [&]<int S>() {
+                constexpr uint32_t ALL = (1u << S) - 1u;
+                unsigned long long* const flags = counters + sk_first * S;
+                const uint32_t mine = 1u << split_z;
+                // (keeps the offsets of all pieces from being worked out ahead of the branches and held in registers)
+                auto here = [](uint32_t& rows, uint32_t& cols) { asm volatile("" : "+v"(rows), "+v"(cols)); };
+                auto store_parts = [&](uint32_t parts) {
+                    const __amdgpu_buffer_rsrc_t rs = slot_of(split_z);
+                    here(rows_in, cols_in);
+#pragma unroll
+                    for (int x = 0; x < NG; x++)
+                        if ((parts >> owner(x, S)) & 1u) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, acc[x / C::NT][x % C::NT]), rs, piece(x), 0, AUX_AGENT);
+                };
+                auto sum_part = [&]<int Z>() {
+                    constexpr int X0 = (Z * NG + S - 1) / S, X1 = ((Z + 1) * NG + S - 1) / S, N = X1 - X0;      // owner(x) == Z for x in [X0, X1)
+                    if constexpr (N > 0) {
+                        here(rows_in, cols_in);
+                        v4f part[S - 1][N];                                          // the other partitions, ascending
+#pragma unroll
+                        for (int j = 0; j < S - 1; j++) {
+                            const __amdgpu_buffer_rsrc_t rs = slot_of(j + (j >= split_z ? 1 : 0));
+#pragma unroll
+                            for (int i = 0; i < N; i++) part[j][i] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rs, piece(X0 + i), 0, AUX_AGENT));
+                        }
+#pragma unroll
+                        for (int i = 0; i < N; i++) {
+                            v4f& own = acc[(X0 + i) / C::NT][(X0 + i) % C::NT];
+                            v4f sum = part[0][i];
+                            if (split_z == 0) sum = own + sum;                        // (the same bits as sum + own)
+#pragma unroll
+                            for (int j = 1; j < S - 1; j++) {
+                                if (j == split_z) sum += own;
+                                sum += part[j][i];
+                            }
+                            if (split_z == S - 1) sum += own;
+                            own = sum;
+                        }
+                    }
+                };
+                auto sum_parts = [&](uint32_t parts) {
+                    if (wave_active)
+                        [&]<int... Z>(std::integer_sequence<int, Z...>) {
+                            (((parts >> Z) & 1u ? sum_part.template operator()<Z>() : (void)0), ...);
+                        }(std::make_integer_sequence<int, S>{});
+                };
+                auto read_flags = [&]() -> unsigned long long { return lane < S ? __hip_atomic_load(&flags[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : tag | 1ull; };
+                auto claim = [&](unsigned long long f) -> uint32_t {                  // the marked parts that this workgroup takes
+                    unsigned long long left = tag | 2ull;
+                    const bool got = lane < S && f == left && __hip_atomic_compare_exchange_strong(&flags[lane], &left, tag | 3ull, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    return (uint32_t)__ballot(got);
+                };
+                if (wave_active) store_parts(ALL & ~mine);
+                wait_vmcnt<0>();                                                      // acknowledged from the agent's point of coherence
+                __syncthreads();
+                if (wave == 0) {
+                    if (lane == 0) __hip_atomic_store(&flags[split_z], tag | 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    bool all = false;
+                    for (int polls = p.sk_spin;; polls--) {
+                        all = __ballot((read_flags() & ~0xFFFFull) != tag) == 0;
+                        if (all || polls <= 0) break;
+                        __builtin_amdgcn_s_sleep(1);
+                    }
+                    if (lane == 0) all_in = all ? 1 : 0;
+                }
+                __syncthreads();
+                const bool all = __builtin_amdgcn_readfirstlane(all_in) != 0;
+                if (!all) {
+                    if (wave_active) store_parts(mine);
+                    wait_vmcnt<0>();
+                    __syncthreads();
+                    if (wave == 0 && lane == 0) __hip_atomic_store(&flags[split_z], tag | 2ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                unsigned long long f = 0;
+                if (wave == 0) {
+                    wait_vmcnt<0>();                                                  // this workgroup's flag or mark is visible
+                    f = read_flags();
+                }
+                if (all) sum_parts(mine);
+                if (wave == 0) {
+                    const uint32_t got = __ballot((f & ~0xFFFFull) != tag) == 0 ? claim(f) : 0u;
+                    if (lane == 0) last_in = (int)got;
+                }
+                __syncthreads();
+                const uint32_t taken = (uint32_t)__builtin_amdgcn_readfirstlane(last_in);
+                if (taken) sum_parts(taken);
+                out_parts = (all ? mine : 0u) | taken;
+            };
+            switch (p.split_k) {
+                case 2: shared.template operator()<2>(); break;
+                case 3: shared.template operator()<3>(); break;
+                case 4: shared.template operator()<4>(); break;
+                case 6: shared.template operator()<6>(); break;
+                default: shared.template operator()<8>(); break;
+            }
+            store_output = out_parts != 0;
+            summed = true;
+        }
+        if (!summed) {
+        // (the counter is read ahead of the stores: the value only seeds the exchange below, which finds out if it is stale)
+        unsigned long long seen = 0;
+        if (tid == 0) seen = __hip_atomic_load(&counters[sk_first], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (wave_active) {
             __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)(tile_slots + (size_t)split_z * SLOT_BYTES), 0, SLOT_BYTES, 0x00020000);
 #pragma unroll
@@ -995,7 +1120,6 @@ void gemm_tr_kernel(const GemmArgs p) {
         __syncthreads();
         store_output = __builtin_amdgcn_readfirstlane(last_in) != 0;
         if (store_output && wave_active) {
-            auto slot_of = [&](int z) { return __builtin_amdgcn_make_buffer_rsrc((void*)(tile_slots + (size_t)z * SLOT_BYTES), 0, SLOT_BYTES, 0x00020000); };
             // S partitions known at compile time: the loads of all other partitions' pieces of a batch are in flight
             // together (up to 16 of 16 bytes per lane); S = 0: any number, one partition at a time
             [[maybe_unused]] auto sum_planes = [&]<int S>() {
@@ -1083,6 +1207,7 @@ void gemm_tr_kernel(const GemmArgs p) {
                     default: sum_planes.template operator()<0>(); break;
                 }
             }
+        }
         }
     }
 
@@ -1209,7 +1334,11 @@ void gemm_tr_kernel(const GemmArgs p) {
                 const v4i val = *(const v4i*)(region + r * RSTRIDE + ((lane_chunk ^ sw) << 4));
                 const int pass_row0 = half * HALF_ROWS + q * ROWS_PER_PASS;            // compile-time
                 const int row = m0 + wave_row0 + pass_row0 + lane_r;
-                const bool ok = col_ok && row >= row_lo && row < row_hi;
+                bool ok = col_ok && row >= row_lo && row < row_hi;
+                if constexpr (SHARED_SUM) {
+                    const int x = ((pass_row0 + lane_r) >> 4) * C::NT + (EPI == 1 ? lane_chunk : lane_chunk >> 1);
+                    ok = ok && ((out_parts >> (p.sum_shared ? x * p.split_k / (C::MT * C::NT) : 0)) & 1u);
+                }
                 __amdgpu_buffer_rsrc_t c_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(c_tile + (size_t)pass_row0 * ldc), 0, 0xFFFFFFF0u, 0x00020000);
                 if constexpr (!TAILS) {
                     // Written once and not read again here: nontemporal where rows of c are whole 128-byte lines.
@@ -1296,12 +1425,14 @@ static inline hipError_t launch_shape(const GemmArgs& a, int mode, hipStream_t s
         return launch_tr<BM, BN, WM, WN, 3, 0, NSTAGE>(a, dim3((unsigned)a.sk_grid), stream);
     }
     const dim3 grid((unsigned)(total < resident ? total : resident));
+    GemmArgs sa = a;
+    if constexpr (shares_sum<BM, BN, WM, WN>()) sa.sum_shared = (mode == 4 || mode == 5) && can_share_sum(total, resident, a.split_k, stream);
     if (mode == 5) {
         if constexpr (GROUPED_SPLIT) {
             const long tiles = total / a.split_k;
             if (a.split_k < 2 || a.split_k > 0xFFFF || tiles > StreamK::MAX_GRID || (long)a.split_k * BM * BN * 4 >= (1L << 32)) return hipErrorInvalidValue;
-            if constexpr (WITH_EPI) { if (a.epi == 1) return launch_tr<BM, BN, WM, WN, 5, 1, NSTAGE>(a, grid, stream); }
-            return a.epi == 0 ? launch_tr<BM, BN, WM, WN, 5, 0, NSTAGE>(a, grid, stream) : hipErrorInvalidValue;
+            if constexpr (WITH_EPI) { if (a.epi == 1) return launch_tr<BM, BN, WM, WN, 5, 1, NSTAGE>(sa, grid, stream); }
+            return a.epi == 0 ? launch_tr<BM, BN, WM, WN, 5, 0, NSTAGE>(sa, grid, stream) : hipErrorInvalidValue;
         } else {
             return hipErrorInvalidValue;
         }
@@ -1310,8 +1441,8 @@ static inline hipError_t launch_shape(const GemmArgs& a, int mode, hipStream_t s
         // K split summed by the last workgroup of every tile: one counter per tile in the workspace's head
         const long tiles = total / a.split_k;
         if (a.split_k < 2 || a.split_k > 0xFFFF || tiles > StreamK::MAX_GRID || (long)a.split_k * BM * BN * 4 >= (1L << 32)) return hipErrorInvalidValue;
-        if constexpr (WITH_EPI) { if (a.epi == 1) return launch_tr<BM, BN, WM, WN, 4, 1, NSTAGE>(a, grid, stream); }
-        return a.epi == 0 ? launch_tr<BM, BN, WM, WN, 4, 0, NSTAGE>(a, grid, stream) : hipErrorInvalidValue;
+        if constexpr (WITH_EPI) { if (a.epi == 1) return launch_tr<BM, BN, WM, WN, 4, 1, NSTAGE>(sa, grid, stream); }
+        return a.epi == 0 ? launch_tr<BM, BN, WM, WN, 4, 0, NSTAGE>(sa, grid, stream) : hipErrorInvalidValue;
     }
     if (a.epi != 0) {
         // (with the reduce launch of a K split the planes are plain sums and the reduce kernel applies the epilogue)

@@ -83,8 +83,10 @@ typedef struct fp8bs_plan_t {
     int32_t stream_k;       /* > 0: K blocks, not tiles, are dealt to this many workgroups (one launch;
                                partial tiles meet in the workspace); split_k is 1 then           */
     int32_t sum_in_kernel;  /* 1 (with split_k > 1): one launch - the workgroups of a tile's K partitions leave fp32
-                               partial tiles in the workspace and the last one to finish adds them in ascending K and
-                               writes c; 0: partial planes and a reduce kernel (two launches)      */
+                               partial tiles in the workspace and the sum, in ascending K, is shared out among them or
+                               done by the last one to finish; 0: partial planes and a reduce kernel (two launches; a
+                               call with 4, 6 or 8 partitions whose workspace also holds 16384 + tiles * split_k *
+                               tile_m * tile_n * 4 bytes may still take one launch, with the same bits)      */
     int32_t form;           /* form of the variant (0 unless the variant has two); a plan is run again by forcing
                                FP8BS_VARIANT_FORM(variant, form), the variant alone names its first form, another
                                tile with another workspace need where form is 1                    */
@@ -130,9 +132,11 @@ int fp8bs_gemm(const void* a, const void* b, const float* a_scale, const float* 
  * split_k | FP8BS_SPLIT_SUM_IN_KERNEL: the same K partitions in ONE launch - the role of the reference's split
  * kernel plus merge kernel (1-amd-fp8-mm/amd-fp8-mm-submission.py:371-511) without the second launch, and what
  * fp8bs_plan chooses for splits in two or three (sum_in_kernel of the plan).  Every workgroup writes its fp32
- * partial tile to the workspace and then counts itself in at the tile's counter there; the one that finds all
- * the others counted in adds the partial tiles in ascending K, its own from its registers - the order of the
- * reduce kernel, so c holds the same bits as with two launches - and writes c.  Nobody waits for anybody.  The
+ * partial tile to the workspace; then either each adds its share of the tile, once all of them have raised a flag there,
+ * and writes that part of c (the 64x64, 64x256 and eight-wave 128x128 tiles where all workgroups are on the chip at once and
+ * the launch is not captured), or the one that finds all the others counted in at the tile's counter adds them all.  The order
+ * is ascending K, the reduce kernel's, so c holds the same bits as with two launches.  Nobody depends on another
+ * workgroup being on the chip: one that waits in vain leaves its share to a later one.  The
  * tiled variants only (else FP8BS_ERR_BAD_VARIANT); with more than 2016 tiles or more than 255 partitions the
  * call takes the two-launch form.  Workspace: 16384 + tiles * split_k * tile_m * tile_n * 4 bytes
  * (FP8BS_ERR_WORKSPACE if smaller), contents unspecified on entry (a counter carries the call's own tag, so
