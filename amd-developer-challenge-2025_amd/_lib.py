@@ -34,7 +34,7 @@ class Plan(ctypes.Structure):
     ]
 
 
-SECOND_FORM_NAMES = {4: "t64x64s4", 12: "t128x128s4"}
+FORM_NAMES = {(4, 1): "t64x64s4", (12, 1): "t128x128s4", (12, 2): "waves16x64", (12, 3): "waves32x64"}
 SPLIT_SUM_IN_KERNEL = 1 << 30        # FP8BS_SPLIT_SUM_IN_KERNEL
 MIN_VERSION = 400                    # fp8bs_version() of the first library whose fp8bs_plan_t has form
 
@@ -46,8 +46,9 @@ def planned_variant(plan: Plan) -> int:
 
 def tile_name(variant: int) -> str:
     """Name of a variant argument, plain or with a form."""
-    names = SECOND_FORM_NAMES if variant >> 8 == 2 else VARIANT_NAMES
-    return names.get(variant & 255, "variant %d" % variant)
+    if variant >> 8 > 1:
+        return FORM_NAMES.get((variant & 255, (variant >> 8) - 1), "variant %d" % variant)
+    return VARIANT_NAMES.get(variant & 255, "variant %d" % variant)
 
 
 _lib = None

@@ -42,6 +42,8 @@ bool variant_info(int tile, VariantInfo* out) {
         case FP8BS_VARIANT_T256x128S3: *out = {256, 128, 512}; return true;
         case FP8BS_VARIANT_T192x192S3: *out = {192, 192, 512}; return true;
         case FP8BS_VARIANT_T64x256S3: *out = {64, 256, 512}; return true;
+        case FP8BS_VARIANT_T64x256S3 | 2 * FORM1: *out = {16, 64, 512}; return true;
+        case FP8BS_VARIANT_T64x256S3 | 3 * FORM1: *out = {32, 64, 512}; return true;
         default: return false;
     }
 }
@@ -67,6 +69,10 @@ int streamk_grid(int tile, int m, int n, int k, int num_cus) {
 // The tile of a forced variant argument: FP8BS_VARIANT_FORM(variant, form) names a form, a plain variant its first.
 int forced_tile(int variant) { return variant < 256 ? variant : variant_of(variant) | ((variant >> 8) - 1) * FORM1; }
 
+// The small tiles whose workgroups hold all partitions of K (fp8bs_waves.h): up to eight, one launch, no workspace.
+constexpr int WAVES_MAX = 8;
+bool is_waves_tile(int tile) { return tile == (FP8BS_VARIANT_T64x256S3 | 2 * FORM1) || tile == (FP8BS_VARIANT_T64x256S3 | 3 * FORM1); }
+
 bool is_streaming_variant(int v) { return v == FP8BS_VARIANT_SKINNY64x144 || v == FP8BS_VARIANT_SKINNY64x256 || v == FP8BS_VARIANT_SKINNY64x288; }
 
 // The fp32 partial planes of a K split followed by the reduce kernel.
@@ -90,7 +96,7 @@ bool has_epilogue(int tile) {
     switch (tile) {
         case FP8BS_VARIANT_T256x256: case FP8BS_VARIANT_T256x128S3: case FP8BS_VARIANT_T64x128: case FP8BS_VARIANT_T64x128 | FORM1:
         case FP8BS_VARIANT_T64x256S3: case FP8BS_VARIANT_T64x256S3 | FORM1: return true;
-        default: return false;
+        default: return is_waves_tile(tile);
     }
 }
 
@@ -109,6 +115,7 @@ void fill_plan(int m, int n, int k, int tile, int split_k, fp8bs_plan_t* out, in
     if (stream_k > 0) split_k = 1;
     if (split_k < 1) split_k = 1;
     if (split_k > kbt) split_k = kbt > 0 ? kbt : 1;
+    if (is_waves_tile(tile)) in_kernel = in_kernel || split_k <= 3 || kbt < 16;       // (see choose_tiled)
     out->variant = variant_of(tile);
     out->form = form_of(tile);
     out->tile_m = vi.bm;
@@ -121,7 +128,7 @@ void fill_plan(int m, int n, int k, int tile, int split_k, fp8bs_plan_t* out, in
     if (tile == FP8BS_VARIANT_GENERIC) {
         out->grid_x = (int)cdiv(n, 16); out->grid_y = (int)cdiv(m, 16); out->grid_z = 1;
     } else {
-        out->grid_x = stream_k > 0 ? stream_k : (int)(cdiv(m, vi.bm) * cdiv(n, vi.bn) * split_k); out->grid_y = 1; out->grid_z = 1;
+        out->grid_x = stream_k > 0 ? stream_k : (int)(cdiv(m, vi.bm) * cdiv(n, vi.bn) * (is_waves_tile(tile) ? 1 : split_k)); out->grid_y = 1; out->grid_z = 1;
     }
     if (stream_k > 0) out->workspace_bytes = (uint64_t)fp8bs::StreamK::bytes(stream_k, vi.bm, vi.bn);
     else if (out->sum_in_kernel)   // the counters, then one fp32 tile per (tile, K partition)
@@ -239,6 +246,23 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
             cost = issued(gpu, s == 1 || fuse ? 5.3 : 8.5);
             // (among equals, which the host alone makes, the shorter kernel)
             if (best_tile == 0 || cost < best_cost || (cost == best_cost && gpu < best_gpu)) { best_tile = c.tile; best_split = s; best_cost = cost; best_gpu = gpu; best_fused = fuse; }
+        }
+    }
+    // The small tiles that hold all K partitions in a workgroup: a launch, first copies and output, a chain of kbt / 8 blocks, and
+    // the requests that all workgroups make of the L2 (in units of K blocks per CU).  Fits to 264 shapes (M 1 .. 1024, N 512 ..
+    // 12288, K 384 .. 4096, operands from HBM and from the caches): where they are taken for any of these shapes, the calls take 0.81 of
+    // the time of the other tiles in the geometric mean, within 1.6 % of the best; at most 1.19 of it where the two are
+    // modelled level.  Not beyond 24 K blocks, where the others' splits over workgroups are ahead.  Up to eight blocks the sum is the
+    // unsplit one; beyond, eight partitions: the plan reports them like any K split's, sum_in_kernel says one launch up to 15
+    // K blocks and, as for the other tiles' four partitions and more, leaves it open beyond.  No workspace is used.
+    if (kbt >= 2 && (kbt <= WAVES_MAX || (may_split && kbt <= 24))) {
+        struct Waves { int tile, bm; double fixed, block, load; };
+        const Waves waves[2] = {{FP8BS_VARIANT_T64x256S3 | 2 * FORM1, 16, 2.12, 1.223, 0.312}, {FP8BS_VARIANT_T64x256S3 | 3 * FORM1, 32, 2.31, 1.485, 0.385}};
+        for (const Waves& w : waves) {
+            const int s = kbt <= WAVES_MAX ? 1 : WAVES_MAX;
+            const double gpu = w.fixed + w.block * (double)cdiv(kbt, WAVES_MAX) + w.load * (double)(cdiv(m, w.bm) * cdiv(n, 64)) * kbt / 256.0;
+            const double cost = gpu > 5.3 ? gpu : 5.3;
+            if (cost < best_cost || (cost == best_cost && gpu < best_gpu)) { best_tile = w.tile; best_split = s; best_cost = cost; best_gpu = gpu; best_fused = false; }
         }
     }
     fill_plan(m, n, k, best_tile, best_split, &out->plan, 0, best_fused && best_split <= 3);
@@ -550,10 +574,11 @@ static int dense_call(const void* a, const void* b, const float* a_scale, const 
         const Planned planned = choose(m, n, k, cus, true, epi != 0);
         plan = planned.plan;
         const int tile = plan.variant | plan.form * FORM1;
-        if (split_k > 0) fill_plan(m, n, k, tile, split_k & ~FP8BS_SPLIT_SUM_IN_KERNEL, &plan, 0, (split_k & FP8BS_SPLIT_SUM_IN_KERNEL) != 0);
+        // (a forced split may be any: the small tiles of up to eight partitions give way to 64 x 64)
+        if (split_k > 0) fill_plan(m, n, k, is_waves_tile(tile) ? FP8BS_VARIANT_T64x128 | FORM1 : tile, split_k & ~FP8BS_SPLIT_SUM_IN_KERNEL, &plan, 0, (split_k & FP8BS_SPLIT_SUM_IN_KERNEL) != 0);
         else if (split_k < 0) fill_plan(m, n, k, plan.variant, 1, &plan, streamk_grid(plan.variant, m, n, k, cus));   // (the first form only)
         // the plan needs a workspace the caller did not bring: the best plan that needs none
-        else if (plan.workspace_bytes > 0 && (!ws || ws_bytes < plan.workspace_bytes)) {
+        else if (plan.workspace_bytes > 0 && !is_waves_tile(tile) && (!ws || ws_bytes < plan.workspace_bytes)) {
             // too small for the partial tiles of a sum in the kernel but not for the planes (tiles that overhang
             // the matrix): the same split with the reduce kernel
             if (plan.sum_in_kernel && ws && ws_bytes >= planes_bytes(m, n, plan.split_k)) fill_plan(m, n, k, tile, plan.split_k, &plan);
@@ -579,9 +604,11 @@ static int dense_call(const void* a, const void* b, const float* a_scale, const 
             const bool in_kernel = split_k > 0 && (split_k & FP8BS_SPLIT_SUM_IN_KERNEL) != 0;
             if (in_kernel && (is_streaming_variant(variant) || variant == FP8BS_VARIANT_GENERIC)) return FP8BS_ERR_BAD_VARIANT;   // the tiled kernel only
             fill_plan(m, n, k, tile, split_k > 0 ? (split_k & ~FP8BS_SPLIT_SUM_IN_KERNEL) : 1, &plan, 0, in_kernel);
+            if (is_waves_tile(tile) && plan.split_k > WAVES_MAX) return FP8BS_ERR_BAD_VARIANT;
         }
     }
-    if (plan.workspace_bytes > 0 && (!ws || ws_bytes < plan.workspace_bytes)) return FP8BS_ERR_WORKSPACE;
+    const bool waves = is_waves_tile(plan.variant | plan.form * FORM1);
+    if (plan.workspace_bytes > 0 && !waves && (!ws || ws_bytes < plan.workspace_bytes)) return FP8BS_ERR_WORKSPACE;
     if (epi && plan.variant != FP8BS_VARIANT_GENERIC && (!has_epilogue(plan.variant | plan.form * FORM1) || plan.stream_k > 0)) return FP8BS_ERR_BAD_VARIANT;
 
     fp8bs::GemmArgs g{};
@@ -593,8 +620,8 @@ static int dense_call(const void* a, const void* b, const float* a_scale, const 
     g.band_h = 4;
     g.num_experts = 0;
     g.epi = epi;
-    int mode = plan.split_k > 1 ? 1 : 0;
-    if (plan.sum_in_kernel && plan.split_k > 1) {
+    int mode = plan.split_k > 1 && !waves ? 1 : 0;
+    if (plan.sum_in_kernel && plan.split_k > 1 && !waves) {
         mode = 4;
         g.sk_nonce = next_nonce();
         g.sk_spin = sum_polls();
@@ -633,7 +660,7 @@ int fp8bs_gemm_noalloc(const void* a, const void* b, const float* a_scale, const
         plan = choose(m, n, k, fp8bs::device_cus()).plan;
         uint64_t need = plan.workspace_bytes;
         if (plan.sum_in_kernel && planes_bytes(m, n, plan.split_k) < need) need = planes_bytes(m, n, plan.split_k);   // fp8bs_gemm_ex falls back to the planes
-        if (need > (uint64_t)FP8BS_NOALLOC_SCRATCH_BYTES) return FP8BS_ERR_SCRATCH_LIMIT;
+        if (need > (uint64_t)FP8BS_NOALLOC_SCRATCH_BYTES && !is_waves_tile(plan.variant | plan.form * FORM1)) return FP8BS_ERR_SCRATCH_LIMIT;
     }
     void* ws = nullptr;
     st = scratch_address(&ws, (hipStream_t)stream);
@@ -676,7 +703,7 @@ static int grouped_call(const void* a, const void* b, const float* a_scale, cons
         }
     } else {
         VariantInfo vi{};
-        if (!variant_info(plan.tile, &vi) || is_streaming_variant(plan.tile)) return FP8BS_ERR_BAD_VARIANT;   // no grouped mode in the streaming kernels
+        if (!variant_info(plan.tile, &vi) || is_streaming_variant(plan.tile) || is_waves_tile(plan.tile)) return FP8BS_ERR_BAD_VARIANT;   // no grouped mode in these kernels
         if (plan.tile != FP8BS_VARIANT_GENERIC && k == 0) return FP8BS_ERR_BAD_VARIANT;
         if (epi && plan.tile != FP8BS_VARIANT_GENERIC && !has_epilogue(plan.tile)) return FP8BS_ERR_BAD_VARIANT;
         if (plan.split > 1 && !can_split_grouped(plan, num_experts, rows, n, k)) return FP8BS_ERR_BAD_VARIANT;
@@ -697,6 +724,7 @@ size_t fp8bs_grouped_workspace_bytes(int num_experts, int total_rows, int n, int
 size_t fp8bs_silu_mul_workspace_bytes(int rows, int n, int k) {
     if (rows <= 0 || n <= 0 || k <= 0 || (k % KBLK) != 0) return 0;
     const Planned& p = choose(rows, n, k, fp8bs::device_cus(), true, true);
+    if (is_waves_tile(p.plan.variant | p.plan.form * FORM1)) return 0;
     return (size_t)(p.share ? summed_in_kernel(rows, n, k, p.plan) : p.plan).workspace_bytes;
 }
 

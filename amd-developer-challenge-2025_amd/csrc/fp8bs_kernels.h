@@ -104,6 +104,10 @@ hipError_t launch_tile_64x128(const GemmArgs& args, int mode, hipStream_t stream
 hipError_t launch_tile_64x64(const GemmArgs& args, int mode, hipStream_t stream);
 hipError_t launch_tile_192x192s3(const GemmArgs& args, int mode, hipStream_t stream);
 hipError_t launch_tile_64x256s3(const GemmArgs& args, int mode, hipStream_t stream);
+// the small tiles whose workgroups hold all K partitions (fp8bs_waves.h): split_k up to eight
+hipError_t launch_waves_16x64(const GemmArgs& args, hipStream_t stream);
+hipError_t launch_waves_32x64(const GemmArgs& args, hipStream_t stream);
+int waves_lds_bytes(int tile_m);
 hipError_t launch_splitk_reduce(const float* ws, uint16_t* c, size_t mn, int split_k, int epi, hipStream_t stream);
 int variant_lds_bytes(int tile);
 

@@ -418,6 +418,8 @@ hipError_t launch_gemm(int tile, int mode, const GemmArgs& a, hipStream_t stream
         case 11: return launch_tile_192x192s3(a, mode, stream);
         case 12: return launch_tile_64x256s3(a, mode, stream);
         case 12 | 256: return launch_tile_128x128s4(a, mode, stream);
+        case 12 | 512: return mode == 0 ? launch_waves_16x64(a, stream) : hipErrorInvalidValue;
+        case 12 | 768: return mode == 0 ? launch_waves_32x64(a, stream) : hipErrorInvalidValue;
         default: return hipErrorInvalidValue;
     }
 }
@@ -460,6 +462,8 @@ int variant_lds_bytes(int tile) {
         case 11: return TileCfg<192, 192, 48, 96, 0, 3>::LDS_BYTES;
         case 12: return TileCfg<64, 256, 32, 64, 0, 3>::LDS_BYTES;
         case 12 | 256: return TileCfg<128, 128, 32, 64, 0, 4>::LDS_BYTES;
+        case 12 | 512: return waves_lds_bytes(16);
+        case 12 | 768: return waves_lds_bytes(32);
         default: return 0;
     }
 }

@@ -195,6 +195,8 @@ def plan(m: int, n: int, k: int) -> _lib.Plan:
 def _wanted_bytes(p) -> int:
     """What a plan's call makes use of: its workspace_bytes, and room for the counters and partial tiles with which four and
     more partitions are summed in the kernel where the library finds that faster than planes and a reduce kernel."""
+    if p.variant == 12 and p.form >= 2:                # all partitions in a workgroup: none
+        return 0
     tiles = p.grid_x // p.split_k
     return max(int(p.workspace_bytes), 16384 + tiles * p.split_k * p.tile_m * p.tile_n * 4 if p.split_k > 3 and tiles * p.split_k <= 512 else 0)
 

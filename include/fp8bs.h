@@ -64,11 +64,14 @@ enum {
     FP8BS_VARIANT_T256x128S3 = 10, /* 256 x 128 tile, three LDS stages (a copy has two K blocks' time to land) */
     FP8BS_VARIANT_T192x192S3 = 11, /* 192 x 192 tile, 8 waves of 48 x 96, three LDS stages     */
     FP8BS_VARIANT_T64x256S3 = 12,  /* 8 waves of 32 x 64.  Form 0: 64(m) x 256(n) tile, three LDS stages: few rows against much of
-                                     b; form 1: 128 x 128 tile, four stages: mid-size, one tile per CU */
+                                     b; form 1: 128 x 128 tile, four stages: mid-size, one tile per CU;
+                                     forms 2 and 3: 16 x 64 and 32 x 64 tiles whose eight waves each multiply the whole
+                                     tile over a K partition of their own: small products, dense calls, split_k
+                                     up to 8, no workspace whatever the plan's workspace_bytes      */
     FP8BS_VARIANT_COUNT = 13
 };
 
-/* A forced variant argument that names one of the two forms of a variant (without it: the first form). */
+/* A forced variant argument that names one of the forms of a variant (without it: the first form). */
 #define FP8BS_VARIANT_FORM(variant, form) ((variant) | (((form) + 1) << 8))
 
 /* What fp8bs_plan() decides for a shape. Replaces the exact-(m,n,k) if-ladder of the reference
@@ -87,7 +90,7 @@ typedef struct fp8bs_plan_t {
                                done by the last one to finish; 0: partial planes and a reduce kernel (two launches; a
                                call with 4, 6 or 8 partitions whose workspace also holds 16384 + tiles * split_k *
                                tile_m * tile_n * 4 bytes may still take one launch, with the same bits)      */
-    int32_t form;           /* form of the variant (0 unless the variant has two); a plan is run again by forcing
+    int32_t form;           /* form of the variant (0 unless the variant has several); a plan is run again by forcing
                                FP8BS_VARIANT_FORM(variant, form), the variant alone names its first form, another
                                tile with another workspace need where form is 1                    */
     uint64_t workspace_bytes;
