@@ -120,6 +120,26 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+def _extension(name):
+    """A host module built next to this file, or None where it has not been built or cannot be imported (one warning)."""
+    load()                                            # the library must be there first; raises if it is not
+    path = os.path.join(HERE, name + ".so")
+    if not os.path.exists(path):
+        return None
+    import importlib.machinery
+    import importlib.util
+    try:
+        loader = importlib.machinery.ExtensionFileLoader(name, path)
+        spec = importlib.util.spec_from_file_location(name, path, loader=loader)
+        mod = importlib.util.module_from_spec(spec)
+        loader.exec_module(mod)
+        return mod
+    except (ImportError, OSError) as ex:              # built for another Python or torch, or its libraries cannot be resolved
+        import warnings
+        warnings.warn("%s.so cannot be imported (%s); going without it, which costs host time in every call" % (name, ex))
+        return None
+
+
 _pycall = False
 
 
@@ -129,22 +149,26 @@ def pycall():
     imported (one warning); callers then use the ctypes functions of load().  Either way the work is done by libfp8bs.so, which has no substitute."""
     global _pycall
     if _pycall is False:
-        load()                                        # the library must be there first; raises if it is not
-        path = os.path.join(HERE, "_fp8bs_pycall.so")
-        _pycall = None
-        if os.path.exists(path):
-            import importlib.machinery
-            import importlib.util
-            try:
-                loader = importlib.machinery.ExtensionFileLoader("_fp8bs_pycall", path)
-                spec = importlib.util.spec_from_file_location("_fp8bs_pycall", path, loader=loader)
-                mod = importlib.util.module_from_spec(spec)
-                loader.exec_module(mod)
-                _pycall = mod
-            except (ImportError, OSError) as ex:      # built for another Python, or its libfp8bs.so cannot be resolved
-                import warnings
-                warnings.warn("_fp8bs_pycall.so cannot be imported (%s); binding libfp8bs.so through ctypes instead" % ex)
+        _pycall = _extension("_fp8bs_pycall")
     return _pycall
+
+
+_dense = False
+
+
+def dense():
+    """custom_kernel's checks and call on torch tensors (csrc/fp8bs_torch.cpp's dense), or None where the module has not been
+    built, cannot be imported, or was built against another torch (one warning)."""
+    global _dense
+    if _dense is False:
+        import torch
+        mod = _extension("_fp8bs_torch")
+        if mod is not None and mod.torch_version != torch.__version__:
+            import warnings
+            warnings.warn("_fp8bs_torch.so was built against torch %s; going without it, which costs host time in every call" % mod.torch_version)
+            mod = None
+        _dense = mod.dense if mod is not None else None
+    return _dense
 
 
 _CALLS = ("gemm_ex", "gemm_grouped_ws", "gemm_silu_mul_ws", "quantize_a", "quantize_b", "gather_a", "moe_topk", "moe_route", "moe_combine")

@@ -17,7 +17,6 @@ the split-K workspace is cached per device instead of allocated per call
 branch overwrites them, :570-571).
 """
 import ctypes
-import weakref
 
 import torch
 
@@ -95,20 +94,10 @@ _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 _plan_cache = {}   # (m, n, k) and ("grouped" | "silu" | "route", sizes ...) -> workspace bytes the call asks for
 _PLANS_MAX = 4096
 
-# Operands that passed the checks once: a caller that hands over the same tensor objects again (a benchmark
-# loop, a layer called every step) skips the dtype / device / K-major checks, which cost more host time than a
-# small GEMM takes on the GPU.  An entry is keyed by the identities of the tensors and holds weak references,
-# so a recycled id() cannot alias a dead tensor; what can change under one identity (resize_, set_, as_strided_,
-# t_, .data = ...) is caught by comparing addresses, shapes and strides with the ones that were checked.
+# Dense sizes that the native call of custom_kernel may take, with the workspace bytes that each asks for.  It checks the tensors
+# themselves at every call; what it is told here is a fact about the sizes alone.
 _CHECKED_MAX = 64
-_checked = {}      # ids -> (weakrefs, addresses, shapes, strides, sizes ..., device index)
-
-
-def _remember(key, data, *rest):
-    if len(_checked) >= _CHECKED_MAX:
-        _checked.pop(next(iter(_checked)))
-    _checked[key] = (tuple(weakref.ref(t) for t in data), tuple(t.data_ptr() for t in data), tuple(t.shape for t in data),
-                     tuple(t.stride() for t in data)) + rest
+_checked = {}      # (m, n, k) -> bytes
 
 
 def _grouped_workspace(device, stream, num_experts, rows, n, k):
@@ -212,29 +201,20 @@ def custom_kernel(data, variant: int = 0, split_k: int = 0):
     (``split_k | SPLIT_SUM_IN_KERNEL``: the partitions summed in the one kernel; ``split_k < 0``: K blocks
     dealt to the workgroups); the defaults let the library's planner decide.
     """
+    if variant == 0 and split_k == 0:
+        dense = _lib.dense()
+        if dense is not None:
+            st = dense(data, _checked, 0, 0)
+            if st < -1:                               # all is well, and it wants a workspace
+                dev = data[0].device
+                ws = _workspace(dev, -st, _stream_ptr(dev))
+                st = dense(data, _checked, ws.data_ptr(), ws.numel())
+            if st == 0:
+                return data[4]
+            if st > 0:
+                _lib.check(st)
     a, b, a_scale, b_scale, c = data
     gemm_ex = _lib.calls().gemm_ex
-    key = None
-    if variant == 0 and split_k == 0:
-        key = (id(a), id(b), id(a_scale), id(b_scale), id(c))
-        hit = _checked.get(key)
-        if hit is not None:
-            refs, ptrs, shapes, strides, m, n, k, need, dev_index = hit
-            pa, pb, pas, pbs, pc = a.data_ptr(), b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(), c.data_ptr()
-            if refs[0]() is a and refs[1]() is b and refs[2]() is a_scale and refs[3]() is b_scale and refs[4]() is c \
-                    and (pa, pb, pas, pbs, pc) == ptrs \
-                    and a.shape == shapes[0] and b.shape == shapes[1] and a_scale.shape == shapes[2] and b_scale.shape == shapes[3] and c.shape == shapes[4] \
-                    and a.stride() == strides[0] and b.stride() == strides[1] and a_scale.stride() == strides[2] \
-                    and b_scale.stride() == strides[3] and c.stride() == strides[4] and dev_index == torch.cuda.current_device():
-                stream = _stream_ptr(a.device)
-                ws_ptr, ws_len = None, 0
-                if need:
-                    ws = _workspace(a.device, need, stream)
-                    ws_ptr, ws_len = ws.data_ptr(), ws.numel()
-                st = gemm_ex(pa, pb, pas, pbs, pc, ws_ptr, ws_len, m, n, k, 0, 0, stream)
-                if st:
-                    _lib.check(st)
-                return c
     m, k = a.shape
     n = b.shape[0]
     _check_operands(a, b, a_scale, b_scale, c, m, n, k)
@@ -250,7 +230,10 @@ def custom_kernel(data, variant: int = 0, split_k: int = 0):
             if len(_plan_cache) >= _PLANS_MAX:
                 _plan_cache.clear()
             _plan_cache[(m, n, k)] = need
-        _remember(key, data, m, n, k, need, a.device.index)
+        if (m, n, k) not in _checked:
+            if len(_checked) >= _CHECKED_MAX:
+                _checked.clear()
+            _checked[(m, n, k)] = need
     else:
         # a forced K split's planes; K blocks dealt to the workgroups (split_k < 0): a header and one fp32 tile per
         # workgroup, at most 64 MiB for every tile shape on 256 CUs
