@@ -30,7 +30,6 @@ struct GemmArgs {
     unsigned long long sk_nonce;   // value a flag takes when its workgroup's partial tile is complete: differs from call to call
     int sk_grid;            // workgroups of such a call: at most the places on the chip and the number of (tile, K block) pairs
     int sk_spin;            // polls of a flag before the wait gives up (< 0: give up at once - tests of the error path); with a shared-out sum: before a part is left to another workgroup
-    int sum_shared;         // K split summed in the kernel: the sum of a tile is shared out among its workgroups (set by the launcher)
 };
 
 // Workspace of a call that deals K blocks (all offsets from the 16-byte aligned workspace base):

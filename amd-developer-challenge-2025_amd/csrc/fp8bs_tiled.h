@@ -235,12 +235,15 @@ constexpr int waves_per_simd() {
 // the tiles with more than eight accumulators a wave, which the planner splits in two or three only where the chip is full.
 template <int BM, int BN, int WM, int WN> constexpr bool shares_sum() { return (BM == 64 && BN == 64) || (WM == 32 && WN == 64); }
 
-template <int BM, int BN, int WM, int WN, int MODE, int EPI = 0, int NSTAGE = 2, bool TAILS = false>
+// SHARED_SUM: the sum of a tile is shared out among its workgroups; without, the last of them does it.  An instantiation each, chosen
+// by the launcher: with both forms in one kernel the sum by one workgroup - all that a captured launch can have - was 2 to 5 % slower
+// (us, replayed: 448 x 924 x 4480 12.9 and 12.3, 22 x 4544 x 3200 9.8 and 9.3, 1876 x 571 x 4608 20.8 and 20.0).
+template <int BM, int BN, int WM, int WN, int MODE, int EPI = 0, int NSTAGE = 2, bool TAILS = false, bool SHARED_SUM = false>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) __attribute__((amdgpu_waves_per_eu(waves_per_simd<BM, BN, WM, WN, MODE, NSTAGE>())))
 void gemm_tr_kernel(const GemmArgs p) {
     using C = TileCfg<BM, BN, WM, WN, MODE, NSTAGE>;
     constexpr bool GROUPED = MODE == 2 || MODE == 5, SUMMED = MODE == 4 || MODE == 5;
-    constexpr bool SHARED_SUM = SUMMED && shares_sum<BM, BN, WM, WN>();
+    static_assert(!SHARED_SUM || (SUMMED && shares_sum<BM, BN, WM, WN>()));
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
 
     // global store instructions per wave and tile in the bf16 epilogue (always this many: lanes without
@@ -976,8 +979,7 @@ void gemm_tr_kernel(const GemmArgs p) {
             return ((rows_in >> (x / C::NT)) & (cols_in >> (x % C::NT)) & 1u) ? voff + (uint32_t)x * 1024u : 0xFFFFFFFFu;
         };
         auto slot_of = [&](int z) { return __builtin_amdgcn_make_buffer_rsrc((void*)(tile_slots + (size_t)z * SLOT_BYTES), 0, SLOT_BYTES, 0x00020000); };
-        bool summed = false;
-        if constexpr (SHARED_SUM) if (p.sum_shared) {
+        if constexpr (SHARED_SUM) {
             // The sum is shared out: of every wave's accumulators partition z adds the z-th S-th part and writes that part of c,
             // so a workgroup stores and loads (S-1)/S of a tile, all of a tile's workgroups at once, where below every one
             // stores a tile and then one loads S-1.  Each raises a flag of its own - one store, no exchange that S workgroups
@@ -1090,9 +1092,7 @@ void gemm_tr_kernel(const GemmArgs p) {
                 default: shared.template operator()<8>(); break;
             }
             store_output = out_parts != 0;
-            summed = true;
-        }
-        if (!summed) {
+        } else {
         // (the counter is read ahead of the stores: the value only seeds the exchange below, which finds out if it is stale)
         unsigned long long seen = 0;
         if (tid == 0) seen = __hip_atomic_load(&counters[sk_first], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1337,7 +1337,7 @@ void gemm_tr_kernel(const GemmArgs p) {
                 bool ok = col_ok && row >= row_lo && row < row_hi;
                 if constexpr (SHARED_SUM) {
                     const int x = ((pass_row0 + lane_r) >> 4) * C::NT + (EPI == 1 ? lane_chunk : lane_chunk >> 1);
-                    ok = ok && ((out_parts >> (p.sum_shared ? x * p.split_k / (C::MT * C::NT) : 0)) & 1u);
+                    ok = ok && ((out_parts >> (x * p.split_k / (C::MT * C::NT))) & 1u);
                 }
                 __amdgpu_buffer_rsrc_t c_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(c_tile + (size_t)pass_row0 * ldc), 0, 0xFFFFFFF0u, 0x00020000);
                 if constexpr (!TAILS) {
@@ -1380,22 +1380,33 @@ void gemm_tr_kernel(const GemmArgs p) {
 // ---------------------------------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------------------------------
-template <int BM, int BN, int WM, int WN, int MODE, int EPI = 0, int NSTAGE = 2>
+// Rows of a that are not a multiple of four, columns that are not a multiple of eight, operands that start off the 16-byte
+// grid: the instantiation that repairs the last bytes of a and b and stores c without assuming any alignment of its rows.
+// (with the fused epilogue the rows of the output have n/2 columns: 16-byte stores need n/2 on the 8-column grid; MODE 1 writes
+// planes of n columns, not c)
+template <int EPI>
+static inline bool needs_tails(const GemmArgs& a) {
+    const int out_cols = EPI == 1 ? a.n / 2 : a.n;
+    return (a.lda & 3) != 0 || (a.n & 7) != 0 || (out_cols & 7) != 0 || (((uintptr_t)a.a | (uintptr_t)a.b | (uintptr_t)a.c) & 15) != 0;
+}
+
+// The instantiation of a call, its LDS limit raised.
+template <int BM, int BN, int WM, int WN, int MODE, int EPI, int NSTAGE, bool SHARED_SUM>
+static inline hipError_t ready_tr(const GemmArgs& a, void (**kern)(const GemmArgs)) {
+    const bool tails = needs_tails<EPI>(a);
+    *kern = tails ? gemm_tr_kernel<BM, BN, WM, WN, MODE, EPI, NSTAGE, true, SHARED_SUM> : gemm_tr_kernel<BM, BN, WM, WN, MODE, EPI, NSTAGE, false, SHARED_SUM>;
+    static int raised[2][MAX_DEVICES];
+    return raise_lds_limit((const void*)*kern, TileCfg<BM, BN, WM, WN, MODE, NSTAGE>::LDS_BYTES, raised[tails ? 1 : 0]);
+}
+
+template <int BM, int BN, int WM, int WN, int MODE, int EPI = 0, int NSTAGE = 2, bool SHARED_SUM = false>
 static inline hipError_t launch_tr(const GemmArgs& a, dim3 grid, hipStream_t stream) {
     using C = TileCfg<BM, BN, WM, WN, MODE, NSTAGE>;
-    // rows of a that are not a multiple of four, columns that are not a multiple of eight, operands that
-    // start off the 16-byte grid: the instantiation that repairs the last bytes of a and b and stores c
-    // without assuming any alignment of its rows
-    // (with the fused epilogue the rows of the output have n/2 columns: 16-byte stores need n/2 on the 8-column grid)
-    const int out_cols = EPI == 1 ? a.n / 2 : a.n;
-    // (MODE 1 writes planes of n columns, not c)
-    const bool tails = (a.lda & 3) != 0 || (a.n & 7) != 0 || (out_cols & 7) != 0 || (((uintptr_t)a.a | (uintptr_t)a.b | (uintptr_t)a.c) & 15) != 0;
-    GemmArgs args = a;
-    args.c_whole_lines = ((size_t)out_cols * 2u) % 128u == 0 && ((uintptr_t)a.c & 127) == 0;
-    void (*kern)(const GemmArgs) = tails ? gemm_tr_kernel<BM, BN, WM, WN, MODE, EPI, NSTAGE, true> : gemm_tr_kernel<BM, BN, WM, WN, MODE, EPI, NSTAGE, false>;
-    static int raised[2][MAX_DEVICES];
-    hipError_t e = raise_lds_limit((const void*)kern, C::LDS_BYTES, raised[tails ? 1 : 0]);
+    void (*kern)(const GemmArgs);
+    hipError_t e = ready_tr<BM, BN, WM, WN, MODE, EPI, NSTAGE, SHARED_SUM>(a, &kern);
     if (e != hipSuccess) return e;
+    GemmArgs args = a;
+    args.c_whole_lines = ((size_t)(EPI == 1 ? a.n / 2 : a.n) * 2u) % 128u == 0 && ((uintptr_t)a.c & 127) == 0;
     hipLaunchKernelGGL(kern, grid, dim3(C::NTHREADS), C::LDS_BYTES, stream, args);
     return hipGetLastError();
 }
@@ -1425,24 +1436,36 @@ static inline hipError_t launch_shape(const GemmArgs& a, int mode, hipStream_t s
         return launch_tr<BM, BN, WM, WN, 3, 0, NSTAGE>(a, dim3((unsigned)a.sk_grid), stream);
     }
     const dim3 grid((unsigned)(total < resident ? total : resident));
-    GemmArgs sa = a;
-    if constexpr (shares_sum<BM, BN, WM, WN>()) sa.sum_shared = (mode == 4 || mode == 5) && can_share_sum(total, resident, a.split_k, stream);
+    // K partitions summed in the kernel, the sum shared out or not.  A call that shares it readies the kernel that a capture of the
+    // same call will launch too: the LDS limit is not a thing to be raised there.
+    auto launch_summed = [&](auto mode_tag, auto epi_tag) {
+        constexpr int M = decltype(mode_tag)::value, E = decltype(epi_tag)::value;
+        if constexpr (shares_sum<BM, BN, WM, WN>())
+            if (can_share_sum(total, resident, a.split_k, stream)) {
+                void (*captured)(const GemmArgs);
+                hipError_t e = ready_tr<BM, BN, WM, WN, M, E, NSTAGE, false>(a, &captured);
+                if (e != hipSuccess) return e;
+                return launch_tr<BM, BN, WM, WN, M, E, NSTAGE, true>(a, grid, stream);
+            }
+        return launch_tr<BM, BN, WM, WN, M, E, NSTAGE>(a, grid, stream);
+    };
+    using std::integral_constant;
     if (mode == 5) {
         if constexpr (GROUPED_SPLIT) {
             const long tiles = total / a.split_k;
             if (a.split_k < 2 || a.split_k > 0xFFFF || tiles > StreamK::MAX_GRID || (long)a.split_k * BM * BN * 4 >= (1L << 32)) return hipErrorInvalidValue;
-            if constexpr (WITH_EPI) { if (a.epi == 1) return launch_tr<BM, BN, WM, WN, 5, 1, NSTAGE>(sa, grid, stream); }
-            return a.epi == 0 ? launch_tr<BM, BN, WM, WN, 5, 0, NSTAGE>(sa, grid, stream) : hipErrorInvalidValue;
+            if constexpr (WITH_EPI) { if (a.epi == 1) return launch_summed(integral_constant<int, 5>{}, integral_constant<int, 1>{}); }
+            return a.epi == 0 ? launch_summed(integral_constant<int, 5>{}, integral_constant<int, 0>{}) : hipErrorInvalidValue;
         } else {
             return hipErrorInvalidValue;
         }
     }
     if (mode == 4) {
-        // K split summed by the last workgroup of every tile: one counter per tile in the workspace's head
+        // K split summed in the kernel: one counter per tile, or one flag per workgroup, in the workspace's head
         const long tiles = total / a.split_k;
         if (a.split_k < 2 || a.split_k > 0xFFFF || tiles > StreamK::MAX_GRID || (long)a.split_k * BM * BN * 4 >= (1L << 32)) return hipErrorInvalidValue;
-        if constexpr (WITH_EPI) { if (a.epi == 1) return launch_tr<BM, BN, WM, WN, 4, 1, NSTAGE>(sa, grid, stream); }
-        return a.epi == 0 ? launch_tr<BM, BN, WM, WN, 4, 0, NSTAGE>(sa, grid, stream) : hipErrorInvalidValue;
+        if constexpr (WITH_EPI) { if (a.epi == 1) return launch_summed(integral_constant<int, 4>{}, integral_constant<int, 1>{}); }
+        return a.epi == 0 ? launch_summed(integral_constant<int, 4>{}, integral_constant<int, 0>{}) : hipErrorInvalidValue;
     }
     if (a.epi != 0) {
         // (with the reduce launch of a K split the planes are plain sums and the reduce kernel applies the epilogue)

@@ -1,0 +1,88 @@
+"""What a call launches when its stream is captured, and what an eager call of the same shape has made ready for it.
+
+On the CPU: a small library loaded ahead of the HIP runtime says whether the stream is capturing, and takes the launches and the
+attribute calls instead of the runtime.  No pointer is dereferenced."""
+import json
+import subprocess
+import sys
+
+import pytest
+
+SHIM = r"""
+#include <stdint.h>
+#include <stdio.h>
+typedef struct { uint32_t x, y, z; } grid3;
+static int capturing;
+static grid3 g_, b_; static size_t lds_;
+void shim_capture(int on) { capturing = on; }
+int hipStreamIsCapturing(void* stream, int* status) { (void)stream; *status = capturing; return 0; }
+int __hipPushCallConfiguration(grid3 g, grid3 b, size_t lds, void* stream) { (void)stream; g_ = g; b_ = b; lds_ = lds; return 0; }
+int __hipPopCallConfiguration(grid3* g, grid3* b, size_t* lds, void** stream) { *g = g_; *b = b_; *lds = lds_; *stream = 0; return 0; }
+int hipLaunchKernel(const void* f, grid3 g, grid3 b, void** args, size_t lds, void* stream) {
+    (void)args; (void)stream;
+    printf("{\"launch\": %zu, \"grid\": %u, \"threads\": %u, \"lds\": %zu}\n", (size_t)f, g.x, b.x, lds); fflush(stdout);
+    return 0;
+}
+int hipGetLastError(void) { return 0; }
+int hipGetDevice(int* device) { *device = 0; return 0; }
+int hipDeviceGetAttribute(int* value, int attr, int device) { (void)attr; (void)device; *value = 256; return 0; }       /* CUs */
+int hipFuncSetAttribute(const void* f, int attr, int value) { (void)attr; (void)value; printf("{\"raise\": %zu}\n", (size_t)f); fflush(stdout); return 0; }
+"""
+CALLS = r"""
+import ctypes, json, sys
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+lib = ctypes.CDLL(sys.argv[2])
+one = ctypes.c_void_p(1 << 20)
+for fn, capture, m, n, k, variant, split, ws_bytes in json.loads(sys.argv[3]):
+    shim.shim_capture(capture)
+    print(json.dumps({"call": [fn, capture, m, n, k, variant, split]}), flush=True)
+    ws = (one, ctypes.c_size_t(ws_bytes)) if ws_bytes else (None, ctypes.c_size_t(0))
+    if fn == "gemm":
+        st = lib.fp8bs_gemm_ex(one, one, one, one, one, *ws, m, n, k, variant, split, None)
+    elif fn == "silu":
+        st = lib.fp8bs_gemm_silu_mul_ws(one, one, one, one, one, None, 0, m, n, k, variant, split, *ws, None)
+    else:
+        st = lib.fp8bs_gemm_grouped_ws(one, one, one, one, one, one, 4, m, n, k, variant, split, *ws, None)
+    assert st == 0, st
+"""
+FORM = lambda variant, form: variant | (form + 1) << 8           # FP8BS_VARIANT_FORM
+SUM = 1 << 30                                                    # FP8BS_SPLIT_SUM_IN_KERNEL
+MUCH = 256 << 20
+
+
+@pytest.fixture(scope="module")
+def run(pkg, tmp_path_factory):
+    """run(calls): for every call ("gemm" | "silu" | "grouped", capturing, m, n, k, variant, split, workspace bytes) in one fresh
+    process, the list of what it launched and the list of the kernels whose LDS limit it raised."""
+    d = tmp_path_factory.mktemp("shim")
+    (d / "shim.c").write_text(SHIM)
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", str(d / "shim.so"), str(d / "shim.c")], check=True)
+
+    def call(calls):
+        out = subprocess.run([sys.executable, "-c", CALLS, str(d / "shim.so"), pkg._lib.LIB_PATH, json.dumps(calls)],
+                             check=True, stdout=subprocess.PIPE, text=True, timeout=100).stdout
+        seen = []
+        for line in map(json.loads, out.splitlines()):
+            if "call" in line:
+                seen.append(([], []))
+            elif "launch" in line:
+                seen[-1][0].append(line)
+            else:
+                seen[-1][1].append(line["raise"])
+        assert len(seen) == len(calls)
+        return seen
+    return call
+
+
+@pytest.mark.parametrize("fn,variant,m,n,k,split", [("gemm", FORM(4, 1), 448, 924, 4480, 2), ("gemm", 12, 64, 18432, 7168, 3), ("gemm", FORM(12, 1), 1876, 571, 4608, 3),
+                                                    ("gemm", FORM(12, 1), 250, 4096, 7168, 4), ("silu", FORM(12, 1), 250, 4096, 7168, 2), ("grouped", FORM(4, 1), 96, 832, 1024, 2)])
+def test_a_captured_sum_has_a_kernel_without_the_shared_one(run, fn, variant, m, n, k, split):
+    """A captured launch cannot share out its sums.  Its kernel is the one that an eager call takes where there is nothing to
+    share (eight tiles and fewer), not one that carries both forms and is the slower for it."""
+    few = (fn, 0, 16, 66 if m % 4 or n % 8 else 64, k, variant, split | SUM, MUCH)              # (rows as whole or as odd: the same instantiation)
+    (eager, _), (captured, raised), (small, _) = run([(fn, capture, m, n, k, variant, split | SUM, MUCH) for capture in (0, 1)] + [few])
+    assert len(eager) == len(captured) == len(small) == 1
+    assert not raised                                                 # the eager call has readied the captured one's kernel
+    assert eager[0]["launch"] != captured[0]["launch"]
+    assert (eager[0]["grid"], eager[0]["threads"], eager[0]["lds"]) == (captured[0]["grid"], captured[0]["threads"], captured[0]["lds"])
+    assert captured[0]["launch"] == small[0]["launch"]
