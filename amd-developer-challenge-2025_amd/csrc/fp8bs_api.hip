@@ -169,7 +169,7 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
     // split, form) of 93 shapes - the 18 of the upstream benchmark, 60 log-uniform draws of M 1 .. 8192, N 512 .. 18432,
     // K 256 .. 7168, and 15 others.  Picking by the model costs 0.7 % against the measured best of each of the 93 shapes
     // in the geometric mean, worst 14 % (measured with the line at 80 K blocks, below, at 48).
-    struct Cand { int tile; int rmax; double t_alone, t_power, t_fixed, shared; int kb_min; double t_sum = 0; };
+    struct Cand { int tile; int rmax; double t_alone, t_power, t_fixed, shared; int kb_min; double t_sum = 0; int shares_from = 0; };
     // kb_min: the fewest K blocks a workgroup of a split keeps.  4; 8 with the 64x256 tile, whose short blocks leave a
     // workgroup's first copies and its partial plane as most of its time (1024 x 512 x 7168: split 8 20.9 us, split 4
     // 18.6); 2 with the small tiles, where the splits are what fills the chip (1 x 2048 x 2048: split 8 6.5 us, 4 6.9).
@@ -182,10 +182,10 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
         // few output tiles or few K blocks: the call is a chain of K blocks and barriers, so the tile with the shortest
         // block wins (512 x 2048 x 1024: 64x64 5.8 us, 64x128 6.3, 128x128 in eight waves 7.5, 64x256 7.7)
         {FP8BS_VARIANT_T64x128, 2, 0.398, 0.093, 4.76, 1.90, 2},
-        {FP8BS_VARIANT_T64x128 | FORM1, 2, 0.323, 0.108, 4.00, 1.76, 2, 2.17},
-        {FP8BS_VARIANT_T64x256S3, 1, 0.552, 0.540, 5.00, 1.0, 8, 3.20},
+        {FP8BS_VARIANT_T64x128 | FORM1, 2, 0.323, 0.108, 4.00, 1.76, 2, 2.17, 4},
+        {FP8BS_VARIANT_T64x256S3, 1, 0.552, 0.540, 5.00, 1.0, 8, 3.20, 2},
         // 128x128 in eight waves: see fp8bs_tile_64x256s3.hip (2048^3 12.6 us against 14.2 with 64x256, the best of the others)
-        {FP8BS_VARIANT_T64x256S3 | FORM1, 1, 0.467, 0.531, 4.57, 1.0, 4, 2.80},
+        {FP8BS_VARIANT_T64x256S3 | FORM1, 1, 0.467, 0.531, 4.57, 1.0, 4, 2.80, 2},
     };
     const int splits[6] = {1, 2, 3, 4, 6, 8};
     int best_tile = 0, best_split = 1; double best_cost = 0, best_gpu = 0; bool best_fused = false;
@@ -237,7 +237,7 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
             // there (1 x 512 x 7168 in eight 7.7 us, shared 8.7) and which the tests run at those sizes.
             // (Four and more partitions from 16 K blocks on: below, a caller who brings no more than workspace_bytes, and gets the
             // reduce launch, would lose more than the others gain.)
-            const bool share = c.t_sum > 0 && tiles > 8 && wgs <= per_round && wgs <= fp8bs::StreamK::MAX_GRID && (s <= 3 || kbt >= 16);
+            const bool share = c.t_sum > 0 && s >= c.shares_from && tiles > 8 && wgs <= per_round && wgs <= fp8bs::StreamK::MAX_GRID && (s <= 3 || kbt >= 16);
             const double rows = m < vi.bm ? m : vi.bm, cols = n < vi.bn ? n : vi.bn;
             const double shared_sum = c.t_sum * (1.0 + 0.027 * s) + 49.0 * (s - 1) / s * rows * cols * 4e-6 * (double)cdiv(wgs, num_cus);
             const double one = s > 1 ? cost + (share ? shared_sum : in_kernel) : cost, two = cost + planes;

@@ -234,6 +234,10 @@ constexpr int waves_per_simd() {
 // registers a wave, and the sums spill (128 x 7168 x 7168 in three 26.9 us against 24.9 with one workgroup summing); not
 // the tiles with more than eight accumulators a wave, which the planner splits in two or three only where the chip is full.
 template <int BM, int BN, int WM, int WN> constexpr bool shares_sum() { return (BM == 64 && BN == 64) || (WM == 32 && WN == 64); }
+// The fewest partitions it is shared out in.  64x64 has four accumulators a wave: in two parts nothing is gained, in three, of which
+// one is twice the others, 1.8 % lost over 210 shapes, 5.5 % where all rows start on 16 bytes (192 x 1280 x 3072: one workgroup summing
+// 8.8 us, shared 9.5).  The other tiles gain 2.4 % in three and up to 1 % in two (280 and 310 shapes).
+template <int BM, int BN> constexpr int shares_from() { return BM == 64 && BN == 64 ? 4 : 2; }
 
 // SHARED_SUM: the sum of a tile is shared out among its workgroups; without, the last of them does it.  An instantiation each, chosen
 // by the launcher: with both forms in one kernel the sum by one workgroup - all that a captured launch can have - was 2 to 5 % slower
@@ -1085,8 +1089,8 @@ void gemm_tr_kernel(const GemmArgs p) {
                 out_parts = (all ? mine : 0u) | taken;
             };
             switch (p.split_k) {
-                case 2: shared.template operator()<2>(); break;
-                case 3: shared.template operator()<3>(); break;
+                case 2: if constexpr (shares_from<BM, BN>() <= 2) shared.template operator()<2>(); break;
+                case 3: if constexpr (shares_from<BM, BN>() <= 3) shared.template operator()<3>(); break;
                 case 4: shared.template operator()<4>(); break;
                 case 6: shared.template operator()<6>(); break;
                 default: shared.template operator()<8>(); break;
@@ -1441,7 +1445,7 @@ static inline hipError_t launch_shape(const GemmArgs& a, int mode, hipStream_t s
     auto launch_summed = [&](auto mode_tag, auto epi_tag) {
         constexpr int M = decltype(mode_tag)::value, E = decltype(epi_tag)::value;
         if constexpr (shares_sum<BM, BN, WM, WN>())
-            if (can_share_sum(total, resident, a.split_k, stream)) {
+            if (a.split_k >= shares_from<BM, BN>() && can_share_sum(total, resident, a.split_k, stream)) {
                 void (*captured)(const GemmArgs);
                 hipError_t e = ready_tr<BM, BN, WM, WN, M, E, NSTAGE, false>(a, &captured);
                 if (e != hipSuccess) return e;

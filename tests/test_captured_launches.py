@@ -74,8 +74,8 @@ def run(pkg, tmp_path_factory):
     return call
 
 
-@pytest.mark.parametrize("fn,variant,m,n,k,split", [("gemm", FORM(4, 1), 448, 924, 4480, 2), ("gemm", 12, 64, 18432, 7168, 3), ("gemm", FORM(12, 1), 1876, 571, 4608, 3),
-                                                    ("gemm", FORM(12, 1), 250, 4096, 7168, 4), ("silu", FORM(12, 1), 250, 4096, 7168, 2), ("grouped", FORM(4, 1), 96, 832, 1024, 2)])
+@pytest.mark.parametrize("fn,variant,m,n,k,split", [("gemm", FORM(4, 1), 448, 924, 4480, 4), ("gemm", 12, 64, 18432, 7168, 3), ("gemm", FORM(12, 1), 1876, 571, 4608, 3),
+                                                    ("gemm", FORM(12, 1), 250, 4096, 7168, 4), ("silu", FORM(12, 1), 250, 4096, 7168, 2), ("grouped", FORM(4, 1), 96, 832, 1024, 4)])
 def test_a_captured_sum_has_a_kernel_without_the_shared_one(run, fn, variant, m, n, k, split):
     """A captured launch cannot share out its sums.  Its kernel is the one that an eager call takes where there is nothing to
     share (eight tiles and fewer), not one that carries both forms and is the slower for it."""
@@ -86,3 +86,11 @@ def test_a_captured_sum_has_a_kernel_without_the_shared_one(run, fn, variant, m,
     assert eager[0]["launch"] != captured[0]["launch"]
     assert (eager[0]["grid"], eager[0]["threads"], eager[0]["lds"]) == (captured[0]["grid"], captured[0]["threads"], captured[0]["lds"])
     assert captured[0]["launch"] == small[0]["launch"]
+
+
+@pytest.mark.parametrize("fn,m,n,k", [("gemm", 192, 1280, 3072), ("gemm", 448, 512, 3456), ("silu", 128, 1472, 2304), ("grouped", 96, 832, 1024)])
+def test_two_or_three_partitions_of_64x64_are_not_shared(run, fn, m, n, k):
+    """Four accumulators a wave in three parts: the shared sum is slower than the sum by one workgroup, which is what runs."""
+    calls = [(fn, capture, m, n, k, FORM(4, 1), split | SUM, MUCH) for split in (2, 3, 4) for capture in (0, 1)]
+    kernels = [launched[0]["launch"] for launched, _ in run(calls)]
+    assert kernels[0] == kernels[1] == kernels[2] == kernels[3] == kernels[5] != kernels[4]
