@@ -169,7 +169,7 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
     // split, form) of 93 shapes - the 18 of the upstream benchmark, 60 log-uniform draws of M 1 .. 8192, N 512 .. 18432,
     // K 256 .. 7168, and 15 others.  Picking by the model costs 0.7 % against the measured best of each of the 93 shapes
     // in the geometric mean, worst 14 % (measured with the line at 80 K blocks, below, at 48).
-    struct Cand { int tile; int rmax; double t_alone, t_power, t_fixed, shared; int kb_min; double t_sum = 0; int shares_from = 0; };
+    struct Cand { int tile; int rmax; double t_alone, t_power, t_fixed, shared; int kb_min; double t_sum = 0, t_part = 0; int shares_from = 0; };
     // kb_min: the fewest K blocks a workgroup of a split keeps.  4; 8 with the 64x256 tile, whose short blocks leave a
     // workgroup's first copies and its partial plane as most of its time (1024 x 512 x 7168: split 8 20.9 us, split 4
     // 18.6); 2 with the small tiles, where the splits are what fills the chip (1 x 2048 x 2048: split 8 6.5 us, 4 6.9).
@@ -182,10 +182,10 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
         // few output tiles or few K blocks: the call is a chain of K blocks and barriers, so the tile with the shortest
         // block wins (512 x 2048 x 1024: 64x64 5.8 us, 64x128 6.3, 128x128 in eight waves 7.5, 64x256 7.7)
         {FP8BS_VARIANT_T64x128, 2, 0.398, 0.093, 4.76, 1.90, 2},
-        {FP8BS_VARIANT_T64x128 | FORM1, 2, 0.323, 0.108, 4.00, 1.76, 2, 2.17, 4},
-        {FP8BS_VARIANT_T64x256S3, 1, 0.552, 0.540, 5.00, 1.0, 8, 3.20, 2},
+        {FP8BS_VARIANT_T64x128 | FORM1, 2, 0.323, 0.108, 4.00, 1.76, 2, 2.17, 20.0, 4},
+        {FP8BS_VARIANT_T64x256S3, 1, 0.552, 0.540, 5.00, 1.0, 8, 2.90, 9.0, 2},
         // 128x128 in eight waves: see fp8bs_tile_64x256s3.hip (2048^3 12.6 us against 14.2 with 64x256, the best of the others)
-        {FP8BS_VARIANT_T64x256S3 | FORM1, 1, 0.467, 0.531, 4.57, 1.0, 4, 2.80, 2},
+        {FP8BS_VARIANT_T64x256S3 | FORM1, 1, 0.467, 0.531, 4.57, 1.0, 4, 2.50, 9.0, 2},
     };
     const int splits[6] = {1, 2, 3, 4, 6, 8};
     int best_tile = 0, best_split = 1; double best_cost = 0, best_gpu = 0; bool best_fused = false;
@@ -229,17 +229,20 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
             // These are Python callers' launches; a captured graph or a C program, whose launches cost less, is given the same plan.
             auto issued = [](double gpu, double host) { return gpu > host ? gpu : host; };
             // Where every (tile, partition) has a workgroup of its own the sums can be shared out (see the kernel): a base that is
-            // the tile's plus the S - 1 of S parts of a tile that a workgroup stores and loads.  The constants are fits, with all
-            // others held, to every (tile, split, form) of 232 shapes (M 1 .. 2048, N 512 .. 8192, K 1024 .. 7168, operands from HBM
-            // and from the caches): with these splits in one launch the picks are 1.9 % behind the best of each shape, 4.1 %
-            // before; 250 x 4096 x 7168 in four 128x128 tiles' partitions 19.0 us (three, one workgroup summing: 20.9), 300 x 2112 x
-            // 7168 16.6 (19.0), 1 x 1230 x 4864 8.5 (10.8).  Eight tiles and fewer stay with the reduce launch, which is as fast
-            // there (1 x 512 x 7168 in eight 7.7 us, shared 8.7) and which the tests run at those sizes.
+            // the tile's, the S - 1 of S parts of a tile that a workgroup stores and loads, and, with S, ever smaller parts: pieces
+            // of lines of c, written from as many XCDs.  The constants are fits, with all others held, to every (tile, split, form) of 267
+            // shapes (M 1 .. 8000, N 190 .. 18100, K 1024 .. 7168, operands from HBM and from the caches), 200 of them with another plan than
+            // without shared sums: the picks are 2.7 and 3.9 % behind the best of each shape, 6.1 and 4.9 % without the last term,
+            // which priced eight partitions of full tiles like four (1024 x 512 x 7168 in eight of 128x128 20.4 us, 64x128 in four and a
+            // reduce launch 15.1; 619 x 768 x 6272 21.3 in eight, 15.9 in two of 64x64).  250 x 4096 x 7168 in four 128x128 tiles' partitions
+            // 19.0 us (three, one workgroup summing: 20.9), 300 x 2112 x 7168 16.6 (19.0), 1 x 1230 x 4864 8.5 (10.8).  Eight tiles and fewer stay
+            // with the reduce launch, which is as fast there (1 x 512 x 7168 in eight 7.7 us, shared 8.7) and which the tests run at
+            // those sizes.
             // (Four and more partitions from 16 K blocks on: below, a caller who brings no more than workspace_bytes, and gets the
             // reduce launch, would lose more than the others gain.)
             const bool share = c.t_sum > 0 && s >= c.shares_from && tiles > 8 && wgs <= per_round && wgs <= fp8bs::StreamK::MAX_GRID && (s <= 3 || kbt >= 16);
             const double rows = m < vi.bm ? m : vi.bm, cols = n < vi.bn ? n : vi.bn;
-            const double shared_sum = c.t_sum * (1.0 + 0.027 * s) + 49.0 * (s - 1) / s * rows * cols * 4e-6 * (double)cdiv(wgs, num_cus);
+            const double shared_sum = c.t_sum * (1.0 + 0.027 * s) + (20.0 * (s - 1) / s + c.t_part * s) * rows * cols * 4e-6 * (double)cdiv(wgs, num_cus);
             const double one = s > 1 ? cost + (share ? shared_sum : in_kernel) : cost, two = cost + planes;
             const bool fuse = (share || s == 2 || s == 3) && s > 1 && can_sum_in_kernel(m, n, c.tile, s) && issued(one, 5.3) < issued(two, 8.5);
             const double gpu = s == 1 || fuse ? one : two;

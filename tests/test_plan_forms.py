@@ -78,6 +78,16 @@ def test_small_products_take_one_launch_where_that_is_faster(pkg):
         assert p.split_k >= 4 and not p.sum_in_kernel, (m, n, k)
 
 
+@pytest.mark.parametrize("m,n,k,tile,split", [(1024, 512, 7168, (64, 128), 4), (86, 3392, 5632, (64, 128), 4), (107, 3520, 4736, (64, 64), 2), (384, 1728, 3840, (64, 64), 1),
+                                              (92, 3478, 4480, (64, 64), 2), (1115, 1088, 2944, (64, 128), 1), (619, 768, 6272, (64, 64), 2), (565, 640, 6656, (64, 128), 4),
+                                              (112, 3712, 6144, (64, 128), 4), (891, 768, 4864, (64, 128), 3), (250, 4096, 7168, (128, 128), 4), (1024, 1536, 7168, (128, 128), 2)])
+def test_many_partitions_of_full_tiles_are_not_planned_for_a_shared_sum(pkg, m, n, k, tile, split):
+    """Six and eight partitions of full 128x128 tiles, three of few K blocks: 4 to 40 % slower, operands from HBM and from the caches, than
+    the plans here; and two sizes where sharing the sum pays."""
+    p = pkg.plan(m, n, k)
+    assert ((p.tile_m, p.tile_n), p.split_k) == (tile, split)
+
+
 def test_an_incomplete_binding_is_named(pkg, monkeypatch):
     """A CPython binding built before a function was added to it gives way to ctypes with a warning that says so."""
     lib_mod, whole = pkg._lib, pkg._lib.pycall()
