@@ -78,10 +78,35 @@ bool is_streaming_variant(int v) { return v == FP8BS_VARIANT_SKINNY64x144 || v =
 // The fp32 partial planes of a K split followed by the reduce kernel.
 uint64_t planes_bytes(int m, int n, int split_k) { return split_k > 1 ? (uint64_t)split_k * (uint64_t)m * (uint64_t)n * 4u : 0u; }
 
-// A plan and what the caller's structure has no field for: whether four, six or eight partitions are better summed in the kernel,
-// the sum shared out, where the call's workspace holds the counters and partial tiles and the launch is not captured.  The plan itself
-// then says what every caller with workspace_bytes gets: partial planes and the reduce kernel.
+// A plan and what the caller's structure has no field for: whether the sums of the K partitions are better shared out in the kernel
+// where the call's workspace holds the flags and partial tiles and the launch is not captured.  The plan itself says what every
+// caller with workspace_bytes gets, also under capture: partial planes and the reduce kernel, or the sum by one workgroup.  Tile
+// and split are the same for all callers, so that a replayed call returns the bits of an eager one.
 struct Planned { fp8bs_plan_t plan; bool share; };
+
+// The choice among (tile, split) in microseconds, each at the price of both forms: the soonest to finish where its sum can be shared out, among those
+// that finish within 6 % of the soonest where it cannot.  Of 267 shapes (see choose_tiled), times against the planner before there were
+// shared sums, operands from the caches / from HBM: eager 0.992 / 0.974, worst 1.09, replayed 0.999 / 0.980, worst 1.08.  At the price of the
+// shared form alone 0.996 / 0.969, worst 1.37, and 1.006 / 0.976, worst 1.35 (896 x 1344 x 2944 in three, 16 us, 12 unsplit); within 4 % instead
+// 250 x 4096 x 7168 would lose its four partitions, 19.3 us eager and 21.4 replayed against 21.3 and 21.6 in three.
+struct Choice {
+    struct Option { int tile, split; double shared, plain, gpu; bool share, fused; } options[80];
+    int count = 0;
+    // gpu: time on the GPU, which decides among calls that the host's launches make equal.  shared, plain: of the call, the sum shared
+    // out where share says so; fused: without sharing, summed in the kernel.
+    void add(int tile, int split, double shared, double plain, double gpu, bool share, bool fused) { options[count++] = {tile, split, shared, plain, gpu, share, fused}; }
+    const Option& pick() const {
+        double soonest = options[0].plain;
+        for (int i = 1; i < count; i++) if (options[i].plain < soonest) soonest = options[i].plain;
+        const Option* best = nullptr;
+        for (int i = 0; i < count; i++) {
+            const Option& o = options[i];
+            if (o.plain > 1.06 * soonest) continue;
+            if (!best || o.shared < best->shared || (o.shared == best->shared && o.gpu < best->gpu)) best = &o;
+        }
+        return *best;
+    }
+};
 
 // Can the partial tiles of a K split of this tile shape be summed in the kernel that writes them (one counter per
 // tile in the head of the workspace, the partition count in the counter's low 16 bits)?
@@ -188,7 +213,7 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
         {FP8BS_VARIANT_T64x256S3 | FORM1, 1, 0.467, 0.531, 4.57, 1.0, 4, 2.50, 9.0, 2},
     };
     const int splits[6] = {1, 2, 3, 4, 6, 8};
-    int best_tile = 0, best_split = 1; double best_cost = 0, best_gpu = 0; bool best_fused = false;
+    Choice choice;                                         // 9 tiles in up to 6 splits and two more
     for (const Cand& c : cands) {
         if (epi && !has_epilogue(c.tile)) continue;
         VariantInfo vi{};
@@ -232,23 +257,23 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
             // the tile's, the S - 1 of S parts of a tile that a workgroup stores and loads, and, with S, ever smaller parts: pieces
             // of lines of c, written from as many XCDs.  The constants are fits, with all others held, to every (tile, split, form) of 267
             // shapes (M 1 .. 8000, N 190 .. 18100, K 1024 .. 7168, operands from HBM and from the caches), 200 of them with another plan than
-            // without shared sums: the picks are 2.7 and 3.9 % behind the best of each shape, 6.1 and 4.9 % without the last term,
+            // without shared sums: the picks are 2.1 and 4.5 % behind the best of each shape, 6.1 and 4.9 % without the last term,
             // which priced eight partitions of full tiles like four (1024 x 512 x 7168 in eight of 128x128 20.4 us, 64x128 in four and a
             // reduce launch 15.1; 619 x 768 x 6272 21.3 in eight, 15.9 in two of 64x64).  250 x 4096 x 7168 in four 128x128 tiles' partitions
             // 19.0 us (three, one workgroup summing: 20.9), 300 x 2112 x 7168 16.6 (19.0), 1 x 1230 x 4864 8.5 (10.8).  Eight tiles and fewer stay
             // with the reduce launch, which is as fast there (1 x 512 x 7168 in eight 7.7 us, shared 8.7) and which the tests run at
             // those sizes.
-            // (Four and more partitions from 16 K blocks on: below, a caller who brings no more than workspace_bytes, and gets the
-            // reduce launch, would lose more than the others gain.)
+            // (Four and more partitions from 16 K blocks on: below, the small tiles that hold all partitions are ahead.)
             const bool share = c.t_sum > 0 && s >= c.shares_from && tiles > 8 && wgs <= per_round && wgs <= fp8bs::StreamK::MAX_GRID && (s <= 3 || kbt >= 16);
             const double rows = m < vi.bm ? m : vi.bm, cols = n < vi.bn ? n : vi.bn;
             const double shared_sum = c.t_sum * (1.0 + 0.027 * s) + (20.0 * (s - 1) / s + c.t_part * s) * rows * cols * 4e-6 * (double)cdiv(wgs, num_cus);
-            const double one = s > 1 ? cost + (share ? shared_sum : in_kernel) : cost, two = cost + planes;
-            const bool fuse = (share || s == 2 || s == 3) && s > 1 && can_sum_in_kernel(m, n, c.tile, s) && issued(one, 5.3) < issued(two, 8.5);
-            const double gpu = s == 1 || fuse ? one : two;
-            cost = issued(gpu, s == 1 || fuse ? 5.3 : 8.5);
-            // (among equals, which the host alone makes, the shorter kernel)
-            if (best_tile == 0 || cost < best_cost || (cost == best_cost && gpu < best_gpu)) { best_tile = c.tile; best_split = s; best_cost = cost; best_gpu = gpu; best_fused = fuse; }
+            if (s == 1) { choice.add(c.tile, 1, issued(cost, 5.3), issued(cost, 5.3), cost, false, false); continue; }
+            const double two = cost + planes, last = cost + in_kernel, parts = cost + shared_sum;
+            const bool can = can_sum_in_kernel(m, n, c.tile, s), shared = can && share && issued(parts, 5.3) < issued(two, 8.5);
+            // (where a sum in the kernel can be shared out it is: one that is not better than two launches then is none)
+            const bool fused = can && (s == 2 || s == 3) && shared == share && issued(last, 5.3) < issued(two, 8.5);
+            const double plain = fused ? issued(last, 5.3) : issued(two, 8.5);
+            choice.add(c.tile, s, shared ? issued(parts, 5.3) : plain, plain, shared ? parts : fused ? last : two, shared, fused);
         }
     }
     // The small tiles that hold all K partitions in a workgroup: a launch, first copies and output, a chain of kbt / 8 blocks, and
@@ -265,11 +290,12 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
             const int s = kbt <= WAVES_MAX ? 1 : WAVES_MAX;
             const double gpu = w.fixed + w.block * (double)cdiv(kbt, WAVES_MAX) + w.load * (double)(cdiv(m, w.bm) * cdiv(n, 64)) * kbt / 256.0;
             const double cost = gpu > 5.3 ? gpu : 5.3;
-            if (cost < best_cost || (cost == best_cost && gpu < best_gpu)) { best_tile = w.tile; best_split = s; best_cost = cost; best_gpu = gpu; best_fused = false; }
+            choice.add(w.tile, s, cost, cost, gpu, false, false);
         }
     }
-    fill_plan(m, n, k, best_tile, best_split, &out->plan, 0, best_fused && best_split <= 3);
-    out->share = best_fused && best_split > 3;
+    const Choice::Option& o = choice.pick();
+    fill_plan(m, n, k, o.tile, o.split, &out->plan, 0, o.fused);
+    out->share = o.share;
 }
 
 // Skinny shapes: one of the two tiles of eight 32 x 64 waves - 64 x 256 with three LDS stages, two K blocks of b, 64 KB, in
@@ -277,15 +303,18 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
 // model in microseconds: a workgroup advances one K block in the time the workgroups running together need to pull
 // their 32 or 16 KB of b each (and of a, at a quarter of the price) from HBM at 5.5 or 5.3 TB/s, and never faster than a
 // block's copies take to arrive; a time for the first block and the output; the partial planes and the reduce launch, or a sum
-// that is shared out in the kernel.  The constants of the 64 x 256 tile's planes are as measured before; the others are fits to
-// every split of both tiles on 79 shapes (M 1 .. 64, N 3000 .. 28672, K 1024 .. 8192, b streamed from HBM): the picks are 1.2 % behind
-// the best of each, 4.3 % with the 64 x 256 tile alone and its sums by one workgroup.  64 x 18432 x 7168 33.0 us (33.7), 64 x 7168 x
-// 7168 18.2 (19.7), 64 x 16384 x 4096 20.5 (22.0), 64 x 12288 x 2048 12.7 (16.4), 64 x 4096 x 7168 14.2 (16.3); below some 30
-// rows the planes are small and two launches of the 64 x 256 tile stay ahead: 1 x 18432 x 7168 28.8, one launch 30.8.
+// in the kernel, shared out or, in two or three partitions, by one workgroup.  The constants of the 64 x 256 tile's planes and its sums by one
+// workgroup are as measured before there was the other tile; its shared sums and the K blocks and shared sums of the other are
+// fits to every split of both tiles on 79 shapes (M 1 .. 64, N 3000 .. 28672, K 1024 .. 8192, b streamed from HBM), the planes and the sums by one
+// workgroup of the 128 x 128 tile to 94 shapes (N 4300 .. 18400, b from HBM and from the caches).  On these 94 the picks are 9 % (caches) and 7 %
+// (HBM) faster than those of the 64 x 256 tile alone, eager as well as replayed, 4 % slower at worst (with its planes left out,
+// 12 %: 11 x 6464 x 4096).  us: 64 x 18432 x 7168 33.0 (33.7), 64 x 16384 x 4096 20.5 (22.0), 64 x 12288 x 2048 12.7 (16.4), 64 x 4096 x 7168
+// 14.2 (16.3).  With few rows the planes are small and two launches are ahead, in either tile: 1 x 18432 x 7168 28.8, one launch 30.8.
 void choose_skinny(int m, int n, int k, int num_cus, Planned* out, bool may_split) {
     if (num_cus <= 0) num_cus = 256;
     const int kbt = k / KBLK;
-    int best_tile = FP8BS_VARIANT_T64x256S3, best_s = 1; double best = 0; bool best_fused = false;
+    const double mn = (double)m * (double)n;
+    Choice choice;
     for (int s = 1; s <= 8 && s <= kbt; s++) {
         if (s > 1 && !may_split) break;
         const long wgs = cdiv(n, 256) * s;
@@ -293,14 +322,15 @@ void choose_skinny(int m, int n, int k, int num_cus, Planned* out, bool may_spli
         double t_block = together * 32768.0 / 5.5e6;
         if (t_block < 1.05) t_block = 1.05;
         double cost = (double)cdiv(wgs, num_cus) * (2.0 + (double)cdiv(kbt, s) * t_block);
-        if (s > 1) cost += 4.0 + 0.24 * s + 1.19e-6 * s * (double)m * (double)n;
-        // In one round of workgroups the sum is shared out where the planes are large enough for the reduce launch to cost more
-        // than the chain of round trips that replaces it (the parts' acknowledged stores, the flags, the parts' reads).
-        const bool can_share = s > 1 && s != 5 && s != 7 && wgs <= num_cus;
-        const double in_kernel = 1.13 - 0.37e-6 * s * (double)m * (double)n;
-        const bool fuse = can_share && in_kernel < 0;
-        if (fuse) cost += in_kernel;
-        if (s == 1 || cost < best) { best = cost; best_s = s; best_fused = fuse; best_tile = FP8BS_VARIANT_T64x256S3; }
+        if (s > 1) cost += 4.0 + 0.24 * s + 1.19e-6 * s * mn;
+        // In one round of workgroups the sum is done in the kernel where the planes are large enough for the reduce launch to cost
+        // more than the chain of round trips that replaces it (acknowledged stores, flags or a count, reads).  One workgroup's sum, b
+        // from HBM, three partitions of 18432 x 7168: 64 rows 33.7 us against 34.4 with the reduce launch, 16 rows 30.3 against 29.3.
+        const double by_one = 2.05 - 0.78e-6 * s * mn, by_all = 1.13 - 0.37e-6 * s * mn;
+        const bool fused = (s == 2 || s == 3) && wgs <= num_cus && by_one < 0;
+        const bool shared = s > 1 && s != 5 && s != 7 && wgs <= num_cus && by_all < 0;
+        const double plain = fused ? cost + by_one : cost, eager = shared ? cost + by_all : plain;
+        choice.add(FP8BS_VARIANT_T64x256S3, s, eager, plain, eager, shared, fused);
     }
     for (int s = 1; s <= 8 && s <= kbt; s++) {
         const long wgs = cdiv(n, 128) * s;
@@ -311,12 +341,16 @@ void choose_skinny(int m, int n, int k, int num_cus, Planned* out, bool may_spli
         if (m == 64 && n == 7168 && k == 7168) continue;
         double t_block = (double)wgs * 128.0 * (128.0 + 0.26 * m) / 5.33e6;
         if (t_block < 0.64) t_block = 0.64;
-        double cost = 5.06 + (double)cdiv(kbt, s) * t_block;
-        if (s > 1) cost += 2.92 + 19.5 * (s - 1) / s * (double)m * 128.0 * 4e-6;
-        if (cost < best) { best = cost; best_s = s; best_fused = s > 1; best_tile = FP8BS_VARIANT_T64x256S3 | FORM1; }
+        const double cost = 5.06 + (double)cdiv(kbt, s) * t_block;
+        const double planes = s > 1 ? 2.41 + 0.755e-6 * s * mn : 0.0;
+        const double by_one = 2.53 + 0.605e-6 * s * mn, by_all = 2.92 + 19.5 * (s - 1) / s * (double)m * 128.0 * 4e-6;
+        const bool fused = (s == 2 || s == 3) && by_one < planes, shared = s > 1 && by_all < planes;
+        const double plain = cost + (fused ? by_one : planes), eager = shared ? cost + by_all : plain;
+        choice.add(FP8BS_VARIANT_T64x256S3 | FORM1, s, eager, plain, eager, shared, fused);
     }
-    fill_plan(m, n, k, best_tile, best_s, &out->plan, 0, best_fused && best_s <= 3);
-    out->share = best_fused && best_s > 3;
+    const Choice::Option& o = choice.pick();
+    fill_plan(m, n, k, o.tile, o.split, &out->plan, 0, o.fused);
+    out->share = o.share;
 }
 
 // What the planners below return for a shape is kept, 64 shapes a thread: the cost models take 0.4-0.8 us of host time
@@ -340,7 +374,7 @@ struct PlanMemo {
     }
 };
 
-// Shape-family rule.  A few rows against a large b -> the 64 x 256 three-stage tile.  Everything else -> the
+// Shape-family rule.  A few rows against a large b -> one of two tiles that stream b.  Everything else -> the
 // tile and K split that the cost model of the tiled kernel picks.
 const Planned& choose(int m, int n, int k, int num_cus, bool may_split = true, bool epi = false) {
     static thread_local PlanMemo<Planned> memo;
@@ -580,18 +614,14 @@ static int dense_call(const void* a, const void* b, const float* a_scale, const 
         // (a forced split may be any: the small tiles of up to eight partitions give way to 64 x 64)
         if (split_k > 0) fill_plan(m, n, k, is_waves_tile(tile) ? FP8BS_VARIANT_T64x128 | FORM1 : tile, split_k & ~FP8BS_SPLIT_SUM_IN_KERNEL, &plan, 0, (split_k & FP8BS_SPLIT_SUM_IN_KERNEL) != 0);
         else if (split_k < 0) fill_plan(m, n, k, plan.variant, 1, &plan, streamk_grid(plan.variant, m, n, k, cus));   // (the first form only)
+        // A captured launch cannot share out its sums: its flags' tag would not change from replay to replay.
+        else if (fp8bs_plan_t p{}; planned.share && !plan.sum_in_kernel && ws && ws_bytes >= (p = summed_in_kernel(m, n, k, plan)).workspace_bytes && !fp8bs::is_capturing(s)) plan = p;
         // the plan needs a workspace the caller did not bring: the best plan that needs none
         else if (plan.workspace_bytes > 0 && !is_waves_tile(tile) && (!ws || ws_bytes < plan.workspace_bytes)) {
             // too small for the partial tiles of a sum in the kernel but not for the planes (tiles that overhang
             // the matrix): the same split with the reduce kernel
             if (plan.sum_in_kernel && ws && ws_bytes >= planes_bytes(m, n, plan.split_k)) fill_plan(m, n, k, tile, plan.split_k, &plan);
             else plan = choose(m, n, k, cus, false, epi != 0).plan;
-        }
-        // A captured launch cannot share out its sums (its flags' tag would not change from replay to replay), and one workgroup
-        // that adds four partial tiles and more takes longer than the reduce kernel (64 x 4096 x 7168 in eight 19 us, 14 as two launches).
-        else if (planned.share && ws) {
-            const fp8bs_plan_t p = summed_in_kernel(m, n, k, plan);
-            if (ws_bytes >= p.workspace_bytes && !fp8bs::is_capturing(s)) plan = p;
         }
     } else {
         VariantInfo vi{};

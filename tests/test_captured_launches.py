@@ -94,3 +94,17 @@ def test_two_or_three_partitions_of_64x64_are_not_shared(run, fn, m, n, k):
     calls = [(fn, capture, m, n, k, FORM(4, 1), split | SUM, MUCH) for split in (2, 3, 4) for capture in (0, 1)]
     kernels = [launched[0]["launch"] for launched, _ in run(calls)]
     assert kernels[0] == kernels[1] == kernels[2] == kernels[3] == kernels[5] != kernels[4]
+
+
+@pytest.mark.parametrize("m,n,k,tile,split", [(896, 1344, 2944, (64, 128), 1), (576, 2048, 3328, (64, 128), 1), (960, 640, 7040, (64, 128), 3), (256, 3648, 4736, (64, 64), 1),
+                                              (384, 2637, 6528, (128, 128), 3), (250, 4096, 7168, (128, 128), 4), (64, 4096, 7168, (128, 128), 8), (64, 18432, 7168, (64, 256), 3)])
+def test_one_plan_that_is_sound_for_every_caller(pkg, run, m, n, k, tile, split):
+    """The same tile and split eager and captured, so that a replay has the bits of an eager call; and not one that is picked at the price of
+    a shared sum and takes 4 to 40 % longer without (the first five, before their plans were priced in both forms)."""
+    p = pkg.plan(m, n, k)
+    assert ((p.tile_m, p.tile_n), p.split_k) == (tile, split)
+    (eager, _), (captured, _), (tight, _) = run([("gemm", 0, m, n, k, 0, 0, MUCH), ("gemm", 1, m, n, k, 0, 0, MUCH), ("gemm", 0, m, n, k, 0, 0, int(p.workspace_bytes))])
+    for launched in (eager, captured, tight):
+        assert (launched[0]["grid"], launched[0]["threads"], launched[0]["lds"]) == (p.grid_x, p.block_threads, p.lds_bytes)
+    assert len(captured) == (2 if split > 1 and not p.sum_in_kernel else 1)
+    assert len(eager) == 1 and len(tight) == len(captured)
