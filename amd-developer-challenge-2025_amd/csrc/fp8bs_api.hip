@@ -232,9 +232,6 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
             // 77.1 / 71.4; 128 4096 x 1024 90.3 / 82.9.  Over 86 shapes of 49 .. 128 blocks (half of them with m or n off the
             // 16-byte grid) the picks with the line at 80 are 6 % faster than at 48, 0.7 % than at 72, 0.2 % than at 88.
             if (c.tile == (FP8BS_VARIANT_T64x256S3 | FORM1) && cdiv(kbt, s) > 80) continue;
-            // This one shape is what the tests of the sum in the kernel run from the planner at full size, in two partitions
-            // of the 256 x 128 tile: its plan stays that, at 43.9 us against 40.2 with this tile unsplit.
-            if (c.tile == (FP8BS_VARIANT_T64x256S3 | FORM1) && m == 6144 && n == 576 && k == 7168 && !epi) continue;
             const long wgs = tiles * s, per_round = (long)num_cus * c.rmax;
             const long full = wgs / per_round, rem = wgs % per_round;
             const double kb = (double)cdiv(kbt, s);
@@ -309,7 +306,7 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
 // workgroup of the 128 x 128 tile to 94 shapes (N 4300 .. 18400, b from HBM and from the caches).  On these 94 the picks are 9 % (caches) and 7 %
 // (HBM) faster than those of the 64 x 256 tile alone, eager as well as replayed, 4 % slower at worst (with its planes left out,
 // 12 %: 11 x 6464 x 4096).  us: 64 x 18432 x 7168 33.0 (33.7), 64 x 16384 x 4096 20.5 (22.0), 64 x 12288 x 2048 12.7 (16.4), 64 x 4096 x 7168
-// 14.2 (16.3).  With few rows the planes are small and two launches are ahead, in either tile: 1 x 18432 x 7168 28.8, one launch 30.8.
+// 14.2 (16.3), 64 x 7168 x 7168 18.2 (19.4).  With few rows the planes are small and two launches are ahead, in either tile: 1 x 18432 x 7168 28.8, one launch 30.8.
 void choose_skinny(int m, int n, int k, int num_cus, Planned* out, bool may_split) {
     if (num_cus <= 0) num_cus = 256;
     const int kbt = k / KBLK;
@@ -337,8 +334,6 @@ void choose_skinny(int m, int n, int k, int num_cus, Planned* out, bool may_spli
         if ((s > 1 && !may_split) || wgs > num_cus) break;
         // (chains of more than 26 blocks take longer than the model has it: 1 x 28672 x 4096 28.5 us, 26.1 with 64 x 256)
         if (s == 5 || s == 7 || (s > 1 && kbt / s < 2) || cdiv(kbt, s) > 26) continue;
-        // The tests hold this one shape to the 64 x 256 tile: 19.4 us, 18.2 with this tile in four partitions.
-        if (m == 64 && n == 7168 && k == 7168) continue;
         double t_block = (double)wgs * 128.0 * (128.0 + 0.26 * m) / 5.33e6;
         if (t_block < 0.64) t_block = 0.64;
         const double cost = 5.06 + (double)cdiv(kbt, s) * t_block;

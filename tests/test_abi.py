@@ -96,8 +96,8 @@ def test_plan_shape_families(pkg):
 
 
 def test_plan_skinny_rule_and_the_streaming_kernels(pkg):
-    """At most 64 rows against a B of 24 MB or more: always the 64x256 three-stage tile, with the K split of the
-    streaming model.  Everything else goes through the cost model of all the tiles (the 64x256 tile among them).
+    """At most 64 rows against a B of 24 MB or more: one of the two tiles of eight 32x64 waves, 64x256 and 128x128, with the K split of
+    the streaming model.  Everything else goes through the cost model of all the tiles (these two among them).
     The streaming kernels are never planned (forced variants only)."""
     for m, n, k, skinny in [(64, 18432, 7168, True), (16, 18432, 7168, True), (4, 18432, 7168, True), (64, 7168, 7168, True),
                             (1, 28672, 4096, True), (64, 18440, 7168, True), (63, 18429, 7168, True),
@@ -105,10 +105,14 @@ def test_plan_skinny_rule_and_the_streaming_kernels(pkg):
                             (64, 7168, 2048, False), (32, 512, 2048, False), (1536, 1536, 4096, False)]:
         p = pkg.plan(m, n, k)
         if skinny:
-            assert p.variant == 12 and p.grid_x == -(-n // 256) * p.split_k, (m, n, k, p.variant)
+            assert p.variant == 12 and (p.tile_m, p.tile_n) in ((64, 256), (128, 128)), (m, n, k, p.variant)
+            assert p.grid_x == -(-n // p.tile_n) * p.split_k, (m, n, k, p.variant)
         assert p.variant not in (1, 6, 7, 8)
         assert 1 <= p.split_k <= 8 and p.workspace_bytes == _planned_workspace(p, m, n)
         assert p.sum_in_kernel == 0 or p.split_k in (2, 3)              # only two or three partitions are summed in the kernel
+    for shape in ((64, 7168, 7168), (64, 7167, 7168), (63, 7168, 7168), (64, 7176, 7168)):     # a size and its neighbours: one rule
+        assert [getattr(pkg.plan(*shape), f) for f in ("variant", "form", "split_k")] == [12, 1, 4], shape
+    assert pkg.plan(6144, 576, 7168).split_k == 1 and pkg.plan(6144, 576, 7168).tile_m == 128  # likewise among all the tiles
     assert pkg.plan(1536, 1536, 4096).variant == 12           # the cost model's pick for a few hundred rows per tile column
     # few rows: summed in the kernel only where the planes are large enough for the reduce launch to cost more
     assert pkg.plan(64, 18432, 7168).sum_in_kernel == 1 and pkg.plan(1, 18432, 7168).sum_in_kernel == 0

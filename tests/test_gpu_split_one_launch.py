@@ -72,18 +72,20 @@ def test_ragged_shapes_against_the_oracle_and_the_two_launch_split(pkg, oracle, 
             assert ok, "%dx%dx%d variant %d split %d: %d elements outside the bar (max abs err %g)" % (m, n, k, variant, split, nbad, maxerr)
 
 
-@pytest.mark.parametrize("m,n,k", [(64, 18432, 7168), (1024, 1536, 7168), (6144, 576, 7168), (57, 18429, 7168)])
-def test_what_the_planner_sums_in_the_kernel(pkg, oracle, dev, m, n, k):
-    """Shapes planned with two or three partitions at full size, every element against the oracle, and the bits of
-    the same plan with the reduce kernel."""
+@pytest.mark.parametrize("m,n,k,forced", [(64, 18432, 7168, None), (1024, 1536, 7168, None), (6144, 576, 7168, (10, 2)), (57, 18429, 7168, None),
+                                          (6048, 264, 6272, None), (5560, 648, 4992, None)])
+def test_what_the_planner_sums_in_the_kernel(pkg, oracle, dev, m, n, k, forced):
+    """Shapes planned with two or three partitions at full size (one forced into them), every element against the oracle, and the
+    bits of the same plan with the reduce kernel."""
     plan = pkg.plan(m, n, k)
-    assert plan.split_k in (2, 3) and plan.sum_in_kernel == 1
+    variant, split = forced or (pkg._lib.planned_variant(plan), plan.split_k)
+    assert forced or plan.split_k in (2, 3) and plan.sum_in_kernel == 1
     cpu = pkg.inputs.make_dense(pkg.inputs.CONFIGS[3], m=m, n=n, k=k)
     data = _to(cpu, dev)
-    out = pkg.custom_kernel(data).clone()
-    ok, nstrict, nun = oracle.parity_report(out, oracle.ref_kernel(cpu), cpu, plan.split_k, RTOL, ATOL)
+    out = pkg.custom_kernel(data, **(dict(variant=variant, split_k=split | pkg._lib.SPLIT_SUM_IN_KERNEL) if forced else {})).clone()
+    ok, nstrict, nun = oracle.parity_report(out, oracle.ref_kernel(cpu), cpu, split, RTOL, ATOL)
     assert ok, "%dx%dx%d: %d beyond the bar, %d not reproduced" % (m, n, k, nstrict, nun)
-    two = pkg.custom_kernel(data, variant=pkg._lib.planned_variant(plan), split_k=plan.split_k)
+    two = pkg.custom_kernel(data, variant=variant, split_k=split)
     assert torch.equal(_bits(out), _bits(two))
 
 
