@@ -602,6 +602,7 @@ static int dense_call(const void* a, const void* b, const float* a_scale, const 
     }
     const bool simple = aligned && vector_shape(n);      // streaming kernels possible
     const int cus = fp8bs::device_cus();
+    bool ready_planes = false;
     if (variant == FP8BS_VARIANT_AUTO) {
         const Planned planned = choose(m, n, k, cus, true, epi != 0);
         plan = planned.plan;
@@ -610,7 +611,10 @@ static int dense_call(const void* a, const void* b, const float* a_scale, const 
         if (split_k > 0) fill_plan(m, n, k, is_waves_tile(tile) ? FP8BS_VARIANT_T64x128 | FORM1 : tile, split_k & ~FP8BS_SPLIT_SUM_IN_KERNEL, &plan, 0, (split_k & FP8BS_SPLIT_SUM_IN_KERNEL) != 0);
         else if (split_k < 0) fill_plan(m, n, k, plan.variant, 1, &plan, streamk_grid(plan.variant, m, n, k, cus));   // (the first form only)
         // A captured launch cannot share out its sums: its flags' tag would not change from replay to replay.
-        else if (fp8bs_plan_t p{}; planned.share && !plan.sum_in_kernel && ws && ws_bytes >= (p = summed_in_kernel(m, n, k, plan)).workspace_bytes && !fp8bs::is_capturing(s)) plan = p;
+        else if (fp8bs_plan_t p{}; planned.share && !plan.sum_in_kernel && ws && ws_bytes >= (p = summed_in_kernel(m, n, k, plan)).workspace_bytes && !fp8bs::is_capturing(s)) {
+            plan = p;
+            ready_planes = true;                 // a capture of this call takes the two launches
+        }
         // the plan needs a workspace the caller did not bring: the best plan that needs none
         else if (plan.workspace_bytes > 0 && !is_waves_tile(tile) && (!ws || ws_bytes < plan.workspace_bytes)) {
             // too small for the partial tiles of a sum in the kernel but not for the planes (tiles that overhang
@@ -648,6 +652,11 @@ static int dense_call(const void* a, const void* b, const float* a_scale, const 
     g.band_h = 4;
     g.num_experts = 0;
     g.epi = epi;
+    if (ready_planes) {
+        g.ready_only = 1;
+        if (fp8bs::launch_gemm(plan.variant | plan.form * FORM1, 1, g, s) != hipSuccess) return FP8BS_ERR_LAUNCH;
+        g.ready_only = 0;
+    }
     int mode = plan.split_k > 1 && !waves ? 1 : 0;
     if (plan.sum_in_kernel && plan.split_k > 1 && !waves) {
         mode = 4;

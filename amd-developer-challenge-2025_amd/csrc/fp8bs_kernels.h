@@ -29,6 +29,7 @@ struct GemmArgs {
     // 8-byte flag per workgroup) and one fp32 partial tile per workgroup, see StreamK below
     unsigned long long sk_nonce;   // value a flag takes when its workgroup's partial tile is complete: differs from call to call
     int sk_grid;            // workgroups of such a call: at most the places on the chip and the number of (tile, K block) pairs
+    int ready_only;         // host: the launcher raises the LDS limit of the kernel that these arguments take and launches nothing
     int sk_spin;            // polls of a flag before the wait gives up (< 0: give up at once - tests of the error path); with a shared-out sum: before a part is left to another workgroup
 };
 

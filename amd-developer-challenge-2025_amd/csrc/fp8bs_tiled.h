@@ -1408,7 +1408,7 @@ static inline hipError_t launch_tr(const GemmArgs& a, dim3 grid, hipStream_t str
     using C = TileCfg<BM, BN, WM, WN, MODE, NSTAGE>;
     void (*kern)(const GemmArgs);
     hipError_t e = ready_tr<BM, BN, WM, WN, MODE, EPI, NSTAGE, SHARED_SUM>(a, &kern);
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess || a.ready_only) return e;
     GemmArgs args = a;
     args.c_whole_lines = ((size_t)(EPI == 1 ? a.n / 2 : a.n) * 2u) % 128u == 0 && ((uintptr_t)a.c & 127) == 0;
     hipLaunchKernelGGL(kern, grid, dim3(C::NTHREADS), C::LDS_BYTES, stream, args);

@@ -108,3 +108,12 @@ def test_one_plan_that_is_sound_for_every_caller(pkg, run, m, n, k, tile, split)
         assert (launched[0]["grid"], launched[0]["threads"], launched[0]["lds"]) == (p.grid_x, p.block_threads, p.lds_bytes)
     assert len(captured) == (2 if split > 1 and not p.sum_in_kernel else 1)
     assert len(eager) == 1 and len(tight) == len(captured)
+
+
+@pytest.mark.parametrize("fn,m,n,k", [("gemm", 250, 4096, 7168), ("silu", 250, 4096, 7168), ("gemm", 64, 4096, 7168), ("gemm", 448, 1537, 5120), ("gemm", 1024, 1536, 7168),
+                                      ("gemm", 256, 512, 1024), ("gemm", 64, 512, 7168), ("grouped", 96, 832, 7168)])
+def test_one_eager_call_readies_a_capture(run, fn, m, n, k):
+    """In a process that has launched nothing else: whatever kernel a captured call of the shape takes, an eager call with the same
+    arguments has raised its LDS limit, which is no thing to be done under capture."""
+    (eager, _), (captured, raised) = run([(fn, capture, m, n, k, 0, 0, MUCH) for capture in (0, 1)])
+    assert eager and captured and not raised

@@ -80,3 +80,23 @@ def test_captured_calls_and_the_epilogue(pkg, m, n, k, split):
     g = want.float()
     ref = torch.nn.functional.silu(g[:, 0::2]) * g[:, 1::2]
     assert bool(((h.float() - ref).abs() <= 1e-3 + 2 * 2e-2 * ref.abs()).all())
+
+
+def test_capture_after_one_eager_call_in_a_fresh_process():
+    """Four partitions, shared out when eager and in two launches when captured, by a process that has launched nothing else."""
+    code = """import importlib, sys, torch
+sys.path.insert(0, %r)
+pkg = importlib.import_module('amd-developer-challenge-2025_amd')
+a, b, sa, sb, c = (t.to('cuda:0') for t in pkg.inputs.make_dense(pkg.inputs.CONFIGS[2], m=250, n=4096, k=7168))
+want = pkg.custom_kernel((a, b, sa, sb, torch.empty_like(c))).clone()
+graph = torch.cuda.CUDAGraph()
+with torch.cuda.graph(graph):
+    pkg.custom_kernel((a, b, sa, sb, c))
+for _ in range(3):
+    c.fill_(3.0)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(c.view(torch.int16), want.view(torch.int16))
+print('all equal')""" % ROOT
+    res = subprocess.run([sys.executable, "-c", code], stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True, timeout=110)
+    assert res.returncode == 0 and "all equal" in res.stdout, res.stdout[-500:] + res.stderr[-2000:]
