@@ -277,7 +277,9 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
     // the requests that all workgroups make of the L2 (in units of K blocks per CU).  Fits to 264 shapes (M 1 .. 1024, N 512 ..
     // 12288, K 384 .. 4096, operands from HBM and from the caches): where they are taken for any of these shapes, the calls take 0.81 of
     // the time of the other tiles in the geometric mean, within 1.6 % of the best; at most 1.19 of it where the two are
-    // modelled level.  Not beyond 24 K blocks, where the others' splits over workgroups are ahead.  Up to eight blocks the sum is the
+    // modelled level.  Only where all workgroups are on the chip at once - one or two fit a CU -, the model has no second round: of 34
+    // shapes with more, M 17 .. 4203, N 126 .. 18300, all but one were slower than with the other tiles, 14 % in the geometric mean, 36 at
+    // worst (320 x 1664 x 384 5.2 us, 64 x 64 3.9); of 90 with fewer, outside the fitted sizes too, none (0.74).  Not beyond 24 K blocks, where the others' splits over workgroups are ahead.  Up to eight blocks the sum is the
     // unsplit one; beyond, eight partitions: the plan reports them like any K split's, sum_in_kernel says one launch up to 15
     // K blocks and, as for the other tiles' four partitions and more, leaves it open beyond.  No workspace is used.
     if (kbt >= 2 && (kbt <= WAVES_MAX || (may_split && kbt <= 24))) {
@@ -285,6 +287,7 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
         const Waves waves[2] = {{FP8BS_VARIANT_T64x256S3 | 2 * FORM1, 16, 2.12, 1.223, 0.312}, {FP8BS_VARIANT_T64x256S3 | 3 * FORM1, 32, 2.31, 1.485, 0.385}};
         for (const Waves& w : waves) {
             const int s = kbt <= WAVES_MAX ? 1 : WAVES_MAX;
+            if (cdiv(m, w.bm) * cdiv(n, 64) > (long)num_cus * (163840 / fp8bs::waves_lds_bytes(w.bm))) continue;
             const double gpu = w.fixed + w.block * (double)cdiv(kbt, WAVES_MAX) + w.load * (double)(cdiv(m, w.bm) * cdiv(n, 64)) * kbt / 256.0;
             const double cost = gpu > 5.3 ? gpu : 5.3;
             choice.add(w.tile, s, cost, cost, gpu, false, false);

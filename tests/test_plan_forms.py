@@ -78,6 +78,17 @@ def test_small_products_take_one_launch_where_that_is_faster(pkg):
         assert p.split_k >= 4 and not p.sum_in_kernel, (m, n, k)
 
 
+def test_waves_tiles_in_one_round_only(pkg):
+    """The tiles that hold all K partitions are planned where all their workgroups are on the chip at once (256 of 32x64, 512 of 16x64):
+    sizes measured 4 to 36 % slower in two rounds, and sizes at the edge that are faster."""
+    for m, n, k in [(320, 1664, 384), (612, 896, 256), (64, 8448, 256), (20, 17920, 896), (2130, 242, 256), (4203, 126, 256), (28, 17878, 384), (867, 637, 256)]:
+        p = pkg.plan(m, n, k)
+        assert not (p.variant == 12 and p.form >= 2), (m, n, k)
+    for m, n, k in [(8000, 64, 256), (256, 512, 1024), (18, 13764, 896), (41, 8128, 256)]:
+        p = pkg.plan(m, n, k)
+        assert p.variant == 12 and p.form >= 2 and p.grid_x <= 163840 // p.lds_bytes * 256, (m, n, k)
+
+
 @pytest.mark.parametrize("m,n,k,tile,split", [(1024, 512, 7168, (64, 128), 4), (86, 3392, 5632, (64, 128), 4), (107, 3520, 4736, (64, 64), 2), (384, 1728, 3840, (64, 64), 1),
                                               (92, 3478, 4480, (64, 64), 2), (1115, 1088, 2944, (64, 128), 1), (619, 768, 6272, (64, 64), 2), (565, 640, 6656, (64, 128), 4),
                                               (112, 3712, 6144, (64, 128), 4), (891, 768, 4864, (64, 128), 3), (250, 4096, 7168, (128, 128), 4), (1024, 1536, 7168, (128, 128), 2)])
