@@ -140,7 +140,7 @@ void fill_plan(int m, int n, int k, int tile, int split_k, fp8bs_plan_t* out, in
     if (stream_k > 0) split_k = 1;
     if (split_k < 1) split_k = 1;
     if (split_k > kbt) split_k = kbt > 0 ? kbt : 1;
-    if (is_waves_tile(tile)) in_kernel = in_kernel || split_k <= 3 || kbt < 16;       // (see choose_tiled)
+    const bool waves = is_waves_tile(tile);                                          // (all partitions in a workgroup: one launch, no workspace)
     out->variant = variant_of(tile);
     out->form = form_of(tile);
     out->tile_m = vi.bm;
@@ -149,13 +149,14 @@ void fill_plan(int m, int n, int k, int tile, int split_k, fp8bs_plan_t* out, in
     out->block_threads = vi.threads;
     out->lds_bytes = fp8bs::variant_lds_bytes(tile);
     out->stream_k = stream_k > 0 ? stream_k : 0;
-    out->sum_in_kernel = in_kernel && stream_k <= 0 && can_sum_in_kernel(m, n, tile, split_k) ? 1 : 0;
+    out->sum_in_kernel = waves ? split_k > 1 : in_kernel && stream_k <= 0 && can_sum_in_kernel(m, n, tile, split_k) ? 1 : 0;
     if (tile == FP8BS_VARIANT_GENERIC) {
         out->grid_x = (int)cdiv(n, 16); out->grid_y = (int)cdiv(m, 16); out->grid_z = 1;
     } else {
-        out->grid_x = stream_k > 0 ? stream_k : (int)(cdiv(m, vi.bm) * cdiv(n, vi.bn) * (is_waves_tile(tile) ? 1 : split_k)); out->grid_y = 1; out->grid_z = 1;
+        out->grid_x = stream_k > 0 ? stream_k : (int)(cdiv(m, vi.bm) * cdiv(n, vi.bn) * (waves ? 1 : split_k)); out->grid_y = 1; out->grid_z = 1;
     }
-    if (stream_k > 0) out->workspace_bytes = (uint64_t)fp8bs::StreamK::bytes(stream_k, vi.bm, vi.bn);
+    if (waves) out->workspace_bytes = 0;
+    else if (stream_k > 0) out->workspace_bytes = (uint64_t)fp8bs::StreamK::bytes(stream_k, vi.bm, vi.bn);
     else if (out->sum_in_kernel)   // the counters, then one fp32 tile per (tile, K partition)
         out->workspace_bytes = (uint64_t)fp8bs::StreamK::SLOTS_OFF + (uint64_t)(cdiv(m, vi.bm) * cdiv(n, vi.bn)) * (uint64_t)split_k * (uint64_t)vi.bm * (uint64_t)vi.bn * 4u;
     else out->workspace_bytes = planes_bytes(m, n, split_k);
@@ -280,8 +281,7 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
     // modelled level.  Only where all workgroups are on the chip at once - one or two fit a CU -, the model has no second round: of 34
     // shapes with more, M 17 .. 4203, N 126 .. 18300, all but one were slower than with the other tiles, 14 % in the geometric mean, 36 at
     // worst (320 x 1664 x 384 5.2 us, 64 x 64 3.9); of 90 with fewer, outside the fitted sizes too, none (0.74).  Not beyond 24 K blocks, where the others' splits over workgroups are ahead.  Up to eight blocks the sum is the
-    // unsplit one; beyond, eight partitions: the plan reports them like any K split's, sum_in_kernel says one launch up to 15
-    // K blocks and, as for the other tiles' four partitions and more, leaves it open beyond.  No workspace is used.
+    // unsplit one; beyond, eight partitions, summed in the kernel without a workspace.
     if (kbt >= 2 && (kbt <= WAVES_MAX || (may_split && kbt <= 24))) {
         struct Waves { int tile, bm; double fixed, block, load; };
         const Waves waves[2] = {{FP8BS_VARIANT_T64x256S3 | 2 * FORM1, 16, 2.12, 1.223, 0.312}, {FP8BS_VARIANT_T64x256S3 | 3 * FORM1, 32, 2.31, 1.485, 0.385}};
@@ -619,7 +619,7 @@ static int dense_call(const void* a, const void* b, const float* a_scale, const 
             ready_planes = true;                 // a capture of this call takes the two launches
         }
         // the plan needs a workspace the caller did not bring: the best plan that needs none
-        else if (plan.workspace_bytes > 0 && !is_waves_tile(tile) && (!ws || ws_bytes < plan.workspace_bytes)) {
+        else if (plan.workspace_bytes > 0 && (!ws || ws_bytes < plan.workspace_bytes)) {
             // too small for the partial tiles of a sum in the kernel but not for the planes (tiles that overhang
             // the matrix): the same split with the reduce kernel
             if (plan.sum_in_kernel && ws && ws_bytes >= planes_bytes(m, n, plan.split_k)) fill_plan(m, n, k, tile, plan.split_k, &plan);
@@ -643,7 +643,7 @@ static int dense_call(const void* a, const void* b, const float* a_scale, const 
         }
     }
     const bool waves = is_waves_tile(plan.variant | plan.form * FORM1);
-    if (plan.workspace_bytes > 0 && !waves && (!ws || ws_bytes < plan.workspace_bytes)) return FP8BS_ERR_WORKSPACE;
+    if (plan.workspace_bytes > 0 && (!ws || ws_bytes < plan.workspace_bytes)) return FP8BS_ERR_WORKSPACE;
     if (epi && plan.variant != FP8BS_VARIANT_GENERIC && (!has_epilogue(plan.variant | plan.form * FORM1) || plan.stream_k > 0)) return FP8BS_ERR_BAD_VARIANT;
 
     fp8bs::GemmArgs g{};
@@ -700,7 +700,7 @@ int fp8bs_gemm_noalloc(const void* a, const void* b, const float* a_scale, const
         plan = choose(m, n, k, fp8bs::device_cus()).plan;
         uint64_t need = plan.workspace_bytes;
         if (plan.sum_in_kernel && planes_bytes(m, n, plan.split_k) < need) need = planes_bytes(m, n, plan.split_k);   // fp8bs_gemm_ex falls back to the planes
-        if (need > (uint64_t)FP8BS_NOALLOC_SCRATCH_BYTES && !is_waves_tile(plan.variant | plan.form * FORM1)) return FP8BS_ERR_SCRATCH_LIMIT;
+        if (need > (uint64_t)FP8BS_NOALLOC_SCRATCH_BYTES) return FP8BS_ERR_SCRATCH_LIMIT;
     }
     void* ws = nullptr;
     st = scratch_address(&ws, (hipStream_t)stream);
@@ -764,7 +764,6 @@ size_t fp8bs_grouped_workspace_bytes(int num_experts, int total_rows, int n, int
 size_t fp8bs_silu_mul_workspace_bytes(int rows, int n, int k) {
     if (rows <= 0 || n <= 0 || k <= 0 || (k % KBLK) != 0) return 0;
     const Planned& p = choose(rows, n, k, fp8bs::device_cus(), true, true);
-    if (is_waves_tile(p.plan.variant | p.plan.form * FORM1)) return 0;
     return (size_t)(p.share ? summed_in_kernel(rows, n, k, p.plan) : p.plan).workspace_bytes;
 }
 

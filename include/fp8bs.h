@@ -67,7 +67,7 @@ enum {
                                      b; form 1: 128 x 128 tile, four stages: mid-size, one tile per CU;
                                      forms 2 and 3: 16 x 64 and 32 x 64 tiles whose eight waves each multiply the whole
                                      tile over a K partition of their own: small products, dense calls, split_k
-                                     up to 8, no workspace whatever the plan's workspace_bytes      */
+                                     up to 8, always one launch and no workspace                   */
     FP8BS_VARIANT_COUNT = 13
 };
 
@@ -79,7 +79,7 @@ enum {
 typedef struct fp8bs_plan_t {
     int32_t variant;        /* FP8BS_VARIANT_*                                   */
     int32_t tile_m, tile_n; /* workgroup tile                                    */
-    int32_t split_k;        /* number of K partitions (1 = no workspace needed)  */
+    int32_t split_k;        /* number of K partitions (1 = none)                 */
     int32_t grid_x, grid_y, grid_z;
     int32_t block_threads;
     int32_t lds_bytes;
@@ -87,7 +87,8 @@ typedef struct fp8bs_plan_t {
                                partial tiles meet in the workspace); split_k is 1 then           */
     int32_t sum_in_kernel;  /* 1 (with split_k > 1): one launch - the workgroups of a tile's K partitions leave fp32
                                partial tiles in the workspace and the sum, in ascending K, is shared out among them or
-                               done by the last one to finish; 0: partial planes and a reduce kernel (two launches; a
+                               done by the last one to finish (in forms 2 and 3 of FP8BS_VARIANT_T64x256S3 they are
+                               waves of one workgroup, and there is no workspace); 0: partial planes and a reduce kernel (two launches; a
                                call with 4, 6 or 8 partitions whose workspace also holds 16384 + tiles * split_k *
                                tile_m * tile_n * 4 bytes may still take one launch, with the same bits)      */
     int32_t form;           /* form of the variant (0 unless the variant has several); a plan is run again by forcing

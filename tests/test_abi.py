@@ -52,8 +52,8 @@ def test_plan_with_the_devices_cu_count(pkg):
 
 def _planned_workspace(p, m, n):
     """What a plan's K split needs: counters and one fp32 tile per (tile, partition) when the partitions are summed in
-    the kernel, whole fp32 planes when a reduce kernel follows."""
-    if p.split_k == 1:
+    the kernel, whole fp32 planes when a reduce kernel follows; nothing where a workgroup's waves hold the partitions."""
+    if p.split_k == 1 or (p.variant == 12 and p.form >= 2):
         return 0
     if p.sum_in_kernel:
         return 16384 + -(-m // p.tile_m) * -(-n // p.tile_n) * p.split_k * p.tile_m * p.tile_n * 4
@@ -109,7 +109,8 @@ def test_plan_skinny_rule_and_the_streaming_kernels(pkg):
             assert p.grid_x == -(-n // p.tile_n) * p.split_k, (m, n, k, p.variant)
         assert p.variant not in (1, 6, 7, 8)
         assert 1 <= p.split_k <= 8 and p.workspace_bytes == _planned_workspace(p, m, n)
-        assert p.sum_in_kernel == 0 or p.split_k in (2, 3)              # only two or three partitions are summed in the kernel
+        # only two or three partitions are summed in the kernel, or those of one workgroup's waves
+        assert p.sum_in_kernel == (p.split_k > 1) if p.variant == 12 and p.form >= 2 else p.sum_in_kernel == 0 or p.split_k in (2, 3)
     for shape in ((64, 7168, 7168), (64, 7167, 7168), (63, 7168, 7168), (64, 7176, 7168)):     # a size and its neighbours: one rule
         assert [getattr(pkg.plan(*shape), f) for f in ("variant", "form", "split_k")] == [12, 1, 4], shape
     assert pkg.plan(6144, 576, 7168).split_k == 1 and pkg.plan(6144, 576, 7168).tile_m == 128  # likewise among all the tiles

@@ -78,6 +78,15 @@ def test_small_products_take_one_launch_where_that_is_faster(pkg):
         assert p.split_k >= 4 and not p.sum_in_kernel, (m, n, k)
 
 
+@pytest.mark.parametrize("m,n,k", [(64, 512, 1536), (64, 512, 2048), (1, 1088, 1664), (32, 512, 2048), (64, 2304, 2048), (256, 512, 1024)])
+def test_a_plan_of_the_waves_tiles_says_what_runs(pkg, m, n, k):
+    """One launch and no workspace at every number of K blocks: nothing for a caller to allocate, and nothing that is refused without."""
+    p = pkg.plan(m, n, k)
+    assert p.variant == 12 and p.form >= 2
+    assert (p.sum_in_kernel, p.workspace_bytes, pkg.workspace_bytes(m, n, k)) == (int(p.split_k > 1), 0, 0)
+    assert p.split_k == (8 if k > 1024 else 1)
+
+
 def test_waves_tiles_in_one_round_only(pkg):
     """The tiles that hold all K partitions are planned where all their workgroups are on the chip at once (256 of 32x64, 512 of 16x64):
     sizes measured 4 to 36 % slower in two rounds, and sizes at the edge that are faster."""
