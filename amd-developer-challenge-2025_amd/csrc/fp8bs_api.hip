@@ -391,6 +391,9 @@ fp8bs_plan_t summed_in_kernel(int m, int n, int k, const fp8bs_plan_t& plan) {
     return p;
 }
 
+// The workspace that every form of a planned call finds room in: the flags and partial tiles of a sum shared out are no less than planes.
+uint64_t useful_bytes(int m, int n, int k, const Planned& p) { return (p.share ? summed_in_kernel(m, n, k, p.plan) : p.plan).workspace_bytes; }
+
 // Order of the tiles of a grouped call (the row counts themselves are on the device).  With a tile or more of
 // rows per expert on average the tiles go expert by expert: the tile that holds an expert's last rows then runs
 // beside the full tiles that read the same weights (32 experts of 1040 rows x 4096 x 7168: 956 us against 1014;
@@ -580,9 +583,8 @@ int fp8bs_plan(int m, int n, int k, int num_cus, fp8bs_plan_t* out) {
 }
 
 size_t fp8bs_workspace_bytes(int m, int n, int k) {
-    fp8bs_plan_t p{};
-    if (fp8bs_plan(m, n, k, fp8bs::device_cus(), &p) != FP8BS_OK) return 0;
-    return (size_t)p.workspace_bytes;
+    if (m <= 0 || n <= 0 || k <= 0 || (k % KBLK) != 0) return 0;
+    return (size_t)useful_bytes(m, n, k, choose(m, n, k, fp8bs::device_cus()));
 }
 
 // A dense call, plain or with the silu-mul epilogue (epi 1: c has n/2 columns).
@@ -763,8 +765,7 @@ size_t fp8bs_grouped_workspace_bytes(int num_experts, int total_rows, int n, int
 
 size_t fp8bs_silu_mul_workspace_bytes(int rows, int n, int k) {
     if (rows <= 0 || n <= 0 || k <= 0 || (k % KBLK) != 0) return 0;
-    const Planned& p = choose(rows, n, k, fp8bs::device_cus(), true, true);
-    return (size_t)(p.share ? summed_in_kernel(rows, n, k, p.plan) : p.plan).workspace_bytes;
+    return (size_t)useful_bytes(rows, n, k, choose(rows, n, k, fp8bs::device_cus(), true, true));
 }
 
 int fp8bs_gemm_grouped_ex(const void* a, const void* b, const float* a_scale, const float* b_scale,

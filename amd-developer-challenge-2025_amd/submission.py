@@ -181,16 +181,8 @@ def plan(m: int, n: int, k: int) -> _lib.Plan:
     return p
 
 
-def _wanted_bytes(p) -> int:
-    """What a plan's call makes use of: its workspace_bytes, and room for the counters and partial tiles with which four and
-    more partitions are summed in the kernel where the library finds that faster than planes and a reduce kernel."""
-    if p.variant == 12 and p.form >= 2:                # all partitions in a workgroup: none
-        return 0
-    tiles = p.grid_x // p.split_k
-    return max(int(p.workspace_bytes), 16384 + tiles * p.split_k * p.tile_m * p.tile_n * 4 if p.split_k > 3 and tiles * p.split_k <= 512 else 0)
-
-
 def workspace_bytes(m: int, n: int, k: int) -> int:
+    """Bytes of workspace that a dense call of a shape can make use of (no GPU needed)."""
     return int(_lib.load().fp8bs_workspace_bytes(m, n, k))
 
 
@@ -226,7 +218,7 @@ def custom_kernel(data, variant: int = 0, split_k: int = 0):
     if variant == 0 and split_k == 0:
         need = _plan_cache.get((m, n, k))
         if need is None:
-            need = _wanted_bytes(plan(m, n, k)) if (m > 0 and n > 0 and k > 0) else 0
+            need = workspace_bytes(m, n, k) if (m > 0 and n > 0 and k > 0) else 0
             if len(_plan_cache) >= _PLANS_MAX:
                 _plan_cache.clear()
             _plan_cache[(m, n, k)] = need

@@ -89,8 +89,8 @@ typedef struct fp8bs_plan_t {
                                partial tiles in the workspace and the sum, in ascending K, is shared out among them or
                                done by the last one to finish (in forms 2 and 3 of FP8BS_VARIANT_T64x256S3 they are
                                waves of one workgroup, and there is no workspace); 0: partial planes and a reduce kernel (two launches; a
-                               call with 4, 6 or 8 partitions whose workspace also holds 16384 + tiles * split_k *
-                               tile_m * tile_n * 4 bytes may still take one launch, with the same bits)      */
+                               call that is not captured and whose workspace has fp8bs_workspace_bytes may still take
+                               one launch, with the same bits)                                       */
     int32_t form;           /* form of the variant (0 unless the variant has several); a plan is run again by forcing
                                FP8BS_VARIANT_FORM(variant, form), the variant alone names its first form, another
                                tile with another workspace need where form is 1                    */
@@ -113,8 +113,9 @@ const char* fp8bs_strerror(int status);
  * fp8bs_gemm runs the best plan that needs none (slower, same result up to the summation order). */
 int fp8bs_plan(int m, int n, int k, int num_cus, fp8bs_plan_t* out);
 
-/* Bytes of device workspace fp8bs_gemm needs for this shape (0 when split_k == 1; the partial planes, or the
- * counters and partial tiles of a split summed in the kernel). Replaces the
+/* Bytes of device workspace fp8bs_gemm makes use of for this shape: the plan's workspace_bytes (0 when split_k == 1; the partial planes, or
+ * the counters and partial tiles of a split summed in the kernel), or more where a call that is not captured is faster with the sum
+ * of its partitions shared out in the kernel, 16384 + tiles * split_k * tile_m * tile_n * 4. Replaces the
  * per-call `torch.empty(m*n*4)` of 1-amd-fp8-mm/amd-fp8-mm-submission.py:600: the caller owns and
  * reuses the workspace. */
 size_t fp8bs_workspace_bytes(int m, int n, int k);

@@ -117,3 +117,13 @@ def test_one_eager_call_readies_a_capture(run, fn, m, n, k):
     arguments has raised its LDS limit, which is no thing to be done under capture."""
     (eager, _), (captured, raised) = run([(fn, capture, m, n, k, 0, 0, MUCH) for capture in (0, 1)])
     assert eager and captured and not raised
+
+
+@pytest.mark.parametrize("fn,m,n,k", [("gemm", 250, 4096, 7168), ("gemm", 64, 4096, 7168), ("gemm", 64, 7168, 7168), ("gemm", 448, 1537, 5120), ("silu", 250, 4096, 7168)])
+def test_a_workspace_of_the_reported_size_lets_a_sum_be_shared(pkg, run, fn, m, n, k):
+    """What fp8bs_workspace_bytes and fp8bs_silu_mul_workspace_bytes say is room for the fastest form, one launch, and for a capture's
+    two; a byte less is not, and takes the same split in two."""
+    nbytes = pkg._lib.load().fp8bs_silu_mul_workspace_bytes(m, n, k) if fn == "silu" else pkg.workspace_bytes(m, n, k)
+    assert nbytes >= pkg.plan(m, n, k).workspace_bytes
+    counts = [len(launched) for launched, _ in run([(fn, 0, m, n, k, 0, 0, nbytes), (fn, 1, m, n, k, 0, 0, nbytes), (fn, 0, m, n, k, 0, 0, nbytes - 1)])]
+    assert counts == [1, 2, 2]
