@@ -86,8 +86,9 @@ struct Planned { fp8bs_plan_t plan; bool share; };
 
 // The choice among (tile, split) in microseconds, each at the price of both forms: the soonest to finish where its sum can be shared out, among those
 // that finish within 6 % of the soonest where it cannot.  Of 267 shapes (see choose_tiled), times against the planner before there were
-// shared sums, operands from the caches / from HBM: eager 0.992 / 0.974, worst 1.09, replayed 0.999 / 0.980, worst 1.08.  At the price of the
-// shared form alone 0.996 / 0.969, worst 1.37, and 1.006 / 0.976, worst 1.35 (896 x 1344 x 2944 in three, 16 us, 12 unsplit); within 4 % instead
+// shared sums, operands from the caches / from HBM: eager 0.987 / 0.972, worst 1.09, replayed 0.996 / 0.978, worst 1.08 (of 270 others, 0.965 /
+// 0.970 and 0.997 / 0.997, 1.10 and 1.07).  At the price of the shared form alone 0.996 / 0.969, worst 1.37, and 1.006 / 0.976, worst 1.35
+// (896 x 1344 x 2944 in three, 16 us, 12 unsplit); within 4 % instead
 // 250 x 4096 x 7168 would lose its four partitions, 19.3 us eager and 21.4 replayed against 21.3 and 21.6 in three.
 struct Choice {
     struct Option { int tile, split; double shared, plain, gpu; bool share, fused; } options[80];
@@ -242,7 +243,9 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
             // launch and no pass over whole planes, but the last workgroup of a tile reads s - 1 partial tiles alone
             // (measured on the same 38 shapes: two partitions 1-50 us faster than with the reduce launch, median 4.7;
             // three: median 2.3 faster; four and more: the serial sums cost more than the launch)
-            const double planes = 2.66 + 1.656e-6 * s * (double)m * (double)n;
+            // (Few rows, and n off the 8-column grid: the planes take 0.2 us each more than the constants have, 14 x 3373 x 6144 in eight of
+            // 64x64 14.1 us, the sum shared out 11.2.  The picks for 150 shapes of up to 80 rows are 2 and 3 % behind the best, 4 and 4 without.)
+            const double planes = 2.66 + 1.656e-6 * s * (double)m * (double)n + ((n & 7) != 0 && m <= 64 ? 0.2 * s : 0.0);
             const double in_kernel = 2.34 + 0.891e-6 * s * (double)m * (double)n
                                      + 13.2 * (s - 1) * (vi.bm * vi.bn * 4e-6) * (double)cdiv(wgs, num_cus);
             // calls issued one after another are never faster than the host launches them: 5.2 to 6.2 us, or 7.7 to 10.2 with the
@@ -255,7 +258,7 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
             // the tile's, the S - 1 of S parts of a tile that a workgroup stores and loads, and, with S, ever smaller parts: pieces
             // of lines of c, written from as many XCDs.  The constants are fits, with all others held, to every (tile, split, form) of 267
             // shapes (M 1 .. 8000, N 190 .. 18100, K 1024 .. 7168, operands from HBM and from the caches), 200 of them with another plan than
-            // without shared sums: the picks are 2.1 and 4.5 % behind the best of each shape, 6.1 and 4.9 % without the last term,
+            // without shared sums: the picks are 1.7 and 4.2 % behind the best of each shape, 6.1 and 4.9 % without the last term,
             // which priced eight partitions of full tiles like four (1024 x 512 x 7168 in eight of 128x128 20.4 us, 64x128 in four and a
             // reduce launch 15.1; 619 x 768 x 6272 21.3 in eight, 15.9 in two of 64x64).  250 x 4096 x 7168 in four 128x128 tiles' partitions
             // 19.0 us (three, one workgroup summing: 20.9), 300 x 2112 x 7168 16.6 (19.0), 1 x 1230 x 4864 8.5 (10.8).  Eight tiles and fewer stay
