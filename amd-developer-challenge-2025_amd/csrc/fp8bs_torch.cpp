@@ -1,9 +1,9 @@
 // custom_kernel on torch tensors, for callers that issue many small products from Python: its checks and its call in one native
 // function.  In Python they were some forty attribute reads and comparisons; here they are read from the tensors themselves, at
 // every call.  Calls issued one after another: 256 x 512 x 1024 5.2 us before, 4.1 now (the kernel takes 3.8), 3 x 2092 x 384 5.2
-// and 3.6; with tensors that were not seen before 24 and 16, waiting for each.
-// Whatever is not the usual case (another layout, type or device, a dimension of few elements, a tensor subclass, a size that has
-// not been planned yet) is handed back: the Python path takes it, or says what is wrong with it.
+// and 3.6, 1 x 3968 x 384 5.3 and 3.9; with tensors that were not seen before 24 and 16, waiting for each.
+// Whatever is not the usual case (another layout, type or device, an empty product, a tensor subclass, a size that has not been
+// planned yet) is handed back: the Python path takes it, or says what is wrong with it.
 // Built by build.py with the host compiler against torch's headers; without this module the Python path takes every call.
 #define PY_SSIZE_T_CLEAN
 #include <torch/csrc/autograd/python_variable.h>
@@ -19,7 +19,8 @@ namespace {
 
 constexpr long NOT_HERE = -1;
 
-bool kmajor(const at::Tensor& t) { return t.stride(0) == 1 && t.stride(1) == t.size(0); }
+// (the stride of a dimension of one element is immaterial)
+bool kmajor(const at::Tensor& t) { return (t.size(0) == 1 || t.stride(0) == 1) && (t.size(1) == 1 || t.stride(1) == t.size(0)); }
 
 // The call's status code, NOT_HERE, or -(bytes) where a larger workspace is wanted than the one given.
 // Throws what torch throws.
@@ -29,10 +30,9 @@ long dense_call(const at::Tensor* const* t, PyObject* planned, void* ws, size_t 
     for (int i = 0; i < 5; i++)
         if (t[i]->scalar_type() != types[i] || !t[i]->is_cuda() || t[i]->layout() != at::kStrided || t[i]->dim() != 2 || t[i]->device() != a.device()) return NOT_HERE;
     const int64_t m = a.size(0), k = a.size(1), n = b.size(0), nb = (n + 127) / 128, kb = k / 128;
-    // no dimension of one element, the scales' included: its stride would be immaterial, which the Python path knows about
-    if (m < 2 || n <= 128 || k < 256 || k % 128 != 0 || m > INT32_MAX || n > INT32_MAX || k > INT32_MAX) return NOT_HERE;
+    if (m < 1 || n < 1 || k < 128 || k % 128 != 0 || m > INT32_MAX || n > INT32_MAX || k > INT32_MAX) return NOT_HERE;
     if (b.size(1) != k || as.size(0) != m || as.size(1) != kb || bs.size(0) != nb || bs.size(1) != kb || c.size(0) != m || c.size(1) != n) return NOT_HERE;
-    if (!kmajor(a) || !kmajor(b) || !kmajor(as) || !kmajor(bs) || c.stride(0) != n || c.stride(1) != 1) return NOT_HERE;
+    if (!kmajor(a) || !kmajor(b) || !kmajor(as) || !kmajor(bs) || !c.is_contiguous()) return NOT_HERE;
     int device = -1;
     if (hipGetDevice(&device) != hipSuccess || device != a.get_device()) return NOT_HERE;
     PyObject* const key = Py_BuildValue("(LLL)", (long long)m, (long long)n, (long long)k);
@@ -52,10 +52,10 @@ PyObject* dense(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (PyErr_Occurred()) return nullptr;
     const size_t ws_bytes = PyLong_AsSize_t(args[3]);
     if (PyErr_Occurred()) return nullptr;
-    if (!PyTuple_CheckExact(args[0]) || PyTuple_GET_SIZE(args[0]) != 5) return PyLong_FromLong(NOT_HERE);
+    if (!(PyTuple_CheckExact(args[0]) || PyList_CheckExact(args[0])) || PySequence_Fast_GET_SIZE(args[0]) != 5) return PyLong_FromLong(NOT_HERE);
     const at::Tensor* t[5];
     for (int i = 0; i < 5; i++) {
-        PyObject* const o = PyTuple_GET_ITEM(args[0], i);
+        PyObject* const o = PySequence_Fast_GET_ITEM(args[0], i);
         if (!THPVariable_CheckExact(o)) return PyLong_FromLong(NOT_HERE);      // a subclass has rules of its own
         t[i] = &THPVariable_Unpack(o);
     }

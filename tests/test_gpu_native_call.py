@@ -49,7 +49,7 @@ FORMS = {
 }
 
 
-# (96 x 384 x 512: no workspace.  64 x 1536 x 7168: one.  The rest: dimensions of one element, and of one block)
+# (96 x 384 x 512: no workspace.  64 x 1536 x 7168: one.  The rest: dimensions of one element, and of one block, whose strides may be any)
 @pytest.mark.parametrize("m,n,k", [(96, 384, 512), (64, 1536, 7168), (1, 384, 512), (96, 128, 512), (96, 1, 512), (96, 384, 128), (2, 129, 256)])
 def test_forms(pkg, dev, m, n, k, monkeypatch):
     lib = importlib.import_module("amd-developer-challenge-2025_amd._lib")
@@ -78,8 +78,8 @@ def test_forms(pkg, dev, m, n, k, monkeypatch):
         got, same = outcome(form, counted)
         assert got is want, (name, got, want)
         assert want is not None or torch.equal(bits, same), name
-        if name in ("tuple", "a offset by a byte"):
-            assert (taken[-1] == 0) == (m > 1 and n > 128 and k > 128), (name, taken)      # who took it
+        if name in ("tuple", "list", "parameter", "a offset by a byte"):
+            assert taken[-1] == 0, (name, taken)                                           # who took it
 
 
 def test_goes_to_the_current_stream(pkg, dev):
