@@ -86,8 +86,8 @@ struct Planned { fp8bs_plan_t plan; bool share; };
 
 // The choice among (tile, split) in microseconds, each at the price of both forms: the soonest to finish where its sum can be shared out, among those
 // that finish within 6 % of the soonest where it cannot.  Of 267 shapes (see choose_tiled), times against the planner before there were
-// shared sums, operands from the caches / from HBM: eager 0.987 / 0.972, worst 1.09, replayed 0.996 / 0.978, worst 1.08 (of 270 others, 0.965 /
-// 0.970 and 0.997 / 0.997, 1.10 and 1.07).  At the price of the shared form alone 0.996 / 0.969, worst 1.37, and 1.006 / 0.976, worst 1.35
+// shared sums, operands from the caches / from HBM: eager 0.988 / 0.975, worst 1.09, replayed 0.996 / 0.979, worst 1.08 (of 270 others, 0.963 /
+// 0.970 and 0.997 / 0.997, 1.10 and 1.07).  At the price of the shared form alone 0.994 / 0.970, worst 1.37, and 1.009 / 0.977, worst 1.38
 // (896 x 1344 x 2944 in three, 16 us, 12 unsplit); within 4 % instead
 // 250 x 4096 x 7168 would lose its four partitions, 19.3 us eager and 21.4 replayed against 21.3 and 21.6 in three.
 struct Choice {
@@ -258,7 +258,7 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
             // the tile's, the S - 1 of S parts of a tile that a workgroup stores and loads, and, with S, ever smaller parts: pieces
             // of lines of c, written from as many XCDs.  The constants are fits, with all others held, to every (tile, split, form) of 267
             // shapes (M 1 .. 8000, N 190 .. 18100, K 1024 .. 7168, operands from HBM and from the caches), 200 of them with another plan than
-            // without shared sums: the picks are 1.7 and 4.2 % behind the best of each shape, 6.1 and 4.9 % without the last term,
+            // without shared sums: the picks are 1.8 and 4.5 % behind the best of each shape, 6.1 and 4.9 % without the last term,
             // which priced eight partitions of full tiles like four (1024 x 512 x 7168 in eight of 128x128 20.4 us, 64x128 in four and a
             // reduce launch 15.1; 619 x 768 x 6272 21.3 in eight, 15.9 in two of 64x64).  250 x 4096 x 7168 in four 128x128 tiles' partitions
             // 19.0 us (three, one workgroup summing: 20.9), 300 x 2112 x 7168 16.6 (19.0), 1 x 1230 x 4864 8.5 (10.8).  Eight tiles and fewer stay
@@ -269,8 +269,12 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
             const double rows = m < vi.bm ? m : vi.bm, cols = n < vi.bn ? n : vi.bn;
             const double shared_sum = c.t_sum * (1.0 + 0.027 * s) + (20.0 * (s - 1) / s + c.t_part * s) * rows * cols * 4e-6 * (double)cdiv(wgs, num_cus);
             if (s == 1) { choice.add(c.tile, 1, issued(cost, 5.3), issued(cost, 5.3), cost, false, false); continue; }
-            const double two = cost + planes, last = cost + in_kernel, parts = cost + shared_sum;
-            const bool can = can_sum_in_kernel(m, n, c.tile, s), shared = can && share && issued(parts, 5.3) < issued(two, 8.5);
+            // 64x64 always shares where it can: its planes are as fast on the GPU (0.95 to 1.22 of the shared time in the geometric mean, by rows
+            // and n on the 8-column grid, 300 shapes), and a second launch costs a caller's host 2 us (quantise, gate/up, quantise and
+            // down of 41 x 1280 x 3456, bound by the host, 25.1 us and 27.0).
+            const bool level = c.tile == (FP8BS_VARIANT_T64x128 | FORM1);
+            const double two = cost + planes, last = cost + in_kernel, parts = cost + (level && planes < shared_sum ? planes : shared_sum);
+            const bool can = can_sum_in_kernel(m, n, c.tile, s), shared = can && share && (level || issued(parts, 5.3) < issued(two, 8.5));
             // (where a sum in the kernel can be shared out it is: one that is not better than two launches then is none)
             const bool fused = can && (s == 2 || s == 3) && shared == share && issued(last, 5.3) < issued(two, 8.5);
             const double plain = fused ? issued(last, 5.3) : issued(two, 8.5);

@@ -129,9 +129,10 @@ def test_a_workspace_of_the_reported_size_lets_a_sum_be_shared(pkg, run, fn, m, 
     assert counts == [1, 2, 2]
 
 
-@pytest.mark.parametrize("m,n,k,split", [(7, 1516, 7040, 8), (14, 3373, 6144, 4), (1, 827, 6656, 8), (11, 2882, 5120, 4), (21, 777, 5888, 8), (46, 2489, 4736, 6)])
-def test_a_few_odd_rows_share_their_sums(pkg, run, m, n, k, split):
-    """One launch of 64x64 tiles: with planes and a reduce launch, 10 to 26 % slower at these sizes."""
+@pytest.mark.parametrize("m,n,k,split", [(7, 1516, 7040, 8), (14, 3373, 6144, 4), (1, 827, 6656, 8), (11, 2882, 5120, 4), (21, 777, 5888, 8), (46, 2489, 4736, 6),
+                                        (41, 1280, 3456, 8), (16, 2096, 3712, 6)])
+def test_a_few_rows_share_their_sums(pkg, run, m, n, k, split):
+    """One launch of 64x64 tiles: with planes and a reduce launch 10 to 26 % slower where n is odd, and one launch more where it is not."""
     p = pkg.plan(m, n, k)
     assert (p.tile_m, p.tile_n, p.split_k) == (64, 64, split)
     (eager, _), = run([("gemm", 0, m, n, k, 0, 0, pkg.workspace_bytes(m, n, k))])
