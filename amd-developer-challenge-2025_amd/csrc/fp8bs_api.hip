@@ -248,11 +248,12 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
             const double planes = 2.66 + 1.656e-6 * s * (double)m * (double)n + ((n & 7) != 0 && m <= 64 ? 0.2 * s : 0.0);
             const double in_kernel = 2.34 + 0.891e-6 * s * (double)m * (double)n
                                      + 13.2 * (s - 1) * (vi.bm * vi.bn * 4e-6) * (double)cdiv(wgs, num_cus);
-            // calls issued one after another are never faster than the host launches them: 5.2 to 6.2 us, or 7.7 to 10.2 with the
-            // reduce launch of a split, by the machine.  The latter stands as 8.5 here: the constants are 0.5 to 1.2 us over
+            // calls issued one after another are never faster than the host launches them: 5.2 to 6.2 us with the checks in Python, or 7.7
+            // to 10.2 with the reduce launch of a split, by the machine.  The latter stands as 8.5 here: the constants are 0.5 to 1.2 us over
             // what such small calls take, and at 8.5 neither side loses much on a fast or a slow host (12 x 512 x 1536 unsplit 5.4,
             // in four partitions and two launches 8.1 and 9.1; 1 x 512 x 3456 in three, one launch, 8.8, in eight 7.7 and 9.1).
-            // These are Python callers' launches; a captured graph or a C program, whose launches cost less, is given the same plan.
+            // custom_kernel's native call issues one launch in 3 to 4 us.  Calls below 5.3 us are equals here, and the time on the GPU
+            // decides among them; so all that the floors do for such a caller is to ask 3.2 us on the GPU of a second launch.
             auto issued = [](double gpu, double host) { return gpu > host ? gpu : host; };
             // Where every (tile, partition) has a workgroup of its own the sums can be shared out (see the kernel): a base that is
             // the tile's, the S - 1 of S parts of a tile that a workgroup stores and loads, and, with S, ever smaller parts: pieces

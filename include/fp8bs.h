@@ -138,8 +138,8 @@ int fp8bs_gemm(const void* a, const void* b, const float* a_scale, const float* 
  * kernel plus merge kernel (1-amd-fp8-mm/amd-fp8-mm-submission.py:371-511) without the second launch, and what
  * fp8bs_plan chooses for splits in two or three (sum_in_kernel of the plan).  Every workgroup writes its fp32
  * partial tile to the workspace; then either each adds its share of the tile, once all of them have raised a flag there,
- * and writes that part of c (the 64x64, 64x256 and eight-wave 128x128 tiles where all workgroups are on the chip at once and
- * the launch is not captured), or the one that finds all the others counted in at the tile's counter adds them all.  The order
+ * and writes that part of c (the 64x256 and eight-wave 128x128 tiles, and 64x64 from four partitions on, where all workgroups
+ * are on the chip at once and the launch is not captured), or the one that finds all the others counted in at the tile's counter adds them all.  The order
  * is ascending K, the reduce kernel's, so c holds the same bits as with two launches.  Nobody depends on another
  * workgroup being on the chip: one that waits in vain leaves its share to a later one.  The
  * tiled variants only (else FP8BS_ERR_BAD_VARIANT); with more than 2016 tiles or more than 255 partitions the
@@ -166,7 +166,7 @@ int fp8bs_gemm_ex(const void* a, const void* b, const float* a_scale, const floa
 /* fp8bs_gemm for callers that cannot allocate device memory or hand over a workspace: code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc.  No counterpart in the reference
  * (its split-K path allocates a tensor per call, 1-amd-fp8-mm/amd-fp8-mm-submission.py:600).  Same
- * arguments, plan, kernels and results as fp8bs_gemm, but the fp32 partial planes or tiles of a K split live in an
+ * arguments, plan, kernels and results as fp8bs_gemm, eager and captured alike, but the fp32 partial planes or tiles of a K split live in an
  * array of FP8BS_NOALLOC_SCRATCH_BYTES that is part of the library's device code (every GPU the library
  * runs on holds it until the process ends).  Calls no hipMalloc / hipFree or any allocating routine.
  * A shape whose planned K split needs more workspace than that returns FP8BS_ERR_SCRATCH_LIMIT
