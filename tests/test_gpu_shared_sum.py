@@ -122,16 +122,18 @@ def test_parts_that_are_left_behind():
     assert res.returncode == 0 and "all equal" in res.stdout, res.stdout[-500:] + res.stderr[-2000:]
 
 
-@pytest.mark.parametrize("m,n,k,split", [(250, 4096, 7168, 4), (64, 4096, 7168, 8), (300, 500, 2048, 2)])
+@pytest.mark.parametrize("m,n,k,split", [(250, 4096, 7168, 4), (64, 4096, 7168, 8), (1024, 1536, 7168, 2), (64, 18432, 7168, 3), (21, 778, 5888, 8)])
 def test_captured_calls_and_the_epilogue(pkg, m, n, k, split):
-    """The planner's own calls: eager, captured and replayed with changed operands, and with the silu-mul epilogue."""
+    """The planner's own calls: eager, shared out; captured and replayed with changed operands, not shared; and with the silu-mul epilogue."""
     dev, moe = torch.device("cuda:0"), importlib.import_module("amd-developer-challenge-2025_amd.moe")
     a, b, sa, sb, c = _operands(pkg, m, n, k, dev)
     plan = pkg.plan(m, n, k)
-    if split > 2:
-        assert plan.split_k == split and not plan.sum_in_kernel      # what a caller with no more than workspace_bytes gets
+    assert plan.split_k == split and plan.sum_in_kernel == (split in (2, 3))      # what a captured call gets
     want = pkg.custom_kernel((a, b, sa, sb, torch.empty_like(c)), variant=3, split_k=plan.split_k)
+    ws = importlib.import_module("amd-developer-challenge-2025_amd.submission")._workspace(dev, 64 << 20, torch.cuda.current_stream().cuda_stream)
+    ws[:16384].fill_(0)
     assert torch.equal(pkg.custom_kernel((a, b, sa, sb, c)).view(torch.int16), want.view(torch.int16))
+    assert len(_flags(ws)) == plan.grid_x
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         pkg.custom_kernel((a, b, sa, sb, c))
