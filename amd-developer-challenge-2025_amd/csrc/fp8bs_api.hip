@@ -84,12 +84,12 @@ uint64_t planes_bytes(int m, int n, int split_k) { return split_k > 1 ? (uint64_
 // and split are the same for all callers, so that a replayed call returns the bits of an eager one.
 struct Planned { fp8bs_plan_t plan; bool share; };
 
-// The choice among (tile, split) in microseconds, each at the price of both forms: the soonest to finish where its sum can be shared out, among those
-// that finish within 6 % of the soonest where it cannot.  Of 267 shapes (see choose_tiled), times against the planner before there were
+// The choice among (tile, split) in microseconds, each at the price of both forms: the soonest to finish where its sum can be
+// shared out, among those that finish within 6 % of the soonest where it cannot.  Of 267 shapes (see choose_tiled), times against the planner before there were
 // shared sums, operands from the caches / from HBM: eager 0.988 / 0.975, worst 1.09, replayed 0.996 / 0.979, worst 1.08 (of 270 others, 0.963 /
 // 0.970 and 0.997 / 0.997, 1.10 and 1.07).  At the price of the shared form alone 0.994 / 0.970, worst 1.37, and 1.009 / 0.977, worst 1.38
-// (896 x 1344 x 2944 in three, 16 us, 12 unsplit); within 4 % instead
-// 250 x 4096 x 7168 would lose its four partitions, 19.3 us eager and 21.4 replayed against 21.3 and 21.6 in three.
+// (896 x 1344 x 2944 in three, 16 us, 12 unsplit); within 4 % instead 250 x 4096 x 7168 would lose its four partitions, 19.3 us eager
+// and 21.4 replayed against 21.3 and 21.6 in three.
 struct Choice {
     struct Option { int tile, split; double shared, plain, gpu; bool share, fused; } options[80];
     int count = 0;
@@ -288,7 +288,8 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
     // the time of the other tiles in the geometric mean, within 1.6 % of the best; at most 1.19 of it where the two are
     // modelled level.  Only where all workgroups are on the chip at once - one or two fit a CU -, the model has no second round: of 34
     // shapes with more, M 17 .. 4203, N 126 .. 18300, all but one were slower than with the other tiles, 14 % in the geometric mean, 36 at
-    // worst (320 x 1664 x 384 5.2 us, 64 x 64 3.9); of 90 with fewer, outside the fitted sizes too, none (0.74).  Not beyond 24 K blocks, where the others' splits over workgroups are ahead.  Up to eight blocks the sum is the
+    // worst (320 x 1664 x 384 5.2 us, 64 x 64 3.9); of 90 with fewer, outside the fitted sizes too, none (0.74).  Not beyond 24 K
+    // blocks, where the others' splits over workgroups are ahead.  Up to eight blocks the sum is the
     // unsplit one; beyond, eight partitions, summed in the kernel without a workspace.
     if (kbt >= 2 && (kbt <= WAVES_MAX || (may_split && kbt <= 24))) {
         struct Waves { int tile, bm; double fixed, block, load; };
@@ -317,7 +318,8 @@ void choose_tiled(int m, int n, int k, int num_cus, Planned* out, bool may_split
 // workgroup of the 128 x 128 tile to 94 shapes (N 4300 .. 18400, b from HBM and from the caches).  On these 94 the picks are 9 % (caches) and 7 %
 // (HBM) faster than those of the 64 x 256 tile alone, eager as well as replayed, 4 % slower at worst (with its planes left out,
 // 12 %: 11 x 6464 x 4096).  us: 64 x 18432 x 7168 33.0 (33.7), 64 x 16384 x 4096 20.5 (22.0), 64 x 12288 x 2048 12.7 (16.4), 64 x 4096 x 7168
-// 14.2 (16.3), 64 x 7168 x 7168 18.2 (19.4).  With few rows the planes are small and two launches are ahead, in either tile: 1 x 18432 x 7168 28.8, one launch 30.8.
+// 14.2 (16.3), 64 x 7168 x 7168 18.2 (19.4).  With few rows the planes are small and two launches are ahead, in either tile:
+// 1 x 18432 x 7168 28.8, one launch 30.8.
 void choose_skinny(int m, int n, int k, int num_cus, Planned* out, bool may_split) {
     if (num_cus <= 0) num_cus = 256;
     const int kbt = k / KBLK;
