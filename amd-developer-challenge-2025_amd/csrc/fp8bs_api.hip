@@ -667,11 +667,7 @@ static int dense_call(const void* a, const void* b, const float* a_scale, const 
     g.band_h = 4;
     g.num_experts = 0;
     g.epi = epi;
-    if (ready_planes) {
-        g.ready_only = 1;
-        if (fp8bs::launch_gemm(plan.variant | plan.form * FORM1, 1, g, s) != hipSuccess) return FP8BS_ERR_LAUNCH;
-        g.ready_only = 0;
-    }
+    if (ready_planes && fp8bs::launch_gemm(plan.variant | plan.form * FORM1, 1 | fp8bs::READY_ONLY, g, s) != hipSuccess) return FP8BS_ERR_LAUNCH;
     int mode = plan.split_k > 1 && !waves ? 1 : 0;
     if (plan.sum_in_kernel && plan.split_k > 1 && !waves) {
         mode = 4;

@@ -29,9 +29,14 @@ struct GemmArgs {
     // 8-byte flag per workgroup) and one fp32 partial tile per workgroup, see StreamK below
     unsigned long long sk_nonce;   // value a flag takes when its workgroup's partial tile is complete: differs from call to call
     int sk_grid;            // workgroups of such a call: at most the places on the chip and the number of (tile, K block) pairs
-    int ready_only;         // host: the launcher raises the LDS limit of the kernel that these arguments take and launches nothing
     int sk_spin;            // polls of a flag before the wait gives up (< 0: give up at once - tests of the error path); with a shared-out sum: before a part is left to another workgroup
 };
+// (A kernel's arguments are read cold at its start: with eight bytes more an unsplit grouped product of 64 tokens to 8 of 16 experts,
+// 960 x 768, took 8.27 us instead of 8.18, means of three processes each in turn.)
+static_assert(sizeof(GemmArgs) <= 120);
+
+// Or'ed into a mode: raise the LDS limit of the kernel that the arguments take and launch nothing (tiles of gemm_tr_kernel).
+constexpr int READY_ONLY = 256;
 
 // Workspace of a call that deals K blocks (all offsets from the 16-byte aligned workspace base):
 //   [0, 4)                          status word: set to FP8BS_ERR_TIMEOUT by a workgroup whose bounded wait gave up

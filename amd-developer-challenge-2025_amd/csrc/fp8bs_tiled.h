@@ -1408,7 +1408,7 @@ static inline hipError_t launch_tr(const GemmArgs& a, dim3 grid, hipStream_t str
     using C = TileCfg<BM, BN, WM, WN, MODE, NSTAGE>;
     void (*kern)(const GemmArgs);
     hipError_t e = ready_tr<BM, BN, WM, WN, MODE, EPI, NSTAGE, SHARED_SUM>(a, &kern);
-    if (e != hipSuccess || a.ready_only) return e;
+    if (e != hipSuccess || grid.x == 0) return e;                       // no workgroups: the kernel was to be readied only
     GemmArgs args = a;
     args.c_whole_lines = ((size_t)(EPI == 1 ? a.n / 2 : a.n) * 2u) % 128u == 0 && ((uintptr_t)a.c & 127) == 0;
     hipLaunchKernelGGL(kern, grid, dim3(C::NTHREADS), C::LDS_BYTES, stream, args);
@@ -1418,6 +1418,8 @@ static inline hipError_t launch_tr(const GemmArgs& a, dim3 grid, hipStream_t str
 // WITH_EPI: the fused silu-mul epilogue is instantiated for this tile; GROUPED_SPLIT: the grouped walk with a K split is
 template <int BM, int BN, int WM, int WN, bool WITH_EPI = false, int NSTAGE = 2, bool GROUPED_SPLIT = false>
 static inline hipError_t launch_shape(const GemmArgs& a, int mode, hipStream_t stream) {
+    const bool ready_only = (mode & READY_ONLY) != 0;
+    mode &= ~READY_ONLY;
     using C = TileCfg<BM, BN, WM, WN, 0, NSTAGE>;
     // persistent workgroups: as many as fit the chip at once (LDS and thread limits), each walks
     // tiles  blockIdx.x, blockIdx.x + grid, ...
@@ -1439,7 +1441,7 @@ static inline hipError_t launch_shape(const GemmArgs& a, int mode, hipStream_t s
         if (a.sk_grid < 1 || a.sk_grid > resident || a.sk_grid > pairs || a.sk_grid > StreamK::MAX_GRID) return hipErrorInvalidValue;
         return launch_tr<BM, BN, WM, WN, 3, 0, NSTAGE>(a, dim3((unsigned)a.sk_grid), stream);
     }
-    const dim3 grid((unsigned)(total < resident ? total : resident));
+    const dim3 grid(ready_only ? 0u : (unsigned)(total < resident ? total : resident));
     // K partitions summed in the kernel, the sum shared out or not.  A call that shares it readies the kernel that a capture of the
     // same call will launch too: the LDS limit is not a thing to be raised there.
     auto launch_summed = [&](auto mode_tag, auto epi_tag) {
