@@ -738,11 +738,28 @@ void gemm_tr_kernel(const GemmArgs p) {
             }(std::make_integer_sequence<int, NL_LATE>{});
         }
 
+        // A block's scales are read ahead of its first operands, behind the barrier that publishes it, and the operands in the
+        // order in which they are multiplied, here as in the loop: an LDS wait names how many younger reads may still be out, and
+        // where two ways lead into the loop the compiler takes the lower number.  (Read at the block's start, the scales were
+        // the youngest, and the first MFMA waited for every read there was: 1024 x 1536 x 7168 unsplit, us, 128x128 in eight waves
+        // 30.0 -> 29.3, in four 39.8 -> 38.1, 256x128 46.3 -> 44.3, 64x256 33.3 -> 33.5; 2048 x 2048 x 2048 17.7 -> 17.1 in 256x128.)
         v8i areg[C::MT], breg[2];
-        if (wave_active) {
+        float asv[C::MT], bsv, bsv1;
+        auto read_scales = [&](const unsigned char* sb) {
 #pragma unroll
-            for (int t = 0; t < C::MT; t++) read_a(areg[t], t, lds);
+            for (int t = 0; t < C::MT; t++) asv[t] = *(const float*)(sb + as_lane_off + t * 64);
+            bsv = *(const float*)(sb + bs_off);
+            bsv1 = C::SPLIT_SCALES ? *(const float*)(sb + bs_off + 4) : 0.f;
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        if (wave_active) {
+            read_scales(lds);
+            read_a(areg[0], 0, lds);
+            __builtin_amdgcn_sched_barrier(0);
             read_b(breg[0], 0, lds);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int t = 1; t < C::MT; t++) { read_a(areg[t], t, lds); __builtin_amdgcn_sched_barrier(0); }
         }
 
         // All K blocks of the tile.  UB: the wave's n tiles [UB, NT) belong to the next b_scale block
@@ -791,14 +808,8 @@ void gemm_tr_kernel(const GemmArgs p) {
             const unsigned char* sbase = lds + cur_stage * C::STAGE_BYTES;
             const unsigned char* snext = lds + next_stage * C::STAGE_BYTES;
             float sc[C::MT], sc1[C::MT];
-            const float bsv = *(const float*)(sbase + bs_off);
-            const float bsv1 = UB < C::NT ? *(const float*)(sbase + bs_off + 4) : 0.f;
-#pragma unroll
-            for (int t = 0; t < C::MT; t++) {
-                const float asv = *(const float*)(sbase + as_lane_off + t * 64);
-                sc[t] = asv * bsv;
-                sc1[t] = UB < C::NT ? asv * bsv1 : 0.f;
-            }
+            // the step that works out the block's scales: the one that folds first, but before the next block's are read
+            constexpr int BARRIER_STEP = STEPS - C::MT, SCALE_STEP = LAG < BARRIER_STEP ? LAG : BARRIER_STEP - 1;
             v4f ring[RING];
             auto step = [&](auto s_tag) {
                 constexpr int s = decltype(s_tag)::value;
@@ -821,6 +832,7 @@ void gemm_tr_kernel(const GemmArgs p) {
                         wait_next_block();
                         __syncthreads();
                         if constexpr (TAILS && LANDS_LAST) FP8BS_PATCH_TAILS(next_stage, cur_stage);
+                        if constexpr (HAS_NEXT) read_scales(snext);
                     }
                     const v4f z = {0.f, 0.f, 0.f, 0.f};
                     ring[s % RING] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(breg[u & 1], areg[t], z, 0, 0, 0, 0, 0, 0);
@@ -831,6 +843,13 @@ void gemm_tr_kernel(const GemmArgs p) {
                     }
                     if constexpr (u == C::NT - 1 && HAS_LATE && t < NL_LATE)
                         issue_one(cp, cur_stage, j + NSTAGE, std::integral_constant<int, t>{});
+                }
+                if constexpr (s == SCALE_STEP) {
+#pragma unroll
+                    for (int t = 0; t < C::MT; t++) {
+                        sc[t] = asv[t] * bsv;
+                        sc1[t] = UB < C::NT ? asv[t] * bsv1 : 0.f;
+                    }
                 }
                 if constexpr (s >= LAG) {
                     constexpr int sp = s - LAG, u = sp / C::MT, t = sp % C::MT;
