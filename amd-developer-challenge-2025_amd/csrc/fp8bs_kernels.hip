@@ -5,6 +5,26 @@
 
 namespace fp8bs {
 
+// Repair of the last bytes of a in the streaming kernel (gemm_tr_kernel does without a second barrier).  cand[i]: see tail_candidate; bits
+// 8-31 of `last` = the bytes themselves.  tile: the tile of a of the last K block, x0 its first row, spare: a byte of LDS
+// nobody reads.  No control flow: a store that does not apply goes to the spare byte.
+template <int BX, int CPR>
+__device__ __forceinline__ void patch_tail_bytes(unsigned char* tile, unsigned char* spare, bool enable, int x0,
+                                                 uint32_t cand0, uint32_t cand1, uint32_t cand2, uint32_t last, int tid) {
+    const uint32_t cand[3] = {cand0, cand1, cand2};
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        const int xt = (int)(cand[c] & 0x1FFFFFFFu) - x0;                 // row / column inside the tile
+        const int kl = KBLK - 3 + (int)((cand[c] >> 29) & 3u);            // k row inside the last block
+        int xc = xt < 0 ? 0 : xt;                                         // in range whatever xt is
+        xc = xc < BX ? xc : BX - 1;
+        unsigned char* dst = tile + kl * BX + (chunk_to_stored<CPR>(xc >> 4, swz_of_krow<CPR>(kl)) << 4) + (xc & 15);
+        int apply = (enable && (cand[c] >> 31) != 0 && xt >= 0 && xt < BX && tid == 0) ? 1 : 0;
+        asm volatile("" : "+v"(apply));       // opaque to the optimiser: a select follows, never a branch
+        *(apply != 0 ? dst : spare) = (unsigned char)(last >> (8 * (c + 1)));
+    }
+}
+
 // ---------------------------------------------------------------------------------------------------
 // Skinny-M streaming kernel (bandwidth-bound shapes: a few rows of A against a long B).
 //
@@ -150,10 +170,10 @@ void gemm_skinny_kernel(const GemmArgs p) {
     uint32_t acand0 = 0, acand1 = 0, acand2 = 0, a_last = 0;
     if (a_tail) {
         const uint32_t end = (uint32_t)p.k * (uint32_t)p.lda;
-        acand0 = tail_candidate(end - 3, (uint32_t)p.lda, end, (uint32_t)p.k);
-        acand1 = tail_candidate(end - 2, (uint32_t)p.lda, end, (uint32_t)p.k);
-        acand2 = tail_candidate(end - 1, (uint32_t)p.lda, end, (uint32_t)p.k);
-        a_last = load_last_dword(p.a + (end - 4));
+        acand0 = tail_candidate(3, (uint32_t)p.lda, (uint32_t)p.k);
+        acand1 = tail_candidate(2, (uint32_t)p.lda, (uint32_t)p.k);
+        acand2 = tail_candidate(1, (uint32_t)p.lda, (uint32_t)p.k);
+        a_last = load_last_dword(p.a + end);
     }
     acand0 = __builtin_amdgcn_readfirstlane(acand0); acand1 = __builtin_amdgcn_readfirstlane(acand1);
     acand2 = __builtin_amdgcn_readfirstlane(acand2); a_last = __builtin_amdgcn_readfirstlane(a_last);

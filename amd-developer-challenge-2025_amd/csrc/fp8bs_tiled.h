@@ -174,35 +174,20 @@ __device__ __forceinline__ int stored_to_chunk(int st, int swz) {
     else { int x = st - swz; return x < 0 ? x + CPR : x; }
 }
 
-// Repair of the last bytes of a or b (see the main kernel).  cand[i]: bit 31 = the byte is lost, bits
-// 29-30 = its k row inside the last K block minus 125, bits 0-28 = its row (of a) or column (of b); bits
-// 8-31 of `last` = the bytes themselves.  tile: the operand's tile of the tile's last K block, x0 its first
-// row / column, spare: a byte of LDS nobody reads.  No control flow: a store that does not apply goes to
-// the spare byte.  (A branch at this place, in the middle of a K block's step sequence, makes the compiler
-// move the folds of the MFMAs before it below it, which costs some thirty registers.)
-template <int BX, int CPR>
-__device__ __forceinline__ void patch_tail_bytes(unsigned char* tile, unsigned char* spare, bool enable, int x0,
-                                                 uint32_t cand0, uint32_t cand1, uint32_t cand2, uint32_t last, int tid) {
-    const uint32_t cand[3] = {cand0, cand1, cand2};
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        const int xt = (int)(cand[c] & 0x1FFFFFFFu) - x0;                 // row / column inside the tile
-        const int kl = KBLK - 3 + (int)((cand[c] >> 29) & 3u);            // k row inside the last block
-        int xc = xt < 0 ? 0 : xt;                                         // in range whatever xt is
-        xc = xc < BX ? xc : BX - 1;
-        unsigned char* dst = tile + kl * BX + (chunk_to_stored<CPR>(xc >> 4, swz_of_krow<CPR>(kl)) << 4) + (xc & 15);
-        int apply = (enable && (cand[c] >> 31) != 0 && xt >= 0 && xt < BX && tid == 0) ? 1 : 0;
-        asm volatile("" : "+v"(apply));       // opaque to the optimiser: a select follows, never a branch
-        *(apply != 0 ? dst : spare) = (unsigned char)(last >> (8 * (c + 1)));
-    }
+// The four bytes before `end`, which may be any address (the same in all lanes), from the one or two dwords that hold them.  Scalar
+// loads: nothing waits for them but what uses them, where a vector load would be waited for together with the copies.
+__device__ __forceinline__ uint32_t load_last_dword(const uint8_t* end) {
+    typedef const __attribute__((address_space(4))) uint32_t* dword;
+    const uintptr_t at = (uintptr_t)end - 4;
+    const uint32_t lo = *(dword)(at & ~(uintptr_t)3), hi = *(dword)((at + 3) & ~(uintptr_t)3);
+    return (uint32_t)((((uint64_t)hi << 32) | lo) >> (8 * (at & 3)));
 }
-// The last four bytes of an operand, which may start on any byte.
-__device__ __forceinline__ uint32_t load_last_dword(const uint8_t* q) {
-    return (uint32_t)q[0] | ((uint32_t)q[1] << 8) | ((uint32_t)q[2] << 16) | ((uint32_t)q[3] << 24);
-}
-// The three candidates of an operand whose k rows are ld bytes long and whose buffer ends at `end`.
-__device__ __forceinline__ uint32_t tail_candidate(uint32_t o, uint32_t ld, uint32_t end, uint32_t k) {
-    const uint32_t krow = o / ld, x = o - krow * ld;
+// The byte `back` = 1, 2 or 3 before the end of an operand of k rows of ld bytes.
+// The byte `back` = 1, 2 or 3 before the end of an operand of k rows of ld bytes: bit 31 = the range check cuts it off, bits 29-30 = its k row
+// minus k - 3, bits 0-28 = its row (of a) or column (of b).
+__device__ __forceinline__ uint32_t tail_candidate(uint32_t back, uint32_t ld, uint32_t k) {
+    const uint32_t rows = ld > 2 ? 0 : ld == 2 ? (back - 1) >> 1 : back - 1;       // whole k rows behind its own
+    const uint32_t krow = k - 1 - rows, x = (rows + 1) * ld - back, end = k * ld;
     const bool lost = krow * ld + (x & ~3u) + 4u > end;                   // its dword crosses the end
     return lost ? (0x80000000u | ((krow - (k - 3u)) << 29) | x) : 0u;
 }
@@ -217,7 +202,7 @@ __device__ __forceinline__ float silu_mul(float gate, float up) {
 }
 
 // TAILS: lda is not a multiple of four or n not a multiple of eight; the kernel then repairs the last
-// bytes of a and b in LDS (one more barrier per tile) and stores a row's last, partial 16-byte chunk of c
+// bytes of a and b in LDS and stores a row's last, partial 16-byte chunk of c
 // in pieces, see below.
 // Waves per SIMD when as many workgroups as LDS and thread count allow share a CU.  The modes that exchange partial
 // tiles must keep their registers within that (their sums would otherwise take registers the K loop does not need
@@ -628,6 +613,15 @@ void gemm_tr_kernel(const GemmArgs p) {
     const int as_lane_off = C::A_BYTES + C::B_BYTES + (wave_m * WM + i16) * 4;
     const int bs_base = C::A_BYTES + C::B_BYTES + C::AS_AREA;     // slot i: b_scale of n block n0/128 + i
 
+    Tile cur = pick_tile(0);
+    if (!cur.valid) return;
+    CopyPlan cp = copy_plan(cur);
+    bool prefetched = false;                // the first blocks of `cur` are already on their way
+    if (TAILS && cur.kb_end > cur.kb_begin) {
+        issue_first(cp, cur.kb_end - cur.kb_begin);
+        prefetched = true;
+    }
+
     // ---- rows of a that are not a multiple of four, columns of b that are not ------------------------
     // The buffer of a ends on a dword boundary (K is a multiple of 128), but with lda % 4 != 0 the copies
     // fetch its last one to three bytes in dwords that start inside and end beyond it; the range check
@@ -635,53 +629,45 @@ void gemm_tr_kernel(const GemmArgs p) {
     // arrives intact (a dword that crosses the end of a k row just runs on into the next one).  The
     // workgroup whose tile holds those bytes writes them into LDS itself once the last K block has
     // landed: they all lie in the last aligned dword of a.  The same holds for b with n % 4 != 0.
-    // The three candidates (byte offsets end-3 .. end-1) are worked out once, here, where registers are
-    // plentiful, and kept in scalar registers.
+    // Each is written by the wave whose copy brought the bytes around it, between its wait for the copy and the barrier that
+    // publishes the block: lane l < 6 of every wave has one candidate, a's for l < 3, in patch_at and patch_byte, worked out at a tile's
+    // start while the first copies are on their way; a lane whose candidate is not lost, not in the tile or another
+    // wave's writes to a byte of the stage that nobody reads.  So the store has no condition: a branch at this place, in the middle of
+    // a K block's step sequence, makes the compiler move the folds of the MFMAs before it below it, which costs some thirty registers.
+    // (Worked out ahead of the first copies, from vector loads, six bytes one after the other behind the barrier and with a second
+    // barrier, the repair was 0.4 to 0.9 us of every call that takes this instantiation, and the pieces of c below, stored by all
+    // waves, 0.1 to 1.1: 1023 x 3141 x 2048 in 128x128 19.2 -> 18.1 us, 250 x 4096 x 1792 12.5 -> 11.5, 130 x 1000 x 128 5.6 -> 4.4, in
+    // 64x64 4.2 -> 3.5; 45 products on five tiles 0.88 of the time in the geometric mean.)
     const bool a_tail = TAILS && (p.lda & 3) != 0 && p.k > 0;
     const bool b_tail = TAILS && (p.n & 3) != 0 && p.k > 0;
-    uint32_t acand0 = 0, acand1 = 0, acand2 = 0, a_last = 0, bcand0 = 0, bcand1 = 0, bcand2 = 0, b_last = 0;
-    if (a_tail) {
-        const uint32_t end = (uint32_t)p.k * (uint32_t)p.lda;
-        acand0 = tail_candidate(end - 3, (uint32_t)p.lda, end, (uint32_t)p.k);
-        acand1 = tail_candidate(end - 2, (uint32_t)p.lda, end, (uint32_t)p.k);
-        acand2 = tail_candidate(end - 1, (uint32_t)p.lda, end, (uint32_t)p.k);
-        a_last = load_last_dword(p.a + (end - 4));
-    }
-    if (b_tail) {
-        const uint32_t end = (uint32_t)p.k * (uint32_t)p.n;
-        bcand0 = tail_candidate(end - 3, (uint32_t)p.n, end, (uint32_t)p.k);
-        bcand1 = tail_candidate(end - 2, (uint32_t)p.n, end, (uint32_t)p.k);
-        bcand2 = tail_candidate(end - 1, (uint32_t)p.n, end, (uint32_t)p.k);
-        if (!GROUPED) b_last = load_last_dword(p.b + (end - 4));     // grouped: every expert's matrix has last bytes of its own, read per tile
-    }
-    // (the loads are consumed here, not inside the K loop)
-    acand0 = __builtin_amdgcn_readfirstlane(acand0); acand1 = __builtin_amdgcn_readfirstlane(acand1);
-    acand2 = __builtin_amdgcn_readfirstlane(acand2); a_last = __builtin_amdgcn_readfirstlane(a_last);
-    bcand0 = __builtin_amdgcn_readfirstlane(bcand0); bcand1 = __builtin_amdgcn_readfirstlane(bcand1);
-    bcand2 = __builtin_amdgcn_readfirstlane(bcand2); b_last = __builtin_amdgcn_readfirstlane(b_last);
-    // stage: the tile's last K block; called by every wave right behind the barrier that publishes that
-    // block; ends with a second barrier
-#define FP8BS_PATCH_TAILS(stage, spare_stage)                                                                                              \
-    do {                                                                                                                                   \
-        patch_tail_bytes<BM, C::CPR_A>(lds + (stage) * C::STAGE_BYTES, lds + (spare_stage) * C::STAGE_BYTES + C::STAGE_BYTES - 1,          \
-                                       patch_tile && a_tail, m0, acand0, acand1, acand2, a_last, tid);                                     \
-        patch_tail_bytes<BN, C::CPR_B>(lds + (stage) * C::STAGE_BYTES + C::A_BYTES, lds + (spare_stage) * C::STAGE_BYTES + C::STAGE_BYTES - 1, \
-                                       patch_tile && b_tail, n0, bcand0, bcand1, bcand2, b_last, tid);                                     \
-        __syncthreads();                                                                                                                   \
-    } while (0)
+    [[maybe_unused]] int patch_at = 0;
+    [[maybe_unused]] uint32_t patch_byte = 0;
+    [[maybe_unused]] auto plan_patch = [&](const Tile& t) {
+        const bool of_b = lane >= 3;
+        const uint32_t back = 3u - (uint32_t)(of_b ? lane - 3 : lane) % 3u;
+        const uint32_t cand = tail_candidate(back, (uint32_t)(of_b ? p.n : p.lda), (uint32_t)p.k);
+        const int xt = (int)(cand & 0x1FFFFFFFu) - (of_b ? t.n0 : t.m0);                // row / column inside the tile
+        const int kl = KBLK - 3 + (int)((cand >> 29) & 3u);                             // k row inside the last block
+        const int cpr = of_b ? C::CPR_B : C::CPR_A;
+        const int stored = of_b ? chunk_to_stored<C::CPR_B>((xt >> 4) & 15, swz_of_krow<C::CPR_B>(kl)) : chunk_to_stored<C::CPR_A>((xt >> 4) & 15, swz_of_krow<C::CPR_A>(kl));
+        const int slot = kl * cpr + stored;                                             // of 16 bytes; 64 of them are a wave's copy
+        const bool mine = lane < 6 && (of_b ? b_tail : a_tail) && (cand >> 31) != 0 && t.kb_end * KBLK == p.k
+                          && xt >= 0 && xt < (of_b ? BN : BM) && (slot >> 6) % C::NWAVES == wave;
+        uint32_t a_last = 0, b_last = 0;
+        if (a_tail) a_last = load_last_dword(p.a + a_bytes);
+        if (b_tail) b_last = load_last_dword(t.bptr + b_bytes);                         // grouped: every expert's matrix has last bytes of its own
+        patch_byte = (of_b ? b_last : a_last) >> (8u * (4u - back));
+        patch_at = mine ? (of_b ? C::A_BYTES : 0) + slot * 16 + (xt & 15) : C::STAGE_BYTES - 1;
+    };
+    // stage: the tile's last K block, which this wave's copies have just reached
+    [[maybe_unused]] auto patch = [&](int stage) { *(volatile unsigned char*)(lds + stage * C::STAGE_BYTES + patch_at) = (unsigned char)patch_byte; };
 
-    Tile cur = pick_tile(0);
-    if (!cur.valid) return;
-    CopyPlan cp = copy_plan(cur);
-    bool prefetched = false;                // block 0 of `cur` is already on its way into stage 0
     bool stores_behind = false;             // ... and this wave's output stores of the previous tile were issued after it
     for (int it = 0;; it++) {
     const int m0 = cur.m0, n0 = cur.n0, kb_begin = cur.kb_begin, kb_end = cur.kb_end, split_z = cur.split_z;
     const int row_lo = cur.row_lo, row_hi = cur.row_hi;
     [[maybe_unused]] const int sk_contrib = cur.sk_contrib, sk_first = cur.sk_first;
-    if constexpr (TAILS && GROUPED) {
-        if (b_tail) b_last = __builtin_amdgcn_readfirstlane(load_last_dword(cur.bptr + ((uint32_t)p.k * (uint32_t)p.n - 4u)));
-    }
+    if constexpr (TAILS) plan_patch(cur);
     // a_scale: lane's output row of m-tile t is tile row wave_m*WM + 16t + i16, read from the stage's
     // copy of the a_scale row.
     // does any element of this wave's tile get stored?  (rows of the expert / matrix, columns of the matrix)
@@ -699,7 +685,6 @@ void gemm_tr_kernel(const GemmArgs p) {
         for (int u = 0; u < C::NT; u++) acc[t][u] = (v4f){0.f, 0.f, 0.f, 0.f};
 
     const int nkb = kb_end - kb_begin;
-    const bool patch_tile = TAILS && kb_end * KBLK == p.k;        // this tile's last K block is the last of a and b
     if (nkb > 0) {
         constexpr int STEPS = C::MT * C::NT;
         constexpr int LAG = 3, RING = 4;      // fold the result of step s-LAG while step s runs
@@ -730,8 +715,8 @@ void gemm_tr_kernel(const GemmArgs p) {
                 ((behind == I ? (sb ? wait_vmcnt<I * NLOADS + EPI_STORES>() : wait_vmcnt<I * NLOADS>()) : (void)0), ...);
             }(std::make_integer_sequence<int, NSTAGE - 1>{});
         }
+        if (TAILS && nkb == 1) patch(0);
         __syncthreads();
-        if (TAILS && nkb == 1) FP8BS_PATCH_TAILS(0, 1);
         if (nkb > NSTAGE - 1) {
             [&]<int... Q>(std::integer_sequence<int, Q...>) {
                 (issue_one(cp, NSTAGE - 1, NSTAGE - 1, std::integral_constant<int, Q>{}), ...);
@@ -796,8 +781,8 @@ void gemm_tr_kernel(const GemmArgs p) {
                     }(std::make_integer_sequence<int, NL_EARLY>{});
                 }
                 wait_next_block();
+                if constexpr (TAILS && LANDS_LAST) patch(next_stage);
                 __syncthreads();
-                if constexpr (TAILS && LANDS_LAST) FP8BS_PATCH_TAILS(next_stage, cur_stage);
                 if constexpr (HAS_LATE) {
                     [&]<int... Q>(std::integer_sequence<int, Q...>) {
                         (issue_one(cp, cur_stage, j + NSTAGE, std::integral_constant<int, Q>{}), ...);
@@ -830,8 +815,8 @@ void gemm_tr_kernel(const GemmArgs p) {
                         // of the next block, then meet the other waves: after the barrier the next
                         // block is complete in the other stage and this stage may be overwritten.
                         wait_next_block();
+                        if constexpr (TAILS && LANDS_LAST) patch(next_stage);
                         __syncthreads();
-                        if constexpr (TAILS && LANDS_LAST) FP8BS_PATCH_TAILS(next_stage, cur_stage);
                         if constexpr (HAS_NEXT) read_scales(snext);
                     }
                     const v4f z = {0.f, 0.f, 0.f, 0.f};
@@ -1349,6 +1334,7 @@ void gemm_tr_kernel(const GemmArgs p) {
             const bool lane_live = ROW_POW2 || lane_r < ROWS_PER_PASS;
             const int wave_row0 = wave_m * WM, wave_col0 = wave_n * WNO;              // inside the tile, output columns
             const bool col_ok = lane_live && col0 + wave_col0 + lane_chunk * 8 < ldc;
+            [[maybe_unused]] const bool row_ends = (ldc & 7) != 0 && col0 + wave_col0 + WNO > ldc;      // the wave's tile holds rows' last, partial chunks
             const uint32_t lane_off = ((uint32_t)(wave_row0 + lane_r) * (uint32_t)ldc + (uint32_t)(wave_col0 + lane_chunk * 8)) * 2u;
 #pragma unroll
             for (int q = 0; q < PASSES; q++) {
@@ -1373,7 +1359,7 @@ void gemm_tr_kernel(const GemmArgs p) {
                 } else {
                     // n not a multiple of eight: the chunk that holds a row's last columns is stored in
                     // pieces of 4, 2 and 1 elements (the bits of the number of columns left), every piece
-                    // its own instruction that the other lanes sit out; rows then start on 2-, 4- or
+                    // its own instruction that the other lanes sit out, by the waves whose tile holds such a chunk; rows then start on 2-, 4- or
                     // 8-byte boundaries only, which the stores take in their stride (plain stores: the lines a
                     // row segment shares with the neighbouring tiles are put together in the L2)
                     int left = ldc - (col0 + wave_col0 + lane_chunk * 8);                  // columns from this chunk's first to the row's end
@@ -1381,6 +1367,7 @@ void gemm_tr_kernel(const GemmArgs p) {
                     const bool part = ok && left < 8;
                     const v4u v = __builtin_bit_cast(v4u, val);
                     __builtin_amdgcn_raw_buffer_store_b128(v, c_rsrc, ok && left == 8 ? lane_off : 0xFFFFFFFFu, 0, 0);
+                    if (row_ends) {
                     const v2i lo = {val[0], val[1]};
                     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, lo), c_rsrc, part && (left & 4) ? lane_off : 0xFFFFFFFFu, 0, 0);
                     const uint32_t d2 = (left & 4) ? v[2] : v[0];                          // elements (left & 4), +1
@@ -1388,6 +1375,7 @@ void gemm_tr_kernel(const GemmArgs p) {
                     const int e1 = left & 6;                                               // element (left & 6)
                     const uint32_t d1 = e1 == 0 ? v[0] : e1 == 2 ? v[1] : e1 == 4 ? v[2] : v[3];
                     __builtin_amdgcn_raw_buffer_store_b16((unsigned short)(d1 & 0xFFFFu), c_rsrc, part && (left & 1) ? lane_off + (uint32_t)e1 * 2u : 0xFFFFFFFFu, 0, 0);
+                    }
                 }
             }
         }
@@ -1397,8 +1385,6 @@ void gemm_tr_kernel(const GemmArgs p) {
     cur = nxt; cp = ncp;
     }   // tiles
 }
-
-#undef FP8BS_PATCH_TAILS
 
 // ---------------------------------------------------------------------------------------------------
 // Launchers

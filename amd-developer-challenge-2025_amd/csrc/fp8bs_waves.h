@@ -123,7 +123,7 @@ void gemm_waves_kernel(const GemmArgs p) {
                     constexpr int CPR = decltype(cpr_tag)::value;
                     const uint32_t end = (uint32_t)p.k * ld;
                     if (lane < 3) {
-                        const uint32_t cand = tail_candidate(end - 3u + lane, ld, end, (uint32_t)p.k);
+                        const uint32_t cand = tail_candidate(3u - lane, ld, (uint32_t)p.k);
                         const int x = (int)(cand & 0x1FFFFFFFu) - x0, kl = KBLK - 3 + (int)((cand >> 29) & 3u);
                         if ((cand >> 31) != 0 && x >= 0 && x < CPR * 16)
                             tile[kl * CPR * 16 + (chunk_to_stored<CPR>(x >> 4, swz_of_krow<CPR>(kl)) << 4) + (x & 15)] = src[end - 3u + lane];
