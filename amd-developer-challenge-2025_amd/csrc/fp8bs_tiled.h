@@ -260,7 +260,7 @@ void gemm_tr_kernel(const GemmArgs p) {
     // tile's output and the next tile's first loads overlap (with K = 2048 the per-tile prologue and
     // epilogue are a third of a tile's time otherwise).
     struct Tile {
-        int valid, m0, n0, kb_begin, kb_end, split_z, row_lo, row_hi;
+        int valid, m0, n0, n_hi, kb_begin, kb_end, split_z, row_lo, row_hi;
         int sk_contrib, sk_first;             // MODE 3: the segment ends before the tile's last K block; first workgroup of the tile's earlier segments (-1: none)
         const uint8_t* bptr;
         const float* bsptr;
@@ -312,10 +312,41 @@ void gemm_tr_kernel(const GemmArgs p) {
             total_slots = total_slots < bound ? total_slots : bound;
         }
     }
+    // The tile that this workgroup takes in round `it`, -1: none.  The gridDim.x tiles in flight together are dealt to the XCDs in
+    // contiguous runs, those of a last round that is not full as well: in runs of a full round's length they kept some XCDs busy and
+    // left the others, and their share of the memory's rate, idle.  Where they leave half of the chip, or three quarters, they are cut in
+    // two or four by columns (1 << cut parts, the most: one wave's columns each): waves without columns only copy and
+    // columns of other parts are not fetched, so a part costs little more than what its columns do.
+    // us, before and now: 46 tokens to 8 of 16 experts, 766 x 1536, 15.6 and 9.4; 46 to 4 of 32, 2485 x 2432, 64.1 and 50.4; 900 to 8 of 16,
+    // 3072 x 1536, 48.0 and 41.8; 64 to 8 of 32, 7168 x 2048 (3.5 rounds), 101.2 and 97.4; dense 6144 x 4608 x 7168 195 and 177. 90 grouped
+    // products (1 .. 4096 tokens) 0.93 of the time in the geometric mean, at worst 1.04 (1920 tokens to 4 of 32 experts, 832 x 4992).
+    constexpr int MOST_CUT = (MODE == 0 || MODE == 2) && BN == 256 ? (BN / WN >= 4 ? 2 : 1) : 0;
+    auto place = [&](int it, int total, int& part, int& cut) -> int {
+        const int G = gridDim.x, first = it * G, here = total - first;
+        if (here <= 0) return -1;
+        if (here >= G) return first + xcd_virtual_id(blockIdx.x, G);
+        if constexpr (MOST_CUT > 0)
+            if (it > 0 || MODE == 2) cut = MOST_CUT > 1 && here * 4 <= G ? 2 : here * 2 <= G ? 1 : 0;
+        const int pieces = here << cut;
+        if ((int)blockIdx.x >= pieces) return -1;
+        const int v = xcd_virtual_id(blockIdx.x, pieces);
+        part = v - (v >> cut << cut);
+        return first + (v >> cut);
+    };
+    auto take_part = [&](Tile& t, int part, int cut) -> bool {       // false: no columns in it
+        if constexpr (MOST_CUT > 0) {
+            if (cut > 0) {
+                t.n0 += part * (BN >> cut);
+                if (t.n0 >= p.n) { t.valid = 0; return false; }
+                if (t.n0 + (BN >> cut) < p.n) t.n_hi = t.n0 + (BN >> cut);
+            }
+        }
+        return true;
+    };
     [[maybe_unused]] const int sk_self = xcd_virtual_id(blockIdx.x, gridDim.x);
     auto pick_tile = [&](int it) -> Tile {
         Tile t;
-        t.valid = 0; t.m0 = 0; t.n0 = 0; t.kb_begin = 0; t.kb_end = 0; t.split_z = 0; t.row_lo = 0; t.row_hi = p.m;
+        t.valid = 0; t.m0 = 0; t.n0 = 0; t.n_hi = p.n; t.kb_begin = 0; t.kb_end = 0; t.split_z = 0; t.row_lo = 0; t.row_hi = p.m;
         t.sk_contrib = 0; t.sk_first = -1;
         t.bptr = p.b; t.bsptr = p.bs;
         const int G = gridDim.x;
@@ -369,8 +400,9 @@ void gemm_tr_kernel(const GemmArgs p) {
             // tiles that read the same panel of the expert's weights.
             const int tiles_n = (p.n + BN - 1) / BN;
             const int total = total_slots * tiles_n;
-            int v = it * G + xcd_virtual_id(blockIdx.x, G);
-            if (v >= total * (MODE == 5 ? p.split_k : 1)) return t;
+            int part = 0, cut = 0;
+            int v = place(it, total * (MODE == 5 ? p.split_k : 1), part, cut);
+            if (v < 0) return t;
             if (MODE == 5) {                           // partition by partition; the tile's number: its counter and its slots
                 t.split_z = __builtin_amdgcn_readfirstlane(v / total);
                 v -= t.split_z * total;
@@ -420,6 +452,7 @@ void gemm_tr_kernel(const GemmArgs p) {
             if (!found) return t;                      // uniform for the whole workgroup
             t.valid = 1;
             t.m0 = start; t.n0 = tn * BN;
+            if (!take_part(t, part, cut)) return t;
             t.row_lo = cnt_lo; t.row_hi = cnt_hi;
             t.bptr = p.b + (size_t)e * (size_t)p.k * (size_t)p.n;
             t.bsptr = p.bs + (size_t)e * (size_t)(p.k / KBLK) * (size_t)p.nb;
@@ -429,19 +462,16 @@ void gemm_tr_kernel(const GemmArgs p) {
         } else {
             const int tiles_m = (p.m + BM - 1) / BM, tiles_n = (p.n + BN - 1) / BN;
             const int per_split = tiles_m * tiles_n, total = per_split * p.split_k;
-            // the gridDim.x tiles in flight together: every XCD takes a contiguous run of them
-            const int first = it * G;
-            const int here = total - first < G ? total - first : G;
-            if (here <= 0) return t;
-            const int v = first + xcd_virtual_id(blockIdx.x, G);
-            if (v >= total) return t;
-            (void)here;
+            int part = 0, cut = 0;
+            const int v = place(it, total, part, cut);
+            if (v < 0) return t;
             t.valid = 1;
             t.split_z = v / per_split;
             int tm, tn;
             band_tile(v - t.split_z * per_split, tiles_m, tiles_n, p.band_h, tm, tn);
             if (MODE == 4) t.sk_first = v - t.split_z * per_split;        // the tile's number: its counter and its slots
             t.m0 = tm * BM; t.n0 = tn * BN;
+            if (!take_part(t, part, cut)) return t;
             const int kbt = p.k / KBLK;
             t.kb_begin = t.split_z * p.kb_per_split;
             t.kb_end = t.kb_begin + p.kb_per_split;
@@ -514,7 +544,7 @@ void gemm_tr_kernel(const GemmArgs p) {
         }
         krow = P / C::CPR_B; ch = stored_to_chunk<C::CPR_B>(P % C::CPR_B, swz_of_krow<C::CPR_B>(krow));
         col = t.n0 + 16 * ch;
-        const bool skip_b = col >= p.n && b_bytes < 0x80000000u;      // columns beyond the matrix: not fetched either
+        const bool skip_b = col >= t.n_hi && b_bytes < 0x80000000u;   // columns beyond the matrix, or of another part of the tile: not fetched either
         col = col < p.n ? col : t.n0;
         c.b_voff = skip_b ? b_bytes : (uint32_t)krow * (uint32_t)p.n + (uint32_t)col;
 #pragma unroll
@@ -672,7 +702,7 @@ void gemm_tr_kernel(const GemmArgs p) {
     // copy of the a_scale row.
     // does any element of this wave's tile get stored?  (rows of the expert / matrix, columns of the matrix)
     const bool wave_active = __builtin_amdgcn_readfirstlane((m0 + wave_m * WM < row_hi && m0 + wave_m * WM + WM > row_lo &&
-                                                             n0 + wave_n * WN < p.n) ? 1 : 0) != 0;
+                                                             n0 + wave_n * WN < cur.n_hi) ? 1 : 0) != 0;
     // b_scale of the wave's n tiles: slot bs_off for n tiles [0, ub), the next slot for [ub, NT)
     const int wave_col = (BN % 128 != 0 ? (n0 & 127) : 0) + wave_n * WN;               // from the start of the tile's first n block
     const int bs_off = bs_base + (wave_col >> 7) * 4;
@@ -728,6 +758,9 @@ void gemm_tr_kernel(const GemmArgs p) {
         // where two ways lead into the loop the compiler takes the lower number.  (Read at the block's start, the scales were
         // the youngest, and the first MFMA waited for every read there was: 1024 x 1536 x 7168 unsplit, us, 128x128 in eight waves
         // 30.0 -> 29.3, in four 39.8 -> 38.1, 256x128 46.3 -> 44.3, 64x256 33.3 -> 33.5; 2048 x 2048 x 2048 17.7 -> 17.1 in 256x128.)
+        // (Not with waves of 24 tiles and more, whose registers are full: 1000 tokens to 4 of 32 experts, 4096 x 2048, 70.0 us as it is, 73.5
+        // ahead in 256x256; 1024 x 1536 x 7168 59.6 and 60.1 in 256x192.)
+        constexpr bool SCALES_AHEAD = STEPS < 24;
         v8i areg[C::MT], breg[2];
         float asv[C::MT], bsv, bsv1;
         auto read_scales = [&](const unsigned char* sb) {
@@ -738,7 +771,7 @@ void gemm_tr_kernel(const GemmArgs p) {
             __builtin_amdgcn_sched_barrier(0);
         };
         if (wave_active) {
-            read_scales(lds);
+            if (SCALES_AHEAD) read_scales(lds);
             read_a(areg[0], 0, lds);
             __builtin_amdgcn_sched_barrier(0);
             read_b(breg[0], 0, lds);
@@ -795,6 +828,7 @@ void gemm_tr_kernel(const GemmArgs p) {
             float sc[C::MT], sc1[C::MT];
             // the step that works out the block's scales: the one that folds first, but before the next block's are read
             constexpr int BARRIER_STEP = STEPS - C::MT, SCALE_STEP = LAG < BARRIER_STEP ? LAG : BARRIER_STEP - 1;
+            if constexpr (!SCALES_AHEAD) read_scales(sbase);
             v4f ring[RING];
             auto step = [&](auto s_tag) {
                 constexpr int s = decltype(s_tag)::value;
@@ -817,7 +851,7 @@ void gemm_tr_kernel(const GemmArgs p) {
                         wait_next_block();
                         if constexpr (TAILS && LANDS_LAST) patch(next_stage);
                         __syncthreads();
-                        if constexpr (HAS_NEXT) read_scales(snext);
+                        if constexpr (HAS_NEXT && SCALES_AHEAD) read_scales(snext);
                     }
                     const v4f z = {0.f, 0.f, 0.f, 0.f};
                     ring[s % RING] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(breg[u & 1], areg[t], z, 0, 0, 0, 0, 0, 0);
@@ -1271,7 +1305,7 @@ void gemm_tr_kernel(const GemmArgs p) {
         constexpr int RSTRIDE = ROW_POW2 ? WNO * 2 : WNO * 2 + 16;    // bytes from row to row in the staging area
         static_assert(C::MT % EPI_PARTS == 0 && C::NWAVES * HALF_ROWS * RSTRIDE <= C::STAGE_BYTES, "output staging must fit one stage");
         unsigned char* region = lds + (NSTAGE - 1) * C::STAGE_BYTES + wave * (HALF_ROWS * RSTRIDE);
-        const int ldc = EPI == 1 ? p.n / 2 : p.n;
+        const int ldc = EPI == 1 ? p.n / 2 : p.n, col_hi = EPI == 1 ? cur.n_hi / 2 : cur.n_hi;
         // Stores go through buffer descriptors: an offset of 0xFFFFFFFF drops the lane's store, so the
         // instruction count does not depend on the data.  Each store gets a descriptor based at the first
         // element of its group of rows (scalar arithmetic only); the scalar-offset operand is not used:
@@ -1333,7 +1367,7 @@ void gemm_tr_kernel(const GemmArgs p) {
             const int lane_r = lane / ROW_CHUNKS, lane_chunk = lane % ROW_CHUNKS;
             const bool lane_live = ROW_POW2 || lane_r < ROWS_PER_PASS;
             const int wave_row0 = wave_m * WM, wave_col0 = wave_n * WNO;              // inside the tile, output columns
-            const bool col_ok = lane_live && col0 + wave_col0 + lane_chunk * 8 < ldc;
+            const bool col_ok = lane_live && col0 + wave_col0 + lane_chunk * 8 < col_hi;
             [[maybe_unused]] const bool row_ends = (ldc & 7) != 0 && col0 + wave_col0 + WNO > ldc;      // the wave's tile holds rows' last, partial chunks
             const uint32_t lane_off = ((uint32_t)(wave_row0 + lane_r) * (uint32_t)ldc + (uint32_t)(wave_col0 + lane_chunk * 8)) * 2u;
 #pragma unroll
