@@ -153,20 +153,36 @@ def pycall():
     return _pycall
 
 
+_native = False
 _dense = False
+_NATIVE = ("dense", "quantize", "experts", "topk", "route", "combine")
+
+
+def native():
+    """The entry points' checks and calls on torch tensors (csrc/fp8bs_torch.cpp), or None where the module has not been built, cannot
+    be imported, was built against another torch or lacks some of them (one warning)."""
+    global _native
+    if _native is False:
+        import torch
+        mod = _extension("_fp8bs_torch")
+        why = None
+        if mod is not None and mod.torch_version != torch.__version__:
+            why = "was built against torch %s" % mod.torch_version
+        elif mod is not None and not all(hasattr(mod, name) for name in _NATIVE):
+            why = "is older than this file"
+        if why:
+            import warnings
+            warnings.warn("_fp8bs_torch.so %s; going without it, which costs host time in every call" % why)
+            mod = None
+        _native = mod
+    return _native
 
 
 def dense():
-    """custom_kernel's checks and call on torch tensors (csrc/fp8bs_torch.cpp's dense), or None where the module has not been
-    built, cannot be imported, or was built against another torch (one warning)."""
+    """custom_kernel's checks and call in native code, or None without that module."""
     global _dense
     if _dense is False:
-        import torch
-        mod = _extension("_fp8bs_torch")
-        if mod is not None and mod.torch_version != torch.__version__:
-            import warnings
-            warnings.warn("_fp8bs_torch.so was built against torch %s; going without it, which costs host time in every call" % mod.torch_version)
-            mod = None
+        mod = native()
         _dense = mod.dense if mod is not None else None
     return _dense
 

@@ -11,7 +11,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
-from .submission import _PLANS_MAX, _call, _check_operands, _experts_kmajor, _grouped_workspace, _is_kmajor, _plan_cache, _stream_ptr, _workspace
+from .submission import _PLANS_MAX, _call, _check_operands, _experts_kmajor, _experts_native, _grouped_workspace, _is_kmajor, _plan_cache, _remember, _stream_ptr, _workspace
 
 
 _route_ws = {}     # (device index, stream) -> uint8 tensor: the routing kernels' scratch, grown on demand, reused across
@@ -21,6 +21,13 @@ _route_ws = {}     # (device index, stream) -> uint8 tensor: the routing kernels
 def topk(scores: torch.Tensor, k: int, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """scores fp32 [T, E] row-major on the GPU -> int32 [T, k], best first, lowest index first among equals.
     ``out`` (contiguous int32 [T, k] on the same GPU) is filled and returned if given: no allocation."""
+    native = _lib.native() if out is None else None
+    if native is not None:
+        got = native.topk(scores, k)
+        if type(got) is int:
+            _lib.check(got)
+        if got is not None:
+            return got
     if scores.dtype != torch.float32 or scores.dim() != 2 or not scores.is_cuda or not scores.is_contiguous():
         raise ValueError("scores must be a contiguous float32 [tokens, experts] tensor on the GPU")
     t, e = scores.shape
@@ -46,6 +53,19 @@ def route(top_idx: torch.Tensor, experts: int, out: Optional[Tuple[torch.Tensor,
         raise ValueError("top_idx must be a contiguous int32 [tokens, topk] tensor on the GPU")
     t, k = top_idx.shape
     dev = top_idx.device
+    need = _plan_cache.get(("route", t, experts))
+    if need is None:
+        if len(_plan_cache) >= _PLANS_MAX:
+            _plan_cache.clear()
+        need = _plan_cache[("route", t, experts)] = _lib.load().fp8bs_moe_route_workspace_bytes(t, experts)
+    ws = _workspace(dev, need, _stream_ptr(dev), _route_ws, 4096)
+    native = _lib.native() if out is None else None
+    if native is not None:
+        got = native.route(top_idx, experts, ws.data_ptr(), ws.numel())
+        if type(got) is int:
+            _lib.check(got)
+        if got is not None:
+            return got
     if out is None:
         row_offsets = torch.empty(experts + 1, dtype=torch.int32, device=dev)
         row_map = torch.empty(t * k, dtype=torch.int32, device=dev)
@@ -55,12 +75,6 @@ def route(top_idx: torch.Tensor, experts: int, out: Optional[Tuple[torch.Tensor,
         for name, x, shape in (("row_offsets", row_offsets, (experts + 1,)), ("row_map", row_map, (t * k,)), ("slot_of", slot_of, (t, k))):
             if x.dtype != torch.int32 or tuple(x.shape) != shape or x.device != dev or not x.is_contiguous():
                 raise ValueError("out: %s must be a contiguous int32 tensor of shape %s on top_idx's device" % (name, shape))
-    need = _plan_cache.get(("route", t, experts))
-    if need is None:
-        if len(_plan_cache) >= _PLANS_MAX:
-            _plan_cache.clear()
-        need = _plan_cache[("route", t, experts)] = _lib.load().fp8bs_moe_route_workspace_bytes(t, experts)
-    ws = _workspace(dev, need, _stream_ptr(dev), _route_ws, 4096)
     _call(_lib.calls().moe_route, dev, top_idx.data_ptr(), t, experts, k, row_offsets.data_ptr(), row_map.data_ptr(),
           slot_of.data_ptr(), ws.data_ptr(), ws.numel())
     return row_offsets, row_map, slot_of
@@ -75,6 +89,8 @@ def gate_up_silu(data):
     2-amd-moe/5-amd-fp8-moe-hip-fuse.py:366-408.  Fills and returns ``h``.
     A call that splits K keeps its workspace (grouped: up to 64 MiB) for this device and stream, the one `custom_kernel` uses.
     """
+    if _experts_native(data, True):
+        return data[5]
     a, b, a_scale, b_scale, row_offsets, h = data
     if a.dim() != 2:
         raise ValueError("a must be a [rows, k] tensor")
@@ -104,6 +120,7 @@ def gate_up_silu(data):
     dev = a.device
     if grouped:
         ws_ptr, ws_len = _grouped_workspace(dev, _stream_ptr(dev), num_experts, rows, n, k)
+        _remember(True, num_experts, rows, n, k, _plan_cache.get(("grouped", num_experts, rows, n, k)))
     else:
         need = _plan_cache.get(("silu", rows, n, k))
         if need is None:
@@ -113,6 +130,7 @@ def gate_up_silu(data):
                 need = _plan_cache[("silu", rows, n, k)] = int(_lib.load().fp8bs_silu_mul_workspace_bytes(rows, n, k))
         ws = _workspace(dev, need, _stream_ptr(dev)) if need else None
         ws_ptr, ws_len = (ws.data_ptr(), ws.numel()) if need else (None, 0)
+        _remember(True, 0, rows, n, k, need)
     _call(_lib.calls().gemm_silu_mul_ws, dev, a.data_ptr(), b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(), h.data_ptr(),
           row_offsets.data_ptr() if grouped else None, num_experts, rows, n, k, 0, 0, ws_ptr, ws_len)
     return h
@@ -123,6 +141,13 @@ def combine(y: torch.Tensor, slot_of: torch.Tensor, weights: torch.Tensor) -> to
 
     Role of pack_output (2-amd-moe/amd-moe-submission.py:239-301); fp32 accumulation in the order of j.
     """
+    native = _lib.native()
+    if native is not None:
+        got = native.combine(y, slot_of, weights)
+        if type(got) is int:
+            _lib.check(got)
+        if got is not None:
+            return got
     if y.dtype != torch.bfloat16 or y.dim() != 2 or not y.is_contiguous() or not y.is_cuda:
         raise ValueError("y must be a contiguous bfloat16 [rows, d] tensor on the GPU")
     if slot_of.dtype != torch.int32 or not slot_of.is_contiguous() or weights.dtype != torch.float32 \

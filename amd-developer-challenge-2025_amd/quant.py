@@ -33,6 +33,15 @@ def _k_major(rows: int, k: int, dtype: torch.dtype, device: torch.device) -> tor
     return torch.empty_strided((rows, k), (1, rows or 1), dtype=dtype, device=device)
 
 
+def _native_quantize(x, row_map, of_b: bool):
+    """The native call's result, or None where it does not take this one."""
+    native = _lib.native()
+    out = native.quantize(x, row_map, of_b) if native is not None else None
+    if type(out) is int:
+        _lib.check(out)
+    return out
+
+
 def _quantise_then_gather(dtype: torch.dtype, t: int, m: int, k: int, row_map: torch.Tensor) -> bool:
     """Whether two kernels are faster than one for m gathered rows of t tokens, by measurement (us, one / two): where rows repeat
     often, the output is large and ``gather_a`` has a fast path that keeps 8 or 16 k rows of the source in LDS (T and M multiples
@@ -62,6 +71,10 @@ def quantize_a(x: torch.Tensor, row_map: Optional[torch.Tensor] = None, fused: O
     quantiser (one kernel), or every token quantised once and the bytes gathered by ``gather_a`` (two kernels), see
     ``_quantise_then_gather``.  ``fused`` = True / False forces the one-kernel / two-kernel route.
     """
+    if row_map is None and fused is None:
+        out = _native_quantize(x, None, False)
+        if out is not None:
+            return out
     _check_input(x, "x")
     t, k = x.shape
     if row_map is not None:
@@ -72,6 +85,9 @@ def quantize_a(x: torch.Tensor, row_map: Optional[torch.Tensor] = None, fused: O
             fused = not _quantise_then_gather(x.dtype, t, m, k, row_map)
         if not fused:
             return gather_a(*quantize_a(x), row_map)
+        out = _native_quantize(x, row_map, False)
+        if out is not None:
+            return out
     else:
         m = t
     dev = x.device
@@ -83,6 +99,9 @@ def quantize_a(x: torch.Tensor, row_map: Optional[torch.Tensor] = None, fused: O
 
 def quantize_b(w: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """w [N, K] -> (b e4m3fn [N, K] stride (1, N), b_scale fp32 [ceil(N/128), K/128] stride (1, NB))."""
+    out = _native_quantize(w, None, True)
+    if out is not None:
+        return out
     _check_input(w, "w")
     n, k = w.shape
     dev = w.device

@@ -98,6 +98,31 @@ _PLANS_MAX = 4096
 # themselves at every call; what it is told here is a fact about the sizes alone.
 _CHECKED_MAX = 64
 _checked = {}      # (m, n, k) -> bytes
+_checked_experts = {}      # the same for grouped_kernel and gate_up_silu: (silu, experts or 0, rows, n, k) -> bytes
+
+
+def _remember(silu: bool, experts: int, rows: int, n: int, k: int, need) -> None:
+    """Sizes that the native call may take from now on; called where the Python path has checked a call of them."""
+    key = (int(silu), experts, rows, n, k)
+    if need is not None and key not in _checked_experts:
+        if len(_checked_experts) >= _CHECKED_MAX:
+            _checked_experts.clear()
+        _checked_experts[key] = need
+
+
+def _experts_native(data, silu: bool) -> bool:
+    """grouped_kernel's and gate_up_silu's checks and call in native code: whether it took the call."""
+    native = _lib.native()
+    if native is None:
+        return False
+    st = native.experts(data, _checked_experts, 0, 0, silu)
+    if st < -1:                                   # all is well, and it wants a workspace
+        dev = data[0].device
+        ws = _workspace(dev, -st, _stream_ptr(dev))
+        st = native.experts(data, _checked_experts, ws.data_ptr(), ws.numel(), silu)
+    if st > 0:
+        _lib.check(st)
+    return st == 0
 
 
 def _grouped_workspace(device, stream, num_experts, rows, n, k):
@@ -254,6 +279,8 @@ def grouped_kernel(data, variant: int = 0):
     [E, ceil(n/128), k/128] with stride (nb*kb, 1, nb).  Fills and returns ``c``; no host sync.
     A call that splits K keeps a workspace of up to 64 MiB for this device and stream (the one `custom_kernel` uses).
     """
+    if variant == 0 and _experts_native(data, False):
+        return data[5]
     a, b, a_scale, b_scale, row_offsets, c = data
     rows, k = a.shape
     if b.dim() != 3:
@@ -269,6 +296,8 @@ def grouped_kernel(data, variant: int = 0):
         raise ValueError("row_offsets must be an int32 tensor with num_experts+1 entries on the operands' GPU")
     dev = a.device
     ws_ptr, ws_len = _grouped_workspace(dev, _stream_ptr(dev), num_experts, rows, n, k) if variant == 0 else (None, 0)
+    if variant == 0:
+        _remember(False, num_experts, rows, n, k, _plan_cache.get(("grouped", num_experts, rows, n, k)))
     _call(_lib.calls().gemm_grouped_ws, dev, a.data_ptr(), b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(), c.data_ptr(),
           row_offsets.data_ptr(), num_experts, rows, n, k, variant, 0, ws_ptr, ws_len)
     return c

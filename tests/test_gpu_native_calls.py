@@ -1,0 +1,118 @@
+"""The native calls of the quantisers, routing, combine and the experts' products (csrc/fp8bs_torch.cpp) against the Python paths, over
+the forms of arguments that both see: what one accepts the other accepts with the same bits, layout and type, what one refuses the
+other refuses with the same type of exception."""
+import importlib
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+pkg_name = "amd-developer-challenge-2025_amd"
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+def _lib():
+    return importlib.import_module(pkg_name + "._lib")
+
+
+def _outcome(monkeypatch, native, fn):
+    monkeypatch.setattr(_lib(), "_native", native)
+    try:
+        out = fn()
+    except Exception as ex:
+        return type(ex)
+    out = out if isinstance(out, tuple) else (out,)
+    return [(tuple(t.shape), t.stride(), t.dtype, t.device, t.requires_grad, t.detach().as_subclass(torch.Tensor).cpu().flatten().clone().view(torch.uint8)) for t in out]
+
+
+def _same(monkeypatch, what, fn, counts=None):
+    native = _lib().native()
+    assert native is not None, "build() builds it"
+    want, got = _outcome(monkeypatch, None, fn), _outcome(monkeypatch, native, fn)
+    monkeypatch.setattr(_lib(), "_native", native)
+    if isinstance(want, type) or isinstance(got, type):
+        assert want is got, (what, want, got)
+        return
+    for w, g in zip(want, got, strict=True):
+        assert w[:5] == g[:5] and torch.equal(w[5], g[5]), (what, w[:5], g[:5])
+
+
+MATRICES = {
+    "bf16": lambda x: x.bfloat16(), "fp32": lambda x: x, "half": lambda x: x.half(), "rows apart": lambda x: torch.cat([x, x], 1)[:, :x.shape[1]],
+    "one row": lambda x: x[:1], "no rows": lambda x: x[:0], "transposed": lambda x: x.t().contiguous().t(), "every other column": lambda x: torch.cat([x, x], 1)[:, ::2],
+    "one row expanded": lambda x: x[:1].expand(x.shape[0], x.shape[1]), "k off the blocks": lambda x: x[:, :-1], "3-D": lambda x: x[None], "on the CPU": lambda x: x.cpu(),
+    "subclass": lambda x: x.as_subclass(_Sub), "parameter": lambda x: torch.nn.Parameter(x), "wants a gradient": lambda x: x.clone().requires_grad_(),
+    "off by an element": lambda x: torch.cat([x.reshape(-1)[:1], x.reshape(-1)])[1:].view(x.shape), "none": lambda x: None,
+}
+
+
+@pytest.mark.parametrize("rows,k", [(1, 128), (7, 256), (300, 512)])
+def test_quantisers(pkg, monkeypatch, rows, k):
+    quant = importlib.import_module(pkg_name + ".quant")
+    x = torch.randn(rows, k, device="cuda:0")
+    maps = {"none": None, "map": torch.randint(0, rows, (2 * rows + 1,), dtype=torch.int32, device="cuda:0"), "empty": torch.empty(0, dtype=torch.int32, device="cuda:0"),
+            "long": torch.zeros(4, dtype=torch.int64, device="cuda:0"), "2-D": torch.zeros(2, 2, dtype=torch.int32, device="cuda:0"), "on the CPU": torch.zeros(4, dtype=torch.int32),
+            "apart": torch.zeros(8, dtype=torch.int32, device="cuda:0")[::2]}
+    for name, form in MATRICES.items():
+        y = form(x)
+        _same(monkeypatch, name, lambda: quant.quantize_b(y))
+        for which, row_map in maps.items():
+            _same(monkeypatch, (name, which), lambda: quant.quantize_a(y, row_map))
+
+
+def test_routing_and_combine(pkg, monkeypatch):
+    moe = importlib.import_module(pkg_name + ".moe")
+    scores = torch.randn(37, 16, device="cuda:0")
+    for name, form in MATRICES.items():
+        for k in (1, 4, 16, 17, 0, -1, True, 2.0):
+            _same(monkeypatch, (name, k), lambda: moe.topk(form(scores), k))
+    top = moe.topk(scores, 4)
+    for name, t in {"plain": top, "long": top.long(), "rows apart": torch.cat([top, top], 1)[:, :4], "none of it": top[:0], "subclass": top.as_subclass(_Sub), "on the CPU": top.cpu()}.items():
+        for experts in (16, 20, 3, 0, -2):
+            _same(monkeypatch, (name, experts), lambda: moe.route(t, experts))
+    _, row_map, slot_of = moe.route(top, 16)
+    y, w = torch.randn(row_map.numel(), 520, device="cuda:0").bfloat16(), torch.rand(37, 4, device="cuda:0")
+    forms = {"plain": (y, slot_of, w), "float": (y.float(), slot_of, w), "narrow": (y[:, :256], slot_of, w), "half weights": (y, slot_of, w.half()), "short": (y, slot_of[:-1], w),
+             "fewer": (y, slot_of[:, :2].contiguous(), w[:, :2].contiguous()), "no tokens": (y, slot_of[:0], w[:0]), "subclass": (y.as_subclass(_Sub), slot_of, w), "on the CPU": (y, slot_of.cpu(), w)}
+    for name, f in forms.items():
+        _same(monkeypatch, name, lambda: moe.combine(*f))
+
+
+@pytest.mark.parametrize("silu", [False, True])
+@pytest.mark.parametrize("n,k,grouped", [(256, 512, True), (130, 128, True), (256, 512, False), (8192, 7168, False)])
+def test_products(pkg, monkeypatch, silu, n, k, grouped):
+    moe = importlib.import_module(pkg_name + ".moe")
+    dev, rows, experts = torch.device("cuda:0"), 96, 3
+    f8 = lambda *s: torch.randn(*s, device=dev).to(torch.float8_e4m3fn)
+    a, a_scale = f8(k, rows).t(), torch.rand(k // 128, rows, device=dev).t() + 0.5
+    a_scale = a_scale.t().contiguous().t()
+    e = (experts,) if grouped else ()
+    b, b_scale = f8(*e, k, n).transpose(-1, -2), torch.rand(*e, k // 128, (n + 127) // 128, device=dev).transpose(-1, -2)
+    offsets = torch.tensor([0, 20, 20, 96], dtype=torch.int32, device=dev) if grouped else None
+    plain = [a, b, a_scale, b_scale, offsets, None]
+
+    def form(i, change):
+        d = list(plain)
+        d[i] = change(d[i])
+        return d
+
+    cols = n // 2 if silu else n
+    forms = {"plain": plain, "a row-major": form(0, lambda t: t.contiguous()), "b row-major": form(1, lambda t: t.contiguous()), "a bytes": form(0, lambda t: t.view(torch.uint8)),
+             "b_scale short": form(3, lambda t: t[..., :-1]), "a_scale half": form(2, lambda t: t.half()), "subclass": form(2, lambda t: t.as_subclass(_Sub)), "five": plain[:5],
+             "b on the CPU": form(1, lambda t: t.cpu()), "b 4-D": form(1, lambda t: t[None])}
+    if grouped:
+        forms.update({"offsets long": form(4, lambda t: t.long()), "offsets short": form(4, lambda t: t[:-1]), "offsets on the CPU": form(4, lambda t: t.cpu()),
+                      "offsets apart": form(4, lambda t: torch.stack([t, t], 1)[:, 0]), "one expert less": form(1, lambda t: t[:-1])})
+    for name, d in forms.items():
+        for wide in (cols, cols + 1):
+            for as_list in (False, True):
+                def call():
+                    c = torch.full((rows, wide), float("nan"), dtype=torch.bfloat16, device=dev)
+                    data = (list if as_list else tuple)(d[:5] + [c]) if len(d) == 6 else tuple(d)
+                    out = moe.gate_up_silu(data) if silu else pkg.grouped_kernel(data)
+                    assert out is c
+                    return out
+                _same(monkeypatch, (name, wide, as_list), call)
