@@ -88,12 +88,18 @@ __device__ __forceinline__ int xcd_virtual_id(int wg, int total) {
 }
 
 __device__ __forceinline__ void band_tile(int v, int tiles_m, int tiles_n, int gh, int& tm, int& tn) {
-    int per_band = gh * tiles_n;
-    int band = v / per_band;
-    int rem = v - band * per_band;
+    // (divisions only where they are needed: each is some 25 dependent instructions ahead of a kernel's first copies; 27 x 1408 x 1280 3.85
+    // -> 3.73 us, 128 x 6080 x 896 5.10 -> 4.90, 64 x 6614 x 1152 6.26 -> 6.09, 111 dense products 0.988 in the geometric mean)
+    int band = 0, rem = v;
+    if (tiles_m > gh) {
+        const int per_band = gh * tiles_n;
+        band = v / per_band;
+        rem = v - band * per_band;
+    }
     int rows = tiles_m - band * gh;           // rows in this band (last band may be short)
     rows = rows < gh ? rows : gh;
-    tn = rem / rows;
+    if ((rows & (rows - 1)) == 0) tn = rem >> __builtin_ctz(rows);
+    else tn = rem / rows;
     tm = band * gh + (rem - tn * rows);
 }
 
@@ -496,7 +502,7 @@ void gemm_tr_kernel(const GemmArgs p) {
             const int v = place(it, total, part, cut);
             if (v < 0) return t;
             t.valid = 1;
-            t.split_z = v / per_split;
+            if (MODE != 0) t.split_z = v / per_split;
             int tm, tn;
             band_tile(v - t.split_z * per_split, tiles_m, tiles_n, p.band_h, tm, tn);
             if (MODE == 4) t.sk_first = v - t.split_z * per_split;        // the tile's number: its counter and its slots
@@ -690,7 +696,7 @@ void gemm_tr_kernel(const GemmArgs p) {
     // workgroup whose tile holds those bytes writes them into LDS itself once the last K block has
     // landed: they all lie in the last aligned dword of a.  The same holds for b with n % 4 != 0.
     // Each is written by the wave whose copy brought the bytes around it, between its wait for the copy and the barrier that
-    // publishes the block: lane l < 6 of every wave has one candidate, a's for l < 3, in patch_at and patch_byte, worked out at a tile's
+    // publishes the block: lane l < 6 of every wave has one candidate, a's for l < 3, in patch_at, worked out at a tile's
     // start while the first copies are on their way; a lane whose candidate is not lost, not in the tile or another
     // wave's writes to a byte of the stage that nobody reads.  So the store has no condition: a branch at this place, in the middle of
     // a K block's step sequence, makes the compiler move the folds of the MFMAs before it below it, which costs some thirty registers.
@@ -700,8 +706,8 @@ void gemm_tr_kernel(const GemmArgs p) {
     // 64x64 4.2 -> 3.5; 45 products on five tiles 0.88 of the time in the geometric mean.)
     const bool a_tail = TAILS && (p.lda & 3) != 0 && p.k > 0;
     const bool b_tail = TAILS && (p.n & 3) != 0 && p.k > 0;
-    [[maybe_unused]] int patch_at = 0;
-    [[maybe_unused]] uint32_t patch_byte = 0;
+    [[maybe_unused]] uint32_t patch_at = 0;                       // bits 0-23: the place in the stage, bits 24-31: the byte
+    static_assert(C::STAGE_BYTES <= 1 << 24);
     [[maybe_unused]] auto plan_patch = [&](const Tile& t) {
         const bool of_b = lane >= 3;
         const uint32_t back = 3u - (uint32_t)(of_b ? lane - 3 : lane) % 3u;
@@ -716,11 +722,11 @@ void gemm_tr_kernel(const GemmArgs p) {
         uint32_t a_last = 0, b_last = 0;
         if (a_tail) a_last = load_last_dword(p.a + a_bytes);
         if (b_tail) b_last = load_last_dword(t.bptr + b_bytes);                         // grouped: every expert's matrix has last bytes of its own
-        patch_byte = (of_b ? b_last : a_last) >> (8u * (4u - back));
-        patch_at = mine ? (of_b ? C::A_BYTES : 0) + slot * 16 + (xt & 15) : C::STAGE_BYTES - 1;
+        const uint32_t byte = (of_b ? b_last : a_last) >> (8u * (4u - back));
+        patch_at = (uint32_t)(mine ? (of_b ? C::A_BYTES : 0) + slot * 16 + (xt & 15) : C::STAGE_BYTES - 1) | byte << 24;
     };
     // stage: the tile's last K block, which this wave's copies have just reached
-    [[maybe_unused]] auto patch = [&](int stage) { *(volatile unsigned char*)(lds + stage * C::STAGE_BYTES + patch_at) = (unsigned char)patch_byte; };
+    [[maybe_unused]] auto patch = [&](int stage) { *(volatile unsigned char*)(lds + stage * C::STAGE_BYTES + (patch_at & 0xFFFFFFu)) = (unsigned char)(patch_at >> 24); };
 
     bool stores_behind = false;             // ... and this wave's output stores of the previous tile were issued after it
     for (int it = 0;; it++) {
@@ -1050,6 +1056,8 @@ void gemm_tr_kernel(const GemmArgs p) {
         auto piece = [&](int x) -> uint32_t {               // x = t * NT + u, a compile-time number at every use
             return ((rows_in >> (x / C::NT)) & (cols_in >> (x % C::NT)) & 1u) ? voff + (uint32_t)x * 1024u : 0xFFFFFFFFu;
         };
+        // (keeps the offsets of all pieces from being worked out ahead of the branches and held in registers)
+        [[maybe_unused]] auto here = [](uint32_t& rows, uint32_t& cols) { asm volatile("" : "+v"(rows), "+v"(cols)); };
         auto slot_of = [&](int z) { return __builtin_amdgcn_make_buffer_rsrc((void*)(tile_slots + (size_t)z * SLOT_BYTES), 0, SLOT_BYTES, 0x00020000); };
         if constexpr (SHARED_SUM) {
             // The sum is shared out: of every wave's accumulators partition z adds the z-th S-th part and writes that part of c,
@@ -1073,8 +1081,6 @@ void gemm_tr_kernel(const GemmArgs p) {
                 constexpr uint32_t ALL = (1u << S) - 1u;
                 unsigned long long* const flags = counters + sk_first * S;
                 const uint32_t mine = 1u << split_z;
-                // (keeps the offsets of all pieces from being worked out ahead of the branches and held in registers)
-                auto here = [](uint32_t& rows, uint32_t& cols) { asm volatile("" : "+v"(rows), "+v"(cols)); };
                 auto store_parts = [&](uint32_t parts) {
                     const __amdgpu_buffer_rsrc_t rs = slot_of(split_z);
                     here(rows_in, cols_in);
@@ -1198,6 +1204,7 @@ void gemm_tr_kernel(const GemmArgs p) {
                 constexpr int WANT = S > 1 ? (16 / (S - 1) > 0 ? 16 / (S - 1) : 1) : 4;
                 constexpr int BATCH = WANT >= NG ? NG : (WANT >= 4 && NG % 4 == 0 ? 4 : (WANT >= 3 && NG % 3 == 0 ? 3 : (WANT >= 2 && NG % 2 == 0 ? 2 : 1)));
                 const int nz = S > 0 ? S : p.split_k;
+                here(rows_in, cols_in);
 #pragma unroll
                 for (int base = 0; base < NG; base += BATCH) {
                     if constexpr (S > 0) {
