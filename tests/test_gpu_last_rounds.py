@@ -1,0 +1,58 @@
+"""Rounds of tiles that do not fill the chip: dealt to all XCDs, and tiles of 256 columns cut in two or four by columns where they
+leave half of it, or three quarters, idle (fp8bs_tiled.h, `place` and `take_part`); and the grouped walk with its table in
+registers (up to 64 experts), in LDS, and past that.
+
+The operands are small whole numbers and the scales powers of two that differ from block to block of columns, so every output is
+exact in float32 and the comparison is of bits; c starts as NaN, so that a part left out shows.
+"""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+FORM = lambda variant, form: variant | (form + 1) << 8           # FP8BS_VARIANT_FORM
+K = 256
+
+
+def _codes(gen, *shape):
+    values = torch.tensor([0x00, 0x38, 0xB8, 0x40], dtype=torch.uint8, device="cuda:0")          # 0, 1, -1, 2
+    return values[torch.randint(4, shape, generator=gen, device="cuda:0")].view(torch.float8_e4m3fn)
+
+
+def _column_scales(n, dev):
+    """[K/128, ceil(n/128)]: 1, 2 and 4 in turn over the blocks of columns, and their expansion to [n]."""
+    s = torch.exp2((torch.arange((n + 127) // 128, device=dev) % 3).float())
+    return s.expand(K // 128, -1).contiguous(), s.repeat_interleave(128)[:n]
+
+
+# Tiles beyond the last full round of 256 or 512 workgroups: 256x256: 324 tiles (68 left over), 320 (64), the last tile 250 or 10 columns
+# wide; 64x256: 576 (64 left over, the last tile 10 columns wide) and 648 (136).
+@pytest.mark.parametrize("tile,m,n", [(2, 4608, 4608), (2, 5111, 4090), (2, 5120, 3850), (12, 2304, 3850), (12, 2300, 4601)])
+def test_dense(pkg, tile, m, n):
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(m + n)
+    a, b = _codes(gen, K, m).t(), _codes(gen, K, n).t()
+    b_scale, columns = _column_scales(n, dev)
+    c = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=dev)
+    pkg.custom_kernel((a, b, torch.ones(K // 128, m, device=dev).t(), b_scale.t(), c), variant=tile)
+    assert torch.equal(c, (a.float() @ b.float().t().contiguous() * columns).bfloat16())
+
+
+@pytest.mark.parametrize("experts", [1, 3, 63, 64, 65, 300])
+@pytest.mark.parametrize("n", [70, 250, 266, 520])
+def test_grouped(pkg, experts, n):
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(experts * 1000 + n)
+    counts = torch.randint(0, 40, (experts,), generator=gen, device=dev).mul_(torch.rand(experts, generator=gen, device=dev) < 0.7).tolist()
+    counts[-1] += 131                                              # several tiles of one expert
+    rows = sum(counts)
+    offsets = torch.tensor([0] + counts, device=dev).cumsum(0).int()
+    a, b = _codes(gen, K, rows).t(), _codes(gen, experts, K, n).transpose(1, 2)
+    b_scale, columns = _column_scales(n, dev)
+    b_scale = b_scale.expand(experts, -1, -1).contiguous().transpose(1, 2)
+    bounds = offsets.tolist()
+    want = torch.cat([a[lo:hi].float() @ b[e].float().t().contiguous() * columns for e, (lo, hi) in enumerate(zip(bounds, bounds[1:]))]).bfloat16()
+    for tile in (0, 2, 3, 12, FORM(12, 1)):
+        c = torch.full((rows, n), float("nan"), dtype=torch.bfloat16, device=dev)
+        pkg.grouped_kernel((a, b, torch.ones(K // 128, rows, device=dev).t(), b_scale, offsets, c), variant=tile)
+        assert torch.equal(c, want), "tile %#x" % tile
