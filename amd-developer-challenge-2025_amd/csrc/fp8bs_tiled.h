@@ -188,7 +188,6 @@ __device__ __forceinline__ uint32_t load_last_dword(const uint8_t* end) {
     const uint32_t lo = *(dword)(at & ~(uintptr_t)3), hi = *(dword)((at + 3) & ~(uintptr_t)3);
     return (uint32_t)((((uint64_t)hi << 32) | lo) >> (8 * (at & 3)));
 }
-// The byte `back` = 1, 2 or 3 before the end of an operand of k rows of ld bytes.
 // The byte `back` = 1, 2 or 3 before the end of an operand of k rows of ld bytes: bit 31 = the range check cuts it off, bits 29-30 = its k row
 // minus k - 3, bits 0-28 = its row (of a) or column (of b).
 __device__ __forceinline__ uint32_t tail_candidate(uint32_t back, uint32_t ld, uint32_t k) {
