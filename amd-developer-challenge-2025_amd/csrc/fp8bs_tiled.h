@@ -790,12 +790,17 @@ void gemm_tr_kernel(const GemmArgs p) {
 
         // A block's scales are read ahead of its first operands, behind the barrier that publishes it, and the operands in the
         // order in which they are multiplied, here as in the loop: an LDS wait names how many younger reads may still be out, and
-        // where two ways lead into the loop the compiler takes the lower number.  (Read at the block's start, the scales were
-        // the youngest, and the first MFMA waited for every read there was: 1024 x 1536 x 7168 unsplit, us, 128x128 in eight waves
-        // 30.0 -> 29.3, in four 39.8 -> 38.1, 256x128 46.3 -> 44.3, 64x256 33.3 -> 33.5; 2048 x 2048 x 2048 17.7 -> 17.1 in 256x128.)
-        // (Not with waves of 24 tiles and more, whose registers are full: 1000 tokens to 4 of 32 experts, 4096 x 2048, 70.0 us as it is, 73.5
-        // ahead in 256x256; 1024 x 1536 x 7168 59.6 and 60.1 in 256x192.)
-        constexpr bool SCALES_AHEAD = STEPS < 24;
+        // where two ways lead into the loop the compiler takes the lower number.  (Read at the block's start, the scales are
+        // the youngest, and the first MFMA waits for every read there is.  us, at the start and ahead: 1024 x 1536 x 7168 in 128x128 of eight
+        // waves 29.2 and 29.0, of four 46.0 and 45.0, in 64x128 24.1 and 23.2; 512 x 1024 x 2048 in 64x128 8.76 and 8.40, in 64x64 7.80 and 7.33; in
+        // 64x256 128 x 8192 x 4096 20.75 and 20.41, but 1024 x 1536 x 7168 32.8 and 33.3; in 256x128 with three stages 1024 x 1536 x 7168 44.8 and 45.8,
+        // but 4847 x 480 x 7936 in three partitions 45.1 and 38.0.)
+        // Not with waves of 24 tiles and more, whose registers are full: 1000 tokens to 4 of 32 experts, 4096 x 2048, 70.0 us as it is, 73.5
+        // ahead in 256x256; 1024 x 1536 x 7168 59.6 and 60.1 in 256x192.  Nor in the summed K split of 192x192 on aligned rows, where the two
+        // registers that it spills are reloaded ahead of the loop and waited for inside it, with counts that know nothing of the copies and
+        // wait for those as well: 4096 x 2112 x 7168 in two partitions 79.3 at the start, 95.2 ahead.  (With TAILS it spills either way:
+        // 4523 x 952 x 6016 53.5 and 51.5.)
+        constexpr bool SCALES_AHEAD = STEPS < 24 && !(STEPS >= 18 && SUMMED && !TAILS);
         v8i areg[C::MT], breg[2];
         float asv[C::MT], bsv, bsv1;
         auto read_scales = [&](const unsigned char* sb) {
