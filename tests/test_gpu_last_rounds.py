@@ -26,8 +26,9 @@ def _column_scales(n, dev):
 
 
 # Tiles beyond the last full round of 256 or 512 workgroups: 256x256: 324 tiles (68 left over), 320 (64), the last tile 250 or 10 columns
-# wide; 64x256: 576 (64 left over, the last tile 10 columns wide) and 648 (136).
-@pytest.mark.parametrize("tile,m,n", [(2, 4608, 4608), (2, 5111, 4090), (2, 5120, 3850), (12, 2304, 3850), (12, 2300, 4601)])
+# wide; 64x256: 576 (64 left over, the last tile 10 columns wide) and 648 (136).  The last two: 3100 tiles, 28 of them behind twelve full
+# rounds, where the last round is neither spread nor cut.
+@pytest.mark.parametrize("tile,m,n", [(2, 4608, 4608), (2, 5111, 4090), (2, 5120, 3850), (12, 2304, 3850), (12, 2300, 4601), (2, 12790, 15810), (12, 3190, 15810)])
 def test_dense(pkg, tile, m, n):
     dev = torch.device("cuda:0")
     gen = torch.Generator(device=dev).manual_seed(m + n)
@@ -38,6 +39,21 @@ def test_dense(pkg, tile, m, n):
     assert torch.equal(c, (a.float() @ b.float().t().contiguous() * columns).bfloat16())
 
 
+def _check_grouped(pkg, gen, counts, n, tiles):
+    dev = torch.device("cuda:0")
+    rows, experts = sum(counts), len(counts)
+    offsets = torch.tensor([0, *counts], device=dev).cumsum(0).int()
+    a, b = _codes(gen, K, rows).t(), _codes(gen, experts, K, n).transpose(1, 2)
+    b_scale, columns = _column_scales(n, dev)
+    b_scale = b_scale.expand(experts, -1, -1).contiguous().transpose(1, 2)
+    bounds = offsets.tolist()
+    want = torch.cat([a[lo:hi].float() @ b[e].float().t().contiguous() * columns for e, (lo, hi) in enumerate(zip(bounds, bounds[1:]))]).bfloat16()
+    for tile in tiles:
+        c = torch.full((rows, n), float("nan"), dtype=torch.bfloat16, device=dev)
+        pkg.grouped_kernel((a, b, torch.ones(K // 128, rows, device=dev).t(), b_scale, offsets, c), variant=tile)
+        assert torch.equal(c, want), "tile %#x" % tile
+
+
 @pytest.mark.parametrize("experts", [1, 3, 63, 64, 65, 300])
 @pytest.mark.parametrize("n", [70, 250, 266, 520])
 def test_grouped(pkg, experts, n):
@@ -45,14 +61,10 @@ def test_grouped(pkg, experts, n):
     gen = torch.Generator(device=dev).manual_seed(experts * 1000 + n)
     counts = torch.randint(0, 40, (experts,), generator=gen, device=dev).mul_(torch.rand(experts, generator=gen, device=dev) < 0.7).tolist()
     counts[-1] += 131                                              # several tiles of one expert
-    rows = sum(counts)
-    offsets = torch.tensor([0] + counts, device=dev).cumsum(0).int()
-    a, b = _codes(gen, K, rows).t(), _codes(gen, experts, K, n).transpose(1, 2)
-    b_scale, columns = _column_scales(n, dev)
-    b_scale = b_scale.expand(experts, -1, -1).contiguous().transpose(1, 2)
-    bounds = offsets.tolist()
-    want = torch.cat([a[lo:hi].float() @ b[e].float().t().contiguous() * columns for e, (lo, hi) in enumerate(zip(bounds, bounds[1:]))]).bfloat16()
-    for tile in (0, 2, 3, 12, FORM(12, 1)):
-        c = torch.full((rows, n), float("nan"), dtype=torch.bfloat16, device=dev)
-        pkg.grouped_kernel((a, b, torch.ones(K // 128, rows, device=dev).t(), b_scale, offsets, c), variant=tile)
-        assert torch.equal(c, want), "tile %#x" % tile
+    _check_grouped(pkg, gen, counts, n, (0, 2, 3, 12, FORM(12, 1)))
+
+
+@pytest.mark.parametrize("tile,counts", [(2, (4100, 0, 5000, 3700)), (12, (1030, 0, 1250, 920))])
+def test_grouped_of_many_rounds(pkg, tile, counts):
+    """Some 3300 tiles: the last round behind twelve full ones."""
+    _check_grouped(pkg, torch.Generator(device="cuda:0").manual_seed(tile), counts, 15810, (tile,))
