@@ -108,8 +108,9 @@ def gate_up_silu(data):
             raise ValueError("b / b_scale shapes do not match [E, n, k] / [E, ceil(n/128), k/128]")
         if not _experts_kmajor(b) or not _experts_kmajor(b_scale):
             raise ValueError("every expert of b and b_scale must be K-major")
-        if row_offsets.dtype != torch.int32 or row_offsets.shape != (num_experts + 1,) or row_offsets.device != a.device:
-            raise ValueError("row_offsets must be an int32 tensor with num_experts+1 entries on the operands' GPU")
+        if row_offsets.dtype != torch.int32 or row_offsets.shape != (num_experts + 1,) or row_offsets.device != a.device \
+                or not row_offsets.is_contiguous():
+            raise ValueError("row_offsets must be a contiguous int32 tensor with num_experts+1 entries on the operands' GPU")
     else:
         if b.shape != (n, k) or b_scale.shape != (nb, kb):
             raise ValueError("b / b_scale shapes do not match [n, k] / [ceil(n/128), k/128]")

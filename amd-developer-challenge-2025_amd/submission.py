@@ -292,8 +292,9 @@ def grouped_kernel(data, variant: int = 0):
         raise ValueError("b / b_scale shapes do not match [E, n, k] / [E, ceil(n/128), k/128]")
     if not _experts_kmajor(b) or not _experts_kmajor(b_scale):
         raise ValueError("every expert of b and b_scale must be K-major")
-    if row_offsets.dtype != torch.int32 or row_offsets.shape != (num_experts + 1,) or row_offsets.device != a.device:
-        raise ValueError("row_offsets must be an int32 tensor with num_experts+1 entries on the operands' GPU")
+    if row_offsets.dtype != torch.int32 or row_offsets.shape != (num_experts + 1,) or row_offsets.device != a.device \
+            or not row_offsets.is_contiguous():
+        raise ValueError("row_offsets must be a contiguous int32 tensor with num_experts+1 entries on the operands' GPU")
     dev = a.device
     ws_ptr, ws_len = _grouped_workspace(dev, _stream_ptr(dev), num_experts, rows, n, k) if variant == 0 else (None, 0)
     if variant == 0:

@@ -116,3 +116,19 @@ def test_products(pkg, monkeypatch, silu, n, k, grouped):
                     assert out is c
                     return out
                 _same(monkeypatch, (name, wide, as_list), call)
+
+
+@pytest.mark.parametrize("silu", [False, True])
+def test_row_offsets_that_lie_apart_are_refused(pkg, silu):
+    """The kernels read them one behind the other."""
+    moe = importlib.import_module(pkg_name + ".moe")
+    dev = torch.device("cuda:0")
+    f8 = lambda *s: torch.ones(*s, device=dev).to(torch.float8_e4m3fn)
+    a, b = f8(128, 96).t(), f8(3, 128, 256).transpose(1, 2)
+    scales = torch.ones(1, 96, device=dev).t(), torch.ones(3, 1, 2, device=dev).transpose(1, 2)
+    offsets = torch.tensor([0, 20, 20, 96], dtype=torch.int32, device=dev)
+    c = torch.zeros(96, 128 if silu else 256, dtype=torch.bfloat16, device=dev)
+    call = moe.gate_up_silu if silu else pkg.grouped_kernel
+    call((a, b, *scales, offsets, c))
+    with pytest.raises(ValueError, match="row_offsets"):
+        call((a, b, *scales, torch.stack([offsets, offsets], 1)[:, 0], c))
