@@ -154,11 +154,11 @@ def combine(y: torch.Tensor, slot_of: torch.Tensor, weights: torch.Tensor) -> to
     if slot_of.dtype != torch.int32 or not slot_of.is_contiguous() or weights.dtype != torch.float32 \
             or not weights.is_contiguous() or slot_of.shape != weights.shape or slot_of.dim() != 2:
         raise ValueError("slot_of (int32) and weights (float32) must be contiguous [tokens, topk] tensors")
-    for name, x in (("slot_of", slot_of), ("weights", weights)):
-        if not x.is_cuda and not x.is_pinned():       # (the kernel would fault on pageable host memory)
-            raise ValueError("%s must be on the GPU" % name)
     t, k = slot_of.shape
     d = y.shape[1]
+    for name, x in (("slot_of", slot_of), ("weights", weights)):
+        if t and d and not x.is_cuda and not x.is_pinned():       # (the kernel would fault on pageable host memory; without outputs there is no launch)
+            raise ValueError("%s must be on the GPU" % name)
     out = torch.empty(t, d, dtype=torch.bfloat16, device=y.device)
     _call(_lib.calls().moe_combine, y.device, y.data_ptr(), y.shape[0], slot_of.data_ptr(), weights.data_ptr(), out.data_ptr(), t, k, d)
     return out
