@@ -95,8 +95,9 @@ _plan_cache = {}   # (m, n, k) and ("grouped" | "silu" | "route", sizes ...) -> 
 _PLANS_MAX = 4096
 
 # Dense sizes that the native call of custom_kernel may take, with the workspace bytes that each asks for.  It checks the tensors
-# themselves at every call; what it is told here is a fact about the sizes alone.
-_CHECKED_MAX = 64
+# themselves at every call; what it is told here is a fact about the sizes alone.  As many as plans are kept: a server whose batches
+# vary has two or three sizes of them for each, and a size that is not here pays for the native attempt and the Python path.
+_CHECKED_MAX = _PLANS_MAX
 _checked = {}      # (m, n, k) -> bytes
 _checked_experts = {}      # the same for grouped_kernel and gate_up_silu: (silu, experts or 0, rows, n, k) -> bytes
 
