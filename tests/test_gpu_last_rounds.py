@@ -68,3 +68,39 @@ def test_grouped(pkg, experts, n):
 def test_grouped_of_many_rounds(pkg, tile, counts):
     """Some 3300 tiles: the last round behind twelve full ones."""
     _check_grouped(pkg, torch.Generator(device="cuda:0").manual_seed(tile), counts, 15810, (tile,))
+
+
+def _silu_mul(pkg, a, b, a_scale, b_scale, offsets, rows, n, variant):
+    """gate_up_silu with the tile forced, unsplit; h starts as NaN."""
+    lib = pkg._lib.load()
+    h = torch.full((rows, n // 2), float("nan"), dtype=torch.bfloat16, device="cuda:0")
+    pkg._lib.check(lib.fp8bs_gemm_silu_mul_ws(a.data_ptr(), b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(), h.data_ptr(), None if offsets is None else offsets.data_ptr(),
+                                              0 if offsets is None else offsets.numel() - 1, rows, n, K, variant, 1, None, 0, torch.cuda.current_stream().cuda_stream))
+    assert not torch.isnan(h).any()
+    return h.view(torch.int16)
+
+
+# n/2 on the 8-column grid and off it, the last tile 10 columns wide in two of them.  64x128 is never cut.
+@pytest.mark.parametrize("tile,m,n", [(2, 4608, 4608), (2, 5111, 4090), (2, 5120, 3850), (12, 2304, 3850), (12, 2300, 4602)])
+def test_dense_silu_mul(pkg, tile, m, n):
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(m + n)
+    a, b = _codes(gen, K, m).t(), _codes(gen, K, n).t()
+    data = (a, b, torch.ones(K // 128, m, device=dev).t(), _column_scales(n, dev)[0].t(), None, m, n)
+    assert torch.equal(_silu_mul(pkg, *data, tile), _silu_mul(pkg, *data, 4))
+
+
+@pytest.mark.parametrize("experts", [1, 3, 64, 65])
+@pytest.mark.parametrize("n", [70, 250, 266, 520])
+def test_grouped_silu_mul(pkg, experts, n):
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(experts * 1000 + n)
+    counts = torch.randint(0, 40, (experts,), generator=gen, device=dev).tolist()
+    counts[-1] += 131
+    rows = sum(counts)
+    a, b = _codes(gen, K, rows).t(), _codes(gen, experts, K, n).transpose(1, 2)
+    b_scale = _column_scales(n, dev)[0].expand(experts, -1, -1).contiguous().transpose(1, 2)
+    data = (a, b, torch.ones(K // 128, rows, device=dev).t(), b_scale, torch.tensor([0, *counts], device=dev).cumsum(0).int(), rows, n)
+    want = _silu_mul(pkg, *data, 4)
+    for tile in (2, 12):
+        assert torch.equal(_silu_mul(pkg, *data, tile), want), "tile %d" % tile

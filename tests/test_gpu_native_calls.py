@@ -2,6 +2,7 @@
 the forms of arguments that both see: what one accepts the other accepts with the same bits, layout and type, what one refuses the
 other refuses with the same type of exception."""
 import importlib
+import threading
 
 import pytest
 import torch
@@ -28,7 +29,7 @@ def _outcome(monkeypatch, native, fn):
     return [(tuple(t.shape), t.stride(), t.dtype, t.device, t.requires_grad, t.detach().as_subclass(torch.Tensor).cpu().flatten().clone().view(torch.uint8)) for t in out]
 
 
-def _same(monkeypatch, what, fn, counts=None):
+def _same(monkeypatch, what, fn):
     native = _lib().native()
     assert native is not None, "build() builds it"
     want, got = _outcome(monkeypatch, None, fn), _outcome(monkeypatch, native, fn)
@@ -132,3 +133,109 @@ def test_row_offsets_that_lie_apart_are_refused(pkg, silu):
     call((a, b, *scales, offsets, c))
     with pytest.raises(ValueError, match="row_offsets"):
         call((a, b, *scales, torch.stack([offsets, offsets], 1)[:, 0], c))
+
+
+def _layer(seed, tokens=37, experts=8, k=3, hidden=512, inter=384):
+    """(inputs of a layer, the chain of calls on them)"""
+    moe, quant, pkg = (importlib.import_module(pkg_name + x) for x in (".moe", ".quant", ""))
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(seed)
+    rand = lambda *s: torch.randn(*s, generator=gen, device=dev)
+    f8 = lambda *s: rand(*s).to(torch.float8_e4m3fn).transpose(1, 2)
+    scale = lambda *s: (rand(*s).abs() + 0.5).transpose(1, 2)
+    x, scores, gates = rand(tokens, hidden).bfloat16(), rand(tokens, experts), rand(tokens, k).abs()
+    up, up_scale = f8(experts, hidden, 2 * inter), scale(experts, hidden // 128, inter // 64)
+    down, down_scale = f8(experts, inter, hidden), scale(experts, inter // 128, hidden // 128)
+
+    def run():
+        offsets, row_map, slot_of = moe.route(moe.topk(scores, k), experts)
+        h = torch.full((tokens * k, inter), float("nan"), dtype=torch.bfloat16, device=dev)
+        y = torch.full((tokens * k, hidden), float("nan"), dtype=torch.bfloat16, device=dev)
+        a, a_scale = quant.quantize_a(x, row_map)
+        moe.gate_up_silu((a, up, a_scale, up_scale, offsets, h))
+        a, a_scale = quant.quantize_a(h)
+        pkg.grouped_kernel((a, down, a_scale, down_scale, offsets, y))
+        return moe.combine(y, slot_of, gates), offsets, slot_of, h, y
+    return run
+
+
+def test_native_code_takes_the_plain_calls(pkg, monkeypatch):
+    """Every step of a layer, the quantisers' forms among them, once a size has been seen; and not what it should decline."""
+    quant, moe, sub = (importlib.import_module(pkg_name + x) for x in (".quant", ".moe", ".submission"))
+    native = _lib().native()
+    assert native is not None, "build() builds it"
+    run = _layer(1)
+    run()
+    taken = {}
+
+    class Counted:
+        def __getattr__(self, name):
+            def call(*args):
+                got = getattr(native, name)(*args)
+                taken.setdefault(name, []).append(got)
+                return got
+            return call
+
+    monkeypatch.setattr(_lib(), "_native", Counted())
+    run()
+    assert sorted(taken) == ["combine", "experts", "quantize", "route", "topk"]
+    assert all(type(g) is tuple for name in ("quantize", "route") for g in taken[name]) and len(taken["quantize"]) == 2
+    assert all(torch.is_tensor(g) for name in ("topk", "combine") for g in taken[name])
+    assert taken["experts"].count(0) == 2 and all(g == 0 or g < -1 for g in taken["experts"])       # (less than -1: a workspace of so many bytes first)
+    x = torch.randn(9, 256, device="cuda:0")
+    for plain in (x, x.bfloat16(), x[:1]):
+        assert type(native.quantize(plain, None, False)) is type(native.quantize(plain, None, True)) is tuple
+    for odd in (x.half(), x.as_subclass(_Sub), x.cpu(), x[:, :-1], x.t(), None):
+        assert native.quantize(odd, None, False) is None
+    assert native.topk(x.double(), 2) is None and native.combine(x, x, x) is None
+    assert native.route(x, 8, 0, 0) is None and native.experts((x,) * 6, sub._checked_experts, 0, 0, False) == -1
+
+
+def test_traced_tensors_are_refused(pkg):
+    """A tensor that vmap wraps has no storage: the error of the Python path, and the next call is well."""
+    quant, moe = (importlib.import_module(pkg_name + x) for x in (".quant", ".moe"))
+    dev = torch.device("cuda:0")
+    run = _layer(2)
+    want = run()
+    x, two = torch.randn(2, 5, 128, device=dev), torch.zeros(2, 5, 2, dtype=torch.int32, device=dev)
+    y, w = torch.randn(10, 128, device=dev).bfloat16(), torch.rand(2, 5, 2, device=dev)
+    a, s = quant.quantize_a(torch.randn(96, 128, device=dev))
+    b, bs = torch.zeros(3, 128, 256, device=dev).to(torch.float8_e4m3fn).transpose(1, 2), torch.ones(3, 1, 2, device=dev).transpose(1, 2)
+    offsets = torch.tensor([0, 20, 20, 96], dtype=torch.int32, device=dev)
+    c, h = (torch.zeros(96, n, dtype=torch.bfloat16, device=dev) for n in (256, 128))
+    pkg.grouped_kernel((a, b, s, bs, offsets, c)), moe.gate_up_silu((a, b, s, bs, offsets, h))
+    both = torch.stack([offsets, offsets])
+    for fn, over in ((lambda t: quant.quantize_a(t)[0], x), (lambda t: quant.quantize_b(t)[0], x), (lambda t: moe.topk(t, 2), x), (lambda t: moe.route(t, 4)[0], two),
+                     (lambda t: moe.combine(y, two[0], t), w), (lambda t: pkg.grouped_kernel((a, b, s, bs, t, c)), both), (lambda t: moe.gate_up_silu((a, b, s, bs, t, h)), both)):
+        with pytest.raises((RuntimeError, ValueError)):
+            torch.func.vmap(fn)(over)
+    for g, r in zip(run(), want):
+        assert torch.equal(g.view(torch.int16), r.view(torch.int16))
+
+
+def test_layers_of_two_threads_on_streams_of_their_own(pkg):
+    """Each on its own stream, at the same time, with results and workspaces of its own."""
+    runs = [_layer(3, tokens=37), _layer(4, tokens=300)]
+    want = [[t.clone() for t in run()] for run in runs]
+    torch.cuda.synchronize()
+    start, got, errors = threading.Barrier(2), [None, None], []
+
+    def work(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                start.wait(30)
+                got[i] = [runs[i]() for _ in range(20)]
+                torch.cuda.current_stream().synchronize()
+        except Exception as ex:
+            errors.append(ex)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not errors and not any(t.is_alive() for t in threads), errors
+    for mine, theirs in zip(want, got):
+        for out in theirs:
+            for r, g in zip(mine, out):
+                assert torch.equal(r.view(torch.int16), g.view(torch.int16))
