@@ -344,19 +344,21 @@ void gemm_tr_kernel(const GemmArgs p) {
     // us, before and now: 46 tokens to 8 of 16 experts, 766 x 1536, 15.6 and 9.4; 46 to 4 of 32, 2485 x 2432, 64.1 and 50.4; 900 to 8 of 16,
     // 3072 x 1536, 48.0 and 41.8; 64 to 8 of 32, 7168 x 2048 (3.5 rounds), 101.2 and 97.4; dense 6144 x 4608 x 7168 195 and 177. 90 grouped
     // products (1 .. 4096 tokens) 0.93 of the time in the geometric mean, at worst 1.04.
-    // Tiles of 256 columns: behind twelve full rounds the last one is dealt in runs of a full round's length, and not cut.  By then the workgroups have
+    // Unsplit tiles of 256 columns: behind twelve full rounds the last one is dealt in runs of a full round's length, and not cut.  By then the workgroups have
     // drifted apart by more than a part saves, and parts for nearly all of them lengthen the longest: 4096 tokens to 8 of 32 experts, 7168 x
     // 2048 (16.2 rounds), over four draws of the experts, us, in runs 506.6-508.3, spread and cut 512.0-515.7; 2200 to 8 of 32, 7168 x 2048 in 64x256 (33 rounds)
     // 487.7-493.4 and 493.3-502.0; at 11.5 rounds 379.5-387.4 and 382.8-387.4, at 9.2 909.6-914.7 and 904.3-916.6, at 4.4 262.8-264.0 and 252.6-255.7.
-    constexpr int SPREAD_ROUNDS = BN == 256 ? 12 : 0x7FFFFFFF;
+    [[maybe_unused]] constexpr int SPREAD_ROUNDS = 12;
     constexpr int MOST_CUT = (MODE == 0 || MODE == 2) && BN == 256 ? (BN / WN >= 4 ? 2 : 1) : 0;
     auto place = [&](int it, int total, int& part, int& cut) -> int {
         const int G = gridDim.x, first = it * G, here = total - first;
         if (here <= 0) return -1;
-        if (here >= G || it >= SPREAD_ROUNDS) {
-            const int v = xcd_virtual_id(blockIdx.x, G);
-            return v < here ? first + v : -1;
-        }
+        if (here >= G) return first + xcd_virtual_id(blockIdx.x, G);
+        if constexpr (MOST_CUT > 0)
+            if (it >= SPREAD_ROUNDS) {
+                const int v = xcd_virtual_id(blockIdx.x, G);
+                return v < here ? first + v : -1;
+            }
         if constexpr (MOST_CUT > 0)
             if (it > 0 || MODE == 2) cut = MOST_CUT > 1 && here * 4 <= G ? 2 : here * 2 <= G ? 1 : 0;
         const int pieces = here << cut;
