@@ -182,7 +182,7 @@ void route_scan_kernel(int32_t* __restrict__ block_counts, int nblocks, int expe
 // SCAN_HERE: block_base holds the raw per-block counts and every block derives its own bases and the
 // row offsets from them (few blocks: cheaper than a launch of its own); block 0 writes row_offsets.
 // Bound by latency, so the choices are loaded before anything else and there are few barriers; the bitmaps lie word by word, so that a wave's
-// lanes, which ask for one word of different experts, meet in few banks, and the tokens in an expert's earlier words are counted once. us of both kernels, before -> after: 4096 tokens to 8 of
+// lanes, which ask for one word of different experts, meet in few banks, and the tokens in an expert's earlier words are counted once. us of both kernels, back to back in a graph, before -> after: 4096 tokens to 8 of
 // 32 experts 11.6 -> 9.3, 4096 to 2 of 8 9.4 -> 9.1, 1500 to 4 of 16 9.5 -> 8.5, 3000 to 8 of 256 14.8 -> 12.5, 16384 to 8 of 32 13.4 -> 11.2. (Storing
 // row_map in runs, put in order in LDS first, cost two barriers and more than it gave: 10.5, 10.2, 9.7, 13.4, 12.4.)
 template <bool SCAN_HERE>

@@ -343,7 +343,8 @@ void gemm_tr_kernel(const GemmArgs p) {
     // columns of other parts are not fetched, so a part costs little more than what its columns do.
     // us, before and now: 46 tokens to 8 of 16 experts, 766 x 1536, 15.6 and 9.4; 46 to 4 of 32, 2485 x 2432, 64.1 and 50.4; 900 to 8 of 16,
     // 3072 x 1536, 48.0 and 41.8; 64 to 8 of 32, 7168 x 2048 (3.5 rounds), 101.2 and 97.4; dense 6144 x 4608 x 7168 195 and 177. 90 grouped
-    // products (1 .. 4096 tokens) 0.93 of the time in the geometric mean, at worst 1.04.
+    // products (1 .. 4096 tokens) 0.93 of the time in the geometric mean, at worst 1.04 (1920 tokens to 4 of
+    // 32 experts, 832 x 4992, where it is a matter of which experts the rows fall on: over four draws 0.93 to 0.97 with even experts, 0.97 to 1.02 with skewed ones).
     // Unsplit tiles of 256 columns: behind twelve full rounds the last one is dealt in runs of a full round's length, and not cut.  By then the workgroups have
     // drifted apart by more than a part saves, and parts for nearly all of them lengthen the longest: 4096 tokens to 8 of 32 experts, 7168 x
     // 2048 (16.2 rounds), over four draws of the experts, us, in runs 506.6-508.3, spread and cut 512.0-515.7; 2200 to 8 of 32, 7168 x 2048 in 64x256 (33 rounds)
@@ -703,7 +704,7 @@ void gemm_tr_kernel(const GemmArgs p) {
     // of a buffer load works on whole dwords and hands back zeros for those.  Every other byte of a
     // arrives intact (a dword that crosses the end of a k row just runs on into the next one).  The
     // workgroup whose tile holds those bytes writes them into LDS itself once the last K block has
-    // landed: they all lie in the last aligned dword of a.  The same holds for b with n % 4 != 0.
+    // landed: they are among the last four bytes of a.  The same holds for b with n % 4 != 0.
     // Each is written by the wave whose copy brought the bytes around it, between its wait for the copy and the barrier that
     // publishes the block: lane l < 6 of every wave has one candidate, a's for l < 3, in patch_at, worked out at a tile's
     // start while the first copies are on their way; a lane whose candidate is not lost, not in the tile or another
@@ -1466,7 +1467,7 @@ void gemm_tr_kernel(const GemmArgs p) {
         }
     }
     if (!nxt.valid) break;
-    stores_behind = prefetched && wave_active && MODE != 1 && !TAILS && store_output;   // (with TAILS the store count is four times EPI_STORES: plain wait)
+    stores_behind = prefetched && wave_active && MODE != 1 && !TAILS && store_output;   // (with TAILS the store count differs from wave to wave, EPI_STORES or four times that where the wave holds rows' ends: only a plain wait is right)
     cur = nxt; cp = ncp;
     }   // tiles
 }

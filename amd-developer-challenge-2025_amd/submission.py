@@ -274,7 +274,7 @@ def grouped_kernel(data, variant: int = 0):
     ``variant`` forces a tile (FP8BS_VARIANT_*) for testing; 0 lets the library choose.
 
     Row-offset convention of 2-amd-moe/3-amd-fp8-moe-hip-myhgemm.py:142-148, :328-336 with the
-    total appended: ``row_offsets`` is int32 [E+1] on the GPU, expert e owns rows
+    total appended: ``row_offsets`` is int32 [E+1], contiguous, on the GPU; expert e owns rows
     [row_offsets[e], row_offsets[e+1]) of the expert-contiguous ``a`` ([rows, k], K-major) and ``c``
     ([rows, n]).  ``b`` is [E, n, k] with each expert K-major (stride (n*k, 1, n)); ``b_scale`` is
     [E, ceil(n/128), k/128] with stride (nb*kb, 1, nb).  Fills and returns ``c``; no host sync.
