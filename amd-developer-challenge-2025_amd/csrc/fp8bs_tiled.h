@@ -351,20 +351,38 @@ void gemm_tr_kernel(const GemmArgs p) {
     // 487.7-493.4 and 493.3-502.0; at 11.5 rounds 379.5-387.4 and 382.8-387.4, at 9.2 909.6-914.7 and 904.3-916.6, at 4.4 262.8-264.0 and 252.6-255.7.
     [[maybe_unused]] constexpr int SPREAD_ROUNDS = 12;
     constexpr int MOST_CUT = (MODE == 0 || MODE == 2) && BN == 256 ? (BN / WN >= 4 ? 2 : 1) : 0;
+    // Across the experts, where a call is a stream of their weights, an XCD's workgroups change places from round to round, by a band's
+    // rows - one n tile - each time.  Rows of b that are a multiple of 1024 bytes apart put a column of b into one eighth of the address bits 7 to 9,
+    // and the memory serves one of the eight, 384 to 511, at 0.8 of the others' rate (64x256 tiles of 64 x 18432 x 7168: the fourth that holds
+    // those bytes ends its K blocks at 26.5 us, the others at 20.3; with b 256 bytes further on it is the tiles beside them; rows 4352
+    // apart: none).  A round being a multiple of the period, a workgroup had such a tile in every round or in none.  us, before and
+    // now: 32 tokens to 8 of 32 experts, 4096 x 7168, 177.1 and 170.2; 64 to 8 of 32, 7168 x 2048, 102.7 and 97.1; 8 to 4 of 32, 4096 x 7168, 127.8
+    // and 120.9; 3072 x 7168 142.4 and 142.8.  Not in a round that is cut, whose places are other ones (3072 x 7168, 1.5 rounds: 145.7), and not
+    // expert by expert, where the weights are read once for many rows (4096 tokens, 4096 x 7168: 921 as it is, 929 turned).
+    [[maybe_unused]] int turn = 0;
     auto place = [&](int it, int total, int& part, int& cut) -> int {
         const int G = gridDim.x, first = it * G, here = total - first;
+        int wg = blockIdx.x;
         if (here <= 0) return -1;
-        if (here >= G) return first + xcd_virtual_id(blockIdx.x, G);
+        if constexpr (GROUPED)
+            if (it > 0 && !p.by_expert && (G >> 3) >= p.band_h) {
+                const int x = blockIdx.x & 7, run = (G >> 3) + (x < (G & 7) ? 1 : 0), at = (int)(blockIdx.x >> 3);      // workgroups of this XCD, this one's place among them
+                turn += p.band_h;
+                if (turn >= run) turn -= run;
+                wg = x + 8 * (at + turn >= run ? at + turn - run : at + turn);
+            }
+        if (here >= G) return first + xcd_virtual_id(wg, G);
         if constexpr (MOST_CUT > 0)
             if (it >= SPREAD_ROUNDS) {
-                const int v = xcd_virtual_id(blockIdx.x, G);
+                const int v = xcd_virtual_id(wg, G);
                 return v < here ? first + v : -1;
             }
         if constexpr (MOST_CUT > 0)
             if (it > 0 || MODE == 2) cut = MOST_CUT > 1 && here * 4 <= G ? 2 : here * 2 <= G ? 1 : 0;
+        if (cut > 0) wg = blockIdx.x;
         const int pieces = here << cut;
-        if ((int)blockIdx.x >= pieces) return -1;
-        const int v = xcd_virtual_id(blockIdx.x, pieces);
+        if (wg >= pieces) return -1;
+        const int v = xcd_virtual_id(wg, pieces);
         part = v - (v >> cut << cut);
         return first + (v >> cut);
     };

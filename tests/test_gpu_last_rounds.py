@@ -64,6 +64,15 @@ def test_grouped(pkg, experts, n):
     _check_grouped(pkg, gen, counts, n, (0, 2, 3, 12, FORM(12, 1)))
 
 
+# Few rows an expert, several rounds of 256 or 512 tiles: the workgroups of an XCD change places between them.  64x256: 528 tiles (16 left over), 768 (none),
+# 1080 (56), 700 (188 left over, not cut), 490 of 70 experts, whose table is in LDS (234, not cut); 64x64: 1890 to 4320.
+@pytest.mark.parametrize("experts,n", [(33, 4090), (48, 4096), (60, 4601), (50, 3500), (70, 1700)])
+def test_grouped_across_the_experts_in_rounds(pkg, experts, n):
+    gen = torch.Generator(device="cuda:0").manual_seed(experts)
+    counts = torch.randint(1, 16, (experts,), generator=gen, device="cuda:0").tolist()
+    _check_grouped(pkg, gen, counts, n, (0, 2, 12, FORM(12, 1), FORM(4, 1)))
+
+
 @pytest.mark.parametrize("tile,counts", [(2, (4100, 0, 5000, 3700)), (12, (1030, 0, 1250, 920))])
 def test_grouped_of_many_rounds(pkg, tile, counts):
     """Some 3300 tiles: the last round behind twelve full ones."""
