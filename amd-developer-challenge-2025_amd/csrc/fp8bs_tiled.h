@@ -67,6 +67,11 @@ __device__ __forceinline__ void copy16_global_to_lds(__amdgpu_buffer_rsrc_t rsrc
     asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, %3 offen lds"
                  :: "v"(lane_offset), "s"(rsrc), "s"(lds_base), "s"(wave_offset) : "memory", "m0");
 }
+// same, for bytes that are not read again: neither the L2 nor the 256 MB cache behind it makes room for them
+__device__ __forceinline__ void copy16_global_to_lds_once(__amdgpu_buffer_rsrc_t rsrc, uint32_t lds_base, uint32_t lane_offset, uint32_t wave_offset) {
+    asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, %3 offen nt lds"
+                 :: "v"(lane_offset), "s"(rsrc), "s"(lds_base), "s"(wave_offset) : "memory", "m0");
+}
 // same with 4 bytes per lane: lane l's dword lands at lds_base + 4*l
 __device__ __forceinline__ void copy4_global_to_lds(__amdgpu_buffer_rsrc_t rsrc, uint32_t lds_base, uint32_t lane_offset, uint32_t wave_offset) {
     asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dword %0, %1, %3 offen lds"
@@ -112,6 +117,7 @@ __device__ __forceinline__ void band_tile(int v, int tiles_m, int tiles_n, int g
 //   MODE 3  : dense, K blocks instead of tiles dealt to the workgroups, partial tiles through the workspace, bf16 output
 //   MODE 4  : dense split-K, partial tiles to the workspace, the sum of a tile shared out among its workgroups or done by the last of them, bf16 output
 //   MODE 5  : grouped like MODE 2 with a K split summed like MODE 4's
+//   MODE 6  : MODE 2 with b read past the caches (the hint is part of the load instruction), see the rule at `b_read_once`
 // LDS: NSTAGE stages, each [128 k][BM] bytes of A then [128 k][BN] bytes of B, 16-byte chunks XOR-swizzled
 // so that the 16 k rows touched by half a wave in one transposing read fall on 16 different 16-byte
 // bank groups, then the k block's a_scale row and b_scale values.
@@ -217,7 +223,7 @@ constexpr int waves_per_simd() {
     using C = TileCfg<BM, BN, WM, WN, MODE, NSTAGE>;
     const int by_lds = 163840 / C::LDS_BYTES, by_threads = 2048 / C::NTHREADS;
     const int w = C::NWAVES * (by_lds < by_threads ? by_lds : by_threads) / 4;
-    return MODE >= 3 && w > 1 ? w : 1;
+    return MODE >= 3 && MODE <= 5 && w > 1 ? w : 1;
 }
 
 // Tiles whose K partitions can share out the sum of a tile (see there).  Not 64x128: its two workgroups per CU leave 128
@@ -236,7 +242,7 @@ template <int BM, int BN, int WM, int WN, int MODE, int EPI = 0, int NSTAGE = 2,
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) __attribute__((amdgpu_waves_per_eu(waves_per_simd<BM, BN, WM, WN, MODE, NSTAGE>())))
 void gemm_tr_kernel(const GemmArgs p) {
     using C = TileCfg<BM, BN, WM, WN, MODE, NSTAGE>;
-    constexpr bool GROUPED = MODE == 2 || MODE == 5, SUMMED = MODE == 4 || MODE == 5;
+    constexpr bool GROUPED = MODE == 2 || MODE == 5 || MODE == 6, SUMMED = MODE == 4 || MODE == 5, B_ONCE = MODE == 6;
     static_assert(!SHARED_SUM || (SUMMED && shares_sum<BM, BN, WM, WN>()));
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
 
@@ -350,7 +356,7 @@ void gemm_tr_kernel(const GemmArgs p) {
     // 2048 (16.2 rounds), over four draws of the experts, us, in runs 506.6-508.3, spread and cut 512.0-515.7; 2200 to 8 of 32, 7168 x 2048 in 64x256 (33 rounds)
     // 487.7-493.4 and 493.3-502.0; at 11.5 rounds 379.5-387.4 and 382.8-387.4, at 9.2 909.6-914.7 and 904.3-916.6, at 4.4 262.8-264.0 and 252.6-255.7.
     [[maybe_unused]] constexpr int SPREAD_ROUNDS = 12;
-    constexpr int MOST_CUT = (MODE == 0 || MODE == 2) && BN == 256 ? (BN / WN >= 4 ? 2 : 1) : 0;
+    constexpr int MOST_CUT = (MODE == 0 || MODE == 2 || MODE == 6) && BN == 256 ? (BN / WN >= 4 ? 2 : 1) : 0;
     // Across the experts, where a call is a stream of their weights, an XCD's workgroups change places from round to round, by a band's
     // rows - one n tile - each time.  Rows of b that are a multiple of 1024 bytes apart put a column of b into one eighth of the address bits 7 to 9,
     // and the memory serves one of the eight, 384 to 511, at 0.8 of the others' rate (64x256 tiles of 64 x 18432 x 7168: the fourth that holds
@@ -378,7 +384,7 @@ void gemm_tr_kernel(const GemmArgs p) {
                 return v < here ? first + v : -1;
             }
         if constexpr (MOST_CUT > 0)
-            if (it > 0 || MODE == 2) cut = MOST_CUT > 1 && here * 4 <= G ? 2 : here * 2 <= G ? 1 : 0;
+            if (it > 0 || GROUPED) cut = MOST_CUT > 1 && here * 4 <= G ? 2 : here * 2 <= G ? 1 : 0;
         if (cut > 0) wg = blockIdx.x;
         const int pieces = here << cut;
         if (wg >= pieces) return -1;
@@ -569,6 +575,7 @@ void gemm_tr_kernel(const GemmArgs p) {
     // With 12 chunks per k row of B one copy of the workgroup (NWAVES*64 chunks) does not end on a row
     // boundary: a lane's (k row, chunk) then differs from copy to copy and it keeps one offset per copy.
     constexpr bool B_ROWS_WHOLE = (C::NWAVES * 64) % C::CPR_B == 0;
+    static_assert(!B_ONCE || B_ROWS_WHOLE);
     constexpr bool A_ROWS_WHOLE = (C::NWAVES * 64) % C::CPR_A == 0;
     constexpr int AS_COPIES = BM / 64;
     static_assert(C::NWAVES > AS_COPIES, "some wave must be left to copy the b_scale values");
@@ -657,7 +664,9 @@ void gemm_tr_kernel(const GemmArgs p) {
                 copy16_global_to_lds(a_rsrc, sa + q * C::NWAVES * 1024, cp.a_voffq[q], kb * a_kstep);
         } else if constexpr (q < C::A_LOADS + C::B_LOADS) {
             constexpr int qb = q - C::A_LOADS;
-            if constexpr (B_ROWS_WHOLE)
+            if constexpr (B_ONCE)
+                copy16_global_to_lds_once(cp.b_rsrc, sa + C::A_BYTES + qb * C::NWAVES * 1024, cp.b_voff, kb * b_kstep + (uint32_t)(qb * ROWS_PER_COPY_B) * (uint32_t)p.n);
+            else if constexpr (B_ROWS_WHOLE)
                 copy16_global_to_lds(cp.b_rsrc, sa + C::A_BYTES + qb * C::NWAVES * 1024, cp.b_voff, kb * b_kstep + (uint32_t)(qb * ROWS_PER_COPY_B) * (uint32_t)p.n);
             else
                 copy16_global_to_lds(cp.b_rsrc, sa + C::A_BYTES + qb * C::NWAVES * 1024, cp.b_voffq[qb], kb * b_kstep);
@@ -1524,6 +1533,21 @@ static inline hipError_t launch_tr(const GemmArgs& a, dim3 grid, hipStream_t str
     return hipGetLastError();
 }
 
+// The experts' weights are read past the caches where nothing of them can be found there again: together they are as large as the 256 MB
+// cache, which a pass over them leaves with none of what the next one reads first, and an expert has so few rows that one row of tiles, and so
+// one workgroup for a column of them, reads its weights.  What is left in the caches is then a, of which every workgroup of an XCD reads the same lines
+// (128 bytes for an expert's 16 or so), and the memory answers sooner.  us, as before and so (32 experts, 8 a token, 4096 x 7168 but where said): 32
+// tokens 162.9 and 148.7, 64 tokens 182.7 and 168.4, 7168 x 2048 97.0 and 91.7; 128 tokens in 256x256 197.6 and 183.8, 512 tokens 230.3 and 219.8, unevenly
+// spread 275.6 and 261.8, 768 tokens (24 rows in 32) 252.2 and 239.5, unevenly 302.1 and 301.1.  Beyond that line a second row of tiles reads them from
+// memory again: 256 tokens in 64x256 245.8 and 272.5, 1024 in 256x256 364 and 392.  Weights that the cache would hold: 250 x 4096 x 7168 17.8 and 24.4.
+// Rows of b are whole 128-byte lines: a line that two columns of tiles share would come from memory twice (100 tokens to 4 of 32, 3072 x 4096
+// 86.8 and 81.3, 2944 78.7 and 73.8; 3008 78.6 and 79.8, 3064 88.0 and 93.8, 3001 94.0 and 101.1).
+template <int BM> static inline bool b_read_once(const GemmArgs& a) {
+    const int used = a.m < a.num_experts ? a.m : a.num_experts;          // experts with rows, at most
+    return (size_t)used * (size_t)a.n * (size_t)a.k >= ((size_t)256 << 20) && (long)a.m * 4 <= (long)a.num_experts * (BM * 3)
+           && a.n % 128 == 0 && ((uintptr_t)a.b & 127) == 0;
+}
+
 // WITH_EPI: the fused silu-mul epilogue is instantiated for this tile; GROUPED_SPLIT: the grouped walk with a K split is
 template <int BM, int BN, int WM, int WN, bool WITH_EPI = false, int NSTAGE = 2, bool GROUPED_SPLIT = false>
 static inline hipError_t launch_shape(const GemmArgs& a, int mode, hipStream_t stream) {
@@ -1582,6 +1606,12 @@ static inline hipError_t launch_shape(const GemmArgs& a, int mode, hipStream_t s
         if constexpr (WITH_EPI) { if (a.epi == 1) return launch_summed(integral_constant<int, 4>{}, integral_constant<int, 1>{}); }
         return a.epi == 0 ? launch_summed(integral_constant<int, 4>{}, integral_constant<int, 0>{}) : hipErrorInvalidValue;
     }
+    // the tiles that the planner gives calls of few rows an expert
+    if constexpr (BN == 256 && WITH_EPI)
+        if (mode == 2 && b_read_once<BM>(a)) {
+            if (a.epi != 0 && a.epi != 1) return hipErrorInvalidValue;
+            return a.epi == 1 ? launch_tr<BM, BN, WM, WN, 6, 1, NSTAGE>(a, grid, stream) : launch_tr<BM, BN, WM, WN, 6, 0, NSTAGE>(a, grid, stream);
+        }
     if (a.epi != 0) {
         // (with the reduce launch of a K split the planes are plain sums and the reduce kernel applies the epilogue)
         if constexpr (WITH_EPI) {
