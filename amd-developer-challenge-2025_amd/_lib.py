@@ -34,7 +34,7 @@ class Plan(ctypes.Structure):
     ]
 
 
-FORM_NAMES = {(4, 1): "t64x64s4", (12, 1): "t128x128s4", (12, 2): "waves16x64", (12, 3): "waves32x64"}
+FORM_NAMES = {(4, 1): "t64x64s4", (10, 1): "t128x256s3", (12, 1): "t128x128s4", (12, 2): "waves16x64", (12, 3): "waves32x64"}
 SPLIT_SUM_IN_KERNEL = 1 << 30        # FP8BS_SPLIT_SUM_IN_KERNEL
 MIN_VERSION = 400                    # fp8bs_version() of the first library whose fp8bs_plan_t has form
 

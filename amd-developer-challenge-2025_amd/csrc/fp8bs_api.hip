@@ -40,6 +40,7 @@ bool variant_info(int tile, VariantInfo* out) {
         case FP8BS_VARIANT_SKINNY64x288: *out = {64, 288, 256}; return true;
         case FP8BS_VARIANT_T256x192: *out = {256, 192, 512}; return true;
         case FP8BS_VARIANT_T256x128S3: *out = {256, 128, 512}; return true;
+        case FP8BS_VARIANT_T256x128S3 | FORM1: *out = {128, 256, 512}; return true;
         case FP8BS_VARIANT_T192x192S3: *out = {192, 192, 512}; return true;
         case FP8BS_VARIANT_T64x256S3: *out = {64, 256, 512}; return true;
         case FP8BS_VARIANT_T64x256S3 | 2 * FORM1: *out = {16, 64, 512}; return true;
@@ -72,6 +73,9 @@ int forced_tile(int variant) { return variant < 256 ? variant : variant_of(varia
 // The small tiles whose workgroups hold all partitions of K (fp8bs_waves.h): up to eight, one launch, no workspace.
 constexpr int WAVES_MAX = 8;
 bool is_waves_tile(int tile) { return tile == (FP8BS_VARIANT_T64x256S3 | 2 * FORM1) || tile == (FP8BS_VARIANT_T64x256S3 | 3 * FORM1); }
+
+// The tile that only grouped calls take (fp8bs_tile_128x256s3.hip).
+bool is_grouped_tile(int tile) { return tile == (FP8BS_VARIANT_T256x128S3 | FORM1); }
 
 bool is_streaming_variant(int v) { return v == FP8BS_VARIANT_SKINNY64x144 || v == FP8BS_VARIANT_SKINNY64x256 || v == FP8BS_VARIANT_SKINNY64x288; }
 
@@ -120,8 +124,8 @@ bool can_sum_in_kernel(int m, int n, int tile, int split_k) {
 // Tiles with the fused silu-mul epilogue.
 bool has_epilogue(int tile) {
     switch (tile) {
-        case FP8BS_VARIANT_T256x256: case FP8BS_VARIANT_T256x128S3: case FP8BS_VARIANT_T64x128: case FP8BS_VARIANT_T64x128 | FORM1:
-        case FP8BS_VARIANT_T64x256S3: case FP8BS_VARIANT_T64x256S3 | FORM1: return true;
+        case FP8BS_VARIANT_T256x256: case FP8BS_VARIANT_T256x128S3: case FP8BS_VARIANT_T256x128S3 | FORM1:
+        case FP8BS_VARIANT_T64x128: case FP8BS_VARIANT_T64x128 | FORM1: case FP8BS_VARIANT_T64x256S3: case FP8BS_VARIANT_T64x256S3 | FORM1: return true;
         default: return is_waves_tile(tile);
     }
 }
@@ -451,6 +455,19 @@ GroupedPlan make_grouped_plan(int experts, int rows, int n, int k, int num_cus, 
     for (int r = 0; r < rows && unused > 1e-3; r++) unused *= 1.0 - 1.0 / experts;
     const double active = experts * (1.0 - unused), average = rows / active;
     const int kbt = k / KBLK;
+    // Some tens of rows an expert and weights that come from memory: one row of tiles has to hold an expert, or its weights are read twice. The model's
+    // averages do not see the experts that get more than 64 rows, and 128 rows leave b as many copies under way as 64 do. Measured on some 80 products
+    // (256 to 900 MB of weights, experts of equal and unequal shares) against the best other tile or the model's pick: 1.02 to 1.20 times as fast where some
+    // expert has more than 64 rows (160 tokens to 8 of 64 experts, 2048 x 2304, 68.6 -> 57.6 us; 240 to 8 of 32, 4864 x 3840, 153.0 -> 128.7), 0.97 to 1.02
+    // where none has; up to 16 rows the same. Not where 64x256 tiles, second rows of them too, are all on the chip at once (300 tokens to 4 of 32, 1280 x 7168,
+    // 72.0 us, this 75.9; 64 to 4 of 8, 6144 x 7168, 80.5 and 83.4). Above 44 rows some expert has more than 128 itself: only where an eighth more tiles takes no further round (512
+    // to 4 of 32, 3072 x 4096, 103.5 -> 93.6; where the rounds were full, 256 to 8 of 32, 4096 x 7168, 192.0, this 213.4).
+    if (split <= 1 && fp8bs::weights_past_caches(experts, rows, n, k) && rows > 16L * experts && rows <= 64L * experts) {
+        const long tiles = (long)experts * cdiv(n, 256), cus = num_cus;
+        const double share = (double)rows / experts;
+        const bool low_fit = tiles * (1.0 + share * share / 6400.0) <= cus;      // second rows of 64: 0.06 of the experts at 20 rows, 0.64 at 64, of unequal shares
+        if (!low_fit && (share <= 44.0 || (tiles + tiles / 8 + cus - 1) / cus == (tiles + cus - 1) / cus)) return {FP8BS_VARIANT_T256x128S3 | FORM1, 1};
+    }
     GroupedPlan best{FP8BS_VARIANT_T256x256, 1};
     double best_cost = 0;
     for (const Cand& c : cands) {
@@ -641,7 +658,7 @@ static int dense_call(const void* a, const void* b, const float* a_scale, const 
         VariantInfo vi{};
         const int tile = forced_tile(variant);
         variant = variant_of(variant);
-        if (!variant_info(tile, &vi)) return FP8BS_ERR_BAD_VARIANT;
+        if (!variant_info(tile, &vi) || is_grouped_tile(tile)) return FP8BS_ERR_BAD_VARIANT;
         if (is_streaming_variant(variant) && !simple) return FP8BS_ERR_BAD_VARIANT;
         if (is_streaming_variant(variant) && variant != FP8BS_VARIANT_SKINNY64x144 && (m % 4) != 0) return FP8BS_ERR_BAD_VARIANT;   // only the planner's width repairs a
         if (split_k < 0) {

@@ -35,6 +35,11 @@ struct GemmArgs {
 // 960 x 768, took 8.27 us instead of 8.18, means of three processes each in turn.)
 static_assert(sizeof(GemmArgs) <= 120);
 
+// The weights of a grouped call's experts, as many as can have rows, are as large as the 256 MB cache, and rows of them whole 128-byte lines.
+inline bool weights_past_caches(int experts, int rows, int n, int k) {
+    return (size_t)(rows < experts ? rows : experts) * (size_t)n * (size_t)k >= ((size_t)256 << 20) && n % 128 == 0;
+}
+
 // Or'ed into a mode: raise the LDS limit of the kernel that the arguments take and launch nothing (tiles of gemm_tr_kernel).
 constexpr int READY_ONLY = 256;
 
@@ -103,6 +108,7 @@ hipError_t launch_tile_256x256(const GemmArgs& args, int mode, hipStream_t strea
 hipError_t launch_tile_256x192(const GemmArgs& args, int mode, hipStream_t stream);
 hipError_t launch_tile_256x128(const GemmArgs& args, int mode, hipStream_t stream);
 hipError_t launch_tile_256x128s3(const GemmArgs& args, int mode, hipStream_t stream);
+hipError_t launch_tile_128x256s3(const GemmArgs& args, int mode, hipStream_t stream);
 hipError_t launch_tile_128x128(const GemmArgs& args, int mode, hipStream_t stream);
 hipError_t launch_tile_128x128s4(const GemmArgs& args, int mode, hipStream_t stream);
 hipError_t launch_tile_64x128(const GemmArgs& args, int mode, hipStream_t stream);

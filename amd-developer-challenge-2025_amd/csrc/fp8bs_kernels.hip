@@ -435,6 +435,7 @@ hipError_t launch_gemm(int tile, int mode, const GemmArgs& a, hipStream_t stream
         case 8: return launch_skinny<288, 3>(a, mode, stream);
         case 9: return launch_tile_256x192(a, mode, stream);
         case 10: return launch_tile_256x128s3(a, mode, stream);
+        case 10 | 256: return launch_tile_128x256s3(a, mode, stream);
         case 11: return launch_tile_192x192s3(a, mode, stream);
         case 12: return launch_tile_64x256s3(a, mode, stream);
         case 12 | 256: return launch_tile_128x128s4(a, mode, stream);
@@ -479,6 +480,7 @@ int variant_lds_bytes(int tile) {
         case 8: return SkinnyCfg<288, 3>::LDS_BYTES;
         case 9: return TileCfg<256, 192, 64, 96, 0>::LDS_BYTES;
         case 10: return TileCfg<256, 128, 64, 64, 0, 3>::LDS_BYTES;
+        case 10 | 256: return TileCfg<128, 256, 64, 64, 0, 3>::LDS_BYTES;
         case 11: return TileCfg<192, 192, 48, 96, 0, 3>::LDS_BYTES;
         case 12: return TileCfg<64, 256, 32, 64, 0, 3>::LDS_BYTES;
         case 12 | 256: return TileCfg<128, 128, 32, 64, 0, 4>::LDS_BYTES;

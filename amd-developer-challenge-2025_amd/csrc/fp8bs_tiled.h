@@ -1543,9 +1543,35 @@ static inline hipError_t launch_tr(const GemmArgs& a, dim3 grid, hipStream_t str
 // Rows of b are whole 128-byte lines: a line that two columns of tiles share would come from memory twice (100 tokens to 4 of 32, 3072 x 4096
 // 86.8 and 81.3, 2944 78.7 and 73.8; 3008 78.6 and 79.8, 3064 88.0 and 93.8, 3001 94.0 and 101.1).
 template <int BM> static inline bool b_read_once(const GemmArgs& a) {
-    const int used = a.m < a.num_experts ? a.m : a.num_experts;          // experts with rows, at most
-    return (size_t)used * (size_t)a.n * (size_t)a.k >= ((size_t)256 << 20) && (long)a.m * 4 <= (long)a.num_experts * (BM * 3)
-           && a.n % 128 == 0 && ((uintptr_t)a.b & 127) == 0;
+    return weights_past_caches(a.num_experts, a.m, a.n, a.k) && ((uintptr_t)a.b & 127) == 0 && (long)a.m * 4 <= (long)a.num_experts * (BM * 3);
+}
+
+// Persistent workgroups: as many as fit the chip at once (LDS and thread limits), each walks tiles  blockIdx.x, blockIdx.x + grid, ...
+template <class C>
+static inline long resident_workgroups(bool grouped) {
+    const int by_lds = 163840 / (C::LDS_BYTES + (grouped ? GROUP_TABLE_MAX * 16 : 0)), by_threads = 2048 / C::NTHREADS;   // (grouped: + the table of the experts)
+    return (long)device_cus() * (by_lds < by_threads ? by_lds : by_threads);
+}
+
+// A grouped call whose K is not split.
+template <int BM, int BN, int WM, int WN, bool WITH_EPI, int NSTAGE>
+static inline hipError_t launch_grouped(const GemmArgs& a, dim3 grid, hipStream_t stream) {
+    if constexpr (WITH_EPI) {
+        if (a.epi != 0 && a.epi != 1) return hipErrorInvalidValue;
+        // the tiles that the planner gives calls of few rows an expert
+        if constexpr (BN == 256)
+            if (b_read_once<BM>(a)) return a.epi == 1 ? launch_tr<BM, BN, WM, WN, 6, 1, NSTAGE>(a, grid, stream) : launch_tr<BM, BN, WM, WN, 6, 0, NSTAGE>(a, grid, stream);
+        if (a.epi == 1) return launch_tr<BM, BN, WM, WN, 2, 1, NSTAGE>(a, grid, stream);
+    }
+    return a.epi == 0 ? launch_tr<BM, BN, WM, WN, 2, 0, NSTAGE>(a, grid, stream) : hipErrorInvalidValue;
+}
+
+// A tile for such calls only.
+template <int BM, int BN, int WM, int WN, int NSTAGE>
+static inline hipError_t launch_grouped_shape(const GemmArgs& a, int mode, hipStream_t stream) {
+    if (mode != 2) return hipErrorInvalidValue;
+    const long total = grouped_slots_bound(a.m, a.num_experts, BM) * ((a.n + BN - 1) / BN), resident = resident_workgroups<TileCfg<BM, BN, WM, WN, 0, NSTAGE>>(true);
+    return launch_grouped<BM, BN, WM, WN, true, NSTAGE>(a, dim3((unsigned)(total < resident ? total : resident)), stream);
 }
 
 // WITH_EPI: the fused silu-mul epilogue is instantiated for this tile; GROUPED_SPLIT: the grouped walk with a K split is
@@ -1554,10 +1580,7 @@ static inline hipError_t launch_shape(const GemmArgs& a, int mode, hipStream_t s
     const bool ready_only = (mode & READY_ONLY) != 0;
     mode &= ~READY_ONLY;
     using C = TileCfg<BM, BN, WM, WN, 0, NSTAGE>;
-    // persistent workgroups: as many as fit the chip at once (LDS and thread limits), each walks
-    // tiles  blockIdx.x, blockIdx.x + grid, ...
-    const int by_lds = 163840 / (C::LDS_BYTES + (mode == 2 || mode == 5 ? GROUP_TABLE_MAX * 16 : 0)), by_threads = 2048 / C::NTHREADS;   // (grouped: + the table of the experts)
-    const long resident = (long)device_cus() * (by_lds < by_threads ? by_lds : by_threads);
+    const long resident = resident_workgroups<C>(mode == 2 || mode == 5);
     const int tiles_n = (a.n + BN - 1) / BN;
     long total;
     if (mode == 2 || mode == 5) {
@@ -1606,24 +1629,17 @@ static inline hipError_t launch_shape(const GemmArgs& a, int mode, hipStream_t s
         if constexpr (WITH_EPI) { if (a.epi == 1) return launch_summed(integral_constant<int, 4>{}, integral_constant<int, 1>{}); }
         return a.epi == 0 ? launch_summed(integral_constant<int, 4>{}, integral_constant<int, 0>{}) : hipErrorInvalidValue;
     }
-    // the tiles that the planner gives calls of few rows an expert
-    if constexpr (BN == 256 && WITH_EPI)
-        if (mode == 2 && b_read_once<BM>(a)) {
-            if (a.epi != 0 && a.epi != 1) return hipErrorInvalidValue;
-            return a.epi == 1 ? launch_tr<BM, BN, WM, WN, 6, 1, NSTAGE>(a, grid, stream) : launch_tr<BM, BN, WM, WN, 6, 0, NSTAGE>(a, grid, stream);
-        }
+    if (mode == 2) return launch_grouped<BM, BN, WM, WN, WITH_EPI, NSTAGE>(a, grid, stream);
     if (a.epi != 0) {
         // (with the reduce launch of a K split the planes are plain sums and the reduce kernel applies the epilogue)
         if constexpr (WITH_EPI) {
             if (a.epi != 1) return hipErrorInvalidValue;
             if (mode == 1) return launch_tr<BM, BN, WM, WN, 1, 0, NSTAGE>(a, grid, stream);
-            if (mode == 2) return launch_tr<BM, BN, WM, WN, 2, 1, NSTAGE>(a, grid, stream);
             return launch_tr<BM, BN, WM, WN, 0, 1, NSTAGE>(a, grid, stream);
         } else {
             return hipErrorInvalidValue;
         }
     }
-    if (mode == 2) return launch_tr<BM, BN, WM, WN, 2, 0, NSTAGE>(a, grid, stream);
     if (mode == 1) return launch_tr<BM, BN, WM, WN, 1, 0, NSTAGE>(a, grid, stream);
     return launch_tr<BM, BN, WM, WN, 0, 0, NSTAGE>(a, grid, stream);
 }
