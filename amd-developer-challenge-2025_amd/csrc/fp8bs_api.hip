@@ -10,6 +10,7 @@
 #include <stddef.h>
 #include <stdlib.h>
 #include <unistd.h>
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 
@@ -455,22 +456,23 @@ GroupedPlan make_grouped_plan(int experts, int rows, int n, int k, int num_cus, 
     for (int r = 0; r < rows && unused > 1e-3; r++) unused *= 1.0 - 1.0 / experts;
     const double active = experts * (1.0 - unused), average = rows / active;
     const int kbt = k / KBLK;
+    // 128x256 tiles (fp8bs_tile_128x256s3.hip) by the two rules below, never where 64x256 tiles, second rows of them too, are all on the chip at once (300
+    // tokens to 4 of 32, 1280 x 7168, 72.0 us, 128x256 75.9; 105 to 8 of 16, 2176 x 3584, 35.5 and 37.8).
+    const long tall_tiles = (long)experts * cdiv(n, 256), cus = num_cus;
+    const double share = (double)rows / experts;
+    const bool tall_may = split <= 1 && tall_tiles * (1.0 + share * share / 6400.0) > cus;         // second rows of 64: 0.06 of the experts at 20 rows, 0.64 at 64
     // Some tens of rows an expert and weights that come from memory: one row of tiles has to hold an expert, or its weights are read twice. The model's
     // averages do not see the experts that get more than 64 rows, and 128 rows leave b as many copies under way as 64 do. Measured on some 80 products
     // (256 to 900 MB of weights, experts of equal and unequal shares) against the best other tile or the model's pick: 1.02 to 1.20 times as fast where some
     // expert has more than 64 rows (160 tokens to 8 of 64 experts, 2048 x 2304, 68.6 -> 57.6 us; 240 to 8 of 32, 4864 x 3840, 153.0 -> 128.7), 0.97 to 1.02
-    // where none has; up to 16 rows the same. Not where 64x256 tiles, second rows of them too, are all on the chip at once (300 tokens to 4 of 32, 1280 x 7168,
-    // 72.0 us, this 75.9; 64 to 4 of 8, 6144 x 7168, 80.5 and 83.4). Above 44 rows some expert has more than 128 itself: only where an eighth more tiles takes no further round (512
+    // where none has; up to 16 rows the same. Above 44 rows some expert has more than 128 itself: only where an eighth more tiles takes no further round (512
     // to 4 of 32, 3072 x 4096, 103.5 -> 93.6; where the rounds were full, 256 to 8 of 32, 4096 x 7168, 192.0, this 213.4).
-    if (split <= 1 && fp8bs::weights_past_caches(experts, rows, n, k) && rows > 16L * experts && rows <= 64L * experts) {
-        const long tiles = (long)experts * cdiv(n, 256), cus = num_cus;
-        const double share = (double)rows / experts;
-        const bool low_fit = tiles * (1.0 + share * share / 6400.0) <= cus;      // second rows of 64: 0.06 of the experts at 20 rows, 0.64 at 64, of unequal shares
-        if (!low_fit && (share <= 44.0 || (tiles + tiles / 8 + cus - 1) / cus == (tiles + cus - 1) / cus)) return {FP8BS_VARIANT_T256x128S3 | FORM1, 1};
-    }
+    if (tall_may && fp8bs::weights_past_caches(experts, rows, n, k) && share > 16.0 && share <= 64.0
+        && (share <= 44.0 || (tall_tiles + tall_tiles / 8 + cus - 1) / cus == (tall_tiles + cus - 1) / cus)) return {FP8BS_VARIANT_T256x128S3 | FORM1, 1};
     GroupedPlan best{FP8BS_VARIANT_T256x256, 1};
     double best_cost = 0;
-    for (const Cand& c : cands) {
+    // more: as many tiles as expected, times this
+    auto model = [&](const Cand& c, int s, double more) {
         VariantInfo vi{};
         variant_info(c.tile, &vi);
         double slots = (average + 8.0) / vi.bm + 0.4;
@@ -478,22 +480,26 @@ GroupedPlan make_grouped_plan(int experts, int rows, int n, int k, int num_cus, 
         double fill = (average / slots + 24.0) / vi.bm;
         if (fill > 1.0) fill = 1.0;
         const double t_alone = c.t_few + (c.t_full - c.t_few) * fill;
+        const double wgs = active * slots * more * (double)cdiv(n, vi.bn) * s, per_round = (double)num_cus * c.rmax, kb = (double)cdiv(kbt, s);
+        auto t_block = [&](double w) {
+            double t = t_alone * (w > num_cus && c.rmax > 1 ? c.shared : 1.0);
+            const double power = c.t_power * fill * w / num_cus, stream = w * 128.0 * vi.bn / slots / (c.bw * 1e6);
+            t = power > t ? power : t;
+            return stream > t ? stream : t;
+        };
+        const double full = (double)(long)(wgs / per_round), rem = wgs - full * per_round;
+        double cost = full * (c.t_fixed + kb * t_block(per_round));
+        if (rem > 0.5) cost += c.t_fixed + kb * t_block(rem);
+        if (s > 1) cost += 3.56 + 0.757e-6 * s * (double)rows * (double)n;
+        return cost;
+    };
+    for (const Cand& c : cands) {
         for (int s = split ? split : 1; s <= (split ? split : 4); s++) {
             const GroupedPlan p{c.tile, s};
             if (s > 1 && !can_split_grouped(p, experts, rows, n, k)) break;
             // (partial tiles of 64 MB at most: beyond that a call has tiles enough without a split)
             if (s > 1 && !split && (kbt / s < 2 || grouped_bytes(p, experts, rows, n) > (64u << 20))) break;
-            const double wgs = active * slots * (double)cdiv(n, vi.bn) * s, per_round = (double)num_cus * c.rmax, kb = (double)cdiv(kbt, s);
-            auto t_block = [&](double w) {
-                double t = t_alone * (w > num_cus && c.rmax > 1 ? c.shared : 1.0);
-                const double power = c.t_power * fill * w / num_cus, stream = w * 128.0 * vi.bn / slots / (c.bw * 1e6);
-                t = power > t ? power : t;
-                return stream > t ? stream : t;
-            };
-            const double full = (double)(long)(wgs / per_round), rem = wgs - full * per_round;
-            double cost = full * (c.t_fixed + kb * t_block(per_round));
-            if (rem > 0.5) cost += c.t_fixed + kb * t_block(rem);
-            if (s > 1) cost += 3.56 + 0.757e-6 * s * (double)rows * (double)n;
+            double cost = model(c, s, 1.0);
             // With more than 32 rows per expert the model flatters the smaller tiles against this one: 640 tokens to 4 of 32 experts,
             // 3664 x 5376, 128x128 in eight waves 217 us, this 169; 704 to 8 of 32, 2176 x 1280, 39.2 and 35.2; 931 to 8 of 16, 3806 x
             // 5888, 256x128 278, this 260.  Over 480 further shapes of the same ranges and wider ones any factor from 0.85 to 0.95 brings
@@ -502,6 +508,13 @@ GroupedPlan make_grouped_plan(int experts, int rows, int n, int k, int num_cus, 
             if (best_cost == 0 || cost < best_cost) { best = p; best_cost = cost; }
         }
     }
+    // From 44 to 128 rows an expert one row of 128x256 tiles holds an expert of the average size. The constants are a fit (12 % off in the mean) to 420 drawn
+    // calls (8 to 128 experts, 10 to 420 rows each, 512 .. 7168 x 512 .. 7168). It is taken where it is ahead by 4 % with a twentieth more tiles than
+    // expected: the unequal shares that the averages hide cost it a round where the last is full. 260 further calls of 40 to 132 rows: 81 took it by one of
+    // the rules, 1.11 times as fast in the geometric mean, 0.95 to 1.28 (704 tokens to 4 of 32, 4864 x 4608, 193.0 -> 150.0 us; 344 to 8 of 32, 1536
+    // x 1920, 31.9 -> 24.3). Beyond 128 rows the model errs too often: of the drawn calls it gains 2 %, and loses 12 to 21 % on some.
+    const Cand tall{FP8BS_VARIANT_T256x128S3 | FORM1, 1, 0.960, 0.628, 0.637, 5.33, 1.0, 5.98};
+    if (tall_may && share > 44.0 && share <= 128.0 && best_cost > 1.04 * std::max(model(tall, 1, 1.0), model(tall, 1, 1.05))) best = {tall.tile, 1};
     return best;
 }
 GroupedPlan choose_grouped(int experts, int rows, int n, int k, int num_cus, int split) {
