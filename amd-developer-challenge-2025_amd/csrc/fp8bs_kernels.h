@@ -40,6 +40,12 @@ inline bool weights_past_caches(int experts, int rows, int n, int k) {
     return (size_t)(rows < experts ? rows : experts) * (size_t)n * (size_t)k >= ((size_t)256 << 20) && n % 128 == 0;
 }
 
+// Whether the weights of an expert of so many tile rows are read past the caches, beside so many experts that have rows (see `b_read_once`).
+constexpr unsigned long long ALL_CACHES = 288ull << 20;          // 256 MB and the L2s of the eight XCDs
+__host__ __device__ constexpr bool expert_read_once(int experts_with_rows, int tile_rows, int n, int k) {
+    return tile_rows == 1 && (unsigned long long)experts_with_rows * ((unsigned long long)n * (unsigned long long)k) >= ALL_CACHES;
+}
+
 // Or'ed into a mode: raise the LDS limit of the kernel that the arguments take and launch nothing (tiles of gemm_tr_kernel).
 constexpr int READY_ONLY = 256;
 

@@ -67,10 +67,12 @@ __device__ __forceinline__ void copy16_global_to_lds(__amdgpu_buffer_rsrc_t rsrc
     asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, %3 offen lds"
                  :: "v"(lane_offset), "s"(rsrc), "s"(lds_base), "s"(wave_offset) : "memory", "m0");
 }
-// same, for bytes that are not read again: neither the L2 nor the 256 MB cache behind it makes room for them
-__device__ __forceinline__ void copy16_global_to_lds_once(__amdgpu_buffer_rsrc_t rsrc, uint32_t lds_base, uint32_t lane_offset, uint32_t wave_offset) {
-    asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, %3 offen nt lds"
-                 :: "v"(lane_offset), "s"(rsrc), "s"(lds_base), "s"(wave_offset) : "memory", "m0");
+// same, with the nontemporal hint where `once` is not zero.  (The hint is a bit of the instruction.  The branch stands inside the assembly: the
+// K loop stays one straight-line block to the compiler.  It costs what two runs differ by, 0.6 us at most: 20 experts of 8 MB 30.2 and 30.8.)
+__device__ __forceinline__ void copy16_global_to_lds_once(__amdgpu_buffer_rsrc_t rsrc, uint32_t lds_base, uint32_t lane_offset, uint32_t wave_offset, uint32_t once) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_cmp_eq_u32 %4, 0\n\ts_cbranch_scc1 0f\n\tbuffer_load_dwordx4 %0, %1, %3 offen nt lds\n\ts_branch 1f\n"
+                 "0:\tbuffer_load_dwordx4 %0, %1, %3 offen lds\n1:"
+                 :: "v"(lane_offset), "s"(rsrc), "s"(lds_base), "s"(wave_offset), "s"(once) : "memory", "m0", "scc");
 }
 // same with 4 bytes per lane: lane l's dword lands at lds_base + 4*l
 __device__ __forceinline__ void copy4_global_to_lds(__amdgpu_buffer_rsrc_t rsrc, uint32_t lds_base, uint32_t lane_offset, uint32_t wave_offset) {
@@ -117,7 +119,7 @@ __device__ __forceinline__ void band_tile(int v, int tiles_m, int tiles_n, int g
 //   MODE 3  : dense, K blocks instead of tiles dealt to the workgroups, partial tiles through the workspace, bf16 output
 //   MODE 4  : dense split-K, partial tiles to the workspace, the sum of a tile shared out among its workgroups or done by the last of them, bf16 output
 //   MODE 5  : grouped like MODE 2 with a K split summed like MODE 4's
-//   MODE 6  : MODE 2 with b read past the caches (the hint is part of the load instruction), see the rule at `b_read_once`
+//   MODE 6  : MODE 2 with b read past the caches for the experts of one tile row, see the rule at `b_read_once`
 // LDS: NSTAGE stages, each [128 k][BM] bytes of A then [128 k][BN] bytes of B, 16-byte chunks XOR-swizzled
 // so that the 16 k rows touched by half a wave in one transposing read fall on 16 different 16-byte
 // bank groups, then the k block's a_scale row and b_scale values.
@@ -272,11 +274,13 @@ void gemm_tr_kernel(const GemmArgs p) {
     // epilogue are a third of a tile's time otherwise).
     struct Tile {
         int valid, m0, n0, n_hi, kb_begin, kb_end, split_z, row_lo, row_hi;
+        uint32_t once;                        // MODE 6: b is read past the caches
         int sk_contrib, sk_first;             // MODE 3: the segment ends before the tile's last K block; first workgroup of the tile's earlier segments (-1: none)
         const uint8_t* bptr;
         const float* bsptr;
     };
     int total_slots = 0;                      // grouped: m-tile slots that exist (from row_offsets)
+    [[maybe_unused]] int active = 0;          // MODE 6: experts that have rows
     // Grouped, fewer than GROUP_TABLE_MAX experts: a table in LDS, one entry per expert - first row of its first
     // tile (row_offsets[e] rounded down to 16), its row range, and the number of slots before it - built once
     // by wave 0.  Finding a tile's expert is then one LDS read per lane and a count of the lanes whose experts
@@ -307,6 +311,7 @@ void gemm_tr_kernel(const GemmArgs p) {
             incl += __builtin_amdgcn_update_dpp(0, incl, 0x143, 0xC, 0xF, false);      // row_bcast:31, into rows 2 and 3
             if (lane < p.num_experts) lane_entry = (v4i){s, lo, hi, incl - nt};
             total_slots = __builtin_amdgcn_readlane(incl, 63);
+            if constexpr (B_ONCE) active = __popcll(__ballot(nt > 0));
         } else if (use_table) {
             if (wave == 0) {
                 int carry = 0;
@@ -325,16 +330,19 @@ void gemm_tr_kernel(const GemmArgs p) {
                     }
                     if (x < p.num_experts) gtable_store[x] = (v4i){s, lo, hi, carry + incl - nt};
                     carry += __shfl(incl, 63, 64);
+                    if constexpr (B_ONCE) active += __popcll(__ballot(nt > 0));
                 }
-                if (lane == 0) gtable_store[p.num_experts] = (v4i){0, 0, 0, carry};
+                if (lane == 0) gtable_store[p.num_experts] = (v4i){active, 0, 0, carry};
             }
             __syncthreads();
             total_slots = __builtin_amdgcn_readfirstlane(gtable_store[p.num_experts][3]);
+            if constexpr (B_ONCE) active = __builtin_amdgcn_readfirstlane(gtable_store[p.num_experts][0]);
         } else {
             for (int x = 0; x < p.num_experts; x++) {
                 int lo = p.row_offsets[x], hi = p.row_offsets[x + 1];
                 lo = lo < 0 ? 0 : lo; hi = hi > p.m ? p.m : hi;
                 total_slots += (hi > lo) ? (hi - (lo & ~15) + BM - 1) / BM : 0;
+                if constexpr (B_ONCE) active += hi > lo ? 1 : 0;
             }
         }
         if constexpr (MODE == 5) {             // a malformed table must not reach beyond the workspace either
@@ -406,7 +414,7 @@ void gemm_tr_kernel(const GemmArgs p) {
     auto pick_tile = [&](int it) -> Tile {
         Tile t;
         t.valid = 0; t.m0 = 0; t.n0 = 0; t.n_hi = p.n; t.kb_begin = 0; t.kb_end = 0; t.split_z = 0; t.row_lo = 0; t.row_hi = p.m;
-        t.sk_contrib = 0; t.sk_first = -1;
+        t.sk_contrib = 0; t.sk_first = -1; t.once = 0;
         t.bptr = p.b; t.bsptr = p.bs;
         const int G = gridDim.x;
         if (MODE == 3) {
@@ -503,6 +511,7 @@ void gemm_tr_kernel(const GemmArgs p) {
                     if (by_expert) band_tile(v - before * tiles_n, nt, tiles_n, nt <= 8 ? nt : p.band_h, slot, tn);
                     found = slot < nt;
                     start = s + slot * BM;
+                    if constexpr (B_ONCE) t.once = expert_read_once(active, nt, p.n, p.k) ? 1u : 0u;
                 }
             } else {
                 int acc_slots = 0;
@@ -515,6 +524,7 @@ void gemm_tr_kernel(const GemmArgs p) {
                         int slot = slot_all - acc_slots;
                         if (by_expert) band_tile(v - acc_slots * tiles_n, nt, tiles_n, nt <= 8 ? nt : p.band_h, slot, tn);
                         found = 1; e = x; start = s + slot * BM; cnt_lo = lo; cnt_hi = hi;
+                        if constexpr (B_ONCE) t.once = expert_read_once(active, nt, p.n, p.k) ? 1u : 0u;
                     }
                     acc_slots += nt;
                 }
@@ -587,6 +597,7 @@ void gemm_tr_kernel(const GemmArgs p) {
         uint32_t b_voffq[C::B_LOADS];           // only without B_ROWS_WHOLE
         uint32_t a_voffq[C::A_LOADS];           // only without A_ROWS_WHOLE
         int kb_begin;
+        uint32_t once;                          // only with B_ONCE
         __amdgpu_buffer_rsrc_t b_rsrc, sc_rsrc;
     };
     auto copy_plan = [&](const Tile& t) -> CopyPlan {
@@ -635,6 +646,7 @@ void gemm_tr_kernel(const GemmArgs p) {
         r = r < last ? r : last;
         c.sc_voff = (uint32_t)r * 4u;
         c.kb_begin = t.kb_begin;
+        c.once = __builtin_amdgcn_readfirstlane(t.once);
         c.b_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)t.bptr, 0, b_bytes, 0x00020000);
         c.sc_rsrc = __builtin_amdgcn_make_buffer_rsrc(sc_is_b ? (void*)t.bsptr : (void*)p.as, 0,
                                                       sc_is_b ? (uint32_t)(p.k / KBLK) * (uint32_t)p.nb * 4u
@@ -665,7 +677,7 @@ void gemm_tr_kernel(const GemmArgs p) {
         } else if constexpr (q < C::A_LOADS + C::B_LOADS) {
             constexpr int qb = q - C::A_LOADS;
             if constexpr (B_ONCE)
-                copy16_global_to_lds_once(cp.b_rsrc, sa + C::A_BYTES + qb * C::NWAVES * 1024, cp.b_voff, kb * b_kstep + (uint32_t)(qb * ROWS_PER_COPY_B) * (uint32_t)p.n);
+                copy16_global_to_lds_once(cp.b_rsrc, sa + C::A_BYTES + qb * C::NWAVES * 1024, cp.b_voff, kb * b_kstep + (uint32_t)(qb * ROWS_PER_COPY_B) * (uint32_t)p.n, cp.once);
             else if constexpr (B_ROWS_WHOLE)
                 copy16_global_to_lds(cp.b_rsrc, sa + C::A_BYTES + qb * C::NWAVES * 1024, cp.b_voff, kb * b_kstep + (uint32_t)(qb * ROWS_PER_COPY_B) * (uint32_t)p.n);
             else
@@ -1533,17 +1545,22 @@ static inline hipError_t launch_tr(const GemmArgs& a, dim3 grid, hipStream_t str
     return hipGetLastError();
 }
 
-// The experts' weights are read past the caches where nothing of them can be found there again: together they are as large as the 256 MB
-// cache, which a pass over them leaves with none of what the next one reads first, and an expert has so few rows that one row of tiles, and so
-// one workgroup for a column of them, reads its weights.  What is left in the caches is then a, of which every workgroup of an XCD reads the same lines
-// (128 bytes for an expert's 16 or so), and the memory answers sooner.  us, as before and so (32 experts, 8 a token, 4096 x 7168 but where said): 32
-// tokens 162.9 and 148.7, 64 tokens 182.7 and 168.4, 7168 x 2048 97.0 and 91.7; 128 tokens in 256x256 197.6 and 183.8, 512 tokens 230.3 and 219.8, unevenly
-// spread 275.6 and 261.8, 768 tokens (24 rows in 32) 252.2 and 239.5, unevenly 302.1 and 301.1.  Beyond that line a second row of tiles reads them from
-// memory again: 256 tokens in 64x256 245.8 and 272.5, 1024 in 256x256 364 and 392.  Weights that the cache would hold: 250 x 4096 x 7168 17.8 and 24.4.
+// The experts' weights are read past the caches where nothing of them is found there again: those that the call reads are as large as the caches together,
+// and one row of tiles, so one workgroup for a column of them, holds the expert.  The instantiation is chosen here, by what the host knows; how many
+// experts have rows, and how many tile rows this one has, the kernel sees (`expert_read_once`).  What such a call gives up nothing for and gains by:
+// b does not push out a, of which every workgroup of an XCD reads the same lines (128 bytes for an expert's 16 rows or so).  That this is why is not shown: the
+// figures are.  us, MODE 2 and so (32 experts, rows by chance, 4096 x 7168 but where said): 256 rows 166.0 and 152.1, 7168 x 2048 90.2 and 84.1; 1024
+// rows in 128x256 177.5 and 164.1; 6144 in 256x256, 4096 x 4096, 153.2 and 144.3; one expert with half of 1024 rows 202.0 and 198.4, of 1024 to 64
+// experts, 2048 x 7168, 193.3 and 196.2, the largest loss of 48 (hint for all tiles: 199.5); 3072 rows in 128x256, 4096 x 4096, shares of 2 to 500: 134.3 and 126.7 (140.4).
+// The line on the average: beyond it few experts have one row of tiles, and the gain goes: 64x256 at 32, 64 and 80 rows an expert 1.01-1.10, 1.01-1.04,
+// 1.00-1.04 times as fast, 128x256 at 96, 112 and 128 rows 1.04-1.10, 0.98-1.08, 0.99-1.05, 256x256 at 192 and 250 rows 1.03-1.16, 1.02-1.06 (three shapes, three draws).
+// Bytes: streamed, weights between products of others, the hint gains at any size (20 experts of 8 MB 39.0 -> 35.8), but read again with nothing in between
+// smaller ones are found in the cache: the same 30.2 and 33.8, 28 experts 35.7 and 40.0, 32 of 8 MB 41.1 and 45.7, 28 of 10 MB 47.5 and 48.8, 21 of 14 MB 54.0 and
+// 54.1, 30 of 10 MB 54.0 and 52.8, 32 of 10 MB 63.9 and 56.1: the line is where neither loses.
 // Rows of b are whole 128-byte lines: a line that two columns of tiles share would come from memory twice (100 tokens to 4 of 32, 3072 x 4096
 // 86.8 and 81.3, 2944 78.7 and 73.8; 3008 78.6 and 79.8, 3064 88.0 and 93.8, 3001 94.0 and 101.1).
 template <int BM> static inline bool b_read_once(const GemmArgs& a) {
-    return weights_past_caches(a.num_experts, a.m, a.n, a.k) && ((uintptr_t)a.b & 127) == 0 && (long)a.m * 4 <= (long)a.num_experts * (BM * 3);
+    return expert_read_once(a.m < a.num_experts ? a.m : a.num_experts, 1, a.n, a.k) && a.n % 128 == 0 && ((uintptr_t)a.b & 127) == 0 && (long)a.m * 4 <= (long)a.num_experts * (BM * 3);
 }
 
 // Persistent workgroups: as many as fit the chip at once (LDS and thread limits), each walks tiles  blockIdx.x, blockIdx.x + grid, ...
