@@ -68,7 +68,7 @@ __device__ __forceinline__ void copy16_global_to_lds(__amdgpu_buffer_rsrc_t rsrc
                  :: "v"(lane_offset), "s"(rsrc), "s"(lds_base), "s"(wave_offset) : "memory", "m0");
 }
 // same, with the nontemporal hint where `once` is not zero.  (The hint is a bit of the instruction.  The branch stands inside the assembly: the
-// K loop stays one straight-line block to the compiler.  It costs what two runs differ by, 0.6 us at most: 20 experts of 8 MB 30.2 and 30.8.)
+// K loop stays one straight-line block to the compiler.  It costs nothing that shows: 256 rows to 32 experts, 4096 x 7168, 152.7 and 152.3.)
 __device__ __forceinline__ void copy16_global_to_lds_once(__amdgpu_buffer_rsrc_t rsrc, uint32_t lds_base, uint32_t lane_offset, uint32_t wave_offset, uint32_t once) {
     asm volatile("s_mov_b32 m0, %2\n\ts_cmp_eq_u32 %4, 0\n\ts_cbranch_scc1 0f\n\tbuffer_load_dwordx4 %0, %1, %3 offen nt lds\n\ts_branch 1f\n"
                  "0:\tbuffer_load_dwordx4 %0, %1, %3 offen lds\n1:"
@@ -272,15 +272,18 @@ void gemm_tr_kernel(const GemmArgs p) {
     // issues the first K block of the next tile before it converts and stores the current one, so a
     // tile's output and the next tile's first loads overlap (with K = 2048 the per-tile prologue and
     // epilogue are a third of a tile's time otherwise).
+    // (No member for one mode only: with one more the compiler keeps parts of a tile in scratch memory, also in modes that do not use it, and 2197 rows to 64
+    // experts, 1920 x 1408 in 256x256, takes 50.0 us instead of 47.3.)
     struct Tile {
         int valid, m0, n0, n_hi, kb_begin, kb_end, split_z, row_lo, row_hi;
-        uint32_t once;                        // MODE 6: b is read past the caches
         int sk_contrib, sk_first;             // MODE 3: the segment ends before the tile's last K block; first workgroup of the tile's earlier segments (-1: none)
+                                              // MODE 6: sk_contrib: b is read past the caches
         const uint8_t* bptr;
         const float* bsptr;
     };
     int total_slots = 0;                      // grouped: m-tile slots that exist (from row_offsets)
     [[maybe_unused]] int active = 0;          // MODE 6: experts that have rows
+    [[maybe_unused]] int once_rows = 0;       // the tile rows of an expert whose weights are read past the caches, 0: none
     // Grouped, fewer than GROUP_TABLE_MAX experts: a table in LDS, one entry per expert - first row of its first
     // tile (row_offsets[e] rounded down to 16), its row range, and the number of slots before it - built once
     // by wave 0.  Finding a tile's expert is then one LDS read per lane and a count of the lanes whose experts
@@ -345,6 +348,7 @@ void gemm_tr_kernel(const GemmArgs p) {
                 if constexpr (B_ONCE) active += hi > lo ? 1 : 0;
             }
         }
+        if constexpr (B_ONCE) once_rows = expert_read_once(active, 1, p.n, p.k) ? 1 : 0;
         if constexpr (MODE == 5) {             // a malformed table must not reach beyond the workspace either
             const int bound = (int)grouped_slots_bound(p.m, p.num_experts, BM);
             total_slots = total_slots < bound ? total_slots : bound;
@@ -414,7 +418,7 @@ void gemm_tr_kernel(const GemmArgs p) {
     auto pick_tile = [&](int it) -> Tile {
         Tile t;
         t.valid = 0; t.m0 = 0; t.n0 = 0; t.n_hi = p.n; t.kb_begin = 0; t.kb_end = 0; t.split_z = 0; t.row_lo = 0; t.row_hi = p.m;
-        t.sk_contrib = 0; t.sk_first = -1; t.once = 0;
+        t.sk_contrib = 0; t.sk_first = -1;
         t.bptr = p.b; t.bsptr = p.bs;
         const int G = gridDim.x;
         if (MODE == 3) {
@@ -511,7 +515,7 @@ void gemm_tr_kernel(const GemmArgs p) {
                     if (by_expert) band_tile(v - before * tiles_n, nt, tiles_n, nt <= 8 ? nt : p.band_h, slot, tn);
                     found = slot < nt;
                     start = s + slot * BM;
-                    if constexpr (B_ONCE) t.once = expert_read_once(active, nt, p.n, p.k) ? 1u : 0u;
+                    if constexpr (B_ONCE) t.sk_contrib = nt == once_rows;
                 }
             } else {
                 int acc_slots = 0;
@@ -524,7 +528,7 @@ void gemm_tr_kernel(const GemmArgs p) {
                         int slot = slot_all - acc_slots;
                         if (by_expert) band_tile(v - acc_slots * tiles_n, nt, tiles_n, nt <= 8 ? nt : p.band_h, slot, tn);
                         found = 1; e = x; start = s + slot * BM; cnt_lo = lo; cnt_hi = hi;
-                        if constexpr (B_ONCE) t.once = expert_read_once(active, nt, p.n, p.k) ? 1u : 0u;
+                        if constexpr (B_ONCE) t.sk_contrib = nt == once_rows;
                     }
                     acc_slots += nt;
                 }
@@ -596,8 +600,7 @@ void gemm_tr_kernel(const GemmArgs p) {
         uint32_t a_voff, b_voff, sc_voff;
         uint32_t b_voffq[C::B_LOADS];           // only without B_ROWS_WHOLE
         uint32_t a_voffq[C::A_LOADS];           // only without A_ROWS_WHOLE
-        int kb_begin;
-        uint32_t once;                          // only with B_ONCE
+        int kb_begin;                           // with B_ONCE, whose tiles begin at block 0: whether b is read past the caches
         __amdgpu_buffer_rsrc_t b_rsrc, sc_rsrc;
     };
     auto copy_plan = [&](const Tile& t) -> CopyPlan {
@@ -645,8 +648,7 @@ void gemm_tr_kernel(const GemmArgs p) {
         const int last = (sc_is_b ? p.nb : p.lda) - 1;
         r = r < last ? r : last;
         c.sc_voff = (uint32_t)r * 4u;
-        c.kb_begin = t.kb_begin;
-        c.once = __builtin_amdgcn_readfirstlane(t.once);
+        c.kb_begin = B_ONCE ? __builtin_amdgcn_readfirstlane(t.sk_contrib) : t.kb_begin;
         c.b_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)t.bptr, 0, b_bytes, 0x00020000);
         c.sc_rsrc = __builtin_amdgcn_make_buffer_rsrc(sc_is_b ? (void*)t.bsptr : (void*)p.as, 0,
                                                       sc_is_b ? (uint32_t)(p.k / KBLK) * (uint32_t)p.nb * 4u
@@ -668,7 +670,7 @@ void gemm_tr_kernel(const GemmArgs p) {
     auto issue_one = [&](const CopyPlan& cp, int stage, int blk, auto q_tag) {
         constexpr int q = decltype(q_tag)::value;
         const uint32_t sa = lds_base + stage * C::STAGE_BYTES + wave * 1024;
-        const uint32_t kb = (uint32_t)(cp.kb_begin + blk);
+        const uint32_t kb = (uint32_t)((B_ONCE ? 0 : cp.kb_begin) + blk);
         if constexpr (q < C::A_LOADS) {
             if constexpr (A_ROWS_WHOLE)
                 copy16_global_to_lds(a_rsrc, sa + q * C::NWAVES * 1024, cp.a_voff, kb * a_kstep + (uint32_t)(q * ROWS_PER_COPY_A) * (uint32_t)p.lda);
@@ -677,7 +679,7 @@ void gemm_tr_kernel(const GemmArgs p) {
         } else if constexpr (q < C::A_LOADS + C::B_LOADS) {
             constexpr int qb = q - C::A_LOADS;
             if constexpr (B_ONCE)
-                copy16_global_to_lds_once(cp.b_rsrc, sa + C::A_BYTES + qb * C::NWAVES * 1024, cp.b_voff, kb * b_kstep + (uint32_t)(qb * ROWS_PER_COPY_B) * (uint32_t)p.n, cp.once);
+                copy16_global_to_lds_once(cp.b_rsrc, sa + C::A_BYTES + qb * C::NWAVES * 1024, cp.b_voff, kb * b_kstep + (uint32_t)(qb * ROWS_PER_COPY_B) * (uint32_t)p.n, (uint32_t)cp.kb_begin);
             else if constexpr (B_ROWS_WHOLE)
                 copy16_global_to_lds(cp.b_rsrc, sa + C::A_BYTES + qb * C::NWAVES * 1024, cp.b_voff, kb * b_kstep + (uint32_t)(qb * ROWS_PER_COPY_B) * (uint32_t)p.n);
             else
@@ -1549,9 +1551,9 @@ static inline hipError_t launch_tr(const GemmArgs& a, dim3 grid, hipStream_t str
 // and one row of tiles, so one workgroup for a column of them, holds the expert.  The instantiation is chosen here, by what the host knows; how many
 // experts have rows, and how many tile rows this one has, the kernel sees (`expert_read_once`).  What such a call gives up nothing for and gains by:
 // b does not push out a, of which every workgroup of an XCD reads the same lines (128 bytes for an expert's 16 rows or so).  That this is why is not shown: the
-// figures are.  us, MODE 2 and so (32 experts, rows by chance, 4096 x 7168 but where said): 256 rows 166.0 and 152.1, 7168 x 2048 90.2 and 84.1; 1024
-// rows in 128x256 177.5 and 164.1; 6144 in 256x256, 4096 x 4096, 153.2 and 144.3; one expert with half of 1024 rows 202.0 and 198.4, of 1024 to 64
-// experts, 2048 x 7168, 193.3 and 196.2, the largest loss of 48 (hint for all tiles: 199.5); 3072 rows in 128x256, 4096 x 4096, shares of 2 to 500: 134.3 and 126.7 (140.4).
+// figures are.  us, MODE 2 and so (32 experts, rows by chance, 4096 x 7168 but where said): 256 rows 166.5 and 152.4, 7168 x 2048 90.5 and 84.0; 1024
+// rows in 128x256 177.9 and 164.1; 6144 in 256x256, 4096 x 4096, 153.2 and 144.3; one expert with half of 1024 rows 202.7 and 197.2; of 1024 to 64
+// experts, 2048 x 7168, 194.0 and 196.2, the largest loss of 48 (hint for all tiles: 199.4); 2048 rows in 128x256, 4096 x 4096, shares up to 303: 120.3 and 113.3 (126.1).
 // The line on the average: beyond it few experts have one row of tiles, and the gain goes: 64x256 at 32, 64 and 80 rows an expert 1.01-1.10, 1.01-1.04,
 // 1.00-1.04 times as fast, 128x256 at 96, 112 and 128 rows 1.04-1.10, 0.98-1.08, 0.99-1.05, 256x256 at 192 and 250 rows 1.03-1.16, 1.02-1.06 (three shapes, three draws).
 // Bytes: streamed, weights between products of others, the hint gains at any size (20 experts of 8 MB 39.0 -> 35.8), but read again with nothing in between
