@@ -46,6 +46,9 @@ __host__ __device__ constexpr bool expert_read_once(int experts_with_rows, int t
     return tile_rows == 1 && (unsigned long long)experts_with_rows * ((unsigned long long)n * (unsigned long long)k) >= ALL_CACHES;
 }
 
+// Whether a grouped call across the experts deals a workgroup other columns of b in each round of tiles (see `place` in fp8bs_tiled.h).
+__host__ __device__ constexpr bool turns_rounds(int n) { return n % 512 == 0; }
+
 // Or'ed into a mode: raise the LDS limit of the kernel that the arguments take and launch nothing (tiles of gemm_tr_kernel).
 constexpr int READY_ONLY = 256;
 

@@ -370,20 +370,23 @@ void gemm_tr_kernel(const GemmArgs p) {
     [[maybe_unused]] constexpr int SPREAD_ROUNDS = 12;
     constexpr int MOST_CUT = (MODE == 0 || MODE == 2 || MODE == 6) && BN == 256 ? (BN / WN >= 4 ? 2 : 1) : 0;
     // Across the experts, where a call is a stream of their weights, an XCD's workgroups change places from round to round, by a band's
-    // rows - one n tile - each time.  Rows of b that are a multiple of 1024 bytes apart put a column of b into one eighth of the address bits 7 to 9,
-    // and the memory serves one of the eight, 384 to 511, at 0.8 of the others' rate (64x256 tiles of 64 x 18432 x 7168: the fourth that holds
+    // rows - one n tile - each time, if rows of b are a multiple of 512 bytes apart.  A column of b then has the same address bits 7 and 8 in each row, and
+    // the memory serves one eighth of the bits 7 to 9, 384 to 511, at 0.8 of the others' rate (64x256 tiles of 64 x 18432 x 7168: the fourth that holds
     // those bytes ends its K blocks at 26.5 us, the others at 20.3; with b 256 bytes further on it is the tiles beside them; rows 4352
     // apart: none).  A round being a multiple of the period, a workgroup had such a tile in every round or in none.  us, before and
     // now: 32 tokens to 8 of 32 experts, 4096 x 7168, 177.1 and 170.2; 64 to 8 of 32, 7168 x 2048, 102.7 and 97.1; 8 to 4 of 32, 4096 x 7168, 127.8
-    // and 120.9; 3072 x 7168 142.4 and 142.8.  Not in a round that is cut, whose places are other ones (3072 x 7168, 1.5 rounds: 145.7), and not
-    // expert by expert, where the weights are read once for many rows (4096 tokens, 4096 x 7168: 921 as it is, 929 turned).
+    // and 120.9; 8 rows to each of 32, 3584 x 1536, 38.8 and 37.6, 4608 x 1536 49.8 and 48.9; 3072 x 7168 142.4 and 142.8.  Elsewhere columns drift
+    // through all of the bits, and turning only takes tiles from the panels that their neighbours read: 110 such calls (1 .. 37 rows an expert, 512 .. 7168 columns) 0.25 %
+    // slower in the geometric mean, at worst 1.7 % (64 experts, 3328 x 2816, 118.8 and 120.8), so there it is left.  Not in a round that is cut, whose
+    // places are other ones (3072 x 7168, 1.5 rounds: 145.7), and not expert by expert, where the weights are read once for many rows (4096 tokens, 4096 x
+    // 7168: 921 as it is, 929 turned).
     [[maybe_unused]] int turn = 0;
     auto place = [&](int it, int total, int& part, int& cut) -> int {
         const int G = gridDim.x, first = it * G, here = total - first;
         int wg = blockIdx.x;
         if (here <= 0) return -1;
         if constexpr (GROUPED)
-            if (it > 0 && !p.by_expert && (G >> 3) >= p.band_h) {
+            if (it > 0 && !p.by_expert && (G >> 3) >= p.band_h && turns_rounds(p.n)) {
                 const int x = blockIdx.x & 7, run = (G >> 3) + (x < (G & 7) ? 1 : 0), at = (int)(blockIdx.x >> 3);      // workgroups of this XCD, this one's place among them
                 turn += p.band_h;
                 if (turn >= run) turn -= run;
