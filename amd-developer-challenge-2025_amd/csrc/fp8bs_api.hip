@@ -460,15 +460,8 @@ GroupedPlan make_grouped_plan(int experts, int rows, int n, int k, int num_cus, 
     // tokens to 4 of 32, 1280 x 7168, 72.0 us, 128x256 75.9; 105 to 8 of 16, 2176 x 3584, 35.5 and 37.8).
     const long tall_tiles = (long)experts * cdiv(n, 256), cus = num_cus;
     const double share = (double)rows / experts;
-    const bool tall_may = split <= 1 && tall_tiles * (1.0 + share * share / 6400.0) > cus;         // second rows of 64: 0.06 of the experts at 20 rows, 0.64 at 64
-    // Some tens of rows an expert and weights that come from memory: one row of tiles has to hold an expert, or its weights are read twice. The model's
-    // averages do not see the experts that get more than 64 rows, and 128 rows leave b as many copies under way as 64 do. Measured on some 80 products
-    // (256 to 900 MB of weights, experts of equal and unequal shares) against the best other tile or the model's pick: 1.02 to 1.20 times as fast where some
-    // expert has more than 64 rows (160 tokens to 8 of 64 experts, 2048 x 2304, 68.6 -> 57.6 us; 240 to 8 of 32, 4864 x 3840, 153.0 -> 128.7), 0.97 to 1.02
-    // where none has; up to 16 rows the same. Above 44 rows some expert has more than 128 itself: only where an eighth more tiles takes no further round (512
-    // to 4 of 32, 3072 x 4096, 103.5 -> 93.6; where the rounds were full, 256 to 8 of 32, 4096 x 7168, 192.0, this 213.4).
-    if (tall_may && fp8bs::weights_past_caches(experts, rows, n, k) && share > 16.0 && share <= 64.0
-        && (share <= 44.0 || (tall_tiles + tall_tiles / 8 + cus - 1) / cus == (tall_tiles + cus - 1) / cus)) return {FP8BS_VARIANT_T256x128S3 | FORM1, 1};
+    const double seconds = 1.0 + share * share / 6400.0;           // tile rows of 64 an expert: 1.06 at 20 rows, 1.64 at 64
+    const bool tall_may = split <= 1 && tall_tiles * seconds > cus;
     GroupedPlan best{FP8BS_VARIANT_T256x256, 1};
     double best_cost = 0;
     // more: as many tiles as expected, times this
@@ -508,11 +501,24 @@ GroupedPlan make_grouped_plan(int experts, int rows, int n, int k, int num_cus, 
             if (best_cost == 0 || cost < best_cost) { best = p; best_cost = cost; }
         }
     }
+    // Some tens of rows an expert and weights that come from memory: one row of these tiles holds an expert where other tiles take two, or leave workgroups
+    // without work. Up to 44 rows 64x256 is ahead by 1 to 4 % where no expert has more than 64, and as fast or faster by its second rows, whose weights an L2
+    // holds, where these fit the last round; where they start one more it is far behind. 200 such calls, experts by chance and of shares that differ (a deviation
+    // of scores of 0.5), tile rows that start no round: 0.98 and 0.99 of 64x256's speed, and left; that do: 0.98 and 1.09 (at most 1.44: 23 rows to each of 32 experts,
+    // 4096 x 3712, shares up to 67, 106.8 and 88.1 us; 0.93 at worst), and taken. Against every other pick 1.14 to 1.17 times as fast (28 calls, at worst 0.88; 42
+    // rows to each of 64, 4608 x 1024, 84.9 and 71.5), splits among them (10 shapes 1.01 to 1.10, one draw 0.98; the sum without a split is no further from 64 bits).
+    // Above 44 rows some expert has more than 128 itself: only where an eighth more tiles takes no further round (512 tokens to 4 of 32, 3072 x 4096, 103.5 and
+    // 93.6; where the rounds were full, 256 to 8 of 32, 4096 x 7168, 192.0, this 213.4).
+    auto rounds = [&](double tiles) { return (long)__builtin_ceil(tiles / cus); };
+    const bool streams = best.tile == FP8BS_VARIANT_T64x256S3 && best.split == 1;
+    if (tall_may && fp8bs::weights_past_caches(experts, rows, n, k) && share > 16.0 && share <= 64.0
+        && (share <= 44.0 ? !streams || rounds(tall_tiles * seconds) > rounds(tall_tiles) : rounds(tall_tiles + tall_tiles / 8) == rounds(tall_tiles))) return {FP8BS_VARIANT_T256x128S3 | FORM1, 1};
     // From 44 to 128 rows an expert one row of 128x256 tiles holds an expert of the average size. The constants are a fit (12 % off in the mean) to 420 drawn
     // calls (8 to 128 experts, 10 to 420 rows each, 512 .. 7168 x 512 .. 7168). It is taken where it is ahead by 4 % with a twentieth more tiles than
-    // expected: the unequal shares that the averages hide cost it a round where the last is full. 260 further calls of 40 to 132 rows: 81 took it by one of
-    // the rules, 1.11 times as fast in the geometric mean, 0.95 to 1.28 (704 tokens to 4 of 32, 4864 x 4608, 193.0 -> 150.0 us; 344 to 8 of 32, 1536
-    // x 1920, 31.9 -> 24.3). Beyond 128 rows the model errs too often: of the drawn calls it gains 2 %, and loses 12 to 21 % on some.
+    // expected: the unequal shares that the averages hide cost it a round where the last is full. Of 833 further drawn calls of 16 to 132 rows 247 take it by one
+    // of the rules, 214 of them by this one: 1.16 times as fast in the geometric mean of both (experts by chance 1.17, of shares that differ 1.15), 0.83 to 1.44. The worst
+    // are unequal shares whose tiles start a round that the average does not (3216 rows to 32, 1344 x 640, 15.0 and 18.1 us). Splits that it takes the place of: 24 shapes,
+    // 1.12 to 1.46 (1696 rows to 16, 2176 x 6656, 102.2 and 70.2). Beyond 128 rows the model errs too often: of the drawn calls it gains 2 %, and loses 12 to 21 % on some.
     const Cand tall{FP8BS_VARIANT_T256x128S3 | FORM1, 1, 0.960, 0.628, 0.637, 5.33, 1.0, 5.98};
     if (tall_may && share > 44.0 && share <= 128.0 && best_cost > 1.04 * std::max(model(tall, 1, 1.0), model(tall, 1, 1.05))) best = {tall.tile, 1};
     return best;
