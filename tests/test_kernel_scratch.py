@@ -33,3 +33,10 @@ def test_dense_and_grouped(kernels, tile, tails):
 def test_weights_past_the_caches(kernels, tile, tails):
     for epi in (0, 1):
         assert kernels[tile % epi + ",%s,false" % tails][".private_segment_fixed_size"] == 0
+
+
+@pytest.mark.parametrize("tile", READ_ONCE)
+def test_weights_past_the_caches_without_spills(kernels, tile):
+    """As the instantiations that they stand in for: aligned operands, plain and with the epilogue."""
+    for epi in (0, 1):
+        assert kernels[tile % epi + ",false,false"][".vgpr_spill_count"] == 0
