@@ -601,7 +601,8 @@ static int scratch_address(void** out, hipStream_t stream) {
 
 extern "C" {
 
-int fp8bs_version(void) { return 400; }      // 0.4.0: a plan is (variant, form): fp8bs_plan_t::form in the place of a reserved word
+// 0.4.1: grouped calls take FP8BS_VARIANT_FORM(FP8BS_VARIANT_T256x128S3, 1).  0.4.0: a plan is (variant, form): fp8bs_plan_t::form in the place of a reserved word.
+int fp8bs_version(void) { return 401; }
 
 const char* fp8bs_strerror(int status) {
     switch (status) {

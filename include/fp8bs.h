@@ -62,8 +62,8 @@ enum {
     FP8BS_VARIANT_SKINNY64x288 = 8, /* same, 288-wide tile, 3 stages                             */
     FP8BS_VARIANT_T256x192 = 9,   /* 256(m) x 192(n) tile, 8 waves: fills more CUs when n/256 rounds up badly */
     FP8BS_VARIANT_T256x128S3 = 10, /* form 0: 256 x 128 tile, three LDS stages (a copy has two K blocks' time to land);
-                                     form 1: 128 x 256 tile, three stages, grouped calls without a K split only:
-                                     some tens of rows an expert                              */
+                                     form 1 (from version 401): 128 x 256 tile, three stages, grouped calls without
+                                     a K split only: some tens of rows an expert              */
     FP8BS_VARIANT_T192x192S3 = 11, /* 192 x 192 tile, 8 waves of 48 x 96, three LDS stages     */
     FP8BS_VARIANT_T64x256S3 = 12,  /* 8 waves of 32 x 64.  Form 0: 64(m) x 256(n) tile, three LDS stages: few rows against much of
                                      b; form 1: 128 x 128 tile, four stages: mid-size, one tile per CU;
