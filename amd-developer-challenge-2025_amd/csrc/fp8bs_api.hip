@@ -414,7 +414,9 @@ uint64_t useful_bytes(int m, int n, int k, const Planned& p) { return (p.share ?
 // beside the full tiles that read the same weights (32 experts of 1040 rows x 4096 x 7168: 956 us against 1014;
 // configuration 5: 2-3 % faster).  With fewer rows every expert is one tile row and the call streams the weights;
 // the order across the experts is then 0.7-1.2 % ahead (8 or 100 rows per expert), so it is kept there.
-int group_order(int total_rows, int num_experts) { return (long)total_rows >= 256L * num_experts ? 1 : 0; }
+int group_order(int total_rows, int num_experts, int n) {
+    return (long)total_rows >= 256L * num_experts ? fp8bs::ORDER_BY_EXPERT : fp8bs::turns_rounds(n) ? fp8bs::ORDER_TURNED : fp8bs::ORDER_ACROSS;
+}
 
 struct GroupedPlan { int tile, split; };
 
@@ -775,7 +777,7 @@ static int grouped_call(const void* a, const void* b, const float* a_scale, cons
     g.c = (uint16_t*)c; g.ws = (float*)ws; g.row_offsets = row_offsets;
     g.m = rows; g.n = n; g.k = k; g.lda = rows; g.nb = (n + 127) / 128;
     g.band_h = 4; g.num_experts = num_experts;
-    g.by_expert = group_order(rows, num_experts);
+    g.order = group_order(rows, num_experts, n);
     g.epi = epi;
     GroupedPlan plan{forced_tile(variant), split_k > 1 ? split_k : 1};
     if (k == 0 && variant == FP8BS_VARIANT_AUTO) plan = {FP8BS_VARIANT_GENERIC, 1};

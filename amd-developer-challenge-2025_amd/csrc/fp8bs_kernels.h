@@ -24,7 +24,7 @@ struct GemmArgs {
     int num_experts;
     int epi;                // 0: bf16 of the product; 1: silu(column 2i) * column 2i+1, n/2 output columns
     int c_whole_lines;      // set by the launcher: rows of c start and end on 128-byte lines
-    int by_expert;          // grouped: order of the tiles, 0 across the experts, 1 expert by expert (see the tile walk)
+    int order;              // grouped: order of the tiles, ORDER_.. (see the tile walk)
     // K blocks dealt to the workgroups (MODE 3 of the tiled kernel): `ws` then holds a header (a status word, one
     // 8-byte flag per workgroup) and one fp32 partial tile per workgroup, see StreamK below
     unsigned long long sk_nonce;   // value a flag takes when its workgroup's partial tile is complete: differs from call to call
@@ -46,7 +46,9 @@ __host__ __device__ constexpr bool expert_read_once(int experts_with_rows, int t
     return tile_rows == 1 && (unsigned long long)experts_with_rows * ((unsigned long long)n * (unsigned long long)k) >= ALL_CACHES;
 }
 
-// Whether a grouped call across the experts deals a workgroup other columns of b in each round of tiles (see `place` in fp8bs_tiled.h).
+// Orders of a grouped call's tiles: across the experts, a workgroup's columns of b other ones in each round; expert by expert; across the experts.
+enum { ORDER_TURNED, ORDER_BY_EXPERT, ORDER_ACROSS };
+// Whether a call across the experts turns its rounds (see `place` in fp8bs_tiled.h).
 __host__ __device__ constexpr bool turns_rounds(int n) { return n % 512 == 0; }
 
 // Or'ed into a mode: raise the LDS limit of the kernel that the arguments take and launch nothing (tiles of gemm_tr_kernel).

@@ -386,7 +386,7 @@ void gemm_tr_kernel(const GemmArgs p) {
         int wg = blockIdx.x;
         if (here <= 0) return -1;
         if constexpr (GROUPED)
-            if (it > 0 && !p.by_expert && (G >> 3) >= p.band_h && turns_rounds(p.n)) {
+            if (it > 0 && p.order == ORDER_TURNED && (G >> 3) >= p.band_h) {
                 const int x = blockIdx.x & 7, run = (G >> 3) + (x < (G & 7) ? 1 : 0), at = (int)(blockIdx.x >> 3);      // workgroups of this XCD, this one's place among them
                 turn += p.band_h;
                 if (turn >= run) turn -= run;
@@ -468,7 +468,7 @@ void gemm_tr_kernel(const GemmArgs p) {
             // [row_offsets[e], row_offsets[e+1]) are computed but never stored.  The gridDim.x tiles in
             // flight together are dealt to the XCDs in contiguous runs.  Two orders of the tiles.  Across
             // the experts: the (slot, n tile) grid of all slots in bands of band_h slots, as in the dense case.
-            // Expert by expert (p.by_expert): inside an expert's own grid in bands, an expert of up to eight
+            // Expert by expert: inside an expert's own grid in bands, an expert of up to eight
             // slots being one band, so that the tiles sharing an L2 form a compact block of few A panels and
             // few B panels of one expert and the tile that holds an expert's last rows runs beside the full
             // tiles that read the same panel of the expert's weights.
@@ -482,7 +482,7 @@ void gemm_tr_kernel(const GemmArgs p) {
                 v -= t.split_z * total;
                 t.sk_first = v;
             }
-            const bool by_expert = p.by_expert != 0;
+            const bool by_expert = p.order == ORDER_BY_EXPERT;
             int slot_all = 0, tn = 0;
             if (!by_expert) band_tile(v, total_slots, tiles_n, p.band_h, slot_all, tn);
             int e = 0, found = 0, start = 0, cnt_lo = 0, cnt_hi = 0;
