@@ -459,7 +459,7 @@ GroupedPlan make_grouped_plan(int experts, int rows, int n, int k, int num_cus, 
     const double active = experts * (1.0 - unused), average = rows / active;
     const int kbt = k / KBLK;
     // 128x256 tiles (fp8bs_tile_128x256s3.hip) by the two rules below, never where 64x256 tiles, second rows of them too, are all on the chip at once (300
-    // tokens to 4 of 32, 1280 x 7168, 72.0 us, 128x256 75.9; 105 to 8 of 16, 2176 x 3584, 35.5 and 37.8).
+    // tokens to 4 of 32, 1280 x 7168, 74.2 us, 128x256 77.6; 105 to 8 of 16, 2176 x 3584, 38.1 and 39.8).
     const long tall_tiles = (long)experts * cdiv(n, 256), cus = num_cus;
     const double share = (double)rows / experts;
     const double seconds = 1.0 + share * share / 6400.0;           // tile rows of 64 an expert: 1.06 at 20 rows, 1.64 at 64
@@ -509,8 +509,8 @@ GroupedPlan make_grouped_plan(int experts, int rows, int n, int k, int num_cus, 
     // of scores of 0.5), tile rows that start no round: 0.98 and 0.99 of 64x256's speed, and left; that do: 0.98 and 1.09 (at most 1.44: 23 rows to each of 32 experts,
     // 4096 x 3712, shares up to 67, 106.8 and 88.1 us; 0.93 at worst), and taken. Against every other pick 1.14 to 1.17 times as fast (28 calls, at worst 0.88; 42
     // rows to each of 64, 4608 x 1024, 84.9 and 71.5), splits among them (10 shapes 1.01 to 1.10, one draw 0.98; the sum without a split is no further from 64 bits).
-    // Above 44 rows some expert has more than 128 itself: only where an eighth more tiles takes no further round (512 tokens to 4 of 32, 3072 x 4096, 103.5 and
-    // 93.6; where the rounds were full, 256 to 8 of 32, 4096 x 7168, 192.0, this 213.4).
+    // Above 44 rows some expert has more than 128 itself: only where an eighth more tiles takes no further round (512 tokens to 4 of 32, shares that differ, 3072 x 4096,
+    // 112.9 and 92.4; where the rounds were full, 256 to 8 of 32, 4096 x 7168, 197.9, this 208.2).
     auto rounds = [&](double tiles) { return (long)__builtin_ceil(tiles / cus); };
     const bool streams = best.tile == FP8BS_VARIANT_T64x256S3 && best.split == 1;
     if (tall_may && fp8bs::weights_past_caches(experts, rows, n, k) && share > 16.0 && share <= 64.0

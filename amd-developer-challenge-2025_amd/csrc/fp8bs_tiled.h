@@ -1552,14 +1552,14 @@ static inline hipError_t launch_tr(const GemmArgs& a, dim3 grid, hipStream_t str
 
 // The experts' weights are read past the caches where nothing of them is found there again: those that the call reads are as large as the caches together,
 // and one row of tiles, so one workgroup for a column of them, holds the expert.  The instantiation is chosen here, by what the host knows; how many
-// experts have rows, and how many tile rows this one has, the kernel sees (`expert_read_once`).  What such a call gives up nothing for and gains by:
-// b does not push out a, of which every workgroup of an XCD reads the same lines (128 bytes for an expert's 16 rows or so).  That this is why is not shown: the
-// figures are.  us, MODE 2 and so (32 experts, rows by chance, 4096 x 7168 but where said): 256 rows 166.5 and 152.4, 7168 x 2048 90.5 and 84.0; 1024
+// experts have rows, and how many tile rows this one has, the kernel sees (`expert_read_once`).  Bound: HBM.  With the hint a read of memory is under way for 6 to 9 %
+// less time, and 0.4 to 2.5 % of the reads are saved, lines of a that b no longer pushes out of the L2 (counters of three products).  us, MODE 2 and so
+// (32 experts, rows by chance, 4096 x 7168 but where said): 256 rows 166.5 and 152.4, 7168 x 2048 90.5 and 84.0; 1024
 // rows in 128x256 177.9 and 164.1; 6144 in 256x256, 4096 x 4096, 153.2 and 144.3; one expert with half of 1024 rows 202.7 and 197.2; of 1024 to 64
 // experts, 2048 x 7168, 194.0 and 196.2, the largest loss of 48 (hint for all tiles: 199.4); 2048 rows in 128x256, 4096 x 4096, shares up to 303: 120.3 and 113.3 (126.1).
-// The line on the average: beyond it few experts have one row of tiles, and the gain goes: 64x256 at 32, 64 and 80 rows an expert 1.01-1.10, 1.01-1.04,
+// The line on the average: beyond it few experts have one row of tiles, and the gain goes: 64x256 at 32, 64 and 80 rows an expert 1.00-1.10, 1.01-1.04,
 // 1.00-1.04 times as fast, 128x256 at 96, 112 and 128 rows 1.04-1.10, 0.98-1.08, 0.99-1.05, 256x256 at 192 and 250 rows 1.03-1.16, 1.02-1.06 (three shapes, three draws).
-// Bytes: streamed, weights between products of others, the hint gains at any size (20 experts of 8 MB 39.0 -> 35.8), but read again with nothing in between
+// Bytes: streamed, weights between products of others, the hint gains at any size (20 experts of 8 MB 39.0 and 35.8), but read again with nothing in between
 // smaller ones are found in the cache: the same 30.2 and 33.8, 28 experts 35.7 and 40.0, 32 of 8 MB 41.1 and 45.7, 28 of 10 MB 47.5 and 48.8, 21 of 14 MB 54.0 and
 // 54.1, 30 of 10 MB 54.0 and 52.8, 32 of 10 MB 63.9 and 56.1: the line is where neither loses.
 // Rows of b are whole 128-byte lines: a line that two columns of tiles share would come from memory twice (100 tokens to 4 of 32, 3072 x 4096
